@@ -2811,8 +2811,8 @@ __global__ void k_project(int n, double* bodies, const double* step, int skip_st
 }
 
 // ------------------------------------------- sequential impulses (the solver)
-// After a filtered step: the clusters' pair lists and hit counts, then one
-// thread per cluster walks SequentialImpulses::solve (d2_solver.hpp).
+// After a filtered step: the clusters' pair lists, particles and hit counts,
+// then a block per cluster runs SequentialImpulses::solve (d2_solver.hpp).
 struct SolveArgs {
   int n_pairs, n_clusters, n_bodies;
   const int32_t* pairs;
@@ -2832,22 +2832,31 @@ struct SolveArgs {
   int* ccount;  // [n_clusters + 1] pairs per cluster, then their offsets (poff)
   int* chits;   // [n_clusters + 1] hits per cluster, then offsets (hoff)
   int* cfill;   // [n_clusters]
-  int* cpairs;  // [n_pairs]
+  int* cpart;   // [n_clusters] dynamic particles
+  int* cpairs;  // [n_pairs] as placed
+  int* cps;     // [n_pairs] in index order
   int* inpair;  // [n_bodies] 1 + the cluster of the body's pairs, 0: in no pair
   int* loc;     // [n_bodies] local particle index of a dynamic body
   int* flag;    // set when a dynamic body's pairs lie in two clusters
   int* status;  // [n_clusters]
+  int* ploc;    // [2 n_pairs] local particles of each pair (index order)
+  int* phit;    // [n_pairs] first hit of each pair (index order)
   int* hl;      // [hits][2]
   int* ord;     // [hits]
   int* hrow;    // [hits] output row
   int* hpc;     // [hits] contacts of the hit's pair
   int* pbody;   // [2 n_pairs]
+  int* hint;    // [hits][6] scratch: the sort, then the schedule
+  int* lvlo;    // [hits + n_clusters] schedule: level offsets
+  int* cntl;    // [hits] schedule: contacts per level
+  int* pint;    // [3][2 n_pairs] + n_clusters: per particle scratch of the schedule
   double* hA;   // [hits][3]
   double* hB;   // [hits][3]
   double* heps; // [hits]
   double* hkey; // [hits] |A - B| / (eps_a + eps_b)
-  double* hs;   // [hits][SH]
-  double* ps;   // [2 n_pairs][SP]
+  double* hhot;   // [hits][CH] (clusters above the LDS capacity)
+  double* hcold;  // [hits][CC]
+  double* ps;     // [2 n_pairs][SP] (clusters above the LDS capacity)
   double* out;  // [hits][11], cluster-gathered order
   WarmTable warm;
 };
@@ -2867,70 +2876,426 @@ __global__ void k_sv_count(SolveArgs A) {
     }
   }
 }
-// ccount / chits hold the exclusive offsets here (poff / hoff)
+// ccount / chits hold the exclusive offsets here (poff / hoff).  The pairs to
+// their clusters, the dynamic bodies to their clusters' particles (which
+// particle is which changes no result).
 __global__ void k_sv_place(SolveArgs A) {
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < A.n_pairs; p += gridDim.x * blockDim.x) {
-    const int k = A.cluster_of_pair[p];
-    A.cpairs[A.ccount[k] + atomicAdd(&A.cfill[k], 1)] = p;
+  const int n = A.n_pairs > A.n_bodies ? A.n_pairs : A.n_bodies;
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
+    if (p < A.n_pairs) {
+      const int k = A.cluster_of_pair[p];
+      A.cpairs[A.ccount[k] + atomicAdd(&A.cfill[k], 1)] = p;
+    }
+    if (p < A.n_bodies && A.inpair[p] && A.bodies[40 * (size_t)p + 38] == 0.0) {
+      const int k = A.inpair[p] - 1, q = atomicAdd(&A.cpart[k], 1);
+      A.loc[p] = q;
+      A.pbody[2 * (size_t)A.ccount[k] + q] = p;
+    }
   }
 }
-struct IdLess {
-  D2_HD bool operator()(int x, int y) const { return x < y; }
-};
 struct KeyLess {
   const double* k;
   D2_HD bool operator()(int x, int y) const { return k[x] < k[y]; }
 };
-// One thread per cluster.  The cluster's pairs in index order (the order its
-// interactions were gathered in, separate_clusters.cpp:405-434), its hits per
-// pair in the filtered order (PDE_explicit.cpp:77-95), the std::sort replay
-// of the hits by Contact::operator< (contact.h:14-18), then the solve.
-__global__ void __launch_bounds__(64) k_sv_solve(SolveArgs A) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < A.n_clusters; k += gridDim.x * blockDim.x) {
-    const int p0 = A.ccount[k], np_k = A.ccount[k + 1] - p0;
-    const int h0 = A.chits[k];
-    int* cp = A.cpairs + p0;
-    StdSort<IdLess>{cp, IdLess{}}.sort(0, np_k);
-    int* pb = A.pbody + 2 * (size_t)p0;
-    int n_part = 0, nh = 0;
-    auto local_of = [&](int b) {
-      if (A.bodies[40 * (size_t)b + 38] == 0.0) {  // a dynamic body belongs to one cluster
-        if (A.loc[b] < 0) A.loc[b] = n_part, pb[n_part++] = b;
-        return A.loc[b];
+// Value of the neighbouring lane (lane ^ 1), by DPP (no LDS round trip).
+__device__ __forceinline__ double lane_xor1(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0xB1, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0xB1, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+// One cluster's solve after gathering and scheduling.  Contacts sit in slots
+// ordered by level (a contact's level is one above the highest level of an
+// earlier contact that shares a dynamic particle), so the contacts of a level
+// touch different dynamic particles and any order of them gives the
+// sequential walk's values.  hit: hit of each slot; cab: its two particles;
+// csr: per particle, its contacts' slots (2 slot + side) in sorted order.
+struct SvRun {
+  double *C, *cold, *P;
+  const int *hit, *cab, *lvl_off, *csr, *csr_off;
+  int n_lvl, n_dyn;
+};
+template <int NT> __device__ __forceinline__ bool sv_sync_any(bool v) {
+  if (NT == 64) {
+    wave_sync_lds();
+    return __ballot(v) != 0ull;
+  }
+  return __syncthreads_or(v ? 1 : 0) != 0;
+}
+// Both sweeps with NT threads.  A contact takes two lanes, one per side: each
+// evaluates its particle's point, velocity and prediction, and the two
+// exchange their gaps and speeds by DPP.  Static particles' states never
+// change, so they order nothing; their accumulated impulse (the convergence
+// test reads it) is summed in sorted order after the sweep.
+template <int NT> __device__ __forceinline__ void sv_sweeps(const ClusterSolve& S, const SvRun& R, int tid) {
+  const int nh = S.nh, np = S.np;
+  const double t = S.t;
+  const int side = tid & 1;
+  for (int k = tid; k < np; k += NT) st3(R.P + (size_t)SP * k + SP_LAST, ld3(R.P + (size_t)SP * k + SP_IMP));
+  sv_sync_any<NT>(false);
+  for (int it = 0; it < 1000; ++it) {  // normal pass
+    for (int l = 0; l < R.n_lvl; ++l) {
+      const int end = R.lvl_off[l + 1];
+      for (int i = R.lvl_off[l] + (tid >> 1); i < end; i += NT / 2) {
+        double* c = R.C + (size_t)CH * i;
+        const int li = R.cab[2 * i + side];
+        double* p = R.P + (size_t)SP * li;
+        const v3<double> n = ld3(c + CH_N);
+        const SvSide s = sv_side(p, ld3(c + CH_WA + 3 * side), n);
+        const double odn = lane_xor1(s.dn), ovn = lane_xor1(s.vn);
+        double du, doff;
+        sv_contact_step(c, side ? s.dn - odn : odn - s.dn, side ? ovn - s.vn : s.vn - ovn, t, du, doff);
+        const v3<double> u = scl(sv_neg(n), du), uo = scl(sv_neg(n), doff);
+        if (li < R.n_dyn) {
+          sv_apply(p, side ? sv_neg(u) : u, side ? sv_neg(uo) : uo, s.arm);
+          sv_integrate(p, t);
+        } else {
+          st3(c + CH_U, u);
+        }
       }
-      for (int q = 0; q < n_part; ++q)  // a static body: one particle per cluster it touches
-        if (pb[q] == b) return q;
-      pb[n_part] = b;
-      return n_part++;
-    };
-    for (int i = 0; i < np_k; ++i) {
-      const int p = cp[i];
-      const int la = local_of(A.pairs[2 * p]), lb = local_of(A.pairs[2 * p + 1]);
-      int row = A.out_off[p];
-      for (int t = A.pair_off[p]; t < A.pair_off[p + 1]; ++t) {
-        if (!A.keep[t]) continue;
-        const ContactRec& c = A.contacts[A.perm[t]];
-        const size_t H = (size_t)h0 + nh;
-        for (int j = 0; j < 3; ++j) A.hA[3 * H + j] = c.r[j], A.hB[3 * H + j] = c.r[3 + j];
-        A.heps[H] = c.r[6] + c.r[7];
-        A.hkey[H] = vlen(sub(v3<double>{c.r[0], c.r[1], c.r[2]}, v3<double>{c.r[3], c.r[4], c.r[5]})) / A.heps[H];
-        A.hl[2 * H] = la, A.hl[2 * H + 1] = lb;
-        A.hrow[H] = row++;
-        A.hpc[H] = A.kept_cnt[p];
-        A.ord[H] = nh;
-        ++nh;
+      sv_sync_any<NT>(false);
+    }
+    bool moved = false;
+    for (int k = tid; k < np; k += NT) {
+      double* p = R.P + (size_t)SP * k;
+      if (k >= R.n_dyn) {
+        v3<double> imp = ld3(p + SP_IMP);
+        for (int e = R.csr_off[k]; e < R.csr_off[k + 1]; ++e) {
+          const v3<double> u = ld3(R.C + (size_t)CH * (R.csr[e] >> 1) + CH_U);
+          imp = (R.csr[e] & 1) ? sub(imp, u) : add(imp, u);
+        }
+        st3(p + SP_IMP, imp);
+      }
+      moved = moved || sv_moved(p);
+      st3(p + SP_LAST, ld3(p + SP_IMP));
+    }
+    if (!sv_sync_any<NT>(moved)) break;
+  }
+  for (int it = 0; it < 100; ++it) {  // friction pass
+    bool moved = false;
+    for (int i = tid; i < nh; i += NT)
+      if (sv_friction(S, R.hit[i], R.C + (size_t)CH * i, R.cold + (size_t)CC * i, R.P + (size_t)SP * R.cab[2 * i],
+                      R.P + (size_t)SP * R.cab[2 * i + 1], it & 1))
+        moved = true;
+    moved = sv_sync_any<NT>(moved);
+    for (int k = tid; k < R.n_dyn; k += NT) {
+      double* p = R.P + (size_t)SP * k;
+      SvAcc a = sv_acc(p);
+      for (int e = R.csr_off[k]; e < R.csr_off[k + 1]; ++e)
+        sv_friction_apply(a, R.C + (size_t)CH * (R.csr[e] >> 1), R.csr[e] & 1, it & 1);
+      sv_acc_store(a, p);
+      sv_integrate(p, t);
+    }
+    sv_sync_any<NT>(false);
+    if (!moved) break;
+  }
+}
+// Clusters up to these sizes run from LDS (74 KB, two blocks per CU), larger
+// ones from global scratch.
+constexpr int SV_CAPH = 192, SV_CAPP = 64;
+struct SvLds {
+  double C[SV_CAPH * CH];
+  double P[SV_CAPP * SP];
+  int cab[2 * SV_CAPH], lvl[SV_CAPH], slot[SV_CAPH], csr[2 * SV_CAPH], lvl_off[SV_CAPH + 1], csr_off[SV_CAPP + 1];
+};
+// Setup, sweeps and results of a gathered, sorted cluster whose schedule
+// arrays are at the given pointers (LDS or global).  Returns the status.
+__device__ __forceinline__ bool sv_solve_block(const ClusterSolve& S, double* C, double* cold, double* P, int* cab,
+                                               int* lvl, int* slot, int* csr, int* lvl_off, int* csr_off, int* last,
+                                               int* cur, int* cntl, int n_dyn, int* s_misc, bool lds) {
+  const int tid = threadIdx.x, lane = lane_id(), nh = S.nh, np = S.np;
+  // contacts per particle -> csr offsets
+  for (int k = tid; k <= np; k += blockDim.x) csr_off[k] = 0;
+  for (int k = tid; k < nh; k += blockDim.x) cntl[k] = 0;
+  __syncthreads();
+  for (int c = tid; c < nh; c += blockDim.x) {
+    const int h = S.ord[c];
+    atomicAdd(&csr_off[S.hl[2 * h]], 1), atomicAdd(&csr_off[S.hl[2 * h + 1]], 1);
+  }
+  __syncthreads();
+  int base = 0;
+  for (int k0 = 0; k0 < np; k0 += blockDim.x) {
+    const int k = k0 + tid;
+    int tot;
+    const int ex = block_scan(k < np ? csr_off[k] : 0, tot);
+    if (k < np) csr_off[k] = base + ex, cur[k] = base + ex, last[k] = 0;
+    base += tot;
+  }
+  if (tid == 0) csr_off[np] = base;
+  __syncthreads();
+  // levels and csr entries, contact by contact (one lane; the particles'
+  // last levels and cursors are in LDS up to 5000 particles)
+  if (tid < 64) {
+    int n_lvl = 0;
+    for (int c0 = 0; c0 < nh; c0 += 64) {
+      const int cc = c0 + lane < nh ? c0 + lane : c0;
+      const int h = S.ord[cc], va = S.hl[2 * h], vb = S.hl[2 * h + 1];
+      const int m = nh - c0 < 64 ? nh - c0 : 64;
+      for (int i = 0; i < m; ++i) {
+        const int a = rl(va, i), b = rl(vb, i), c = c0 + i;
+        if (lane == 0) {
+          const int la = a < n_dyn ? last[a] : 0, lb = b < n_dyn ? last[b] : 0;
+          const int lv = la > lb ? la : lb;
+          if (a < n_dyn) last[a] = lv + 1;
+          if (b < n_dyn) last[b] = lv + 1;
+          const int ea = cur[a];
+          cur[a] = ea + 1;
+          const int eb = cur[b];
+          cur[b] = eb + 1;
+          csr[ea] = 2 * c, csr[eb] = 2 * c + 1;
+          const int at = cntl[lv];
+          cntl[lv] = at + 1;
+          lvl[c] = lv, slot[c] = at;
+          n_lvl = lv + 1 > n_lvl ? lv + 1 : n_lvl;
+        }
       }
     }
-    StdSort<KeyLess>{A.ord + h0, KeyLess{A.hkey + h0}}.sort(0, nh);
+    if (lane == 0) s_misc[0] = n_lvl;
+  }
+  __syncthreads();
+  const int n_lvl = s_misc[0];
+  int lbase = 0, wide = 0;
+  for (int k0 = 0; k0 < n_lvl; k0 += blockDim.x) {
+    const int k = k0 + tid;
+    int tot;
+    const int v = k < n_lvl ? cntl[k] : 0;
+    const int ex = block_scan(v, tot);
+    if (k < n_lvl) lvl_off[k] = lbase + ex;
+    wide = v > wide ? v : wide;
+    lbase += tot;
+  }
+  if (tid == 0) lvl_off[n_lvl] = lbase;
+  wide = __syncthreads_or(wide > 32 ? 1 : 0);
+  for (int c = tid; c < nh; c += blockDim.x) slot[c] += lvl_off[lvl[c]];
+  __syncthreads();
+  int* hit = lvl;  // the levels are not read again
+  for (int e = tid; e < 2 * nh; e += blockDim.x) csr[e] = 2 * slot[csr[e] >> 1] + (csr[e] & 1);
+  for (int c = tid; c < nh; c += blockDim.x) {
+    const int h = S.ord[c], i = slot[c];
+    hit[i] = h, cab[2 * i] = S.hl[2 * h], cab[2 * i + 1] = S.hl[2 * h + 1];
+  }
+  __syncthreads();  // (also: last, cur and cntl may share C's and P's memory)
+  bool bad = false;
+  for (int i = tid; i < nh; i += blockDim.x)
+    bad = !sv_contact_setup(S, hit[i], C + (size_t)CH * i, cold + (size_t)CC * i) || bad;
+  if (__syncthreads_or(bad ? 1 : 0)) return false;
+  for (int k = tid; k < np; k += blockDim.x) {
+    double* p = P + (size_t)SP * k;
+    sv_particle_setup(S, S.pbody[k], p);
+    SvAcc a = sv_acc(p);
+    for (int e = csr_off[k]; e < csr_off[k + 1]; ++e) sv_warm_apply(a, C + (size_t)CH * (csr[e] >> 1), csr[e] & 1);
+    sv_acc_store(a, p);
+    if (k < n_dyn) sv_predict(p, S.t);
+  }
+  __syncthreads();
+  for (int i = tid; i < nh; i += blockDim.x)
+    sv_contact_turn(C + (size_t)CH * i, cold + (size_t)CC * i, P + (size_t)SP * cab[2 * i],
+                    P + (size_t)SP * cab[2 * i + 1]);
+  __syncthreads();
+  if (nh > 0) {
+    const SvRun R{C, cold, P, hit, cab, lvl_off, csr, csr_off, n_lvl, n_dyn};
+    // levels of at most 32 contacts fit one wavefront, which needs no
+    // barriers; the block's other wavefronts wait for the end
+    if (lds && !wide) {
+      if (tid < 64) sv_sweeps<64>(S, R, tid);
+    } else {
+      sv_sweeps<256>(S, R, tid);
+    }
+  }
+  __syncthreads();
+  for (int k = tid; k < n_dyn; k += blockDim.x)
+    sv_store_future(P + (size_t)SP * k, S.bodies + 40 * (size_t)S.pbody[k]);
+  for (int i = tid; i < nh; i += blockDim.x) {
+    sv_store_out(C + (size_t)CH * i, cold + (size_t)CC * i, S.out_h + 11 * (size_t)hit[i]);
+    // warm store: each body pair keeps its last contact's impulse (the last
+    // of a's contacts, in sorted order, with b at the other end)
+    const int a = cab[2 * i], b = cab[2 * i + 1];
+    const int k = a < n_dyn ? a : b, o = a < n_dyn ? b : a;
+    for (int e = csr_off[k + 1] - 1; e >= csr_off[k]; --e) {
+      const int j = csr[e] >> 1;
+      if (cab[2 * j + ((csr[e] & 1) ^ 1)] != o) continue;
+      if (j == i) warm_put(S.warm, warm_key(S.pbody[a], S.pbody[b]), C[(size_t)CH * i + CH_IMP]);
+      break;
+    }
+  }
+  return true;
+}
+// One block per cluster.  The cluster's pairs in index order (the order its
+// interactions were gathered in, separate_clusters.cpp:405-434), its hits per
+// pair in the filtered order (PDE_explicit.cpp:77-95), the std::sort order of
+// the hits by Contact::operator< (contact.h:14-18), then the solve.
+//
+// Bound by the latency of the normal pass's chain: a sweep is as many
+// dependent steps as there are levels (about 12 for 80 contacts among 32
+// bodies), each one contact update of FP64 arithmetic and LDS round trips.
+// One thread per cluster walking global memory took 125.2 ms for 24 clusters
+// of 32 bodies; with levels, two lanes per contact, the state in LDS and the
+// rotations hoisted the whole step with that solve takes 6.8 ms (128.7 before),
+// bit for bit the same.
+__global__ void __launch_bounds__(256) k_sv_solve(SolveArgs A) {
+  __shared__ SvLds L;
+  __shared__ int s_misc[8];
+  __shared__ int s_np;
+  const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+  for (int k = blockIdx.x; k < A.n_clusters; k += gridDim.x) {
+    const int p0 = A.ccount[k], np_k = A.ccount[k + 1] - p0;
+    const int h0 = A.chits[k], nh = A.chits[k + 1] - h0;
+    const int* cu = A.cpairs + p0;
+    int* cp = A.cps + p0;
+    // pairs in index order: by rank, or (long lists) from one pass over all pairs
+    if (np_k <= 1024) {
+      for (int i = tid; i < np_k; i += blockDim.x) {
+        const int x = cu[i];
+        int r = 0;
+        for (int j = 0; j < np_k; ++j) r += cu[j] < x ? 1 : 0;
+        cp[r] = x;
+      }
+    } else {
+      int at = 0;
+      for (int q0 = 0; q0 < A.n_pairs; q0 += blockDim.x) {
+        const int q = q0 + tid;
+        const bool mine = q < A.n_pairs && A.cluster_of_pair[q] == k;
+        int tot;
+        const int ex = block_scan(mine ? 1 : 0, tot);
+        if (mine) cp[at + ex] = q;
+        at += tot;
+      }
+    }
+    const int n_dyn = A.cpart[k];
+    int* pb = A.pbody + 2 * (size_t)p0;
+    if (tid == 0) s_np = n_dyn;
+    __syncthreads();
+    // the pairs' first hits and local particles; a static body is one
+    // particle per cluster it touches, listed after the dynamic ones
+    int at = 0;
+    for (int i0 = 0; i0 < np_k; i0 += blockDim.x) {
+      const int i = i0 + tid;
+      const int p = i < np_k ? cp[i] : -1;
+      int tot;
+      const int ex = block_scan(p >= 0 ? A.kept_cnt[p] : 0, tot);
+      if (p >= 0) A.phit[p0 + i] = at + ex;
+      at += tot;
+      for (int e = 0; e < 2; ++e) {
+        const int b = p >= 0 ? A.pairs[2 * p + e] : 0;
+        bool open = false;
+        if (p >= 0) {
+          if (A.bodies[40 * (size_t)b + 38] == 0.0) A.ploc[2 * (size_t)(p0 + i) + e] = A.loc[b];
+          else open = true;
+        }
+        for (;;) {  // one static body joins the list per round
+          const int n_now = s_np;
+          for (int q = n_dyn; open && q < n_now; ++q)
+            if (pb[q] == b) A.ploc[2 * (size_t)(p0 + i) + e] = q, open = false;
+          if (tid == 0) s_misc[1] = 0x7fffffff;
+          __syncthreads();
+          if (open) atomicMin(&s_misc[1], b);
+          __syncthreads();
+          const int add = s_misc[1];
+          if (add == 0x7fffffff) break;
+          if (tid == 0) pb[n_now] = add, s_np = n_now + 1;
+          __syncthreads();
+        }
+        __syncthreads();
+      }
+    }
+    const int np = s_np;
+    __syncthreads();
+    // the hits, one pair per wavefront at a time
+    for (int i = w; i < np_k; i += (int)(blockDim.x >> 6)) {
+      const int p = cp[i], la = A.ploc[2 * (size_t)(p0 + i)], lb = A.ploc[2 * (size_t)(p0 + i) + 1];
+      const int b = A.pair_off[p], e = A.pair_off[p + 1], row = A.out_off[p], cnt = A.kept_cnt[p];
+      int n = 0;
+      for (int t0 = b; t0 < e; t0 += 64) {
+        const int t = t0 + lane;
+        const bool take = t < e && A.keep[t] != 0;
+        const unsigned long long m = __ballot(take);
+        if (take) {
+          const int q = n + __popcll(m & lanes_below());
+          const size_t H = (size_t)h0 + A.phit[p0 + i] + q;
+          const ContactRec& c = A.contacts[A.perm[t]];
+          for (int j = 0; j < 3; ++j) A.hA[3 * H + j] = c.r[j], A.hB[3 * H + j] = c.r[3 + j];
+          A.heps[H] = c.r[6] + c.r[7];
+          A.hkey[H] = vlen(sub(v3<double>{c.r[0], c.r[1], c.r[2]}, v3<double>{c.r[3], c.r[4], c.r[5]})) / A.heps[H];
+          A.hl[2 * H] = la, A.hl[2 * H + 1] = lb;
+          A.hrow[H] = row + q;
+          A.hpc[H] = cnt;
+        }
+        n += __popcll(m);
+      }
+    }
+    if (tid == 0) s_misc[0] = 0;
+    __syncthreads();
+    // std::sort's order: ranks of the keys by counting over tiles in LDS, and
+    // the introsort replay where keys tie
+    const double* key = A.hkey + h0;
+    int* ord = A.ord + h0;
+    int* wi = A.hint + 6 * (size_t)h0;
+    const bool lds = nh <= SV_CAPH && np <= SV_CAPP;
+    constexpr int TILE = 2048;  // keys per tile, in L.C
+    bool tie = false, nan = false;
+    for (int q0 = 0; q0 < nh; q0 += blockDim.x) {
+      const int i = q0 + tid;
+      const double x = key[i < nh ? i : 0];
+      int r = 0, eq = 0;
+      for (int t0 = 0; t0 < nh; t0 += TILE) {
+        const int m = nh - t0 < TILE ? nh - t0 : TILE;
+        __syncthreads();
+        for (int j = tid; j < m; j += blockDim.x) L.C[j] = key[t0 + j];
+        __syncthreads();
+        for (int j = 0; j < m; ++j) {
+          const double y = L.C[j];
+          r += y < x ? 1 : 0, eq += y == x ? 1 : 0;
+        }
+      }
+      if (i < nh) wi[i] = r, tie = tie || eq > 1, nan = nan || !(x == x);
+    }
+    tie = __syncthreads_or(tie ? 1 : 0);
+    nan = __syncthreads_or(nan ? 1 : 0);
+    if (!tie && !nan) {
+      for (int i = tid; i < nh; i += blockDim.x) ord[wi[i]] = i;
+    } else {
+      for (int i = tid; i < nh; i += blockDim.x) ord[i] = i;
+      __syncthreads();
+      if (nan) {  // keys without an order: the sequential sort itself
+        if (tid == 0) StdSort<KeyLess>{ord, KeyLess{key}}.sort(0, nh);
+      } else if (lds) {  // (rk, apos, bpos, mark, segs in LDS)
+        for (int i = tid; i < nh; i += blockDim.x) L.lvl[i] = wi[i], L.slot[i] = i;
+        __syncthreads();
+        block_std_sort(nh, L.slot, L.lvl, L.csr, L.csr + SV_CAPH, L.lvl_off, L.cab, s_misc + 2, blk_segs(nh));
+        for (int i = tid; i < nh; i += blockDim.x) ord[i] = L.slot[i];
+      } else {
+        block_std_sort(nh, ord, wi, wi + nh, wi + 2 * (size_t)nh, wi + 3 * (size_t)nh, wi + 4 * (size_t)nh, s_misc + 2,
+                       blk_segs(nh));
+      }
+    }
+    __syncthreads();
     ClusterSolve S;
-    S.nh = nh, S.np = n_part;
+    S.nh = nh, S.np = np;
     S.hA = A.hA + 3 * (size_t)h0, S.hB = A.hB + 3 * (size_t)h0, S.heps = A.heps + h0, S.hl = A.hl + 2 * (size_t)h0;
     S.hpc = A.hpc + h0;
-    S.ord = A.ord + h0, S.pbody = pb, S.bodies = A.bodies, S.mass = A.mass, S.fric = A.fric;
+    S.ord = ord, S.pbody = pb, S.bodies = A.bodies, S.mass = A.mass, S.fric = A.fric;
     S.t = A.cluster_step[k], S.g = v3<double>{A.gx, A.gy, A.gz}, S.warm = A.warm;
-    S.hs = A.hs + (size_t)SH * h0, S.ps = A.ps + (size_t)SP * 2 * p0;
+    S.hs = nullptr, S.ps = nullptr;
     S.out_h = A.out + 11 * (size_t)h0;
-    A.status[k] = solve_cluster(S) ? 1 : 0;
+    double* cold = A.hcold + (size_t)CC * h0;
+    // during the schedule the particles' ints share C's memory, the level
+    // counts P's (both are filled only after it)
+    int* ci = reinterpret_cast<int*>(L.C);
+    bool ok;
+    if (lds) {
+      ok = sv_solve_block(S, L.C, cold, L.P, L.cab, L.lvl, L.slot, L.csr, L.lvl_off, L.csr_off, ci, ci + SV_CAPP,
+                          reinterpret_cast<int*>(L.P), n_dyn, s_misc, true);
+    } else {
+      constexpr int CI = 5000, PI = 5000;  // ints that fit: 2 x 5000 in C, 5000 in P
+      static_assert(sizeof(L.C) >= 2 * CI * sizeof(int) && sizeof(L.P) >= PI * sizeof(int) &&
+                        SV_CAPH * CH >= TILE, "schedule scratch in LDS");
+      int* pi = A.pint + 3 * 2 * (size_t)p0 + k;  // [np + 1] csr offsets, [np] levels, [np] cursors
+      ok = sv_solve_block(S, A.hhot + (size_t)CH * h0, cold, A.ps + (size_t)SP * 2 * p0, wi + 4 * (size_t)nh, wi,
+                          wi + nh, wi + 2 * (size_t)nh, A.lvlo + h0 + k, pi, np <= CI ? ci : pi + np + 1,
+                          np <= CI ? ci + CI : pi + 2 * (size_t)np + 1,
+                          nh <= PI ? reinterpret_cast<int*>(L.P) : A.cntl + h0, n_dyn, s_misc, false);
+    }
+    if (tid == 0) A.status[k] = ok ? 1 : 0;
+    __syncthreads();  // LDS is reused by the next cluster
   }
 }
 // Bodies in no pair: a cluster of their own without contacts (gravity only).
@@ -3080,8 +3445,8 @@ struct d2_ctx {
   // the solver (d2_solve): per-body mass and friction, per-cluster and per-hit scratch, the warm store
   DBuf<double> sv_mass, sv_fric;
   DBuf<int> sv_ccount, sv_chits, sv_poff, sv_hoff, sv_cfill, sv_cpairs, sv_inpair, sv_loc, sv_status, sv_flag;
-  DBuf<int> sv_hl, sv_ord, sv_hrow, sv_hpc, sv_pbody;
-  DBuf<double> sv_hA, sv_hB, sv_heps, sv_hkey, sv_hs, sv_ps, sv_out, sv_out_csr;
+  DBuf<int> sv_hl, sv_ord, sv_hrow, sv_hpc, sv_pbody, sv_cpart, sv_cps, sv_ploc, sv_phit, sv_hint, sv_lvlo, sv_cntl, sv_pint;
+  DBuf<double> sv_hA, sv_hB, sv_heps, sv_hkey, sv_hhot, sv_hcold, sv_ps, sv_out, sv_out_csr;
   DBuf<unsigned long long> warm_keys, warm_used;
   DBuf<double> warm_vals;
   int last_kind = -1;         // kind of the last finished run
@@ -4186,7 +4551,9 @@ int d2_ctx_destroy(d2_ctx* c) {
       release(c->sv_hoff), release(c->sv_cfill), release(c->sv_cpairs), release(c->sv_inpair), release(c->sv_loc),
       release(c->sv_status), release(c->sv_flag), release(c->sv_hl), release(c->sv_ord), release(c->sv_hrow),
       release(c->sv_hpc), release(c->sv_pbody), release(c->sv_hA), release(c->sv_hB), release(c->sv_heps),
-      release(c->sv_hkey), release(c->sv_hs), release(c->sv_ps), release(c->sv_out), release(c->sv_out_csr),
+      release(c->sv_hkey), release(c->sv_hhot), release(c->sv_hcold), release(c->sv_ps), release(c->sv_out),
+      release(c->sv_out_csr), release(c->sv_cpart), release(c->sv_cps), release(c->sv_ploc), release(c->sv_phit),
+      release(c->sv_hint), release(c->sv_lvlo), release(c->sv_cntl), release(c->sv_pint),
       release(c->warm_keys), release(c->warm_used), release(c->warm_vals);
   release(c->step_bits), release(c->first_any), release(c->first_ns), release(c->cluster_step), release(c->body_step),
       release(c->tmp_cluster), release(c->read_later);
@@ -4628,8 +4995,11 @@ int d2_solve(d2_ctx* c, const double* gravity, int32_t* cluster_status, int* n_f
   const size_t H = (size_t)std::max<long long>(nh, 1);
   RC(ensure(c, c->sv_hl, 2 * H)); RC(ensure(c, c->sv_ord, H)); RC(ensure(c, c->sv_hrow, H)); RC(ensure(c, c->sv_hpc, H));
   RC(ensure(c, c->sv_hA, 3 * H)); RC(ensure(c, c->sv_hB, 3 * H)); RC(ensure(c, c->sv_heps, H)); RC(ensure(c, c->sv_hkey, H));
-  RC(ensure(c, c->sv_hs, (size_t)SH * H)); RC(ensure(c, c->sv_out, 11 * H));
-  RC(ensure(c, c->sv_ps, (size_t)SP * 2 * std::max(np, 1)));
+  const size_t P = (size_t)std::max(np, 1), K = (size_t)std::max(nk, 1);
+  RC(ensure(c, c->sv_hhot, (size_t)CH * H)); RC(ensure(c, c->sv_hcold, (size_t)CC * H)); RC(ensure(c, c->sv_out, 11 * H));
+  RC(ensure(c, c->sv_ps, (size_t)SP * 2 * P)); RC(ensure(c, c->sv_cpart, K)); RC(ensure(c, c->sv_cps, P));
+  RC(ensure(c, c->sv_ploc, 2 * P)); RC(ensure(c, c->sv_phit, P)); RC(ensure(c, c->sv_hint, 6 * H));
+  RC(ensure(c, c->sv_lvlo, H + K)); RC(ensure(c, c->sv_cntl, H)); RC(ensure(c, c->sv_pint, 6 * P + K));
   SolveArgs A;
   A.n_pairs = np, A.n_clusters = nk, A.n_bodies = nb;
   A.pairs = c->pairs.p, A.cluster_of_pair = c->cluster_of_pair.p, A.kept_cnt = c->kept_cnt.p;
@@ -4640,25 +5010,28 @@ int d2_solve(d2_ctx* c, const double* gravity, int32_t* cluster_status, int* n_f
   A.ccount = c->sv_ccount.p, A.chits = c->sv_chits.p, A.cfill = c->sv_cfill.p, A.cpairs = c->sv_cpairs.p;
   A.inpair = c->sv_inpair.p, A.loc = c->sv_loc.p, A.status = c->sv_status.p;
   A.hl = c->sv_hl.p, A.ord = c->sv_ord.p, A.hrow = c->sv_hrow.p, A.hpc = c->sv_hpc.p, A.pbody = c->sv_pbody.p;
-  A.hA = c->sv_hA.p, A.hB = c->sv_hB.p, A.heps = c->sv_heps.p, A.hkey = c->sv_hkey.p, A.hs = c->sv_hs.p;
+  A.hA = c->sv_hA.p, A.hB = c->sv_hB.p, A.heps = c->sv_heps.p, A.hkey = c->sv_hkey.p;
+  A.hhot = c->sv_hhot.p, A.hcold = c->sv_hcold.p, A.cpart = c->sv_cpart.p, A.cps = c->sv_cps.p;
+  A.ploc = c->sv_ploc.p, A.phit = c->sv_phit.p, A.hint = c->sv_hint.p, A.lvlo = c->sv_lvlo.p;
+  A.cntl = c->sv_cntl.p, A.pint = c->sv_pint.p;
   A.ps = c->sv_ps.p, A.out = c->sv_out.p, A.warm = warm_table(c), A.flag = c->sv_flag.p;
   auto fill = [&](int* p, long long n, int v) {
     hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(c, n)), dim3(256), 0, c->stream, p, n, v);
   };
   fill(A.ccount, nk + 1, 0), fill(A.chits, nk + 1, 0), fill(A.cfill, nk, 0);
-  fill(A.inpair, nb, 0), fill(A.loc, nb, -1), fill(c->sv_flag.p, 1, 0);
+  fill(A.inpair, nb, 0), fill(A.cpart, nk, 0), fill(c->sv_flag.p, 1, 0);
   hipLaunchKernelGGL(k_sv_count, dim3(grid_for(c, np)), dim3(256), 0, c->stream, A);
   scan_host_n(c, c->sv_ccount.p, c->sv_poff.p, nk, nullptr);
   scan_host_n(c, c->sv_chits.p, c->sv_hoff.p, nk, nullptr);
   scan_host_n(c, c->kept_cnt.p, c->out_off.p, np, nullptr);
   SolveArgs B = A;
   B.ccount = c->sv_poff.p, B.chits = c->sv_hoff.p;  // the offsets from here on
-  hipLaunchKernelGGL(k_sv_place, dim3(grid_for(c, np)), dim3(256), 0, c->stream, B);
+  hipLaunchKernelGGL(k_sv_place, dim3(grid_for(c, std::max(np, nb))), dim3(256), 0, c->stream, B);
   int bad = 0;
   HIPCHK(c, hipMemcpyAsync(&bad, c->sv_flag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (bad) return fail(c, D2_ERR_ARG, "d2_solve: a dynamic body's pairs lie in more than one cluster");
-  hipLaunchKernelGGL(k_sv_solve, dim3((nk + 63) / 64 > 0 ? (nk + 63) / 64 : 1), dim3(64), 0, c->stream, B);
+  hipLaunchKernelGGL(k_sv_solve, dim3(std::max(1, std::min(nk, 16 * c->cus))), dim3(256), 0, c->stream, B);
   hipLaunchKernelGGL(k_sv_free, dim3(grid_for(c, nb)), dim3(256), 0, c->stream, B);
   HIPCHK(c, hipGetLastError());
   std::vector<int32_t> st(std::max(nk, 1));

@@ -1,9 +1,9 @@
 // d2_solver.hpp -- sequential impulses of one cluster (host/device code).
 //
 // strategy::SequentialImpulses::solve (strategies/contact_force/
-// sequential_impulses.cpp:104-638) over a cluster's filtered contacts, as one
-// sequential walk (the Gauss-Seidel order is the reference's, so the result
-// is its result): setup of the local contacts (:109-163), impulses from
+// sequential_impulses.cpp:104-638) over a cluster's filtered contacts, in
+// the reference's Gauss-Seidel order (so the result is its result): setup of
+// the local contacts (:109-163), impulses from
 // gravity (:171-180, contact_force_strategy.cpp:10-13), warm start
 // (sequential_impulses_warm_start.cpp:12-29) and its impulses (:185-213),
 // the first prediction (:215-227), the normal pass (:231-375, at most 1000
@@ -13,10 +13,20 @@
 // pass's drift terms (:432-438, :455-503; they feed only an offset impulse
 // the reference never applies), unused d1 values and contact_draws.
 //
-// The includer defines D2_HD and includes d2_geom.hpp.  Every array is the
-// cluster's own slice (one thread per cluster on the device; the same code
-// runs on the host for checks).  Evaluation orders match the oracle's
-// restatement (dot left to right, M*v row by row, Hamilton products).
+// The arithmetic is in per-contact and per-particle functions (sv_*).  Two
+// walks call them: solve_cluster below, one thread contact by contact (the
+// host's check against the oracle), and the device's k_sv_solve, a block per
+// cluster, which runs contacts that share no dynamic particle side by side.
+//
+// What does not change during a solve is formed once.  The torques of offset
+// impulses stay zero, so a particle's predicted rotation is the same in every
+// prediction (sequential_impulses.cpp:46-70 turns the future state by its own
+// L): it is turned once, and a contact's local points are rotated once; a
+// prediction then is v = v_f + imp / m, x = x_f + (off / m) t, L = L_f + rot.
+//
+// The includer defines D2_HD and includes d2_geom.hpp.  Evaluation orders
+// match the oracle's restatement (dot left to right, M*v row by row, Hamilton
+// products).
 #pragma once
 
 namespace d2 {
@@ -88,17 +98,19 @@ D2_HD double sv_quad(v3<double> v, const double* M) {
                      (v.x * M[2] + v.y * M[5]) + v.z * M[8]};
   return dot(u, v);
 }
-// model/forces.h:101-108: (-force) x (point - centre of mass)
-D2_HD v3<double> sv_torque(v3<double> f, v3<double> p, v3<double> com) { return cross(sv_neg(f), sub(p, com)); }
+// model/forces.h:101-108: (-force) x (point - centre of mass), arm = point - centre
+D2_HD v3<double> sv_torque(v3<double> f, v3<double> arm) { return cross(sv_neg(f), arm); }
 D2_HD v3<double> sv_normalized(v3<double> a) {
   const double z = dot(a, a);
   return z > 0.0 ? dvs(a, sqrt(z)) : a;
 }
-// transform(p, pose(q, x)): the homogeneous transform with the divide by w.
-D2_HD v3<double> sv_xform(const SolverState& s, v3<double> p) {
-  double m[16];
-  pose(s.q, s.x, m);
-  return xform(m, p);
+// The rotated part of transform(p, pose(q, x)); the point is sv_turn + x (a
+// rigid pose's w is 1, so the homogeneous divide changes nothing).
+D2_HD v3<double> sv_turn(quat q, v3<double> p) {
+  double r[9];
+  qrot(q, r);
+  return {(r[0] * p.x + r[1] * p.y) + r[2] * p.z, (r[3] * p.x + r[4] * p.y) + r[5] * p.z,
+          (r[6] * p.x + r[7] * p.y) + r[8] * p.z};
 }
 // sequential_impulses.cpp:46-70 (the future state's own L drives the turn)
 D2_HD SolverState sv_update(const SolverState& f, double t, v3<double> imp, v3<double> off, v3<double> rimp,
@@ -148,238 +160,269 @@ struct ClusterSolve {
   double t;
   v3<double> g;
   WarmTable warm;
-  // scratch per hit (sorted position): 35 doubles
-  double* hs;  // [nh][SH]
-  // scratch per particle: 28 doubles
-  double* ps;  // [np][SP]
+  double* hs;  // scratch per hit (sorted position): [nh][SH]
+  double* ps;  // scratch per particle: [np][SP]
   double* out_h;  // [nh][11]
 };
-// scratch layout
-constexpr int SH_LA = 0, SH_LB = 3, SH_N = 6, SH_RA = 9, SH_RB = 12, SH_LF = 15, SH_LRA = 18, SH_LRB = 21,
-              SH_UT = 24, SH_VT = 27, SH_START = 30, SH_MEFF = 31, SH_IMP = 32, SH_OFF = 33, SH_OUTER = 34, SH = 35;
-constexpr int SP_Q = 0, SP_X = 4, SP_V = 7, SP_L = 10, SP_IMP = 13, SP_ROT = 16, SP_OFF = 19, SP_ROFF = 22,
-              SP_LAST = 25, SP = 28;
+// Scratch per contact: what every sweep touches (CH doubles: normal, the two
+// rotated local points, outer distance, slop, effective mass, impulse, offset
+// impulse, the last change of impulse, and the friction's torques of the even
+// and the odd sweeps, a's then b's) and the rest (CC: local points, arms at
+// the start, friction impulse, tangential velocity).  Strides of the records
+// are odd, so records side by side start in different LDS banks.
+constexpr int CH_N = 0, CH_WA = 3, CH_WB = 6, CH_OUTER = 9, CH_SLOP = 10, CH_MEFF = 11, CH_IMP = 12, CH_OFF = 13,
+              CH_U = 14, CH_LR = 17, CH = 29;
+constexpr int CC_LA = 0, CC_LB = 3, CC_RA = 6, CC_RB = 9, CC_LF = 12, CC_VT = 15, CC = 18;
+constexpr int SH = CH + CC;
+// Scratch per particle: predicted state, accumulated impulses, the future
+// state the solve started from, mass, body-frame inverse inertia, the
+// impulse at the start of the sweep, predicted rotation.
+constexpr int SP_X = 0, SP_V = 3, SP_L = 6, SP_IMP = 9, SP_ROT = 12, SP_OFF = 15, SP_FX = 18, SP_FV = 21, SP_FL = 24,
+              SP_MASS = 27, SP_IB = 28, SP_LAST = 37, SP_Q = 40, SP = 45;
 
 D2_HD v3<double> ld3(const double* p) { return {p[0], p[1], p[2]}; }
 D2_HD void st3(double* p, v3<double> v) { p[0] = v.x, p[1] = v.y, p[2] = v.z; }
-D2_HD SolverState ps_state(const double* p) {
-  return SolverState{quat{p[SP_Q], p[SP_Q + 1], p[SP_Q + 2], p[SP_Q + 3]}, ld3(p + SP_X), ld3(p + SP_V),
-                     ld3(p + SP_L)};
+
+// A local contact (:109-163) of hit h into c (CH) and k (CC); false where the
+// reference gives the cluster up.
+D2_HD bool sv_contact_setup(const ClusterSolve& S, int h, double* c, double* k) {
+  const int ba = S.pbody[S.hl[2 * h]], bb = S.pbody[S.hl[2 * h + 1]];
+  const double* ra = S.bodies + 40 * (size_t)ba;
+  const double* rb = S.bodies + 40 * (size_t)bb;
+  const v3<double> A = ld3(S.hA + 3 * h), B = ld3(S.hB + 3 * h);
+  const double start = vlen(sub(A, B));
+  if (start < 1e-6 && S.t > 1e-4) return false;
+  const SolverState fa = sv_load(ra + 14), fb = sv_load(rb + 14);
+  double m[16], mi[16];
+  pose(fa.q, fa.x, m);
+  inv44(m, mi);
+  st3(k + CC_LA, xform(mi, A));
+  pose(fb.q, fb.x, m);
+  inv44(m, mi);
+  st3(k + CC_LB, xform(mi, B));
+  const v3<double> gn = dvs(sub(B, A), 2.0);
+  st3(c + CH_N, sv_normalized(gn));
+  const v3<double> r_A = sub(A, fa.x), r_B = sub(B, fb.x);
+  st3(k + CC_RA, r_A), st3(k + CC_RB, r_B);
+  const v3<double> rn_A = cross(r_A, gn), rn_B = cross(r_B, gn);
+  double k_normal = 0.0;
+  if (ra[38] == 0.0) k_normal += 1.0 / S.mass[ba] + sv_quad(rn_A, ra + 28);
+  if (rb[38] == 0.0) k_normal += 1.0 / S.mass[bb] + sv_quad(rn_B, rb + 28);
+  c[CH_MEFF] = k_normal < 1e-6 ? 0.0 : 1.0 / k_normal;
+  c[CH_OFF] = 0.0;
+  const double outer = S.heps[h] * 0.25;
+  const double lower_slop = sv_max(outer * 0.2, outer - start);
+  c[CH_OUTER] = outer, c[CH_SLOP] = lerp(lower_slop, outer * 0.2, 0.3);
+  for (int j = 0; j < 3; ++j) k[CC_LF + j] = 0.0;
+  // warm start (warm_start.cpp:12-29) and its impulses at the states the
+  // solve starts from (:185-213): the change of impulse and both torques
+  double w;
+  c[CH_IMP] = warm_find(S.warm, warm_key(ba, bb), w) ? w * 0.75 : 0.0;
+  const v3<double> u = scl(sv_neg(ld3(c + CH_N)), c[CH_IMP]);
+  st3(c + CH_U, u);
+  st3(c + CH_LR, sv_torque(u, sub(add(sv_turn(fa.q, ld3(k + CC_LA)), fa.x), fa.x)));
+  st3(c + CH_LR + 3, sv_torque(sv_neg(u), sub(add(sv_turn(fb.q, ld3(k + CC_LB)), fb.x), fb.x)));
+  return true;
 }
-D2_HD void ps_store(double* p, const SolverState& s) {
-  p[SP_Q] = s.q.w, p[SP_Q + 1] = s.q.x, p[SP_Q + 2] = s.q.y, p[SP_Q + 3] = s.q.z;
-  st3(p + SP_X, s.x), st3(p + SP_V, s.v), st3(p + SP_L, s.L);
+// A particle at its future state, with the impulse from gravity (:171-180).
+D2_HD void sv_particle_setup(const ClusterSolve& S, int b, double* p) {
+  const double* r = S.bodies + 40 * (size_t)b;
+  for (int j = 0; j < 3; ++j) {
+    p[SP_X + j] = p[SP_FX + j] = r[18 + j];
+    p[SP_V + j] = p[SP_FV + j] = r[21 + j];
+    p[SP_L + j] = p[SP_FL + j] = r[24 + j];
+    p[SP_ROT + j] = 0.0, p[SP_OFF + j] = 0.0;
+  }
+  for (int j = 0; j < 4; ++j) p[SP_Q + j] = r[14 + j];
+  for (int j = 0; j < 9; ++j) p[SP_IB + j] = r[28 + j];
+  p[SP_MASS] = S.mass[b];
+  st3(p + SP_IMP, scl(sclL(S.mass[b], S.g), S.t));
+}
+// A particle's accumulated impulses, for walks over its own contacts.
+struct SvAcc {
+  v3<double> imp, rot, off;
+};
+D2_HD SvAcc sv_acc(const double* p) { return SvAcc{ld3(p + SP_IMP), ld3(p + SP_ROT), ld3(p + SP_OFF)}; }
+D2_HD void sv_acc_store(const SvAcc& a, double* p) {
+  st3(p + SP_IMP, a.imp), st3(p + SP_ROT, a.rot), st3(p + SP_OFF, a.off);
+}
+// One contact's warm-start impulse on its particle of side 0 (a) or 1 (b).
+D2_HD void sv_warm_apply(SvAcc& a, const double* c, int side) {
+  const v3<double> u = ld3(c + CH_U);
+  a.imp = side ? sub(a.imp, u) : add(a.imp, u);
+  a.rot = add(a.rot, ld3(c + CH_LR + 3 * side));
+}
+// sequential_impulses.cpp:46-70 with the rotation already turned.
+D2_HD void sv_integrate(double* p, double t) {
+  const double m = p[SP_MASS];
+  st3(p + SP_V, add(ld3(p + SP_FV), dvs(ld3(p + SP_IMP), m)));
+  st3(p + SP_X, add(ld3(p + SP_FX), scl(dvs(ld3(p + SP_OFF), m), t)));
+  st3(p + SP_L, add(ld3(p + SP_FL), ld3(p + SP_ROT)));
+}
+// The first prediction of a dynamic particle (:215-227): its rotation and state.
+D2_HD void sv_predict(double* p, double t) {
+  const v3<double> z{0.0, 0.0, 0.0};
+  const SolverState f{quat{p[SP_Q], p[SP_Q + 1], p[SP_Q + 2], p[SP_Q + 3]}, ld3(p + SP_FX), ld3(p + SP_FV),
+                      ld3(p + SP_FL)};
+  const quat q = sv_update(f, t, z, z, z, z, p[SP_MASS], p + SP_IB).q;
+  p[SP_Q] = q.w, p[SP_Q + 1] = q.x, p[SP_Q + 2] = q.y, p[SP_Q + 3] = q.z;
+  sv_integrate(p, t);
+}
+// A contact's local points rotated as its particles are from here on, and
+// the friction's torques before its first sweep (zero).
+D2_HD void sv_contact_turn(double* c, const double* k, const double* pa, const double* pb) {
+  st3(c + CH_WA, sv_turn(quat{pa[SP_Q], pa[SP_Q + 1], pa[SP_Q + 2], pa[SP_Q + 3]}, ld3(k + CC_LA)));
+  st3(c + CH_WB, sv_turn(quat{pb[SP_Q], pb[SP_Q + 1], pb[SP_Q + 2], pb[SP_Q + 3]}, ld3(k + CC_LB)));
+  for (int j = 0; j < 6; ++j) c[CH_LR + 6 + j] = 0.0;
+}
+// One side of a contact in the normal pass (:231-375): the point's arm, its
+// position and its velocity along the normal.
+struct SvSide {
+  v3<double> arm;
+  double dn, vn;
+};
+D2_HD SvSide sv_side(const double* p, v3<double> w, v3<double> n) {
+  const v3<double> x = ld3(p + SP_X), p1 = add(w, x);
+  SvSide s;
+  s.arm = sub(p1, x);
+  s.dn = dot(p1, n);
+  s.vn = dot(add(ld3(p + SP_V), cross(mul33v(p + SP_IB, ld3(p + SP_L)), s.arm)), n);
+  return s;
+}
+// The contact's impulses after one visit: d1 the gap, v1 the closing speed.
+D2_HD void sv_contact_step(double* c, double d1, double v1, double t, double& du, double& doff) {
+  const double damp = 0.1, outer = c[CH_OUTER], m = c[CH_MEFF];
+  const double last = c[CH_IMP], last_off = c[CH_OFF];
+  const double dimp = d1 < outer ? (v1 * m) * damp : -last;
+  const double imp = sv_max(last + dimp, 0.0);
+  const double pen = outer - d1;
+  const double dof = d1 < outer ? ((damp * m) * sv_max(0.0, pen - c[CH_SLOP])) / t : -last_off;
+  const double off = sv_max(last_off + dof, 0.0);
+  c[CH_IMP] = imp, c[CH_OFF] = off;
+  du = imp - last, doff = off - last_off;
+}
+// The visit's impulse f, its torque and its offset impulse fo on a particle.
+D2_HD void sv_apply(double* p, v3<double> f, v3<double> fo, v3<double> arm) {
+  st3(p + SP_IMP, add(ld3(p + SP_IMP), f));
+  st3(p + SP_ROT, add(ld3(p + SP_ROT), sv_torque(f, arm)));
+  st3(p + SP_OFF, add(ld3(p + SP_OFF), fo));
+}
+// One contact of a friction sweep (:392-571): both passes' values from the
+// particles' states, which a sweep's impulses do not change before its end.
+// par: the sweep's parity.  Returns whether the impulse still moves.
+D2_HD bool sv_friction(const ClusterSolve& S, int h, double* c, double* k, const double* pa, const double* pb, int par) {
+  const int ba = S.pbody[S.hl[2 * h]], bb = S.pbody[S.hl[2 * h + 1]];
+  const bool sa = S.bodies[40 * (size_t)ba + 38] != 0.0, sb = S.bodies[40 * (size_t)bb + 38] != 0.0;
+  const v3<double> n = ld3(c + CH_N), z{0.0, 0.0, 0.0};
+  const v3<double> xa = ld3(pa + SP_X), xb = ld3(pb + SP_X);
+  const v3<double> armA = sub(add(ld3(c + CH_WA), xa), xa), armB = sub(add(ld3(c + CH_WB), xb), xb);
+  const v3<double> v1A = sa ? z : add(ld3(pa + SP_V), cross(mul33v(pa + SP_IB, ld3(pa + SP_L)), armA));
+  const v3<double> v1B = sb ? z : add(ld3(pb + SP_V), cross(mul33v(pb + SP_IB, ld3(pb + SP_L)), armB));
+  const v3<double> v1AB = sub(v1A, v1B);
+  const v3<double> vt = sub(v1AB, sclL(dot(v1AB, n), n));
+  st3(k + CC_VT, vt);
+  const double mu = sv_min(S.fric[ba], S.fric[bb]);
+  const double max_force = (c[CH_IMP] * mu) * 10;
+  const v3<double> tan = sv_normalized(vt);
+  const v3<double> rtA = cross(ld3(k + CC_RA), tan), rtB = cross(ld3(k + CC_RB), tan);
+  double kt = 0.0;
+  if (!sa) kt += 1.0 / pa[SP_MASS] + sv_quad(rtA, pa + SP_IB);
+  if (!sb) kt += 1.0 / pb[SP_MASS] + sv_quad(rtB, pb + SP_IB);
+  const double mt = kt < 1e-6 ? 0.0 : 1.0 / kt;
+  const v3<double> delta = scl(scl(sv_neg(vt), mt), 0.9);
+  v3<double> fit = add(ld3(k + CC_LF), delta);
+  const double len = vlen(fit);
+  const double cl = (len < 0.0) ? 0.0 : (max_force < len) ? max_force : len;  // std::clamp(len, 0, max)
+  fit = scl(sv_normalized(fit), cl);
+  const v3<double> u = dvs(sub(fit, ld3(k + CC_LF)), (double)S.hpc[h]);
+  st3(k + CC_LF, fit);
+  st3(c + CH_U, u);
+  st3(c + CH_LR + 6 * par, sv_torque(fit, armA));
+  st3(c + CH_LR + 6 * par + 3, sv_torque(sv_neg(fit), armB));
+  return vlen(u) > 1e-4;
+}
+// A contact's friction impulse and torque (the last sweep's taken out) on its
+// particle; the offset friction totals stay zero, (0 - 0) / count.
+D2_HD void sv_friction_apply(SvAcc& a, const double* c, int side, int par) {
+  const v3<double> u = ld3(c + CH_U), z{0.0, 0.0, 0.0};
+  a.imp = side ? sub(a.imp, u) : add(a.imp, u);
+  a.rot = add(sub(a.rot, ld3(c + CH_LR + 6 * (par ^ 1) + 3 * side)), ld3(c + CH_LR + 6 * par + 3 * side));
+  a.off = side ? sub(a.off, z) : add(a.off, z);
+}
+D2_HD bool sv_moved(const double* p) { return vlen(sub(ld3(p + SP_IMP), ld3(p + SP_LAST))) > 1e-6; }
+// The new future state (:624-626) of a dynamic particle.
+D2_HD void sv_store_future(const double* p, double* r) {
+  for (int j = 0; j < 4; ++j) r[14 + j] = p[SP_Q + j];
+  for (int j = 0; j < 3; ++j) r[18 + j] = p[SP_X + j], r[21 + j] = p[SP_V + j], r[24 + j] = p[SP_L + j];
+}
+D2_HD void sv_store_out(const double* c, const double* k, double* o) {
+  for (int j = 0; j < 3; ++j) o[j] = c[CH_N + j], o[5 + j] = k[CC_LF + j], o[8 + j] = k[CC_VT + j];
+  o[3] = c[CH_IMP], o[4] = c[CH_OFF];
 }
 
+// The sequential walk: contact by contact, in sorted order.
 D2_HD bool solve_cluster(const ClusterSolve& S) {
   const int nh = S.nh, np = S.np;
   const double t = S.t;
-  // local contacts, in sorted order (:109-163)
-  for (int c = 0; c < nh; ++c) {
-    const int h = S.ord[c];
-    const int la = S.hl[2 * h], lb = S.hl[2 * h + 1];
-    const double* ra = S.bodies + 40 * (size_t)S.pbody[la];
-    const double* rb = S.bodies + 40 * (size_t)S.pbody[lb];
-    const v3<double> A = ld3(S.hA + 3 * h), B = ld3(S.hB + 3 * h);
-    double* s = S.hs + (size_t)SH * c;
-    s[SH_START] = vlen(sub(A, B));
-    if (s[SH_START] < 1e-6 && t > 1e-4) return false;
-    const SolverState fa = sv_load(ra + 14), fb = sv_load(rb + 14);
-    double m[16], mi[16];
-    pose(fa.q, fa.x, m);
-    inv44(m, mi);
-    st3(s + SH_LA, xform(mi, A));
-    pose(fb.q, fb.x, m);
-    inv44(m, mi);
-    st3(s + SH_LB, xform(mi, B));
-    const v3<double> gn = dvs(sub(B, A), 2.0);
-    st3(s + SH_N, sv_normalized(gn));
-    const v3<double> r_A = sub(A, fa.x), r_B = sub(B, fb.x);
-    st3(s + SH_RA, r_A), st3(s + SH_RB, r_B);
-    const v3<double> rn_A = cross(r_A, gn), rn_B = cross(r_B, gn);
-    double k_normal = 0.0;
-    if (ra[38] == 0.0) k_normal += 1.0 / S.mass[S.pbody[la]] + sv_quad(rn_A, ra + 28);
-    if (rb[38] == 0.0) k_normal += 1.0 / S.mass[S.pbody[lb]] + sv_quad(rn_B, rb + 28);
-    s[SH_MEFF] = k_normal < 1e-6 ? 0.0 : 1.0 / k_normal;
-    s[SH_IMP] = 0.0, s[SH_OFF] = 0.0;
-    s[SH_OUTER] = S.heps[h] * 0.25;
-    for (int k = 0; k < 3; ++k) s[SH_LF + k] = 0.0, s[SH_LRA + k] = 0.0, s[SH_LRB + k] = 0.0, s[SH_UT + k] = 0.0;
-  }
-  // per particle: state, impulses from gravity (:171-180)
-  for (int k = 0; k < np; ++k) {
-    const int b = S.pbody[k];
-    double* p = S.ps + (size_t)SP * k;
-    ps_store(p, sv_load(S.bodies + 40 * (size_t)b + 14));
-    st3(p + SP_IMP, scl(sclL(S.mass[b], S.g), t));
-    for (int j = 0; j < 3; ++j) p[SP_ROT + j] = 0.0, p[SP_OFF + j] = 0.0, p[SP_ROFF + j] = 0.0;
-  }
-  // warm start (warm_start.cpp:12-29) and its impulses (:185-213)
-  for (int c = 0; c < nh; ++c) {
-    const int h = S.ord[c];
-    double w;
-    if (warm_find(S.warm, warm_key(S.pbody[S.hl[2 * h]], S.pbody[S.hl[2 * h + 1]]), w)) S.hs[(size_t)SH * c + SH_IMP] = w * 0.75;
-  }
-  for (int c = 0; c < nh; ++c) {
-    const int h = S.ord[c];
-    const double* s = S.hs + (size_t)SH * c;
-    double* pa = S.ps + (size_t)SP * S.hl[2 * h];
-    double* pb = S.ps + (size_t)SP * S.hl[2 * h + 1];
-    const SolverState fa = ps_state(pa), fb = ps_state(pb);
-    const v3<double> n = ld3(s + SH_N);
-    const v3<double> p1A = sv_xform(fa, ld3(s + SH_LA)), p1B = sv_xform(fb, ld3(s + SH_LB));
-    const v3<double> u = scl(sv_neg(n), s[SH_IMP]);
-    st3(pa + SP_IMP, add(ld3(pa + SP_IMP), u));
-    st3(pb + SP_IMP, sub(ld3(pb + SP_IMP), u));
-    st3(pa + SP_ROT, add(ld3(pa + SP_ROT), sv_torque(u, p1A, fa.x)));
-    st3(pb + SP_ROT, add(ld3(pb + SP_ROT), sv_torque(sv_neg(u), p1B, fb.x)));
-  }
-  auto integrate = [&](int k) {
-    const int b = S.pbody[k];
-    const double* r = S.bodies + 40 * (size_t)b;
-    double* p = S.ps + (size_t)SP * k;
-    ps_store(p, sv_update(sv_load(r + 14), t, ld3(p + SP_IMP), ld3(p + SP_OFF), ld3(p + SP_ROT), ld3(p + SP_ROFF),
-                          S.mass[b], r + 28));
-  };
+  auto hot = [&](int c) { return S.hs + (size_t)SH * c; };
+  auto cold = [&](int c) { return S.hs + (size_t)SH * c + CH; };
+  auto part = [&](int c, int side) { return S.ps + (size_t)SP * S.hl[2 * S.ord[c] + side]; };
   auto is_static = [&](int k) { return S.bodies[40 * (size_t)S.pbody[k] + 38] != 0.0; };
-  for (int k = 0; k < np; ++k)  // first prediction (:215-227)
-    if (!is_static(k)) integrate(k);
+  for (int c = 0; c < nh; ++c)
+    if (!sv_contact_setup(S, S.ord[c], hot(c), cold(c))) return false;
+  for (int k = 0; k < np; ++k) sv_particle_setup(S, S.pbody[k], S.ps + (size_t)SP * k);
+  for (int c = 0; c < nh; ++c)
+    for (int side = 0; side < 2; ++side) {
+      SvAcc a = sv_acc(part(c, side));
+      sv_warm_apply(a, hot(c), side);
+      sv_acc_store(a, part(c, side));
+    }
+  for (int k = 0; k < np; ++k)
+    if (!is_static(k)) sv_predict(S.ps + (size_t)SP * k, t);
+  for (int c = 0; c < nh; ++c) sv_contact_turn(hot(c), cold(c), part(c, 0), part(c, 1));
   if (nh > 0) {
-    // normal pass (:231-375)
-    bool converged = false;
+    bool converged = false;  // normal pass (:231-375)
     for (int it = 0; !converged && it < 1000; ++it) {
-      for (int k = 0; k < np; ++k) {
-        double* p = S.ps + (size_t)SP * k;
-        for (int j = 0; j < 3; ++j) p[SP_LAST + j] = p[SP_IMP + j];
-      }
+      for (int k = 0; k < np; ++k) st3(S.ps + (size_t)SP * k + SP_LAST, ld3(S.ps + (size_t)SP * k + SP_IMP));
       for (int c = 0; c < nh; ++c) {
-        const int h = S.ord[c];
-        double* s = S.hs + (size_t)SH * c;
-        const int la = S.hl[2 * h], lb = S.hl[2 * h + 1];
-        double* pa = S.ps + (size_t)SP * la;
-        double* pb = S.ps + (size_t)SP * lb;
-        const double* ra = S.bodies + 40 * (size_t)S.pbody[la];
-        const double* rb = S.bodies + 40 * (size_t)S.pbody[lb];
-        const SolverState fa = ps_state(pa), fb = ps_state(pb);
-        const v3<double> n = ld3(s + SH_N);
-        const double outer = s[SH_OUTER];
-        const v3<double> p1A = sv_xform(fa, ld3(s + SH_LA)), p1B = sv_xform(fb, ld3(s + SH_LB));
-        const double d1 = dot(p1B, n) - dot(p1A, n);
-        const v3<double> v1A = add(fa.v, cross(mul33v(ra + 28, fa.L), sub(p1A, fa.x)));
-        const v3<double> v1B = add(fb.v, cross(mul33v(rb + 28, fb.L), sub(p1B, fb.x)));
-        const double v1 = dot(v1A, n) - dot(v1B, n);
-        const double m = s[SH_MEFF];
-        const double damp = 0.1;
-        const double dimp = d1 < outer ? (v1 * m) * damp : -s[SH_IMP];
-        const double last = s[SH_IMP];
-        s[SH_IMP] = sv_max(s[SH_IMP] + dimp, 0.0);
-        const v3<double> u = scl(sv_neg(n), s[SH_IMP] - last);
-        st3(pa + SP_IMP, add(ld3(pa + SP_IMP), u));
-        st3(pb + SP_IMP, sub(ld3(pb + SP_IMP), u));
-        st3(pa + SP_ROT, add(ld3(pa + SP_ROT), sv_torque(u, p1A, fa.x)));
-        st3(pb + SP_ROT, add(ld3(pb + SP_ROT), sv_torque(sv_neg(u), p1B, fb.x)));
-        const double lower_slop = sv_max(outer * 0.2, outer - s[SH_START]);
-        const double slop = lerp(lower_slop, outer * 0.2, 0.3);
-        const double pen = outer - d1;
-        const double doff = d1 < outer ? ((damp * m) * sv_max(0.0, pen - slop)) / t : -s[SH_OFF];
-        const double last_off = s[SH_OFF];
-        s[SH_OFF] = sv_max(s[SH_OFF] + doff, 0.0);
-        const v3<double> uo = scl(sv_neg(n), s[SH_OFF] - last_off);
-        st3(pa + SP_OFF, add(ld3(pa + SP_OFF), uo));
-        st3(pb + SP_OFF, sub(ld3(pb + SP_OFF), uo));
-        if (ra[38] == 0.0) integrate(la);
-        if (rb[38] == 0.0) integrate(lb);
+        double *pa = part(c, 0), *pb = part(c, 1), *s = hot(c);
+        const v3<double> n = ld3(s + CH_N);
+        const SvSide A = sv_side(pa, ld3(s + CH_WA), n), B = sv_side(pb, ld3(s + CH_WB), n);
+        double du, doff;
+        sv_contact_step(s, B.dn - A.dn, A.vn - B.vn, t, du, doff);
+        const v3<double> u = scl(sv_neg(n), du), uo = scl(sv_neg(n), doff);
+        sv_apply(pa, u, uo, A.arm);
+        sv_apply(pb, sv_neg(u), sv_neg(uo), B.arm);
+        for (int side = 0; side < 2; ++side)
+          if (!is_static(S.hl[2 * S.ord[c] + side])) sv_integrate(part(c, side), t);
       }
       converged = true;
-      for (int k = 0; k < np && converged; ++k) {
-        const double* p = S.ps + (size_t)SP * k;
-        if (vlen(sub(ld3(p + SP_IMP), ld3(p + SP_LAST))) > 1e-6) converged = false;
-      }
+      for (int k = 0; k < np && converged; ++k)
+        if (sv_moved(S.ps + (size_t)SP * k)) converged = false;
     }
-    // friction pass (:392-571); contacts_per_pair is the hit's pair's count (hpc)
-    converged = false;
+    converged = false;  // friction pass (:392-571)
     for (int it = 0; !converged && it < 100; ++it) {
-      for (int c = 0; c < nh; ++c) {
-        const int h = S.ord[c];
-        double* s = S.hs + (size_t)SH * c;
-        const int la = S.hl[2 * h], lb = S.hl[2 * h + 1];
-        const double* ra = S.bodies + 40 * (size_t)S.pbody[la];
-        const double* rb = S.bodies + 40 * (size_t)S.pbody[lb];
-        const SolverState fa = ps_state(S.ps + (size_t)SP * la), fb = ps_state(S.ps + (size_t)SP * lb);
-        const v3<double> n = ld3(s + SH_N);
-        const v3<double> p1A = sv_xform(fa, ld3(s + SH_LA)), p1B = sv_xform(fb, ld3(s + SH_LB));
-        const bool sa = ra[38] != 0.0, sb = rb[38] != 0.0;
-        const v3<double> v1A = sa ? v3<double>{0.0, 0.0, 0.0} : add(fa.v, cross(mul33v(ra + 28, fa.L), sub(p1A, fa.x)));
-        const v3<double> v1B = sb ? v3<double>{0.0, 0.0, 0.0} : add(fb.v, cross(mul33v(rb + 28, fb.L), sub(p1B, fb.x)));
-        const v3<double> v1AB = sub(v1A, v1B);
-        const v3<double> vt = sub(v1AB, sclL(dot(v1AB, n), n));
-        st3(s + SH_VT, vt);
-        const double mu = sv_min(S.fric[S.pbody[la]], S.fric[S.pbody[lb]]);
-        const double max_force = (s[SH_IMP] * mu) * 10;
-        const v3<double> tan = sv_normalized(vt);
-        const v3<double> rtA = cross(ld3(s + SH_RA), tan), rtB = cross(ld3(s + SH_RB), tan);
-        double kt = 0.0;
-        if (!sa) kt += 1.0 / S.mass[S.pbody[la]] + sv_quad(rtA, ra + 28);
-        if (!sb) kt += 1.0 / S.mass[S.pbody[lb]] + sv_quad(rtB, rb + 28);
-        const double mt = kt < 1e-6 ? 0.0 : 1.0 / kt;
-        const v3<double> delta = scl(scl(sv_neg(vt), mt), 0.9);
-        v3<double> fit = add(ld3(s + SH_LF), delta);
-        const double len = vlen(fit);
-        const double cl = (len < 0.0) ? 0.0 : (max_force < len) ? max_force : len;  // std::clamp(len, 0, max)
-        fit = scl(sv_normalized(fit), cl);
-        st3(s + SH_UT, fit);
-      }
       converged = true;
-      for (int c = 0; c < nh; ++c) {
-        const int h = S.ord[c];
-        double* s = S.hs + (size_t)SH * c;
-        const int la = S.hl[2 * h], lb = S.hl[2 * h + 1];
-        double* pa = S.ps + (size_t)SP * la;
-        double* pb = S.ps + (size_t)SP * lb;
-        const SolverState fa = ps_state(pa), fb = ps_state(pb);
-        const double cpp = (double)S.hpc[h];
-        const v3<double> p1A = sv_xform(fa, ld3(s + SH_LA)), p1B = sv_xform(fb, ld3(s + SH_LB));
-        const v3<double> u = dvs(sub(ld3(s + SH_UT), ld3(s + SH_LF)), cpp);
-        st3(s + SH_LF, ld3(s + SH_UT));
-        st3(pa + SP_IMP, add(ld3(pa + SP_IMP), u));
-        st3(pb + SP_IMP, sub(ld3(pb + SP_IMP), u));
-        if (vlen(u) > 1e-4) converged = false;
-        const v3<double> lf = ld3(s + SH_LF);
-        const v3<double> rA = sv_torque(lf, p1A, fa.x), rB = sv_torque(sv_neg(lf), p1B, fb.x);
-        st3(pa + SP_ROT, sub(ld3(pa + SP_ROT), ld3(s + SH_LRA)));
-        st3(pb + SP_ROT, sub(ld3(pb + SP_ROT), ld3(s + SH_LRB)));
-        st3(s + SH_LRA, rA), st3(s + SH_LRB, rB);
-        st3(pa + SP_ROT, add(ld3(pa + SP_ROT), rA));
-        st3(pb + SP_ROT, add(ld3(pb + SP_ROT), rB));
-        // the offset friction totals stay zero: (0 - 0) / count
-        const v3<double> uo = dvs(sub(v3<double>{0.0, 0.0, 0.0}, v3<double>{0.0, 0.0, 0.0}), cpp);
-        st3(pa + SP_OFF, add(ld3(pa + SP_OFF), uo));
-        st3(pb + SP_OFF, sub(ld3(pb + SP_OFF), uo));
-        st3(pa + SP_ROFF, add(ld3(pa + SP_ROFF), sv_torque(uo, p1A, fa.x)));
-        st3(pb + SP_ROFF, add(ld3(pb + SP_ROFF), sv_torque(sv_neg(uo), p1B, fb.x)));
-      }
+      for (int c = 0; c < nh; ++c)
+        if (sv_friction(S, S.ord[c], hot(c), cold(c), part(c, 0), part(c, 1), it & 1)) converged = false;
+      for (int c = 0; c < nh; ++c)
+        for (int side = 0; side < 2; ++side) {
+          SvAcc a = sv_acc(part(c, side));
+          sv_friction_apply(a, hot(c), side, it & 1);
+          sv_acc_store(a, part(c, side));
+        }
       for (int k = 0; k < np; ++k)
-        if (!is_static(k)) integrate(k);
+        if (!is_static(k)) sv_integrate(S.ps + (size_t)SP * k, t);
     }
   }
-  // the new future states (:624-626; a static body's stays as it was)
-  for (int k = 0; k < np; ++k) {
-    if (is_static(k)) continue;
-    const double* p = S.ps + (size_t)SP * k;
-    double* r = S.bodies + 40 * (size_t)S.pbody[k] + 14;
-    for (int j = 0; j < 13; ++j) r[j] = p[j];
-  }
+  for (int k = 0; k < np; ++k)  // a static body's future state stays as it was
+    if (!is_static(k)) sv_store_future(S.ps + (size_t)SP * k, S.bodies + 40 * (size_t)S.pbody[k]);
   // warm store: each body pair keeps its last contact's impulse
   for (int c = 0; c < nh; ++c) {
     const int h = S.ord[c];
-    warm_put(S.warm, warm_key(S.pbody[S.hl[2 * h]], S.pbody[S.hl[2 * h + 1]]), S.hs[(size_t)SH * c + SH_IMP]);
+    warm_put(S.warm, warm_key(S.pbody[S.hl[2 * h]], S.pbody[S.hl[2 * h + 1]]), hot(c)[CH_IMP]);
   }
-  for (int c = 0; c < nh; ++c) {
-    const int h = S.ord[c];
-    const double* s = S.hs + (size_t)SH * c;
-    double* o = S.out_h + 11 * (size_t)h;
-    o[0] = s[SH_N], o[1] = s[SH_N + 1], o[2] = s[SH_N + 2], o[3] = s[SH_IMP], o[4] = s[SH_OFF];
-    for (int j = 0; j < 3; ++j) o[5 + j] = s[SH_LF + j], o[8 + j] = s[SH_VT + j];
-  }
+  for (int c = 0; c < nh; ++c) sv_store_out(hot(c), cold(c), S.out_h + 11 * (size_t)S.ord[c]);
   return true;
 }
 

@@ -3487,7 +3487,7 @@ struct d2_ctx {
   int gate_phases = 3;       // bit 0: CCD phase, bit 1: discrete phase
   DBuf<float> mlp_w, mlp_m, mlp_v, mlp_wf, mlp_grad;
   DBuf<short> mlp_wb;
-  DBuf<float> tr_x, tr_t, tr_act, tr_dlt, tr_loss;
+  DBuf<float> tr_x, tr_t, tr_part, tr_loss;
   DBuf<int> tr_idx;
   bool mlp_ready = false, learned_on = false, has_max_time = false;
   float gate_t = 1.1f, gate_s = 0.99f;
@@ -4563,7 +4563,7 @@ int d2_ctx_destroy(d2_ctx* c) {
       release(c->bk_count), release(c->bk_hits), release(c->bk_out_r), release(c->bk_counter);
   release(c->tree_radius), release(c->tree_eps_out), release(c->hv), release(c->feat), release(c->pred), release(c->hv_off);
   release(c->cert), release(c->mlp_w), release(c->mlp_m), release(c->mlp_v), release(c->mlp_wf), release(c->mlp_grad);
-  release(c->mlp_wb), release(c->tr_x), release(c->tr_t), release(c->tr_act), release(c->tr_dlt), release(c->tr_loss);
+  release(c->mlp_wb), release(c->tr_x), release(c->tr_t), release(c->tr_part), release(c->tr_loss);
   release(c->tr_idx);
   release(c->tb_box), release(c->tb_rad), release(c->last_state), release(c->bp_R), release(c->tree_depth_d),
       release(c->group);
@@ -5543,14 +5543,15 @@ int mlp_alloc(d2_ctx* c) {
 // Minibatch forward/backward + parameter gradient (grad in c->mlp_grad,
 // per-sample losses in c->tr_loss).
 void mlp_batch_grad(d2_ctx* c, const int* idx, int nb, float lw0, float lw1, float delta) {
-  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3((nb + 255) / 256), dim3(256), 0, c->stream, nb, idx, c->tr_x.p, c->tr_t.p,
-                     c->mlp_wf.p, lw0, lw1, delta, c->tr_act.p, c->tr_dlt.p, c->tr_loss.p);
-  hipLaunchKernelGGL(k_mlp_grad, dim3((MLP_PARAMS + 255) / 256), dim3(256), 0, c->stream, nb, c->tr_act.p, c->tr_dlt.p,
+  const int blocks = std::min((nb + MLP_TILE - 1) / MLP_TILE, MLP_MAX_PART);
+  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(blocks), dim3(256), 0, c->stream, nb, idx, c->tr_x.p, c->tr_t.p,
+                     c->mlp_wf.p, lw0, lw1, delta, c->tr_part.p, c->tr_loss.p);
+  hipLaunchKernelGGL(k_mlp_grad_sum, dim3((MLP_PARAMS + 63) / 64), dim3(512), 0, c->stream, blocks, c->tr_part.p,
                      c->mlp_grad.p);
 }
 int mlp_upload_data(d2_ctx* c, const float* X, const float* T, int n, int batch) {
   RC(ensure(c, c->tr_x, (size_t)n * MLP_IN)); RC(ensure(c, c->tr_t, (size_t)n * MLP_OUT));
-  RC(ensure(c, c->tr_act, (size_t)batch * MLP_ACT)); RC(ensure(c, c->tr_dlt, (size_t)batch * MLP_DELTA));
+  RC(ensure(c, c->tr_part, (size_t)MLP_MAX_PART * MLP_PARAMS));
   RC(ensure(c, c->tr_loss, batch)); RC(ensure(c, c->tr_idx, n));
   HIPCHK(c, hipMemcpyAsync(c->tr_x.p, X, sizeof(float) * MLP_IN * (size_t)n, hipMemcpyHostToDevice, c->stream));
   if (T) HIPCHK(c, hipMemcpyAsync(c->tr_t.p, T, sizeof(float) * MLP_OUT * (size_t)n, hipMemcpyHostToDevice, c->stream));

@@ -18,7 +18,7 @@
 // is always the smallest index of its tree), clusters numbered by their
 // smallest member, roll-back of the members to the cluster's earliest time.
 
-constexpr int BP_SEG = 4096;  // bodies one static body's wave sweeps per item
+constexpr int BP_SEG = 512;  // bodies one item of a static body sweeps (4096 left 48 wavefronts to finish 100 us after the rest)
 constexpr int BP_WAVE_CAP = 512;  // partners a wave sorts in LDS
 enum BpRed : int {  // reductions over the non-static bodies' boxes
   BR_EXT = 0,       // largest box extent (float bits, non-negative)
@@ -44,7 +44,7 @@ __device__ __forceinline__ double ord2d(long long o) {
   return __longlong_as_double(o >= 0 ? o : o ^ 0x7fffffffffffffffll);
 }
 
-struct Box8 {  // float lo xyz, pad, hi xyz, pad
+struct alignas(16) Box8 {  // float lo xyz, pad, hi xyz, pad
   float v[8];
 };
 __device__ __forceinline__ void box_extend(float* lo, float* hi, const float* blo, const float* bhi) {
@@ -61,6 +61,8 @@ __device__ __forceinline__ bool box_overlap(const Box8& a, const Box8& b) {
 __global__ void k_bp_bounds(int n, const double* bodies, const double* last, const int32_t* body_tree,
                             const float* tb_box, const double* tb_rad, const int32_t* group, int mode, double t,
                             Box8* box, double* R, int* meta, int* red) {
+  int best[5];
+  for (int q = 0; q < 5; ++q) best[q] = (int)0x80000000;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const double* r = bodies + 40 * (size_t)i;
     const int tr = body_tree[i];
@@ -114,11 +116,32 @@ __global__ void k_bp_bounds(int n, const double* bodies, const double* last, con
     meta[i] = (group ? group[i] : 0) * 2 + (st ? BM_STATIC : 0);
     if (!st) {
       const float ext = fmaxf(b.v[4] - b.v[0], fmaxf(b.v[5] - b.v[1], b.v[6] - b.v[2]));
-      atomicMax(&red[BR_EXT], __float_as_int(ext > 0.f ? ext : 0.f));
-      atomicMin(&red[BR_LO + 0], f2ord(b.v[0]));
-      atomicMin(&red[BR_LO + 1], f2ord(b.v[1]));
-      atomicMin(&red[BR_LO + 2], f2ord(b.v[2]));
-      atomicMax(&red[BR_HIZ], f2ord(b.v[6]));
+      const int e5[5] = {__float_as_int(ext > 0.f ? ext : 0.f), ~f2ord(b.v[0]), ~f2ord(b.v[1]), ~f2ord(b.v[2]),
+                         f2ord(b.v[6])};  // ~: the minimum as a maximum
+#pragma unroll
+      for (int q = 0; q < 5; ++q) best[q] = e5[q] > best[q] ? e5[q] : best[q];
+    }
+  }
+  // the block's extremes, one atomic each (every body's own, on five shared
+  // addresses, cost 64 us for 65 536 bodies; 14 us now)
+  __shared__ int s_best[4][5];
+#pragma unroll
+  for (int q = 0; q < 5; ++q)
+    for (int off = 32; off > 0; off >>= 1) {
+      const int o = __shfl_xor(best[q], off);
+      best[q] = o > best[q] ? o : best[q];
+    }
+  if (lane_id() == 0)
+    for (int q = 0; q < 5; ++q) s_best[threadIdx.x >> 6][q] = best[q];
+  __syncthreads();
+  if (threadIdx.x < 5) {
+    const int q = threadIdx.x;
+    int v = s_best[0][q];
+    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) v = s_best[k][q] > v ? s_best[k][q] : v;
+    if (v != (int)0x80000000) {
+      if (q == 0) atomicMax(&red[BR_EXT], v);
+      else if (q == 4) atomicMax(&red[BR_HIZ], v);
+      else atomicMin(&red[BR_LO + q - 1], ~v);
     }
   }
 }
@@ -201,10 +224,17 @@ __device__ __forceinline__ long long bp_lookup(unsigned long long key, long long
     s = (s + 1) & (T - 1);
   }
 }
-__global__ void k_bp_scatter(int n, const int* meta, const int* slot_of, const int* rank_of, const int* start,
-                             int* members) {
+// The cells' members: a copy of each body's box with its index and group bits
+// in the two spare words, so a candidate is one 32-byte load next to its
+// cell mates instead of an index, a group word and a box from three arrays.
+__global__ void k_bp_scatter(int n, const Box8* box, const int* meta, const int* slot_of, const int* rank_of,
+                             const int* start, Box8* members) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    if (!(meta[i] & BM_STATIC)) members[start[slot_of[i]] + rank_of[i]] = i;
+    if (!(meta[i] & BM_STATIC)) {
+      Box8 b = box[i];
+      b.v[3] = __int_as_float(i), b.v[7] = __int_as_float(meta[i]);
+      members[start[slot_of[i]] + rank_of[i]] = b;
+    }
 }
 
 // State::interpolate (model/state.cpp:55-70) of translation and velocity.
@@ -271,8 +301,16 @@ __device__ __forceinline__ bool bp_collide(int a, int b, int mode, double t, con
 // list is placed by rank when it is gathered).
 __device__ __forceinline__ void lds_rank_sort(int* buf, int cnt) {
   // distinct body indices: a value's rank is the number of smaller values
-  constexpr int PER = BP_WAVE_CAP / 64;
   const int lane = lane_id();
+  if (cnt <= 64) {  // one value per lane
+    const int v = lane < cnt ? buf[lane] : 0x7fffffff;
+    int r = 0;
+    for (int j = 0; j < cnt; ++j) r += rl(v, j) < v ? 1 : 0;
+    if (lane < cnt) buf[r] = v;
+    wave_sync_lds();
+    return;
+  }
+  constexpr int PER = BP_WAVE_CAP / 64;
   int vals[PER], ranks[PER];
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
@@ -307,93 +345,102 @@ struct BpIn {
   const unsigned long long* keys;
   const int* counts;
   const int* start;
-  const int* members;
+  const Box8* members;
 };
-__device__ __forceinline__ bool bp_test(const BpIn& in, int a, const Box8& ba, int ma, int j, int* red_w) {
-  if (j <= a || (in.meta[j] >> 1) != (ma >> 1)) return false;
-  if ((in.meta[j] & BM_STATIC) && (ma & BM_STATIC)) return false;  // collideFunc: not both static
-  if (!box_overlap(ba, in.box[j])) return false;
+__device__ __forceinline__ bool bp_test_box(const BpIn& in, int a, const Box8& ba, int ma, int j, const Box8& bj, int mj,
+                                            int* red_w) {
+  if (j <= a || (mj >> 1) != (ma >> 1)) return false;
+  if ((mj & BM_STATIC) && (ma & BM_STATIC)) return false;  // collideFunc: not both static
+  if (!box_overlap(ba, bj)) return false;
   return bp_collide(a, j, in.mode, in.t, in.bodies, in.last, in.R, in.meta, red_w);
 }
-
-__global__ void __launch_bounds__(256) k_bp_pairs(BpIn in, int n_items, const int* item_body, const int* item_seg,
+// A wavefront takes BP_BATCH items and keeps their sorted partner lists in
+// LDS; the block then allocates one range for all four wavefronts' lists (an
+// atomic per item, all on one address, was most of this kernel's 654 us for
+// 65 536 bodies; 195 us now).  A list that does not fit the wavefront's LDS
+// any more allocates its own range and is written in a second pass, unsorted
+// above BP_WAVE_CAP partners.
+constexpr int BP_BATCH = 8;
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) k_bp_pairs(BpIn in, int n_items, const int* item_body, const int* item_seg,
                                                   long long cap, int2* chunk, unsigned long long* chunk_fill,
                                                   int* item_cnt, long long* item_pos, int* item_sorted, int* red_w) {
   __shared__ int lds[4][BP_WAVE_CAP];
   __shared__ int nb_pre[4][28], nb_st[4][27];
+  __shared__ int s_fill[4];
+  __shared__ unsigned long long s_base;
   const int w = threadIdx.x >> 6, lane = lane_id();
   const BpGrid g = bp_grid(in.red);
-  for (int it = blockIdx.x * 4 + w; it < n_items; it += gridDim.x * 4) {
-    const int a = item_body[it];
-    const Box8 ba = in.box[a];
-    const int ma = in.meta[a];
-    int cnt = 0, sorted = 1;
-    long long pos = 0;
-    if (ma & BM_STATIC) {
-      // sweep over the bodies after a, in index order (the chunk comes out sorted)
-      const long long lo = (long long)a + 1 + (long long)item_seg[it] * BP_SEG;
-      const long long hi = lo + BP_SEG < in.n ? lo + BP_SEG : in.n;
+  const int n_groups = (n_items + 4 * BP_BATCH - 1) / (4 * BP_BATCH);
+  for (int grp = blockIdx.x; grp < n_groups; grp += gridDim.x) {  // block-uniform
+    const int it0 = grp * 4 + w, step = n_groups * 4;  // strided: a static body's segments spread over wavefronts
+    int fill = 0;                  // partners kept in LDS
+    int my_cnt_kept = 0, my_at = -1, my_body = 0;  // lane b: item b's list in LDS (-1: none there)
+    for (int b = 0; b < BP_BATCH; ++b) {
+      const int it = it0 + b * step;
+      if (it >= n_items) break;
+      const int a = item_body[it];
+      const Box8 ba = in.box[a];
+      const int ma = in.meta[a];
+      int cnt = 0, sorted = 1, kept_at = -1;
+      long long pos = 0;
+      // candidates: a static body sweeps a segment of the bodies after it, in
+      // index order; another body takes the members of the 27 cells around
+      // its own, then the static bodies
+      const bool sweep = ma & BM_STATIC;
+      long long lo = 0;
+      int total = 0, n_cand;
+      if (sweep) {
+        lo = (long long)a + 1 + (long long)item_seg[it] * BP_SEG;
+        const long long hi = lo + BP_SEG < in.n ? lo + BP_SEG : in.n;
+        n_cand = hi > lo ? (int)(hi - lo) : 0;
+      } else {
+        long long c0[3];
+        bp_cell(g, ba, ma >> 1, c0);
+        int my_cnt = 0, my_st = 0;
+        int s = -1;
+        if (lane < 27)
+          s = (int)bp_lookup(bp_key(c0[0] + lane % 3 - 1, c0[1] + (lane / 3) % 3 - 1, c0[2] + lane / 9 - 1), in.T, in.keys);
+        // far-apart cells can share a key (coordinates wrap): visit each slot once
+#pragma unroll 1
+        for (int d = 0; d < 26; ++d) {
+          const int o = rl(s, d);
+          if (d < lane && o == s) s = -1;
+        }
+        if (s >= 0) my_cnt = in.counts[s], my_st = in.start[s];
+        const int incl = wave_incl_scan(my_cnt);
+        if (lane < 27) nb_pre[w][lane + 1] = incl, nb_st[w][lane] = my_st;
+        if (lane == 0) nb_pre[w][0] = 0;
+        wave_sync_lds();
+        total = rl(incl, 26);
+        n_cand = total + in.n_static;
+      }
+      const int room = BP_WAVE_CAP - fill;
       for (int pass = 0; pass < 2; ++pass) {
         int c = 0;
-        for (long long b0 = lo; b0 < hi; b0 += 64) {
-          const long long j = b0 + lane;
-          const bool h = j < hi && bp_test(in, a, ba, ma, (int)j, red_w);
-          const unsigned long long m = __ballot(h);
-          if (pass == 1 && h) chunk[pos + c + __popcll(m & lanes_below())] = make_int2(a, (int)j);
-          c += __popcll(m);
-        }
-        if (pass == 1) break;
-        cnt = c;
-        if (cnt == 0) break;
-        unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(chunk_fill, (unsigned long long)cnt);
-        pos = (long long)__shfl((long long)base, 0);
-        if (pos + cnt > cap) {
-          if (lane == 0) atomicOr(&red_w[BR_OVF], 1);
-          break;
-        }
-      }
-    } else {
-      // candidates: the members of the 27 cells around a's cell, then the static bodies
-      long long c0[3];
-      bp_cell(g, ba, ma >> 1, c0);
-      int my_cnt = 0, my_st = 0;
-      long long s = -1;
-      if (lane < 27)
-        s = bp_lookup(bp_key(c0[0] + lane % 3 - 1, c0[1] + (lane / 3) % 3 - 1, c0[2] + lane / 9 - 1), in.T, in.keys);
-      // far-apart cells can share a key (coordinates wrap): visit each slot once
-      for (int d = 0; d < 27; ++d) {
-        const long long o = __shfl(s, d);
-        if (d < lane && o == s) s = -1;
-      }
-      if (s >= 0) my_cnt = in.counts[s], my_st = in.start[s];
-      int incl = my_cnt;
-#pragma unroll
-      for (int d = 1; d < 32; d <<= 1) {
-        const int o = __shfl_up(incl, d);
-        if (lane >= d) incl += o;
-      }
-      if (lane < 27) nb_pre[w][lane + 1] = incl, nb_st[w][lane] = my_st;
-      if (lane == 0) nb_pre[w][0] = 0;
-      wave_sync_lds();
-      const int total = nb_pre[w][27];
-      for (int pass = 0; pass < 2; ++pass) {
-        int c = 0;
-        for (int k0 = 0; k0 < total + in.n_static; k0 += 64) {
+        for (int k0 = 0; k0 < n_cand; k0 += 64) {
           const int k = k0 + lane;
+          bool h = false;
           int j = -1;
-          if (k < total) {
-            int q = 0;
-            while (nb_pre[w][q + 1] <= k) ++q;
-            j = in.members[nb_st[w][q] + (k - nb_pre[w][q])];
-          } else if (k < total + in.n_static) {
-            j = in.statics[k - total];
+          if (k < n_cand) {
+            Box8 m;
+            int mj;
+            if (!sweep && k < total) {
+              int q = 0;  // the last cell whose first candidate is at or before k
+#pragma unroll
+              for (int half = 16; half > 0; half >>= 1)
+                if (q + half < 27 && nb_pre[w][q + half] <= k) q += half;
+              m = in.members[nb_st[w][q] + (k - nb_pre[w][q])];
+              j = __float_as_int(m.v[3]), mj = __float_as_int(m.v[7]);
+            } else {
+              j = sweep ? (int)(lo + k) : in.statics[k - total];
+              m = in.box[j], mj = in.meta[j];
+            }
+            h = bp_test_box(in, a, ba, ma, j, m, mj, red_w);
           }
-          const bool h = j >= 0 && bp_test(in, a, ba, ma, j, red_w);
           const unsigned long long m = __ballot(h);
           const int at = c + __popcll(m & lanes_below());
           if (h) {
-            if (pass == 0 && at < BP_WAVE_CAP) lds[w][at] = j;
+            if (pass == 0 && at < room) lds[w][fill + at] = j;
             if (pass == 1) chunk[pos + at] = make_int2(a, j);
           }
           c += __popcll(m);
@@ -401,6 +448,13 @@ __global__ void __launch_bounds__(256) k_bp_pairs(BpIn in, int n_items, const in
         if (pass == 1) break;
         cnt = c;
         if (cnt == 0) break;
+        if (cnt <= room) {  // stays in LDS until the block's range is known
+          wave_sync_lds();
+          if (!sweep) lds_rank_sort(lds[w] + fill, cnt);
+          kept_at = fill;
+          fill += cnt;
+          break;
+        }
         unsigned long long base = 0;
         if (lane == 0) base = atomicAdd(chunk_fill, (unsigned long long)cnt);
         pos = (long long)__shfl((long long)base, 0);
@@ -408,21 +462,39 @@ __global__ void __launch_bounds__(256) k_bp_pairs(BpIn in, int n_items, const in
           if (lane == 0) atomicOr(&red_w[BR_OVF], 1);
           break;
         }
-        if (cnt <= BP_WAVE_CAP) {
-          wave_sync_lds();
-          lds_rank_sort(lds[w], cnt);
-          for (int k = lane; k < cnt; k += 64) chunk[pos + k] = make_int2(a, lds[w][k]);
-          break;
-        }
-        sorted = 0;  // second pass writes the list unsorted
+        sorted = sweep ? 1 : 0;  // the second pass writes the list as it comes
+      }
+      if (lane == b) my_cnt_kept = kept_at >= 0 ? cnt : 0, my_at = kept_at, my_body = a;
+      if (lane == 0) {
+        item_cnt[it] = cnt;
+        item_pos[it] = pos;  // (lists kept in LDS: below)
+        item_sorted[it] = sorted;
+      }
+      wave_sync_lds();
+    }
+    if (lane == 0) s_fill[w] = fill;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int tot = s_fill[0] + s_fill[1] + s_fill[2] + s_fill[3];
+      unsigned long long base = tot ? atomicAdd(chunk_fill, (unsigned long long)tot) : 0ull;
+      if ((long long)base + tot > cap) {
+        atomicOr(&red_w[BR_OVF], 1);
+        base = ~0ull;
+      }
+      s_base = base;
+    }
+    __syncthreads();
+    if (s_base != ~0ull) {
+      long long base = (long long)s_base;
+      for (int v = 0; v < w; ++v) base += s_fill[v];
+      if (lane < BP_BATCH && my_at >= 0) item_pos[it0 + lane * step] = base + my_at;
+      for (int b = 0; b < BP_BATCH; ++b) {
+        const int at = rl(my_at, b), cnt = rl(my_cnt_kept, b), a = rl(my_body, b);
+        if (at < 0) continue;
+        for (int k = lane; k < cnt; k += 64) chunk[base + at + k] = make_int2(a, lds[w][at + k]);
       }
     }
-    if (lane == 0) {
-      item_cnt[it] = cnt;
-      item_pos[it] = pos;
-      item_sorted[it] = sorted;
-    }
-    wave_sync_lds();
+    __syncthreads();  // the lists are rewritten by the next group
   }
 }
 
@@ -459,23 +531,39 @@ __global__ void __launch_bounds__(256) k_bp_gather(int n_items, const int* item_
       deepest = dsum > deepest ? dsum : deepest;
     }
   }
-  if (deepest) atomicMax(&red_w[BR_DEPTH], deepest);
+  for (int off = 32; off > 0; off >>= 1) {  // one atomic per wavefront, and only where it raises the value
+    const int o = __shfl_xor(deepest, off);
+    deepest = o > deepest ? o : deepest;
+  }
+  if (lane == 0 && deepest > __hip_atomic_load(&red_w[BR_DEPTH], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&red_w[BR_DEPTH], deepest);
 }
 
 // ---------------------------------------------------------------- clusters
-__device__ __forceinline__ int cc_find(const int* parent, int x) {
-  int p = __atomic_load_n(&parent[x], __ATOMIC_RELAXED);
-  while (p != x) {  // parents only ever point to smaller indices
-    x = p;
-    p = __atomic_load_n(&parent[x], __ATOMIC_RELAXED);
+// The root of x, halving the path on the way: every visited node is pointed
+// at its grandparent.  The loads may come from the caches (wavefront scope):
+// a node's parent only ever changes to an ancestor with a smaller index, so a
+// stale parent is still an ancestor, and whether a root found this way is one
+// still is decided by the CAS that hooks it.  Loads at device scope, all
+// ending on the largest component's root, queued on one line: 260 us of
+// unions for 120 k pairs of 65 536 bodies against 102 us.
+__device__ __forceinline__ int cc_load(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+__device__ __forceinline__ int cc_find(int* parent, int x) {
+  int p = cc_load(&parent[x]);
+  while (p != x) {
+    const int g = cc_load(&parent[p]);
+    if (g != p) __hip_atomic_store(&parent[x], g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    x = p, p = g;
   }
   return x;
 }
 __global__ void k_cc_init(int n, int* parent) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) parent[i] = i;
 }
-// Hooks the larger root under the smaller; a failed CAS means the root was
-// hooked meanwhile, so the loop retries from the new roots.
+// Hooks the larger root under the smaller (or under a node of the smaller's
+// tree); a failed CAS means the root was hooked meanwhile, so the loop goes on
+// from the root of what it was hooked under.
 __global__ void k_cc_union(int n_pairs, const int32_t* pairs, const double* bodies, int* parent, int* red_w) {
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n_pairs; p += gridDim.x * blockDim.x) {
     const int a = pairs[2 * p], b = pairs[2 * p + 1];
@@ -496,7 +584,7 @@ __global__ void k_cc_union(int n_pairs, const int32_t* pairs, const double* bodi
     }
   }
 }
-__global__ void k_cc_roots(int n, const double* bodies, const int* parent, int* label, int* is_root) {
+__global__ void k_cc_roots(int n, const double* bodies, int* parent, int* label, int* is_root) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int r = cc_find(parent, i);
     label[i] = r;
@@ -507,17 +595,23 @@ __global__ void k_cc_roots(int n, const double* bodies, const int* parent, int* 
 // smallest last step per cluster.
 __global__ void k_cc_assign(int n, const double* bodies, const int* label, const int* root_off, int* of_body,
                             int* first, long long* tmin, unsigned long long* smin_bits) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const double* r = bodies + 40 * (size_t)i;
-    if (r[38] != 0.0) {
-      of_body[i] = -1;
-      continue;
+  const int stride = gridDim.x * blockDim.x;
+  for (int i0 = blockIdx.x * blockDim.x; i0 < n; i0 += stride) {  // every lane takes part in the reductions
+    const int i = i0 + threadIdx.x;
+    int c = -1;
+    long long t = 0;
+    unsigned long long st = 0;
+    if (i < n) {
+      const double* r = bodies + 40 * (size_t)i;
+      if (r[38] == 0.0) {
+        c = root_off[label[i]];
+        if (label[i] == i) first[c] = i;
+        t = d2ord(r[13]), st = (unsigned long long)__double_as_longlong(r[39]);
+      }
+      of_body[i] = c;
     }
-    const int c = root_off[label[i]];
-    of_body[i] = c;
-    if (label[i] == i) first[c] = i;
-    atomicMin(&tmin[c], d2ord(r[13]));
-    atomic_min_pos(&smin_bits[c], r[39]);
+    wave_key_min(c, t, tmin);
+    wave_key_min(c, st, smin_bits);
   }
 }
 __global__ void k_cc_init_cl(int n_clusters, long long* tmin, unsigned long long* smin_bits) {

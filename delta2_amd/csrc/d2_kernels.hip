@@ -174,6 +174,34 @@ __device__ __forceinline__ void atomic_min_pos(unsigned long long* addr, double 
   atomicMin(addr, (unsigned long long)__double_as_longlong(v));
 }
 
+__device__ __forceinline__ int rl(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+
+// arr[key] = min(arr[key], v) for every lane (key -1: none).  Most lanes of a
+// wavefront often share one key (a pile is one cluster), and atomics on one
+// address take turns (6 ns each here): the lanes of the first keys met are
+// reduced to one atomic per key, the others go by themselves, and a value
+// that would not lower the entry goes nowhere.  All lanes call it.
+template <class V> __device__ __forceinline__ void wave_key_min(int key, V v, V* arr) {
+  unsigned long long todo = __ballot(key >= 0);
+  for (int round = 0; round < 4 && todo; ++round) {
+    const int l = __ffsll((long long)todo) - 1;
+    const int k0 = rl(key, l);
+    const unsigned long long same = __ballot(key == k0);
+    V x = v;
+    if (__popcll(same) > 1) {
+      if (key != k0) x = (V)(~0ull >> (64 - 8 * sizeof(V) + (V(-1) < V(0) ? 1 : 0)));  // the type's largest value
+      for (int off = 32; off > 0; off >>= 1) {
+        const V o = __shfl_xor(x, off);
+        x = o < x ? o : x;
+      }
+    }
+    if (lane_id() == l && x < __hip_atomic_load(&arr[k0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&arr[k0], x);
+    todo &= ~same;
+    if (key == k0) key = -1;
+  }
+  if (key >= 0 && v < __hip_atomic_load(&arr[key], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&arr[key], v);
+}
+
 template <class R> __device__ __forceinline__ tri<R> load_tri(const double* bucket, int k) {
   return tri<R>{{(R)bucket[0 * 8 + k], (R)bucket[1 * 8 + k], (R)bucket[2 * 8 + k]},
                 {(R)bucket[3 * 8 + k], (R)bucket[4 * 8 + k], (R)bucket[5 * 8 + k]},
@@ -327,12 +355,16 @@ __device__ __forceinline__ void cluster_init_range(const ClusterAcc& A, long lon
   }
 }
 __device__ __forceinline__ void cluster_first_range(const ClusterAcc& A, int n_pairs, long long t0, long long stride) {
-  for (long long p = t0; p < n_pairs; p += stride) {
-    const int k = A.cluster_of_pair[p];
-    atomicMin(&A.first_any[k], (int)p);
-    const bool sa = A.bodies[40 * (size_t)A.pairs[2 * p] + 38] != 0.0;
-    const bool sb = A.bodies[40 * (size_t)A.pairs[2 * p + 1] + 38] != 0.0;
-    if (!(sa && sb)) atomicMin(&A.first_ns[k], (int)p);
+  for (long long p0 = t0 - lane_id(); p0 < n_pairs; p0 += stride) {  // wavefront-uniform
+    const long long p = p0 + lane_id();
+    int k = -1;
+    bool ns = false;
+    if (p < n_pairs) {
+      k = A.cluster_of_pair[p];
+      ns = !(A.bodies[40 * (size_t)A.pairs[2 * p] + 38] != 0.0 && A.bodies[40 * (size_t)A.pairs[2 * p + 1] + 38] != 0.0);
+    }
+    wave_key_min(k, (int)p, A.first_any);
+    wave_key_min(ns ? k : -1, (int)p, A.first_ns);
   }
 }
 
@@ -968,8 +1000,6 @@ __device__ __forceinline__ int expansion_desc(const NodeRec& na, const NodeRec& 
   const NodeRec& par = adv_a ? na : nb;
   return (adv_a ? 1 : 0) | (par.nchild << 1) | (par.child_first << 5);
 }
-__device__ __forceinline__ int rl(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
-// Inclusive prefix sum over the wavefront (every lane active).
 // Discrete lists: the children of a node pair that hits or may hit, at slot,
 // slot + 1, ... of the next list, each naming its parent: parent 0 for a
 // certain hit, list index + 1 when the parent's FP64 tests (k_tri_dist, its
@@ -2728,27 +2758,33 @@ __global__ void k_cluster_first(int n_pairs, ClusterAcc CA) {
 __global__ void k_cluster_min(int n_pairs, const int32_t* pairs, const int32_t* cluster_of_pair, const double* bodies,
                               const int* pair_cnt, const double* scale, const int* first_ns, int* read_later,
                               unsigned long long* step_bits) {
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n_pairs; p += gridDim.x * blockDim.x) {
-    const int k = cluster_of_pair[p], a = pairs[2 * p], b = pairs[2 * p + 1];
-    const double* ra = bodies + 40 * (size_t)a;
-    const double* rb = bodies + 40 * (size_t)b;
-    const bool sa = ra[38] != 0.0, sb = rb[38] != 0.0;
-    if (sa && sb) continue;
-    const bool first = p == first_ns[k];
-    const int id = !sa ? a : b;
-    if (!first) {  // the second loop reads step[id]; a pair with contacts lowers a's and b's steps
-      read_later[id] = 1;
-      if (pair_cnt[p] > 0) read_later[a] = 1, read_later[b] = 1;
-    }
-    const double mt = (rb[39] < ra[39]) ? rb[39] : ra[39];
+  for (int p0 = blockIdx.x * blockDim.x; p0 < n_pairs; p0 += gridDim.x * blockDim.x) {  // block-uniform
+    const int p = p0 + threadIdx.x;
+    int key = -1;
     double v = 1e300;
-    if (pair_cnt[p] > 0 && !(first && sa)) {  // a static first pair's own use: see cluster_step_of
-      const double s = mt * scale[p];
-      v = (s < v) ? s : v;
+    if (p < n_pairs) {
+      const int k = cluster_of_pair[p], a = pairs[2 * p], b = pairs[2 * p + 1];
+      const double* ra = bodies + 40 * (size_t)a;
+      const double* rb = bodies + 40 * (size_t)b;
+      const bool sa = ra[38] != 0.0, sb = rb[38] != 0.0;
+      if (!(sa && sb)) {
+        const bool first = p == first_ns[k];
+        const int id = !sa ? a : b;
+        if (!first) {  // the second loop reads step[id]; a pair with contacts lowers a's and b's steps
+          read_later[id] = 1;
+          if (pair_cnt[p] > 0) read_later[a] = 1, read_later[b] = 1;
+        }
+        const double mt = (rb[39] < ra[39]) ? rb[39] : ra[39];
+        if (pair_cnt[p] > 0 && !(first && sa)) {  // a static first pair's own use: see cluster_step_of
+          const double s = mt * scale[p];
+          v = (s < v) ? s : v;
+        }
+        const double last = first ? ra[39] : bodies[40 * (size_t)id + 39];
+        v = (last < v) ? last : v;
+        key = k;
+      }
     }
-    const double last = first ? ra[39] : bodies[40 * (size_t)id + 39];
-    v = (last < v) ? last : v;
-    atomicMin(&step_bits[k], (unsigned long long)__double_as_longlong(v));
+    wave_key_min(key, (unsigned long long)__double_as_longlong(v), step_bits);
   }
 }
 struct ClusterFinal {
@@ -3468,10 +3504,10 @@ struct d2_ctx {
   std::vector<int> host_static;
   int n_items = 0;
   DBuf<int> bp_statics, bp_item_body, bp_item_seg, bp_item_cnt, bp_item_sorted, bp_item_off, bp_meta, bp_slot,
-      bp_rank, bp_counts, bp_start, bp_members, bp_red;
+      bp_rank, bp_counts, bp_start, bp_red;
   DBuf<long long> bp_item_pos;
   DBuf<unsigned long long> bp_keys, bp_fill;
-  DBuf<Box8> bp_box;
+  DBuf<Box8> bp_box, bp_members;
   DBuf<int2> bp_chunk;
   long long bp_cap = 0;
   int* host_red = nullptr;  // pinned: BR_N reductions + pair total
@@ -5412,15 +5448,16 @@ int d2_broad_phase(d2_ctx* c, int mode, double t, int64_t* n_pairs_out) {
     hipLaunchKernelGGL(k_bp_insert, dim3(g), dim3(256), 0, c->stream, n, c->bp_box.p, c->bp_meta.p, c->bp_red.p, T,
                        c->bp_keys.p, c->bp_counts.p, c->bp_slot.p, c->bp_rank.p);
     scan_host_n(c, c->bp_counts.p, c->bp_start.p, T, nullptr);
-    hipLaunchKernelGGL(k_bp_scatter, dim3(g), dim3(256), 0, c->stream, n, c->bp_meta.p, c->bp_slot.p, c->bp_rank.p,
-                       c->bp_start.p, c->bp_members.p);
+    hipLaunchKernelGGL(k_bp_scatter, dim3(g), dim3(256), 0, c->stream, n, c->bp_box.p, c->bp_meta.p, c->bp_slot.p,
+                       c->bp_rank.p, c->bp_start.p, c->bp_members.p);
     BpIn in;
     in.n = n, in.mode = mode, in.t = t, in.bodies = c->bodies.p, in.last = c->last_state.p, in.box = c->bp_box.p;
     in.R = c->bp_R.p, in.meta = c->bp_meta.p, in.statics = c->bp_statics.p, in.n_static = (int)c->host_static.size();
     in.red = c->bp_red.p, in.T = T, in.keys = c->bp_keys.p, in.counts = c->bp_counts.p, in.start = c->bp_start.p;
     in.members = c->bp_members.p;
     const int gi = (int)std::min<long long>((c->n_items + 3) / 4, (long long)c->cus * 16);
-    hipLaunchKernelGGL(k_bp_pairs, dim3(std::max(gi, 1)), dim3(256), 0, c->stream, in, c->n_items, c->bp_item_body.p,
+    const int gp = (int)std::min<long long>((c->n_items + 4 * BP_BATCH - 1) / (4 * BP_BATCH), (long long)c->cus * 16);
+    hipLaunchKernelGGL(k_bp_pairs, dim3(std::max(gp, 1)), dim3(256), 0, c->stream, in, c->n_items, c->bp_item_body.p,
                        c->bp_item_seg.p, c->bp_cap, c->bp_chunk.p, c->bp_fill.p, c->bp_item_cnt.p, c->bp_item_pos.p,
                        c->bp_item_sorted.p, c->bp_red.p);
     scan_host_n(c, c->bp_item_cnt.p, c->bp_item_off.p, c->n_items, c->bp_fill.p + 1);

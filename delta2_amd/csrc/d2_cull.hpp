@@ -396,4 +396,66 @@ D2_HD int cull_pair(const CullTri& A, const CullTri& B, float thr, bool want_hit
   return 1;
 }
 
+// ---------------------------------------------- the same classification in FP64
+// For the FP64 form's discrete levels (k_tri_full): world-space triangles as
+// the test itself takes them, the bounds of cull_pair, and a margin that
+// holds the float-barycentric acceptance bound (the reference's barycentrics
+// are float whatever the precision) and 1e-9 (1 m + |coords|), far above the
+// rounding of the FP64 expressions here and in the test.  0 certain miss, 1
+// needs the test, 2 certain hit (when want_hit).
+D2_HD double tri_extent64(const tri<double>& t, v3<double> n, double& hi) {
+  const double p0 = dot(t.a, n), p1 = dot(t.b, n), p2 = dot(t.c, n);
+  hi = p0 > p1 ? (p0 > p2 ? p0 : p2) : (p1 > p2 ? p1 : p2);
+  return p0 < p1 ? (p0 < p2 ? p0 : p2) : (p1 < p2 ? p1 : p2);
+}
+D2_HD bool tri_apart64(const tri<double>& a, const tri<double>& b, v3<double> n, double T2) {
+  double ahi, bhi;
+  const double alo = tri_extent64(a, n, ahi), blo = tri_extent64(b, n, bhi);
+  const double g = blo - ahi > alo - bhi ? blo - ahi : alo - bhi;
+  return g > 0.0 && g * g > T2 * dot(n, n);
+}
+D2_HD int cull_pair64(const tri<double>& a, const tri<double>& b, double thr, bool want_hit) {
+  double kappa = 0.0, L2 = 0.0, crd = 0.0;
+  v3<double> nn[2];
+  const tri<double>* T[2] = {&a, &b};
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const tri<double>& t = *T[k];
+    const v3<double> e0 = sub(t.b, t.a), e1 = sub(t.c, t.a), e2 = sub(t.c, t.b);
+    const double d00 = dot(e0, e0), d11 = dot(e1, e1), d01 = dot(e0, e1), d22 = dot(e2, e2);
+    const double den = d00 * d11 - d01 * d01;
+    if (!(den > 1e-4 * d00 * d11)) return 1;  // ill-conditioned barycentrics: no bound on what they accept
+    const double kp = d00 * d11 / den, l2 = d00 > d11 ? (d00 > d22 ? d00 : d22) : (d11 > d22 ? d11 : d22);
+    kappa = kp > kappa ? kp : kappa, L2 = l2 > L2 ? l2 : L2;
+    nn[k] = cross(e0, e1);
+    const v3<double> v[3] = {t.a, t.b, t.c};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) crd = fmax(crd, fmax(fabs(v[q].x), fmax(fabs(v[q].y), fabs(v[q].z))));
+  }
+  const double margin = 64.0 * 5.9604644775390625e-08 * kappa * sqrt(L2) + 1e-9 * (1.0 + crd);
+  const double R = thr + margin, R2 = R * R;
+  if (tri_apart64(a, b, nn[0], R2) || tri_apart64(a, b, nn[1], R2)) return 0;
+  const v3<double> cd = sub(add(add(b.a, b.b), b.c), add(add(a.a, a.b), a.c));
+  if (tri_apart64(a, b, cd, R2)) return 0;
+  if (!want_hit) return 1;
+  const v3<double> va[3] = {a.a, a.b, a.c}, vb[3] = {b.a, b.b, b.c};
+  double dd[3][3], ub = 1e300;
+#pragma unroll
+  for (int x = 0; x < 3; ++x)
+#pragma unroll
+    for (int y = 0; y < 3; ++y) {
+      const v3<double> t = sub(va[x], vb[y]);
+      dd[x][y] = dot(t, t);
+    }
+#pragma unroll
+  for (int x = 0; x < 3; ++x)
+#pragma unroll
+    for (int y = 0; y < 3; ++y) {
+      const int x1 = (x + 1) % 3, y1 = (y + 1) % 3;
+      ub = fmin(ub, fmax(fmax(dd[x][y], dd[x][y1]), fmax(dd[x1][y], dd[x1][y1])));
+    }
+  const double lim = thr - margin;
+  return lim > 0.0 && ub < lim * lim ? 2 : 1;
+}
+
 }  // namespace d2

@@ -1022,9 +1022,9 @@ __device__ __forceinline__ void write_children(const Dev& D, long long slot, con
   }
 }
 // The children of a node pair worth writing: all of them, or (pruning) those
-// nodes_apart does not prove contact-free.  offa/offb: the two trees' first
-// node records.
-template <bool F32>
+// spheres_apart_f32 does not prove contact-free (k_tri_mask runs at five
+// wavefronts per SIMD: the boxes' test, or FP64 poses, would spill there).
+// offa/offb: the two trees' first node records.
 __device__ __forceinline__ unsigned child_mask(const Dev& D, const NP& np, int desc, int offa, int offb) {
   const int nc = (desc >> 1) & 15;
   unsigned m = (1u << nc) - 1u;
@@ -1035,15 +1035,8 @@ __device__ __forceinline__ unsigned child_mask(const Dev& D, const NP& np, int d
   for (int c = 0; c < nc; ++c) {
     const size_t ga = (size_t)offa + (adv_a ? (uint32_t)(first + c) : np.na);
     const size_t gb = (size_t)offb + (adv_a ? np.nb : (uint32_t)(first + c));
-    const float* ba = D.nbound + NB_STRIDE * ga;
-    const float* bb = D.nbound + NB_STRIDE * gb;
-    // the FP32 form's mask kernel runs at five wavefronts per SIMD: the FP32
-    // sphere test only (the boxes' test, or FP64 poses, would spill there);
-    // elsewhere both FP64 tests
-    const bool apart = F32 ? spheres_apart_f32(pr + PR_TA1, pr + PR_TB1, ba, bb, pr[PR_SEARCH])
-                           : spheres_apart(pr + PR_TA1, pr + PR_TB1, ba, bb, pr[PR_SEARCH]) ||
-                                 nodes_apart(pr + PR_TA1, pr + PR_TB1, ba, bb, pr[PR_SEARCH]);
-    if (apart) m &= ~(1u << c);
+    if (spheres_apart_f32(pr + PR_TA1, pr + PR_TB1, D.nbound + NB_STRIDE * ga, D.nbound + NB_STRIDE * gb, pr[PR_SEARCH]))
+      m &= ~(1u << c);
   }
   return m;
 }
@@ -1165,7 +1158,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))
     const bool defer = D.defer && l_inner != 0;
     const int mine = defer && kept > 1 ? 1 : kept, mdef = kept - mine;
     const unsigned cmask =
-        lane < batch && (my_settled || my_keep != 0ull) ? child_mask<true>(D, l_np, l_desc, l_offa, l_offb) : 0u;
+        lane < batch && (my_settled || my_keep != 0ull) ? child_mask(D, l_np, l_desc, l_offa, l_offb) : 0u;
     const int nch = __popc(cmask);
     const int incl = wave_incl_scan(mine), ich = wave_incl_scan(nch), idf = wave_incl_scan(mdef);
     const int par = it & 1;
@@ -1322,34 +1315,93 @@ __global__ void __launch_bounds__(256) k_tri_def(Dev D) {
 }
 
 // FP64 discrete levels in one pass, with no item list (the reference's own
-// form: every triangle pair of a node pair tested in place,
+// form: the triangle pairs of a node pair tested in place,
 // full_tree_comparison.h:26-62 with bucketCompare, discrete_comparison.h).
-// A wavefront takes 64 node pairs at a time and packs their valid triangle
+// A wavefront takes G node pairs at a time and packs their valid triangle
 // pairs (n_a * n_b each) densely over its lanes: a prefix sum over the counts,
 // then each lane finds the node pair of its triangle pair by binary search
 // over the sums.  The FP64 test, the contact record and its emission key are
 // k_tri_dist's, so the contacts are the same bit for bit; hits set the node
 // pair's flag and expansion descriptor for k_disc_expand.
+//
+// G = 1 to 64 is the level's node pairs over the launch's wavefronts: with 64
+// always, a level of 20 000 node pairs ran on 320 of the chip's 2048 resident
+// wavefronts, each a chain of up to 64 tests.
+//
+// CULL (pruning on): FP64 bounds (cull_pair64) first classify every triangle
+// pair; certain misses are not tested, an inner node pair with a certain hit
+// is settled, and of the others an inner node pair's first kept pair is
+// tested before the rest, which run only while it has no hit (an inner node
+// pair only asks whether any pair hits).  The kept pairs of the G node pairs
+// are queued in LDS and tested 64 at a time.  311 bodies (1.6 M triangle pairs
+// in 7 levels): 2734 us of k_tri_full with G = 64 and every pair tested, 363
+// us now; what is left is the latency of a level's one or two tests in a row
+// (4300 instructions each) behind the loads.
+constexpr long long FULL_WAVES = 2048;  // wavefronts resident at its 253 VGPRs: two per SIMD
 struct FullSlot {
   int pair, ga, gb, ntb, excl, inner;
   long long w;
 };
+// The FP64 test of triangle pair (i, j) of slot o: its contact for leaf pairs.
+// Every lane of the wavefront calls it (active: has a pair).
+__device__ __forceinline__ bool full_test(Dev& D, const FullSlot& o, int i, int j, bool active) {
+  bool hit = false, emit = false;
+  v3<double> P{}, Q{};
+  double ea = 0.0, eb = 0.0;
+  if (active) {
+    const double* pr = D.pair_rec + (size_t)PR_STRIDE * o.pair;
+    const double* ba = D.buckets + (size_t)BUCKET * o.ga;
+    const double* bb = D.buckets + (size_t)BUCKET * o.gb;
+    const tri<double> A = xform(pr + PR_TA1, load_tri<double>(ba, i));
+    const tri<double> B = xform(pr + PR_TB1, load_tri<double>(bb, j));
+    const double d = tri_tri_dist(A, B, P, Q);
+    ea = ba[72 + i], eb = bb[72 + j];
+    hit = d < (pr[PR_SEARCH] + ea) + eb;
+    emit = hit && !o.inner;  // an inner node: the hit only expands the node pair
+  }
+  const long long slot = wave_alloc(emit, &D.cnt[C_CONTACTS]);
+  if (!emit) return hit;
+  if (slot >= D.cap_contacts) {
+    atomicOr(&D.cnt[C_OVERFLOW], 2ull);
+    return hit;
+  }
+  atomicAdd(&D.pair_cnt[o.pair], 1);
+  const NP np = D.soup[o.w];
+  const double* pr = D.pair_rec + (size_t)PR_STRIDE * o.pair;
+  const double* ba = D.buckets + (size_t)BUCKET * o.ga;
+  const double* bb = D.buckets + (size_t)BUCKET * o.gb;
+  ContactRec c;
+  c.key = make_key(D.level, 0, np.key, 8 * i + j);
+  c.pair = (int32_t)np.pair, c.na = (int32_t)np.na, c.nb = (int32_t)np.nb, c.kind = 0;
+  c.ia = i, c.ib = j, c.level = D.level, c.pad = 0;
+  c.r[0] = P.x, c.r[1] = P.y, c.r[2] = P.z, c.r[3] = Q.x, c.r[4] = Q.y, c.r[5] = Q.z;
+  c.r[6] = pr[PR_GEOA] + ea, c.r[7] = pr[PR_GEOB] + eb, c.r[8] = ba[80 + i], c.r[9] = bb[80 + j], c.r[10] = 0.0;
+  D.contacts[slot] = c;
+  return hit;
+}
+template <bool CULL>
 __global__ void __launch_bounds__(256) k_tri_full(Dev D) {
   __shared__ FullSlot s_np[4][64];
   __shared__ int s_hit[4][64];
+  __shared__ unsigned long long s_keep[CULL ? 4 : 1][64];  // kept triangle pairs of each node pair (bit 8 i + j)
+  __shared__ uint16_t s_q[CULL ? 4 : 1][4096];             // queued tests: slot << 6 | 8 i + j
   __shared__ unsigned long long s_tested;
   const int lane = lane_id(), wid = threadIdx.x >> 6;
   const long long n = D.n_soup();
-  const long long n_groups = (n + 63) / 64;
   const long long nwaves = (long long)gridDim.x * (blockDim.x >> 6);
+  const long long spread = nwaves < FULL_WAVES ? nwaves : FULL_WAVES;
+  const long long per = (n + spread - 1) / spread;
+  const int G = (int)(per < 1 ? 1 : per > 64 ? 64 : per);
+  const long long n_groups = (n + G - 1) / G;
   if (threadIdx.x == 0) s_tested = 0ull;
   __syncthreads();
   unsigned long long tested = 0ull;  // kept by lane 0
   for (long long g = (long long)blockIdx.x * (blockDim.x >> 6) + wid; g < n_groups; g += nwaves) {
-    const long long w = g * 64 + lane;
+    const long long w = g * G + lane;
+    const bool mine = lane < G && w < n;
     int cnt = 0, desc = 0;
     FullSlot f{0, 0, 0, 1, 0, 0, w};
-    if (w < n) {
+    if (mine) {
       const NP np = D.soup[w];
       // a child of a parent that did not hit: no work, no children
       const int32_t* pi = D.pair_info + 4 * np.pair;
@@ -1371,8 +1423,8 @@ __global__ void __launch_bounds__(256) k_tri_full(Dev D) {
     f.excl = incl - cnt;
     s_np[wid][lane] = f;
     s_hit[wid][lane] = 0;
+    if (CULL) s_keep[wid][lane] = 0ull;
     const int total = rl(incl, 63);
-    tested += (unsigned long long)total;
     wave_sync_lds();
     for (int t0 = 0; t0 < total; t0 += 64) {
       const int t = t0 + lane;
@@ -1382,46 +1434,46 @@ __global__ void __launch_bounds__(256) k_tri_full(Dev D) {
 #pragma unroll
       for (int step = 32; step > 0; step >>= 1)
         if (__shfl(incl, k + step - 1) <= t) k += step;
-      bool hit = false, emit = false;
-      int i = 0, j = 0;
-      v3<double> P{}, Q{};
-      double ea = 0.0, eb = 0.0;
+      k = k < 63 ? k : 63;
       const FullSlot& o = s_np[wid][k];
-      if (t < total) {
-        const int s = t - o.excl;
-        i = s / o.ntb, j = s - i * o.ntb;
+      const int s = t - o.excl, i = s / o.ntb, j = s - i * o.ntb;
+      if (!CULL) {
+        if (full_test(D, o, i, j, t < total)) s_hit[wid][k] = 1;
+      } else if (t < total) {
         const double* pr = D.pair_rec + (size_t)PR_STRIDE * o.pair;
         const double* ba = D.buckets + (size_t)BUCKET * o.ga;
         const double* bb = D.buckets + (size_t)BUCKET * o.gb;
         const tri<double> A = xform(pr + PR_TA1, load_tri<double>(ba, i));
         const tri<double> B = xform(pr + PR_TB1, load_tri<double>(bb, j));
-        const double d = tri_tri_dist(A, B, P, Q);
-        ea = ba[72 + i], eb = bb[72 + j];
-        hit = d < (pr[PR_SEARCH] + ea) + eb;
-        if (hit) s_hit[wid][k] = 1;
-        emit = hit && !o.inner;  // an inner node: the hit only expands the node pair
+        const int cls = cull_pair64(A, B, (pr[PR_SEARCH] + ba[72 + i]) + bb[72 + j], o.inner != 0);
+        if (cls == 2) s_hit[wid][k] = 1;
+        else if (cls == 1) atomicOr(&s_keep[wid][k], 1ull << (8 * i + j));
       }
-      const long long slot = wave_alloc(emit, &D.cnt[C_CONTACTS]);
-      if (!emit) continue;
-      if (slot >= D.cap_contacts) {
-        atomicOr(&D.cnt[C_OVERFLOW], 2ull);
-        continue;
-      }
-      atomicAdd(&D.pair_cnt[o.pair], 1);
-      const NP np = D.soup[o.w];
-      const double* pr = D.pair_rec + (size_t)PR_STRIDE * o.pair;
-      const double* ba = D.buckets + (size_t)BUCKET * o.ga;
-      const double* bb = D.buckets + (size_t)BUCKET * o.gb;
-      ContactRec c;
-      c.key = make_key(D.level, 0, np.key, 8 * i + j);
-      c.pair = (int32_t)np.pair, c.na = (int32_t)np.na, c.nb = (int32_t)np.nb, c.kind = 0;
-      c.ia = i, c.ib = j, c.level = D.level, c.pad = 0;
-      c.r[0] = P.x, c.r[1] = P.y, c.r[2] = P.z, c.r[3] = Q.x, c.r[4] = Q.y, c.r[5] = Q.z;
-      c.r[6] = pr[PR_GEOA] + ea, c.r[7] = pr[PR_GEOB] + eb, c.r[8] = ba[80 + i], c.r[9] = bb[80 + j], c.r[10] = 0.0;
-      D.contacts[slot] = c;
     }
+    if (!CULL) tested += (unsigned long long)total;
     wave_sync_lds();
-    if (w < n) {
+    if (CULL) {
+      // two rounds: leaf pairs' tests and one of each unsettled inner node
+      // pair, then the other tests of the inner node pairs without a hit
+      for (int round = 0; round < 2; ++round) {
+        unsigned long long m = s_hit[wid][lane] ? 0ull : s_keep[wid][lane];
+        if (f.inner) m = round == 0 ? (m & (~m + 1ull)) : (m & (m - 1ull));
+        else if (round == 1) m = 0ull;
+        const int c = __popcll(m), qi = wave_incl_scan(c), nq = rl(qi, 63);
+        for (int at = qi - c; m; m &= m - 1ull) s_q[wid][at++] = (uint16_t)(lane << 6 | (__ffsll((long long)m) - 1));
+        wave_sync_lds();
+        for (int q0 = 0; q0 < nq; q0 += 64) {
+          const bool act = q0 + lane < nq;
+          const int e = s_q[wid][act ? q0 + lane : 0], k = e >> 6;
+          const bool need = act && !(round == 1 && s_hit[wid][k]);
+          if (full_test(D, s_np[wid][k], (e >> 3) & 7, e & 7, need)) s_hit[wid][k] = 1;
+          tested += (unsigned long long)__popcll(__ballot(need));
+          wave_sync_lds();
+        }
+        wave_sync_lds();
+      }
+    }
+    if (mine) {
       const int h = s_hit[wid][lane];
       D.np_hit[w] = h;
       if (h) D.exp_desc[w] = desc;
@@ -1714,26 +1766,40 @@ __global__ void __launch_bounds__(256) k_level_write(Dev D) {
 
 // FP64-mode discrete levels: the children of every hit node pair (from its
 // expansion descriptor) to the next list, one atomic per block and round.
+// Eight lanes per node pair, one per child: each tests its own child's bounds
+// and writes it (18.1 us a launch when one lane walked a node pair's children,
+// 8.7 us now, on levels of up to 20 000 node pairs).
 __global__ void __launch_bounds__(256) k_disc_expand(Dev D) {
   __shared__ int s_tot[4];
   __shared__ unsigned long long s_base;
   const long long n = D.n_soup();
   const int lane = lane_id(), wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long b0 = (long long)blockIdx.x * blockDim.x; b0 < n; b0 += stride) {  // block-uniform
-    const long long w = b0 + threadIdx.x;
-    int desc = 0, nc = 0;
-    unsigned cmask = 0u;
-    NP np{};
+  const int c = lane & 7;
+  const long long stride = (long long)gridDim.x * (blockDim.x >> 3);
+  for (long long b0 = (long long)blockIdx.x * (blockDim.x >> 3); b0 < n; b0 += stride) {  // block-uniform
+    const long long w = b0 + (threadIdx.x >> 3);
+    NP child{};
+    bool keep = false;
     if (w < n && D.np_hit[w]) {
-      desc = D.exp_desc[w];
-      np = D.soup[w];
-      const int32_t* pi = D.pair_info + 4 * np.pair;
-      cmask = child_mask<false>(D, np, desc, pi[2], pi[3]);
-      nc = __popc(cmask);
+      const int desc = D.exp_desc[w];
+      const NP np = D.soup[w];
+      if (c < ((desc >> 1) & 15)) {
+        const bool adv_a = desc & 1;
+        const uint32_t id = (uint32_t)((desc >> 5) + c);
+        child = NP{np.pair, adv_a ? id : np.na, adv_a ? np.nb : id, 0u, np.key * 8ull + (unsigned long long)c};
+        keep = true;
+        if (D.prune) {
+          const int32_t* pi = D.pair_info + 4 * np.pair;
+          const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
+          const float* ba = D.nbound + NB_STRIDE * ((size_t)pi[2] + child.na);
+          const float* bb = D.nbound + NB_STRIDE * ((size_t)pi[3] + child.nb);
+          keep = !(spheres_apart(pr + PR_TA1, pr + PR_TB1, ba, bb, pr[PR_SEARCH]) ||
+                   nodes_apart(pr + PR_TA1, pr + PR_TB1, ba, bb, pr[PR_SEARCH]));
+        }
+      }
     }
-    const int incl = wave_incl_scan(nc);
-    if (lane == 63) s_tot[wid] = incl;
+    const unsigned long long m = __ballot(keep);
+    if (lane == 0) s_tot[wid] = __popcll(m);
     __syncthreads();
     if (threadIdx.x == 0) {
       int tot = 0;
@@ -1746,10 +1812,10 @@ __global__ void __launch_bounds__(256) k_disc_expand(Dev D) {
       s_base = base;
     }
     __syncthreads();
-    long long slot = (long long)s_base + incl - nc;
+    long long slot = (long long)s_base + __popcll(m & lanes_below());
     for (int v = 0; v < wid; ++v) slot += s_tot[v];
+    if (keep && slot < D.cap_np) D.soup_next[slot] = child;
     __syncthreads();  // s_tot and s_base are rewritten by the next round
-    if (nc > 0) write_children(D, slot, np, desc, 0u, cmask);
   }
 }
 
@@ -3918,8 +3984,9 @@ void enqueue_level(d2_ctx* c, int level, int discrete) {
     timed_launch(c, K_TRI_MASK, k_tri_mask, dim3(cg), dim3(256), D);
     timed_launch(c, K_TRI_DIST, k_tri_dist, dim3(sg), dim3(256), D);
     if (D.defer) timed_launch(c, K_TRI_DEF, k_tri_def, dim3(G.def), dim3(256), D);
-  } else if (discrete) {  // one wavefront per 64 node pairs
-    timed_launch(c, K_TRI_FULL, k_tri_full, dim3(eg), dim3(256), D);
+  } else if (discrete) {  // as many wavefronts as there are node pairs, up to the tuned blocks
+    if (D.prune) timed_launch(c, K_TRI_FULL, k_tri_full<true>, dim3(cg), dim3(256), D);
+    else timed_launch(c, K_TRI_FULL, k_tri_full<false>, dim3(cg), dim3(256), D);
   } else {
     timed_launch(c, K_SOUP_CULL, k_soup_cull, dim3(cg), dim3(256), D);
     if (D.fp32) timed_launch(c, K_SOUP_KEEP, k_soup_keep, dim3(sg), dim3(256), D);  // FP32 culls + survivor lists
@@ -3928,7 +3995,7 @@ void enqueue_level(d2_ctx* c, int level, int discrete) {
   }
   if (discrete && c->precision != D2_FP32) {
     Timer tm(c, K_EXPAND, 0.0);
-    hipLaunchKernelGGL(k_disc_expand, dim3(eg), dim3(256), 0, c->stream, D);
+    hipLaunchKernelGGL(k_disc_expand, dim3(cg), dim3(256), 0, c->stream, D);
   } else if (!discrete) {  // FP32 discrete levels are expanded by k_tri_mask
     Timer tm(c, K_EXPAND, 0.0);
     hipLaunchKernelGGL(k_level_count, dim3(eg), dim3(256), 0, c->stream, D);

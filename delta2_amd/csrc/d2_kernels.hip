@@ -2150,7 +2150,7 @@ __global__ void __launch_bounds__(256) k_step_rule(const unsigned long long* cnt
 }
 
 // Contacts a pair may have for the LDS passes of the post-processing: the
-// second pass (one 256-thread block per CU, 142 KB of LDS) takes pairs up to
+// second pass (one 1024-thread block per CU, 143 KB of LDS) takes pairs up to
 // POST_CAP_LARGE; above it a pair takes one block with global scratch.
 constexpr int POST_CAP_LARGE = 2048;
 struct LdsKey {
@@ -2160,6 +2160,72 @@ __device__ __forceinline__ bool lds_less(const LdsKey& x, const LdsKey& y) {
   if (x.eps == y.eps) return x.dist < y.dist;
   return x.eps < y.eps;
 }
+// r + (y < x) by one borrow chain (the rank loops: a pair of 64-bit compares
+// with their mask arithmetic takes three times as long).
+__device__ __forceinline__ int add_less(int r, unsigned long long y, unsigned long long x) {
+  unsigned t;
+  asm("v_sub_co_u32 %1, vcc, %2, %3\n\t"
+      "v_subb_co_u32 %1, vcc, %4, %5, vcc\n\t"
+      "v_addc_co_u32 %0, vcc, 0, %0, vcc"
+      : "+v"(r), "=&v"(t)
+      : "v"((unsigned)y), "v"((unsigned)x), "v"((unsigned)(y >> 32)), "v"((unsigned)(x >> 32))
+      : "vcc");
+  return r;
+}
+__device__ __forceinline__ int add_less(int r, unsigned long long yh, unsigned long long yl, unsigned long long xh,
+                                        unsigned long long xl) {
+  unsigned t;
+  asm("v_sub_co_u32 %1, vcc, %2, %3\n\t"
+      "v_subb_co_u32 %1, vcc, %4, %5, vcc\n\t"
+      "v_subb_co_u32 %1, vcc, %6, %7, vcc\n\t"
+      "v_subb_co_u32 %1, vcc, %8, %9, vcc\n\t"
+      "v_addc_co_u32 %0, vcc, 0, %0, vcc"
+      : "+v"(r), "=&v"(t)
+      : "v"((unsigned)yl), "v"((unsigned)xl), "v"((unsigned)(yl >> 32)), "v"((unsigned)(xl >> 32)), "v"((unsigned)yh),
+        "v"((unsigned)xh), "v"((unsigned)(yh >> 32)), "v"((unsigned)(xh >> 32))
+      : "vcc");
+  return r;
+}
+// rk[i] = how many of n keys (W 64-bit words each, high word first, at kb in
+// LDS) are less than key i.  Wavefront w of NW counts over its share of the
+// keys for every i, 128 of them at a time, and the shares meet in rk by LDS
+// atomics; the loads of eight keys are in flight together (one key per thread
+// against all the others in turn waited out the LDS latency every four keys:
+// 17 us for the (eps, dist) ranks of 318 contacts, 9.6 us now).  All threads
+// call it; ends with a barrier.
+template <int W, int NW>
+__device__ __forceinline__ void block_ranks(int n, const unsigned long long* kb, int* rk, int w) {
+  const int lane = lane_id();
+  for (int i = threadIdx.x; i < n; i += 64 * NW) rk[i] = 0;
+  __syncthreads();
+  const int j0 = n * w / NW, j1 = n * (w + 1) / NW;
+  for (int b = 0; b < n; b += 128) {
+    const int i0 = b + lane, i1 = i0 + 64;
+    unsigned long long x0[W], x1[W];
+#pragma unroll
+    for (int q = 0; q < W; ++q) x0[q] = kb[W * (i0 < n ? i0 : 0) + q], x1[q] = kb[W * (i1 < n ? i1 : 0) + q];
+    int r0 = 0, r1 = 0, j = j0;
+    for (; j + 8 <= j1; j += 8) {
+      unsigned long long y[8 * W];
+#pragma unroll
+      for (int q = 0; q < 8 * W; ++q) y[q] = kb[W * j + q];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        if (W == 1) r0 = add_less(r0, y[q], x0[0]), r1 = add_less(r1, y[q], x1[0]);
+        else r0 = add_less(r0, y[W * q], y[W * q + W - 1], x0[0], x0[W - 1]),
+             r1 = add_less(r1, y[W * q], y[W * q + W - 1], x1[0], x1[W - 1]);
+      }
+    }
+    for (; j < j1; ++j) {
+      if (W == 1) r0 = add_less(r0, kb[j], x0[0]), r1 = add_less(r1, kb[j], x1[0]);
+      else r0 = add_less(r0, kb[W * j], kb[W * j + W - 1], x0[0], x0[W - 1]),
+           r1 = add_less(r1, kb[W * j], kb[W * j + W - 1], x1[0], x1[W - 1]);
+    }
+    if (i0 < n && r0) atomicAdd(&rk[i0], r0);
+    if (i1 < n && r1) atomicAdd(&rk[i1], r1);
+  }
+  __syncthreads();
+}
 // The same permutation computed by the whole wavefront.  Each Hoare partition
 // of [lo, hi) around the pivot at lo-1 is derived from ranks: with A_k the k-th
 // position from the left holding an element not less than the pivot and B_k
@@ -2168,39 +2234,47 @@ __device__ __forceinline__ bool lds_less(const LdsKey& x, const LdsKey& y) {
 // K = #{k : A_k < B_k}, and returns min(A_K, B_{K-1}).  The closing insertion
 // sort never moves an element across a leaf segment's border, so it equals a
 // stable sort of every leaf segment; heapsort (depth exhausted) stays on lane 0.
-__device__ int wave_partition(int lo, int hi, int* ord, const int* rk, int* Apos, int* Bpos) {
+// One pass finds both lists (Bpos is filled from the left: B_k is its k-th
+// entry from the end), four chunks' keys in flight at a time.
+__device__ __forceinline__ int wave_partition(int lo, int hi, int* ord, const int* rk, int* Apos, int* Bpos) {
   const int lane = lane_id();
   const int P = rk[ord[lo - 1]];
   int nA = 0, nB = 0;
-  for (int base = lo; base < hi; base += 64) {
-    const int i = base + lane;
-    const bool ge = i < hi && !(rk[ord[i]] < P);
-    const unsigned long long m = __ballot(ge);
-    if (ge) Apos[nA + __popcll(m & lanes_below())] = i;
-    nA += __popcll(m);
-  }
-  for (int top = hi - 1; top >= lo - 1; top -= 64) {
-    const int i = top - lane;
-    const bool le = i >= lo - 1 && !(P < rk[ord[i]]);
-    const unsigned long long m = __ballot(le);
-    if (le) Bpos[nB + __popcll(m & lanes_below())] = i;
-    nB += __popcll(m);
+  for (int base = lo - 1; base < hi; base += 256) {
+    int key[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = base + 64 * q + lane;
+      key[q] = ord[i < hi ? i : lo - 1];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) key[q] = rk[key[q]];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = base + 64 * q + lane;
+      const bool ge = i >= lo && i < hi && !(key[q] < P), le = i < hi && !(P < key[q]);
+      const unsigned long long ma = __ballot(ge), mb = __ballot(le);
+      if (ge) Apos[nA + __popcll(ma & lanes_below())] = i;
+      if (le) Bpos[nB + __popcll(mb & lanes_below())] = i;
+      nA += __popcll(ma), nB += __popcll(mb);
+    }
   }
   wave_sync_lds();
   const int lim = nA < nB ? nA : nB;
   int K = 0;
   for (int base = 0; base < lim; base += 64) {  // A_k < B_k holds for a prefix of k
     const int q = base + lane;
-    const unsigned long long m = __ballot(q < lim && Apos[q] < Bpos[q]);
+    const unsigned long long m = __ballot(q < lim && Apos[q] < Bpos[nB - 1 - q]);
     K += __popcll(m);
     if (m != ~0ull) break;
   }
   const int ak = K < nA ? Apos[K] : hi;
-  const int bk1 = K > 0 ? Bpos[K - 1] : hi;
+  const int bk1 = K > 0 ? Bpos[nB - K] : hi;
   for (int q = lane; q < K; q += 64) {  // the swapped positions are pairwise distinct
-    const int x = ord[Apos[q]], y = ord[Bpos[q]];
-    ord[Apos[q]] = y;
-    ord[Bpos[q]] = x;
+    const int pa = Apos[q], pb = Bpos[nB - 1 - q];
+    const int x = ord[pa], y = ord[pb];
+    ord[pa] = y;
+    ord[pb] = x;
   }
   wave_sync_lds();
   return ak < bk1 ? ak : bk1;
@@ -2214,14 +2288,87 @@ constexpr int BLK_CAP = 512;
 // queued segments per round (> 16 elements each: at most CAP / 17), 3 ints each
 constexpr int blk_segs(int cap) { return 3 * (cap / 17 + 1); }
 
+// The greedy filter's decisions for one group of up to 64 candidates in
+// order: a candidate is kept unless it is near a contact kept before the
+// group (near_m, one word per wavefront) or a kept candidate before it.
+// strike: per candidate, the later ones near it; each kept candidate takes
+// them out, so the loop runs once per kept candidate.  One wavefront.
+template <int NW>
+__device__ __forceinline__ unsigned long long greedy_keep(int m, const unsigned long long* strike,
+                                                          const unsigned long long* near_m) {
+  const unsigned long long mine = strike[lane_id()];
+  unsigned long long blocked = 0ull;
+#pragma unroll
+  for (int k = 0; k < NW; ++k) blocked |= near_m[k];
+  const unsigned long long b0 = readlane_u64(blocked, 0);
+  unsigned long long open = (m < 64 ? (1ull << m) - 1ull : ~0ull) & ~b0, kept = 0ull;
+  while (open) {
+    const int u = __ffsll((long long)open) - 1;
+    kept |= 1ull << u;
+    open &= ~(readlane_u64(mine, u) | (1ull << u));
+  }
+  return kept;
+}
+
+// near_mid for a group of candidates (one per lane, the same in every
+// wavefront) against points held by the lanes, FP32 first: coordinates are
+// taken relative to an origin among the contacts, each is off by at most 4 u
+// cmax (u = 2^-24, cmax the largest of them), so a distance more than err =
+// 16 u cmax + 1e-6 search away from the search distance is decided, and only
+// the others run the FP64 test (25 FP64 instructions per test were most of
+// the greedy pass).  Distances that FP32 cannot hold, and negative or infinite
+// search distances, always run it.
+struct NearTest {
+  double mx, my, mz, search;
+  float fx, fy, fz, lo2, hi2;
+  bool exact;
+};
+__device__ __forceinline__ NearTest near_test(double mx, double my, double mz, double search, const double* org,
+                                              float cmax) {
+  NearTest t{mx, my, mz, search, (float)(mx - org[0]), (float)(my - org[1]), (float)(mz - org[2]), -1.f, 0.f, false};
+  const float s = (float)search, err = 16.f * 5.9604645e-08f * cmax + 1e-6f * s;
+  const float lo = s - err, hi = s + err;
+  t.lo2 = lo > 0.f ? lo * lo * (1.f - 1e-6f) : -1.f, t.hi2 = hi * hi * (1.f + 1e-6f);
+  t.exact = __ballot(!(search >= 0.0 && search < 1e15 && cmax < 1e15f)) != 0ull;
+  return t;
+}
+__device__ __forceinline__ float rlf(float v, int l) { return __int_as_float(rl(__float_as_int(v), l)); }
+// Candidate against the points lanes u, u + step, ... (four of them, below
+// lim) hold (h doubles, g floats): bit q set when near the q-th.  want: the
+// lanes that need an answer.  One branch for the four.  All lanes call it.
+__device__ __forceinline__ unsigned near_at4(const NearTest& t, int u, int step, int lim, double hx, double hy, double hz,
+                                             float gx, float gy, float gz, bool want) {
+  unsigned near = 0u, open = 0u;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int v = u + q * step, l = v < lim ? v : u;
+    const float dx = t.fx - rlf(gx, l), dy = t.fy - rlf(gy, l), dz = t.fz - rlf(gz, l);
+    const float s2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    const bool in = v < lim;
+    near |= (in && s2 < t.lo2) ? 1u << q : 0u;
+    open |= (in && !(s2 >= t.hi2)) ? 1u << q : 0u;
+  }
+  if (t.exact || __ballot(want && (open & ~near)) != 0ull) {
+#pragma unroll 1
+    for (int q = 0; q < 4; ++q) {
+      const int l = u + q * step;
+      if (l >= lim) break;
+      const bool r =
+          near_mid(v3<double>{t.mx - readlane_d(hx, l), t.my - readlane_d(hy, l), t.mz - readlane_d(hz, l)}, t.search);
+      near = (near & ~(1u << q)) | (r ? 1u << q : 0u);
+    }
+  }
+  return near;
+}
+
 // ord[0, n) := the order std::sort gives, with the
 // partitions of one round's segments spread over the block's wavefronts:
 // partitions of disjoint segments commute, and every segment keeps its own
 // depth budget, so the order equals the sequential introsort's.  Apos/Bpos
 // are indexed by position (a segment's lists stay inside its range).
-__device__ void block_std_sort(int n, int* ord, const int* rk, int* Apos, int* Bpos, int* mark, int* segs,
+__device__ __forceinline__ void block_std_sort(int n, int* ord, const int* rk, int* Apos, int* Bpos, int* mark, int* segs,
                                int* s_cnt, int seg_stride) {
-  const int tid = threadIdx.x, w = tid >> 6, lane = lane_id();
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = lane_id();
   for (int i = tid; i < n; i += blockDim.x) mark[i] = 0;
   if (tid == 0) {  // thread 0 also zeroed mark[0] above
     s_cnt[0] = 0, s_cnt[1] = 0;
@@ -2283,19 +2430,30 @@ __device__ void block_std_sort(int n, int* ord, const int* rk, int* Apos, int* B
     cur ^= 1;
     __syncthreads();
   }
-  // leaf segments tile [0, n): stable-sort each (<= 16 elements)
+  // leaf segments tile [0, n): stable-sort each (<= 16 elements).  A
+  // position's segment comes from the marks within 16 places, all read at
+  // once, and the segment's keys likewise (walking them one by one cost a LDS
+  // round trip each).
+  for (int j = tid; j < n; j += blockDim.x) Apos[j] = rk[ord[j]];
+  __syncthreads();
   for (int j = tid; j < n; j += blockDim.x) {
-    int f = j;
-    while (mark[f] == 0) --f;
+    unsigned back = 0u, ahead = 0u;  // bit q: a segment starts at j - q, at j + 1 + q
+    int kind = 0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int mb = j >= q ? mark[j - q] : 0, ma = j + 1 + q < n ? mark[j + 1 + q] : 1;
+      if (mb && back == 0u) kind = mb;
+      back |= mb ? 1u << q : 0u, ahead |= ma ? 1u << q : 0u;
+    }
     int dst = j;
-    if (mark[f] == 1) {
-      int l = j + 1;
-      while (l < n && mark[l] == 0) ++l;
-      const int kj = rk[ord[j]];
+    if (kind == 1) {  // (0: inside a long heap-sorted segment, 2: at its start)
+      const int f = j - (__ffs((int)back) - 1), l = j + (ahead ? __ffs((int)ahead) : 17);
+      const int kj = Apos[j];
       int r = 0;
-      for (int i = f; i < l; ++i) {
-        const int ki = rk[ord[i]];
-        r += ki < kj || (i < j && !(kj < ki));
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int i = f + q, ki = Apos[i < n ? i : n - 1];
+        r += i < l && (ki < kj || (i < j && !(kj < ki))) ? 1 : 0;
       }
       dst = f + r;
     }
@@ -2306,14 +2464,21 @@ __device__ void block_std_sort(int n, int* ord, const int* rk, int* Apos, int* B
   __syncthreads();
 }
 
-// Post-processing of one pair per 256-thread block: orders by rank counting instead of sorting
+// Post-processing of one pair per block: orders by rank counting instead of sorting
 // networks (emission keys are unique; (eps, dist) ranks equal exactly for tied
 // keys), the tie replay over the block's wavefronts, and the greedy pass of
 // filterContacts 64 candidates at a time with the distance tests spread over
-// the wavefronts and the decisions taken in order by the first one.
+// the wavefronts and the decisions taken in order by the first one.  A serial
+// chain bounds it (the replay of the ties, then the greedy groups in order),
+// so a block's size is what its LDS leaves room for: 256 threads up to 512
+// contacts (four blocks a CU), 1024 up to 2048 (143 KB, one block a CU; with
+// 256 the other three SIMD slots stood empty).  One pair of 701 contacts: 350
+// us with 256 threads, FP64 near tests and the sort's ranks a key per thread,
+// 108 us now; a scene of 4,096 bodies (pairs of up to 318): 149 -> 84 us; a
+// pile in a funnel: 2595 + 1629 -> 1488 + 436 us.
 // A pair above every LDS capacity without the filter (mode 0 or 2), one block:
 // the emission order by rank counting (the keys are unique; each thread ranks
-// up to 8 x 256 contacts at a time against key tiles of CAP staged in LDS),
+// up to 8 per thread at a time against key tiles of CAP staged in LDS),
 // written to perm from a copy of the pair's contact indices in keep (unused
 // by these modes); in mode 2 the step rule's minimum over the block.
 template <int CAP>
@@ -2385,11 +2550,11 @@ struct HugeScratch {
 // (block_std_sort) on global scratch when keys tie, then the greedy pass 64
 // candidates at a time as in the LDS path, with the kept list in scratch.
 // Returns the kept count (every thread).
-template <int CAP>
+template <int CAP, int NT>
 __device__ int pair_filter_huge(int p, const ContactRec* c, const int* pair_off, int* perm, int* keep, int* kept_cnt,
                                 double margin, const HugeScratch& H, unsigned long long* skey, LdsKey* sk,
-                                int* s_misc, unsigned long long (*conf_w)[64], int (*near_w)[64]) {
-  const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+                                int* s_misc, unsigned long long* strike, unsigned long long* near_m) {
+  const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = pair_off[p], n = pair_off[p + 1] - b;
   pair_finish_huge<CAP>(p, c, pair_off, perm, 0, keep, nullptr, nullptr, skey, nullptr);  // perm: emission order
   if (tid == 0) s_misc[0] = 0;
@@ -2463,28 +2628,21 @@ __device__ int pair_filter_huge(int p, const ContactRec* c, const int* pair_off,
       const v3<double> hm =
           dvs(add(v3<double>{hc.r[0], hc.r[1], hc.r[2]}, v3<double>{hc.r[3], hc.r[4], hc.r[5]}), 2.0);
       const int mm = nk - q0 < 64 ? nk - q0 : 64;
-      for (int u = w; u < mm; u += 4) {
+      for (int u = w; u < mm; u += NT / 64) {
         const v3<double> dd{mx - readlane_d(hm.x, u), my - readlane_d(hm.y, u), mz - readlane_d(hm.z, u)};
         near = near || near_mid(dd, search);
       }
     }
-    unsigned long long conf = 0;  // bit u: candidate u (< this one) of the group is near
-    for (int u = w; u < m; u += 4) {
+    for (int u = w; u < m; u += NT / 64) {  // the later candidates of the group near candidate u
       const v3<double> dd{mx - readlane_d(mx, u), my - readlane_d(my, u), mz - readlane_d(mz, u)};
-      if (u < lane && near_mid(dd, search)) conf |= 1ull << u;
+      const unsigned long long later = __ballot(lane > u && near_mid(dd, search));
+      if (lane == 0) strike[u] = later;
     }
-    near_w[w][lane] = near ? 1 : 0;
-    conf_w[w][lane] = conf;
+    const unsigned long long nm = __ballot(near);
+    if (lane == 0) near_m[w] = nm;
     __syncthreads();
     if (w == 0) {
-      const bool nr = (near_w[0][lane] | near_w[1][lane] | near_w[2][lane] | near_w[3][lane]) != 0;
-      const unsigned long long cf = conf_w[0][lane] | conf_w[1][lane] | conf_w[2][lane] | conf_w[3][lane];
-      const unsigned long long blocked = __ballot(nr);
-      unsigned long long kept = 0;
-      for (int i = 0; i < m; ++i) {
-        const unsigned long long ci = readlane_u64(cf, i);
-        if (!((blocked >> i) & 1ull) && !(ci & kept)) kept |= 1ull << i;
-      }
+      const unsigned long long kept = greedy_keep<NT / 64>(m, strike, near_m);
       const bool fresh = (kept >> lane) & 1ull;
       if (valid) keep[b + t] = fresh ? 1 : 0;
       if (fresh) kl[nk + __popcll(kept & lanes_below())] = ord[t];
@@ -2502,8 +2660,8 @@ __device__ int pair_filter_huge(int p, const ContactRec* c, const int* pair_off,
 // CAP = BLK_CAP: every pair (list null); pairs above CAP go to `over` (up to
 // POST_CAP_LARGE contacts) or `huge`.  CAP = POST_CAP_LARGE: the pairs of
 // `list`, then the pairs of `tail` one block each (above every LDS capacity).
-template <int CAP>
-__global__ void __launch_bounds__(256) k_pair_finish_block(int n_pairs, const int* list, const int* n_list,
+template <int CAP, int NT>
+__global__ void __launch_bounds__(NT) k_pair_finish_block(int n_pairs, const int* list, const int* n_list,
                                                            const ContactRec* c, const int* pair_off, int* perm,
                                                            int mode, int* keep, int* kept_cnt,
                                                            const double* pair_rec, double* scale, int* over,
@@ -2520,11 +2678,13 @@ __global__ void __launch_bounds__(256) k_pair_finish_block(int n_pairs, const in
   __shared__ int ord[CAP];
   __shared__ int mark[CAP];  // leaf marks of the tie replay, then the kept list
   __shared__ int segs[2 * SEGS];
-  __shared__ unsigned long long conf_w[4][64];
-  __shared__ int near_w[4][64];
-  __shared__ double s_min[4];
+  __shared__ unsigned long long strike[64];
+  __shared__ unsigned long long near_m[NT / 64];
+  __shared__ double s_min[NT / 64];
+  __shared__ float s_cmax[NT / 64];
   __shared__ int s_misc[4];
-  const int tid = threadIdx.x, w = tid >> 6, lane = lane_id();
+  const int tid = threadIdx.x, lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // visibly uniform: scalar loops and lane indexes
   const int n_items = list ? *n_list : n_pairs;
   unsigned long long kept_sum = 0;  // (thread 0) the filter's kept contacts of this block's pairs
   for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
@@ -2544,21 +2704,20 @@ __global__ void __launch_bounds__(256) k_pair_finish_block(int n_pairs, const in
       }
       continue;
     }
-    for (int i = tid; i < n; i += 256) {
+    for (int i = tid; i < n; i += NT) {
       const int idx = perm[b + i];
       sidx[i] = idx;
       skey[i] = c[idx].key;
     }
     __syncthreads();
-    for (int i = tid; i < n; i += 256) {  // emission position = rank of the (unique) key
-      const unsigned long long k = skey[i];
-      int r = 0, j = 0;
-      for (; j + 4 <= n; j += 4) {  // four independent LDS reads in flight
-        const unsigned long long k0 = skey[j], k1 = skey[j + 1], k2 = skey[j + 2], k3 = skey[j + 3];
-        r += (k0 < k ? 1 : 0) + (k1 < k ? 1 : 0) + (k2 < k ? 1 : 0) + (k3 < k ? 1 : 0);
-      }
-      for (; j < n; ++j) r += skey[j] < k ? 1 : 0;
-      eo[r] = sidx[i];
+    bool asc = true;  // contacts that come in emission order need no ranks
+    for (int i = tid; i + 1 < n; i += NT) asc = asc && skey[i] < skey[i + 1];
+    asc = __syncthreads_and(asc ? 1 : 0);
+    if (asc) {
+      for (int i = tid; i < n; i += NT) eo[i] = sidx[i];
+    } else {  // emission position = rank of the (unique) key
+      block_ranks<1, NT / 64>(n, skey, rk, w);
+      for (int i = tid; i < n; i += NT) eo[rk[i]] = sidx[i];
     }
     __syncthreads();
     if (mode == 2) {  // step rule, separate_clusters.cpp:496-564
@@ -2568,7 +2727,7 @@ __global__ void __launch_bounds__(256) k_pair_finish_block(int n_pairs, const in
       v3<double> xa{pr[PR_XA], pr[PR_XA + 1], pr[PR_XA + 2]};
       v3<double> vb{pr[PR_VB], pr[PR_VB + 1], pr[PR_VB + 2]}, wb{pr[PR_WB], pr[PR_WB + 1], pr[PR_WB + 2]};
       v3<double> xb{pr[PR_XB], pr[PR_XB + 1], pr[PR_XB + 2]};
-      for (int i = tid; i < n; i += 256) {
+      for (int i = tid; i < n; i += NT) {
         const ContactRec& ct = c[eo[i]];
         v3<double> A{ct.r[0], ct.r[1], ct.r[2]}, B{ct.r[3], ct.r[4], ct.r[5]};
         v3<double> nrm = sub(A, B);
@@ -2605,47 +2764,51 @@ __global__ void __launch_bounds__(256) k_pair_finish_block(int n_pairs, const in
       __syncthreads();
       if (tid == 0) {
         double m = s_min[0];
-        for (int k = 1; k < 4; ++k) m = (s_min[k] < m) ? s_min[k] : m;
+        for (int k = 1; k < NT / 64; ++k) m = (s_min[k] < m) ? s_min[k] : m;
         scale[p] = m;
       }
-      for (int i = tid; i < n; i += 256) perm[b + i] = eo[i];
+      for (int i = tid; i < n; i += NT) perm[b + i] = eo[i];
     } else if (mode == 1) {  // filterContacts(.., margin)
-      for (int i = tid; i < n; i += 256) {
+      for (int i = tid; i < n; i += NT) {
         const ContactRec& ct = c[eo[i]];
         const v3<double> A{ct.r[0], ct.r[1], ct.r[2]}, B{ct.r[3], ct.r[4], ct.r[5]};
-        sk[i].eps = ct.r[6] + ct.r[7];
-        sk[i].dist = vlen(sub(A, B));
+        sk[i].eps = (ct.r[6] + ct.r[7]) + 0.0;
+        sk[i].dist = vlen(sub(A, B)) + 0.0;
         const v3<double> m = dvs(add(A, B), 2.0);
         smid[3 * i] = m.x, smid[3 * i + 1] = m.y, smid[3 * i + 2] = m.z;
       }
-      if (tid == 0) s_misc[0] = 0;
       __syncthreads();
-      bool tie = false;
-      for (int i = tid; i < n; i += 256) {  // rank of the (eps, dist) key; equal keys share it
-        const LdsKey x = sk[i];
-        int r = 0, eq = 0, j = 0;
-        for (; j + 4 <= n; j += 4) {
-          const LdsKey y0 = sk[j], y1 = sk[j + 1], y2 = sk[j + 2], y3 = sk[j + 3];
-          r += (lds_less(y0, x) ? 1 : 0) + (lds_less(y1, x) ? 1 : 0) + (lds_less(y2, x) ? 1 : 0) +
-               (lds_less(y3, x) ? 1 : 0);
-          eq += (!lds_less(y0, x) && !lds_less(x, y0) ? 1 : 0) + (!lds_less(y1, x) && !lds_less(x, y1) ? 1 : 0) +
-                (!lds_less(y2, x) && !lds_less(x, y2) ? 1 : 0) + (!lds_less(y3, x) && !lds_less(x, y3) ? 1 : 0);
+      float cmax = 0.f;  // the largest coordinate relative to contact 0
+      for (int i = tid; i < n; i += NT)
+        for (int q = 0; q < 3; ++q) {
+          const float v = fabsf((float)(smid[3 * i + q] - smid[q]));
+          cmax = fmaxf(cmax, v < 1e15f ? v : 1e30f);  // (NaN too)
         }
-        for (; j < n; ++j) {
-          const LdsKey y = sk[j];
-          if (lds_less(y, x)) ++r;
-          else if (!lds_less(x, y)) ++eq;
-        }
-        rk[i] = r;
-        tie = tie || eq > 1;
-      }
-      if (tie) s_misc[0] = 1;
+      for (int off = 32; off > 0; off >>= 1) cmax = fmaxf(cmax, __shfl_xor(cmax, off));
+      if (lane == 0) s_cmax[w] = cmax;
       __syncthreads();
-      if (s_misc[0] == 0) {
-        for (int i = tid; i < n; i += 256) ord[rk[i]] = i;
-        __syncthreads();
+      for (int q = 0; q < NT / 64; ++q) cmax = fmaxf(cmax, s_cmax[q]);
+      // rank of the (eps, dist) key: how many are less; equal keys share it.
+      // Non-negative doubles order like their bits (any other key among the
+      // pair's, NaN included, and the comparisons are the doubles' own)
+      bool plain = true;
+      for (int i = tid; i < n; i += NT) ord[i] = -1, plain = plain && sk[i].eps >= 0.0 && sk[i].dist >= 0.0;
+      plain = __syncthreads_and(plain ? 1 : 0);
+      if (plain) {
+        block_ranks<2, NT / 64>(n, reinterpret_cast<const unsigned long long*>(sk), rk, w);
       } else {
-        for (int i = tid; i < n; i += 256) ord[i] = i;
+        for (int i = tid; i < n; i += NT) {
+          int r = 0;
+          for (int j = 0; j < n; ++j) r += lds_less(sk[j], sk[i]) ? 1 : 0;
+          rk[i] = r;
+        }
+        __syncthreads();
+      }
+      bool tie = false;
+      for (int i = tid; i < n; i += NT) tie = tie || atomicExch(&ord[rk[i]], i) != -1;  // two with one rank: a tie
+      tie = __syncthreads_or(tie ? 1 : 0);
+      if (tie) {
+        for (int i = tid; i < n; i += NT) ord[i] = i;
         __syncthreads();
         int* lists = reinterpret_cast<int*>(skey);
         block_std_sort(n, ord, rk, lists, lists + CAP, mark, segs, s_misc + 2, SEGS);
@@ -2657,35 +2820,34 @@ __global__ void __launch_bounds__(256) k_pair_finish_block(int n_pairs, const in
         const int t = t0 + lane;
         const bool valid = t < n;
         const int pi = valid ? ord[t] : 0;
-        const double mx = smid[3 * pi], my = smid[3 * pi + 1], mz = smid[3 * pi + 2];
-        const double search = sk[pi].eps + margin;
+        const NearTest nt = near_test(smid[3 * pi], smid[3 * pi + 1], smid[3 * pi + 2], sk[pi].eps + margin, smid, cmax);
         bool near = false;
         for (int q0 = 0; q0 < nk; q0 += 64) {  // contacts kept before the block
           const int h = q0 + lane < nk ? mark[q0 + lane] : 0;
           const double hx = smid[3 * h], hy = smid[3 * h + 1], hz = smid[3 * h + 2];
+          const float gx = (float)(hx - smid[0]), gy = (float)(hy - smid[1]), gz = (float)(hz - smid[2]);
           const int mm = nk - q0 < 64 ? nk - q0 : 64;
-          for (int u = w; u < mm; u += 4) {
-            const v3<double> dd{mx - readlane_d(hx, u), my - readlane_d(hy, u), mz - readlane_d(hz, u)};
-            near = near || near_mid(dd, search);
+          for (int u = w; u < mm; u += 4 * (NT / 64)) {
+            const unsigned r = near_at4(nt, u, NT / 64, mm, hx, hy, hz, gx, gy, gz, valid && !near);
+            near = near || r != 0u;
           }
         }
-        unsigned long long conf = 0;  // bit u: candidate u (< this one) of the block is near
-        for (int u = w; u < m; u += 4) {
-          const v3<double> dd{mx - readlane_d(mx, u), my - readlane_d(my, u), mz - readlane_d(mz, u)};
-          if (u < lane && near_mid(dd, search)) conf |= 1ull << u;
+        for (int u = w; u < m; u += 4 * (NT / 64)) {  // the later candidates of the group near candidates u, ...
+          const unsigned r =
+              near_at4(nt, u, NT / 64, m, nt.mx, nt.my, nt.mz, nt.fx, nt.fy, nt.fz, u < lane && valid && !near);
+          unsigned long long later = 0ull;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const unsigned long long b = __ballot(((r >> q) & 1u) && lane > u + q * (NT / 64));
+            if (lane == q) later = b;
+          }
+          if (lane < 4 && u + lane * (NT / 64) < m) strike[u + lane * (NT / 64)] = later;
         }
-        near_w[w][lane] = near ? 1 : 0;
-        conf_w[w][lane] = conf;
+        const unsigned long long nm = __ballot(near);
+        if (lane == 0) near_m[w] = nm;
         __syncthreads();
         if (w == 0) {
-          const bool nr = (near_w[0][lane] | near_w[1][lane] | near_w[2][lane] | near_w[3][lane]) != 0;
-          const unsigned long long cf = conf_w[0][lane] | conf_w[1][lane] | conf_w[2][lane] | conf_w[3][lane];
-          const unsigned long long blocked = __ballot(nr);
-          unsigned long long kept = 0;
-          for (int i = 0; i < m; ++i) {
-            const unsigned long long ci = readlane_u64(cf, i);
-            if (!((blocked >> i) & 1ull) && !(ci & kept)) kept |= 1ull << i;
-          }
+          const unsigned long long kept = greedy_keep<NT / 64>(m, strike, near_m);
           const bool fresh = (kept >> lane) & 1ull;
           if (valid) keep[b + t] = fresh ? 1 : 0;
           if (fresh) mark[nk + __popcll(kept & lanes_below())] = pi;
@@ -2694,10 +2856,10 @@ __global__ void __launch_bounds__(256) k_pair_finish_block(int n_pairs, const in
         __syncthreads();
         nk = s_misc[1];
       }
-      for (int t = tid; t < n; t += 256) perm[b + t] = eo[ord[t]];
+      for (int t = tid; t < n; t += NT) perm[b + t] = eo[ord[t]];
       if (tid == 0) kept_cnt[p] = nk, kept_sum += (unsigned long long)nk;
     } else {
-      for (int i = tid; i < n; i += 256) perm[b + i] = eo[i];
+      for (int i = tid; i < n; i += NT) perm[b + i] = eo[i];
     }
     __syncthreads();
   }
@@ -2705,8 +2867,8 @@ __global__ void __launch_bounds__(256) k_pair_finish_block(int n_pairs, const in
     if (tail) {  // pairs above every LDS capacity (listed by the first launch), one block each
       if (mode == 1) {
         for (int t = blockIdx.x; t < *n_tail; t += gridDim.x) {
-          const int nk = pair_filter_huge<CAP>(tail[t], c, pair_off, perm, keep, kept_cnt, margin, H, skey, sk,
-                                               s_misc, conf_w, near_w);
+          const int nk = pair_filter_huge<CAP, NT>(tail[t], c, pair_off, perm, keep, kept_cnt, margin, H, skey, sk,
+                                               s_misc, strike, near_m);
           if (tid == 0) kept_sum += (unsigned long long)nk;
         }
       } else {
@@ -4030,11 +4192,11 @@ HugeScratch huge_scratch(d2_ctx* c) {
   return HugeScratch{h, h + m, h + 2 * m, h + 3 * m, h + 4 * m, h + 5 * m};
 }
 void launch_finish(d2_ctx* c, int np, int wblocks, int mode, unsigned long long* kept_total, double margin) {
-  hipLaunchKernelGGL(k_pair_finish_block<BLK_CAP>, dim3(wblocks), dim3(256), 0, c->stream, np, (const int*)nullptr,
+  hipLaunchKernelGGL((k_pair_finish_block<BLK_CAP, 256>), dim3(wblocks), dim3(256), 0, c->stream, np, (const int*)nullptr,
                      (const int*)nullptr, c->contacts.p, c->pair_off.p, c->perm.p, mode, c->keep.p, c->kept_cnt.p,
                      c->pair_rec.p, c->scale.p, c->big.p, c->n_big.p, c->huge.p, c->n_big.p + 1,
                      (const int*)nullptr, (const int*)nullptr, kept_total, margin, huge_scratch(c));
-  hipLaunchKernelGGL(k_pair_finish_block<POST_CAP_LARGE>, dim3(std::max(1, std::min(np, c->cus))), dim3(256), 0,
+  hipLaunchKernelGGL((k_pair_finish_block<POST_CAP_LARGE, 1024>), dim3(std::max(1, std::min(np, c->cus))), dim3(1024), 0,
                      c->stream, np, (const int*)c->big.p, (const int*)c->n_big.p, c->contacts.p, c->pair_off.p,
                      c->perm.p, mode, c->keep.p, c->kept_cnt.p, c->pair_rec.p, c->scale.p, c->huge.p,
                      c->n_big.p + 1, c->huge.p, c->n_big.p + 1, (const int*)c->huge.p,

@@ -298,12 +298,11 @@ D2_HD unsigned soup_cull_mask(const double* Ta0, const double* Ta1, const double
 // cull.
 //
 // The per-triangle terms are computed once (cull_prep): vertices in the
-// frame of the pair (b's position as origin), normal, kappa, longest squared
-// edge, own-normal extent, centroid, largest coordinate (of the results and
+// frame of the pair (b's position as origin), normal, kappa, longest edge, own-normal extent, centroid, largest coordinate (of the results and
 // of the transform's inputs), and whether the barycentric system is well
 // conditioned.
 struct alignas(16) CullTri {
-  float c3[3], kap, L2, crd, ok;
+  float c3[3], kap, L, crd, ok;
   float v[9], n[3], nn, pmin, pmax;
   float pad[4];  // 112 bytes: 28 dwords, so 8 consecutive records start in 8 distinct 4-bank groups of LDS
   double eps;    // the triangle's eps from its bucket (read with the triangle)
@@ -329,7 +328,7 @@ D2_HD void cull_prep_f(const float* rot, const float* tr, const float* c9, CullT
   const float den = d00 * d11 - d01 * d01;
   o.ok = (den > 1e-4f * d00 * d11) ? 1.f : 0.f;
   o.kap = o.ok != 0.f ? d00 * d11 / den : 0.f;
-  o.L2 = fmaxf(fmaxf(d00, d11), f3dot(e2, e2));
+  o.L = sqrtf(fmaxf(fmaxf(d00, d11), f3dot(e2, e2)));
   o.nn = f3dot(o.n, o.n);
   const float p0 = f3dot(o.v, o.n), p1 = f3dot(o.v + 3, o.n), p2 = f3dot(o.v + 6, o.n);
   o.pmin = fminf(p0, fminf(p1, p2)), o.pmax = fmaxf(p0, fmaxf(p1, p2));
@@ -344,18 +343,15 @@ D2_HD void cull_prep(const float* rot, const float* tr, const tri<double>& t, Cu
 D2_HD float cull_margin(const CullTri& A, const CullTri& B, float thr) {
   const float EPSF = 5.9604645e-08f;
   const float kappa = fmaxf(A.kap, B.kap);
-  const float L = sqrtf(fmaxf(A.L2, B.L2));
+  const float L = fmaxf(A.L, B.L);
   return 1e-6f + 64.f * EPSF * kappa * L + 16.f * EPSF * fmaxf(A.crd, B.crd) + EPSF * thr;
 }
-// 0 certain miss, 1 needs the FP64 test, 2 certain hit.  The lower bound
-// compares g^2 > T^2 |n|^2 per axis instead of g / |n| > T, with T = (thr +
-// margin)(1 + 2^-20) covering the few roundings of the squared form.  The upper bound
-// (certain hit) is only computed when want_hit: a certain hit only matters
-// for node pairs with an inner node.
-D2_HD int cull_pair(const CullTri& A, const CullTri& B, float thr, bool want_hit = true) {
-  if (A.ok == 0.f || B.ok == 0.f) return 1;
-  const float margin = cull_margin(A, B, thr);
-  const float T = (thr + margin) * (1.f + 9.5367432e-07f);
+// Certain miss.  The lower bound compares g^2 > T^2 |n|^2 per axis instead of
+// g / |n| > T, with T = (thr + margin)(1 + 2^-20) covering the few roundings of
+// the squared form.
+D2_HD bool cull_apart(const CullTri& A, const CullTri& B, float thr) {
+  if (A.ok == 0.f || B.ok == 0.f) return false;
+  const float T = (thr + cull_margin(A, B, thr)) * (1.f + 9.5367432e-07f);
   const float T2 = T * T;
   bool sep = false;
   {  // axis nA
@@ -377,8 +373,12 @@ D2_HD int cull_pair(const CullTri& A, const CullTri& B, float thr, bool want_hit
                           fminf(a0, fminf(a1, a2)) - fmaxf(b0, fmaxf(b1, b2)));
     sep = sep || (nn > 0.f && g > 0.f && g * g > T2 * nn);
   }
-  if (sep) return 0;
-  if (!want_hit) return 1;
+  return sep;
+}
+// Certain hit, for a triangle pair that is no certain miss (it only matters
+// for node pairs with an inner node).
+D2_HD bool cull_sure(const CullTri& A, const CullTri& B, float thr) {
+  if (A.ok == 0.f || B.ok == 0.f) return false;
   float ub2 = 3.4e38f;
   float dd[3][3];
   for (int x = 0; x < 3; ++x)
@@ -391,9 +391,13 @@ D2_HD int cull_pair(const CullTri& A, const CullTri& B, float thr, bool want_hit
       const int x1 = x == 2 ? 0 : x + 1, y1 = y == 2 ? 0 : y + 1;
       ub2 = fminf(ub2, fmaxf(fmaxf(dd[x][y], dd[x][y1]), fmaxf(dd[x1][y], dd[x1][y1])));
     }
-  const float lim = thr - margin;
-  if (lim > 0.f && ub2 < lim * lim) return 2;
-  return 1;
+  const float lim = thr - cull_margin(A, B, thr);
+  return lim > 0.f && ub2 < lim * lim;
+}
+// 0 certain miss, 1 needs the FP64 test, 2 certain hit (when want_hit).
+D2_HD int cull_pair(const CullTri& A, const CullTri& B, float thr, bool want_hit = true) {
+  if (cull_apart(A, B, thr)) return 0;
+  return want_hit && cull_sure(A, B, thr) ? 2 : 1;
 }
 
 // ---------------------------------------------- the same classification in FP64

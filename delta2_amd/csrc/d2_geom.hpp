@@ -186,8 +186,8 @@ D2_HD bool nodes_apart(const double* Ta, const double* Tb, const float* ba, cons
   return gap > thr;
 }
 // nodes_apart over the six face axes only (each box's three face normals):
-// fewer live registers, for the FP32 form's mask kernel, which tests every
-// node pair on arrival.  The face axes find nearly all of the separations
+// what the FP32 form's mask kernel asks of every node pair on arrival, in FP32
+// (boxes_apart_faces_rel below).  The face axes find nearly all of the separations
 // the edge axes add to the spheres' (on a 4096-body funnel pile 98% for
 // funnel pairs, 92% for body pairs).  b's offset along its own face normal
 // j (Rb's column j) is taken as that column times the centre difference.
@@ -243,8 +243,7 @@ D2_HD bool spheres_apart(const double* Ta, const double* Tb, const float* ba, co
   }
   return sqrt(s2) - ((double)ba[7] + (double)bb[7]) > thr;
 }
-// spheres_apart in FP32 for the FP32 form's mask kernel (it runs at five
-// wavefronts per SIMD; the FP64 poses would spill there).  Each world
+// spheres_apart in FP32.  Each world
 // coordinate w = R c + t is off by at most 8 u (|R c|_1 + |t|) after the
 // rounding of the pose, the product and the sums (u = 2^-24), so the centre
 // distance by at most 16 u m + 5 u |d| with m the sum of |w| over both
@@ -262,6 +261,72 @@ D2_HD bool spheres_apart_f32(const double* Ta, const double* Tb, const float* ba
   }
   const double dist = (double)sqrtf(s2);
   return dist - ((double)ba[7] + (double)bb[7]) > thr + 32.0 * 5.9604645e-08 * ((double)mag + dist);
+}
+// A pair's poses for the discrete phase's FP32 tests, PF_FLOATS floats: a's
+// rotation (rows), a's translation relative to b's, b's rotation, the search
+// distance (a float to begin with), in the frame with b's position as origin.
+constexpr int PF_RA = 0, PF_TR = 9, PF_RB = 12, PF_SEARCH = 21, PF_FLOATS = 24;
+D2_HD void pair_pose_f32(const double* Ta, const double* Tb, float search, float* f) {
+  for (int r = 0; r < 3; ++r) {
+    for (int k = 0; k < 3; ++k) f[PF_RA + 3 * r + k] = (float)Ta[4 * r + k], f[PF_RB + 3 * r + k] = (float)Tb[4 * r + k];
+    f[PF_TR + r] = (float)(Ta[4 * r + 3] - Tb[4 * r + 3]);
+  }
+  f[PF_SEARCH] = search;
+}
+// spheres_apart and boxes_apart_faces in FP32 from that record.  With u =
+// 2^-24, each coordinate of a centre in b's frame, w = R c + t, is off by at
+// most 8 u (|c| + |t|) <= 8 u (|w|_1 + 2 |t|_1), the centres' difference d by
+// 14 u m (m = |wa|_1 + |wb|_1 + 2 |t|_1), its projection on a face axis by
+// another 5 u |d|_1 and a rounding of the columns, in all at most 25 u m + 6 u
+// |d|_1, and the boxes' half extents E on an axis by 16 u |E|_1; the threshold
+// and the radii round by 4 u.  Both tests demand 64 u of the sum of all these
+// magnitudes, and the FP64 forms' 1e-9, beyond the threshold.
+D2_HD void rel_centre(const float* f, const float* ca, const float* cb, float* d, float& mag) {
+  mag = 0.f;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const float* a = f + PF_RA + 3 * r;
+    const float* b = f + PF_RB + 3 * r;
+    const float wa = fmaf(a[2], ca[2], fmaf(a[1], ca[1], fmaf(a[0], ca[0], f[PF_TR + r])));
+    const float wb = fmaf(b[2], cb[2], fmaf(b[1], cb[1], b[0] * cb[0]));
+    d[r] = wb - wa;
+    mag += (fabsf(wa) + fabsf(wb)) + (fabsf(d[r]) + 2.f * fabsf(f[PF_TR + r]));
+  }
+}
+D2_HD bool spheres_apart_rel(const float* f, const float* ba, const float* bb) {
+  const float thr = (f[PF_SEARCH] + ba[6]) + bb[6], rad = ba[7] + bb[7];
+  float d[3], mag;
+  rel_centre(f, ba + 8, bb + 8, d, mag);
+  const float lim = fmaf(64.f * 5.9604645e-08f, (mag + thr) + rad, (thr + rad) + 2e-9f);
+  return fmaf(d[2], d[2], fmaf(d[1], d[1], d[0] * d[0])) > lim * lim * (1.f + 1e-6f);
+}
+D2_HD bool boxes_apart_faces_rel(const float* f, const float* ba, const float* bb) {
+  const float thr = (f[PF_SEARCH] + ba[6]) + bb[6];
+  float ca[3], cb[3], ea[3], eb[3], d[3], mag;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    ca[k] = 0.5f * (ba[k] + ba[3 + k]), cb[k] = 0.5f * (bb[k] + bb[3 + k]);
+    ea[k] = 0.5f * (ba[3 + k] - ba[k]), eb[k] = 0.5f * (bb[3 + k] - bb[k]);
+  }
+  rel_centre(f, ca, cb, d, mag);
+  mag += (((ea[0] + ea[1]) + ea[2]) + ((eb[0] + eb[1]) + eb[2])) + thr;
+  const float* A = f + PF_RA;
+  const float* B = f + PF_RB;
+  float ga[3], gb[3];  // per face axis: the centres' offset less the extents
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    ga[i] = fabsf(fmaf(A[6 + i], d[2], fmaf(A[3 + i], d[1], A[i] * d[0]))) - ea[i];
+    gb[i] = fabsf(fmaf(B[6 + i], d[2], fmaf(B[3 + i], d[1], B[i] * d[0]))) - eb[i];
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const float r = fabsf(fmaf(A[6 + i], B[6 + j], fmaf(A[3 + i], B[3 + j], A[i] * B[j])));
+      ga[i] = fmaf(-eb[j], r, ga[i]), gb[j] = fmaf(-ea[i], r, gb[j]);
+    }
+  const float gap = fmaxf(fmaxf(fmaxf(ga[0], ga[1]), fmaxf(ga[2], gb[0])), fmaxf(gb[1], gb[2]));
+  return gap > fmaf(64.f * 5.9604645e-08f, mag, thr + 2e-9f);
 }
 // ---- rigid-body state (model/state.cpp) -----------------------------------
 struct quat {

@@ -97,6 +97,7 @@ enum : int {
   PR_GEOA = 146, PR_GEOB = 147, PR_MAXT = 148, PR_SEARCH = 149,
   PR_STRIDE = 152
 };
+constexpr int PF_STRIDE = 32;  // PF_FLOATS in a cache line of their own
 constexpr int BUCKET = 88;
 constexpr int RES_SLOTS = 15;  // sub-results per soup triangle pair
 // Global counters (atomics) and per-level sizes.  Level L reads its list sizes
@@ -176,6 +177,38 @@ __device__ __forceinline__ void atomic_min_pos(unsigned long long* addr, double 
 
 __device__ __forceinline__ int rl(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
 
+// Marks on the lanes of a wavefront divide it into runs: the lane that starts
+// lane t's run (marked: lane t starts one; lane 0 always does).
+__device__ __forceinline__ int run_start(bool marked) {
+  const unsigned long long m = __ballot(marked) | 1ull;
+  return 63 - __clzll((long long)(m & (~0ull >> (63 - lane_id()))));
+}
+// Lanes own runs of consecutive outputs (len of them from position first, in
+// lane order, together covering the 64 positions from 0 or their start): the
+// lane that owns position lane_id().  own: 64 bytes of LDS of this wavefront.
+// All lanes call it.
+__device__ __forceinline__ int run_owner(unsigned char* own, int first, int len) {
+  own[lane_id()] = 0;
+  wave_sync_lds();
+  if (len > 0 && first < 64 && first + len > 0) own[first > 0 ? first : 0] = (unsigned char)(lane_id() + 1);
+  wave_sync_lds();
+  const int owner = (int)own[run_start(own[lane_id()] != 0)] - 1;
+  wave_sync_lds();  // read before the next call writes
+  return owner;
+}
+// Position of the r-th set bit of m (r < popcount).
+__device__ __forceinline__ int nth_bit(unsigned long long m, int r) {
+  unsigned x = (unsigned)m;
+  int pos = 0, c = __popc(x);
+  if (r >= c) r -= c, x = (unsigned)(m >> 32), pos = 32;
+#pragma unroll
+  for (int w = 16; w; w >>= 1) {
+    c = __popc(x & ((1u << w) - 1u));
+    if (r >= c) r -= c, x >>= w, pos += w;
+  }
+  return pos;
+}
+
 // arr[key] = min(arr[key], v) for every lane (key -1: none).  Most lanes of a
 // wavefront often share one key (a pile is one cluster), and atomics on one
 // address take turns (6 ns each here): the lanes of the first keys met are
@@ -221,6 +254,7 @@ struct Dev {
   // pairs
   const int32_t* pair_info;  // a, b, node offset a, node offset b
   const double* pair_rec;
+  float* pair_f;               // FP32 form, discrete phase: pair_pose_f32 per pair (PF_STRIDE)
   // work lists
   NP* soup;
   NP* conn;
@@ -437,6 +471,18 @@ __global__ void __launch_bounds__(256) k_setup(Dev D, const int32_t* pairs, cons
         k[3] = w.x, k[4] = w.y, k[5] = w.z;  // PR_WA / PR_WB
         k[6] = so.t.x, k[7] = so.t.y, k[8] = so.t.z;  // PR_XA / PR_XB
       }
+    }
+    if (!ccd && D.pair_f && end) {
+      // pair_pose_f32, each lane the half it has the pose of
+      float* f = D.pair_f + (size_t)PF_STRIDE * p;
+      const double t[3] = {so.t.x - sx.t.x, so.t.y - sx.t.y, so.t.z - sx.t.z};
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) f[(of_a ? PF_RA : PF_RB) + 3 * r + k] = (float)To[4 * r + k];
+        if (of_a) f[PF_TR + r] = (float)t[r];
+      }
+      if (!of_a) f[PF_SEARCH] = (float)(ra[37] + rb[37]);
     }
     if (q == 0) {
       pr[PR_GEOA] = ra[37];
@@ -1000,71 +1046,73 @@ __device__ __forceinline__ int expansion_desc(const NodeRec& na, const NodeRec& 
   const NodeRec& par = adv_a ? na : nb;
   return (adv_a ? 1 : 0) | (par.nchild << 1) | (par.child_first << 5);
 }
-// Discrete lists: the children of a node pair that hits or may hit, at slot,
-// slot + 1, ... of the next list, each naming its parent: parent 0 for a
-// certain hit, list index + 1 when the parent's FP64 tests (k_tri_dist, its
-// hit flag) decide; the next level drops the children of parents that did
-// not hit.  The discrete phase's contacts carry their emission keys (child
-// index paths) and are ordered by them afterwards, so its lists need no
-// breadth-first order and children take slots by atomics.
-// Only the children in cmask are written (the others are provably apart:
-// child_mask); the emission keys keep every child's own index.
-__device__ __forceinline__ void write_children(const Dev& D, long long slot, const NP& np, int desc, uint32_t parent,
-                                               unsigned cmask) {
+// The child c of a node pair of the discrete list.  Discrete lists: the
+// children of a node pair that hits or may hit take slots of the next list,
+// each naming its parent: parent 0 for a certain hit, list index + 1 when the
+// parent's FP64 tests (k_tri_dist, its hit flag) decide; the next level drops
+// the children of parents that did not hit.  The discrete phase's contacts
+// carry their emission keys (child index paths) and are ordered by them
+// afterwards, so its lists need no breadth-first order and children take slots
+// by atomics; the keys keep every child's own index.
+__device__ __forceinline__ NP child_of(const NP& np, int desc, int c, uint32_t parent) {
   const bool adv_a = desc & 1;
-  const int nc = (desc >> 1) & 15, first = desc >> 5;
-  for (int c = 0; c < nc; ++c) {
-    if (!((cmask >> c) & 1u)) continue;
-    const uint32_t ca = adv_a ? (uint32_t)(first + c) : np.na;
-    const uint32_t cb = adv_a ? np.nb : (uint32_t)(first + c);
-    if (slot < D.cap_np) D.soup_next[slot] = NP{np.pair, ca, cb, parent, np.key * 8ull + (unsigned long long)c};
-    ++slot;
-  }
+  const uint32_t id = (uint32_t)((desc >> 5) + c);
+  return NP{np.pair, adv_a ? id : np.na, adv_a ? np.nb : id, parent, np.key * 8ull + (unsigned long long)c};
 }
-// The children of a node pair worth writing: all of them, or (pruning) those
-// spheres_apart_f32 does not prove contact-free (k_tri_mask runs at five
-// wavefronts per SIMD: the boxes' test, or FP64 poses, would spill there).
-// offa/offb: the two trees' first node records.
-__device__ __forceinline__ unsigned child_mask(const Dev& D, const NP& np, int desc, int offa, int offb) {
-  const int nc = (desc >> 1) & 15;
-  unsigned m = (1u << nc) - 1u;
-  if (!D.prune) return m;
-  const bool adv_a = desc & 1;
-  const int first = desc >> 5;
-  const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
-  for (int c = 0; c < nc; ++c) {
-    const size_t ga = (size_t)offa + (adv_a ? (uint32_t)(first + c) : np.na);
-    const size_t gb = (size_t)offb + (adv_a ? np.nb : (uint32_t)(first + c));
-    if (spheres_apart_f32(pr + PR_TA1, pr + PR_TB1, D.nbound + NB_STRIDE * ga, D.nbound + NB_STRIDE * gb, pr[PR_SEARCH]))
-      m &= ~(1u << c);
+__device__ __forceinline__ void load_pose_f(const Dev& D, uint32_t pair, float* f) {
+  const float4* p = reinterpret_cast<const float4*>(D.pair_f + (size_t)PF_STRIDE * pair);
+#pragma unroll
+  for (int q = 0; q < PF_FLOATS / 4; ++q) {
+    const float4 v = p[q];
+    f[4 * q] = v.x, f[4 * q + 1] = v.y, f[4 * q + 2] = v.z, f[4 * q + 3] = v.w;
   }
-  return m;
 }
 static_assert(sizeof(CullTri) == 112, "prepared triangle: 28 dwords, a conflict-free LDS stride");
-// Five wavefronts per SIMD (at most 96 VGPRs, no spills) instead of the four
-// its natural 101 VGPRs allow: the kernel waits on dependent loads, and more
-// resident wavefronts hide more of them.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) k_tri_mask(Dev D) {
+// A wavefront takes the node pairs of a batch in groups of at most 64
+// triangles, both buckets' together: a lane prepares one triangle, then the
+// group's triangle pairs go one per lane, 64 at a time; those that are no
+// certain miss, of inner node pairs, move together for the certain-hit bound
+// (a third of the arithmetic, needed by a tenth of them), and the candidate
+// children and the kept items are spread over the lanes in the same way.
+// Buckets at the leaves hold two or three triangles and most node pairs are
+// there: with a pass per node pair 5 of 64 lanes worked.  Vector arithmetic
+// bounds it now (68-82% of issue on the large levels); the poses come as
+// 96-byte float records, which halved the load addresses per node pair.
+// A pile's 37 M node pairs: 16.0 -> 8.4 ms; 5.5 M of 48 small scenes: 2.55 ->
+// 1.5 ms; a 4,096-body scene's 0.7 M in nine levels: 516 -> 405 us.
+//
+// Four wavefronts per SIMD (103 VGPRs); at five it spills, and measures the same.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) k_tri_mask(Dev D) {
   __shared__ int s_tot[2][4], s_ch[2][4], s_df[2][4];
-  __shared__ CullTri s_tri[4][4][16];  // per wavefront: 4 node pairs' 8 + 8 prepared triangles
+  __shared__ union {
+    CullTri tri[64];           // per wavefront: the group's prepared triangles,
+    unsigned short kid[512];   // then the children to write: child | owning lane << 4
+  } s_u[4];
+  __shared__ unsigned short s_job[4][256];      // and its triangle pairs: slot of a's, slot of b's << 6, inner << 12
+  __shared__ unsigned char s_own[4][64];        // run starts: the owning lane + 1
+  __shared__ unsigned long long s_sure[4];      // a's triangles with a certain hit
   __shared__ unsigned long long s_base[2], s_chb[2], s_dfb[2];
   const int lane = lane_id(), nw = blockDim.x >> 6, wid = threadIdx.x >> 6;
   const long long n = D.n_soup();
-  long long rb, re;
-  chunk_of(n, rb, re);
-  // The block walks its range 64 * nw node pairs at a time, wavefront wid
-  // taking rb + wid + nw * k; lane l fetches the record, node offsets and node
-  // records of the wave's l-th node pair in one go, so the per-node-pair
-  // dependent loads reduce to its pose and buckets.
+  // Tiles of up to 64 node pairs per wavefront, a block taking every
+  // gridDim-th (how many node pairs are live, and inner, varies along the list:
+  // with one long range per block the last blocks ran alone).  The wavefronts
+  // of a block take consecutive parts (siblings lie next to each other: their records,
+  // pose and nodes come in few cache lines); lane l fetches the record, node
+  // offsets and node records of the wave's l-th node pair in one go, so the
+  // per-node-pair dependent loads reduce to its pose and buckets.
   int it = 0;
-  for (long long b0 = rb; b0 < re; b0 += 64ll * nw, ++it) {
-    const long long w0 = b0 + wid;
-    const long long wl = w0 + (long long)nw * lane;
-    int l_pair = 0, l_offa = 0, l_offb = 0, l_bka = 0, l_bkb = 0, l_nta = 0, l_ntb = 0, l_inner = 0, l_desc = 0;
-    double l_search = 0.0;
-    NP l_np{};
-    if (wl < re) {
+  const long long waves = (long long)gridDim.x * nw;
+  const int part = n < 64 * waves ? (int)((n + waves - 1) / waves) : 64;  // node pairs per wavefront
+  for (long long b0 = (long long)blockIdx.x * nw * part; b0 < n; b0 += waves * part, ++it) {
+    const long long w0 = b0 + (long long)part * wid;
+    const long long wl = w0 + lane;
+    const bool in_range = lane < part && wl < n;
+    int l_pair = 0, l_ga = 0, l_gb = 0, l_nta = 0, l_ntb = 0, l_inner = 0, l_desc = 0;  // l_ga, l_gb: global buckets
+    int l_offa = 0, l_offb = 0;
+    if (in_range) {
       const NP np = D.soup[wl];
+      const int hit = np.pad != 0u ? D.np_hit_prev[np.pad - 1u] : 1;
       const int32_t* pi = D.pair_info + 4 * np.pair;
       l_pair = (int)np.pair, l_offa = pi[2], l_offb = pi[3];
       // a child of a parent that did not hit, or a node pair whose leaves are
@@ -1072,81 +1120,116 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))
       // child is written (roots here); the boxes' face-axis test runs here,
       // one node pair per lane, before the node records are loaded (few
       // registers are live).
-      bool live = np.pad == 0u || D.np_hit_prev[np.pad - 1u] != 0;
-      if (live && D.prune) {
-        const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
+      bool live = hit != 0;
+      if (live && D.prune && (D.level == 0 || D.box_test)) {
+        float f[PF_FLOATS];
+        load_pose_f(D, np.pair, f);
         const float* bA = D.nbound + NB_STRIDE * ((size_t)l_offa + np.na);
         const float* bB = D.nbound + NB_STRIDE * ((size_t)l_offb + np.nb);
-        live = !((D.level == 0 && spheres_apart_f32(pr + PR_TA1, pr + PR_TB1, bA, bB, pr[PR_SEARCH])) ||
-                 (D.box_test && boxes_apart_faces(pr + PR_TA1, pr + PR_TB1, bA, bB, pr[PR_SEARCH])));
+        live = !((D.level == 0 && spheres_apart_rel(f, bA, bB)) || (D.box_test && boxes_apart_faces_rel(f, bA, bB)));
       }
       if (live) {
         const NodeRec na = D.nodes[l_offa + np.na];
         const NodeRec nb = D.nodes[l_offb + np.nb];
-        l_np = np;
-        l_bka = na.bucket, l_bkb = nb.bucket, l_nta = na.ntris, l_ntb = nb.ntris;
+        l_ga = l_offa + na.bucket, l_gb = l_offb + nb.bucket, l_nta = na.ntris, l_ntb = nb.ntris;
         l_inner = (na.inner || nb.inner) ? 1 : 0;
         l_desc = expansion_desc(na, nb);
-        l_search = D.pair_rec[(size_t)PR_STRIDE * np.pair + PR_SEARCH];
       }
     }
-    const long long left = w0 < re ? (re - w0 + nw - 1) / nw : 0;
-    const int batch = left < 64 ? (int)left : 64;
-    unsigned long long my_keep = 0;
+    unsigned long long my_keep = 0;  // bit i * l_ntb + j: triangle i of a against j of b
     int my_settled = 0;
-    const int i = lane >> 3, j = lane & 7;
-    for (int k0 = 0; k0 < batch; k0 += 4) {
+    const int my_jobs = l_nta * l_ntb, my_tris = my_jobs > 0 ? l_nta + l_ntb : 0;
+    const int tri_incl = wave_incl_scan(my_tris), job_incl = wave_incl_scan(my_jobs);
+    const int tri_all = rl(tri_incl, 63);
+    for (int t0 = 0, j0 = 0; t0 < tri_all;) {
+      const int ts = tri_incl - my_tris - t0, js = job_incl - my_jobs - j0;
+      bool in = my_tris > 0 && ts >= 0 && ts + my_tris <= 64;
+      int last = 63 - __clzll((long long)__ballot(in));
+      // a few triangle pairs over a multiple of 64 wait for the next group
+      const int over = rl(job_incl, last) - j0;
+      if (over > 64 && (over & 63) < 40) {
+        in = in && js + my_jobs <= (over & ~63);
+        last = 63 - __clzll((long long)__ballot(in));
+      }
+      const int t1 = rl(tri_incl, last), j1 = rl(job_incl, last), jobs = j1 - j0;
+      s_own[wid][lane] = 0;
+      wave_sync_lds();
+      if (in) s_own[wid][ts] = (unsigned char)(lane + 1);
+      wave_sync_lds();
       {
-        // the triangles of four node pairs at once: lane l prepares triangle
-        // (l & 15) of node pair k0 + (l >> 4) (lanes 0-7 of a group: bucket a,
-        // 8-15: bucket b), so no lane idles in the preparation
-        const int kp = k0 + (lane >> 4), slot = lane & 15, side = slot >> 3, kk = slot & 7;
-        const int src = kp < batch ? kp : k0;
-        // every lane takes part in every shuffle (a shuffle inside divergent
-        // code may read an inactive source lane)
+        // lane t prepares the group's triangle t.  Every lane takes part in
+        // every shuffle (inside divergent code one may read an inactive
+        // source lane).
+        const int start = run_start(s_own[wid][lane] != 0);
+        const int src = (int)s_own[wid][start] - 1, x = lane - start;
         const int pair = __shfl(l_pair, src), nta = __shfl(l_nta, src), ntb = __shfl(l_ntb, src);
-        const int ga = __shfl(l_offa, src) + __shfl(l_bka, src), gb = __shfl(l_offb, src) + __shfl(l_bkb, src);
-        const int gbk = side ? gb : ga;
-        CullTri mine{};
-        if (kp < batch && kk < (side ? ntb : nta)) {
-          const double* pr = D.pair_rec + (size_t)PR_STRIDE * pair;
-          const double* pm = side ? pr + PR_TB1 : pr + PR_TA1;
-          float rot[9], tr[3];
-          for (int r = 0; r < 3; ++r) {
-            for (int q = 0; q < 3; ++q) rot[3 * r + q] = (float)pm[4 * r + q];
-            tr[r] = side ? 0.f : (float)(pr[PR_TA1 + 4 * r + 3] - pr[PR_TB1 + 4 * r + 3]);
-          }
-          const float4* fb = reinterpret_cast<const float4*>(D.fbuckets + (size_t)FB_STRIDE * (8 * (size_t)gbk + kk));
+        const int ga = __shfl(l_ga, src), gb = __shfl(l_gb, src);
+        const int jstart = __shfl(js, src), inner = __shfl(l_inner, src);
+        const bool side = x >= nta;
+        const int kk = side ? x - nta : x;
+        if (lane < t1 - t0) {
+          CullTri mine{};
+          // (b's rotation, no translation: b's position is the origin)
+          const float4* pf = reinterpret_cast<const float4*>(D.pair_f + (size_t)PF_STRIDE * pair + (side ? PF_RB : PF_RA));
+          const float search = D.pair_f[(size_t)PF_STRIDE * pair + PF_SEARCH];
+          const float4 p0 = pf[0], p1 = pf[1], p2 = pf[2];
+          const float rot[9] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w, p2.x};
+          const float tr[3] = {side ? 0.f : p2.y, side ? 0.f : p2.z, side ? 0.f : p2.w};
+          const float4* fb =
+              reinterpret_cast<const float4*>(D.fbuckets + (size_t)FB_STRIDE * (8 * (size_t)(side ? gb : ga) + kk));
           const float4 q0 = fb[0], q1 = fb[1], q2 = fb[2];
           const float c9[9] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x};
           cull_prep_f(rot, tr, c9, mine);
-          mine.eps = __hiloint2double(__float_as_int(q2.w), __float_as_int(q2.z));
+          const double eps = __hiloint2double(__float_as_int(q2.w), __float_as_int(q2.z));
+          mine.eps = side ? eps : (double)search + eps;  // the reference's sum starts so: (search + eps_a) + eps_b
+          s_u[wid].tri[lane] = mine;
+          if (!side)
+            for (int j = 0; j < ntb; ++j)
+              s_job[wid][jstart + kk * ntb + j] =
+                  (unsigned short)(lane | ((start + nta + j) << 6) | (inner << 12));
         }
-        s_tri[wid][lane >> 4][slot] = mine;
         wave_sync_lds();
       }
-      const int kend = k0 + 4 < batch ? k0 + 4 : batch;
-      for (int k = k0; k < kend; ++k) {
-        const int nta = rl(l_nta, k), ntb = rl(l_ntb, k);
-        const bool inner = rl(l_inner, k) != 0;
-        int cls = 0;
-        if (i < nta && j < ntb) {  // operands read from LDS where they are used (fewer live registers)
-          // no global load on the node pair's chain: the search distance came
-          // with the node pair, the eps values with the prepared triangles
-          const CullTri& A = s_tri[wid][k - k0][i];
-          const CullTri& B = s_tri[wid][k - k0][8 + j];
-          const double search = __longlong_as_double((long long)readlane_u64(
-              (unsigned long long)__double_as_longlong(l_search), k));
-          cls = cull_pair(A, B, (float)((search + A.eps) + B.eps), inner);
+      // which are certain misses; the others of inner node pairs move to the
+      // front of the list
+      int left = 0;
+      for (int q0 = 0; q0 < jobs; q0 += 64) {
+        int job = 0;
+        bool keep = false;
+        if (q0 + lane < jobs) {  // operands read from LDS where they are used (fewer live registers)
+          job = s_job[wid][q0 + lane];
+          const CullTri& A = s_u[wid].tri[job & 63];
+          const CullTri& B = s_u[wid].tri[(job >> 6) & 63];
+          keep = !cull_apart(A, B, (float)(A.eps + B.eps));
         }
-        unsigned long long keep = __ballot(cls == 1 || (cls == 2 && !inner));
-        const bool settled = inner && __ballot(cls == 2) != 0ull;
-        if (settled) keep = 0ull;
-        if (lane == k) my_keep = keep, my_settled = settled ? 1 : 0;
+        const unsigned long long kept = __ballot(keep);
+        // this lane's node pair's share of the 64 answers
+        const int d = js - q0;
+        if (in && d < 64 && d + my_jobs > 0)
+          my_keep |= (d >= 0 ? kept >> d : kept << -d) & (my_jobs < 64 ? (1ull << my_jobs) - 1ull : ~0ull);
+        const bool more = keep && job >> 12;
+        const unsigned long long m = __ballot(more);
+        if (more) s_job[wid][left + __popcll(m & lanes_below())] = (unsigned short)job;
+        left += __popcll(m);
+      }
+      // and which of those are certain hits
+      if (left) {
+        if (lane == 0) s_sure[wid] = 0ull;
+        wave_sync_lds();
+        for (int q = lane; q < left; q += 64) {
+          const int job = s_job[wid][q];
+          const CullTri& A = s_u[wid].tri[job & 63];
+          const CullTri& B = s_u[wid].tri[(job >> 6) & 63];
+          if (cull_sure(A, B, (float)(A.eps + B.eps))) atomicOr(&s_sure[wid], 1ull << (job & 63));
+        }
+        wave_sync_lds();
+        if (in && (s_sure[wid] >> ts & ((1ull << l_nta) - 1ull)) != 0ull) my_settled = 1;
       }
       wave_sync_lds();  // read before the next group overwrites
+      t0 = t1, j0 = j1;
     }
-    if (lane < batch) D.np_hit[wl] = my_settled;
+    if (my_settled) my_keep = 0ull;
+    if (in_range) D.np_hit[wl] = my_settled;
     // The kept triangle pairs go straight to the level's item list, and the
     // children of node pairs that hit (settled) or may hit (kept pairs) to
     // the next list: one slot range each per block and round, one atomic
@@ -1154,15 +1237,33 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))
     // inner node pair's items only decide whether it expands (any FP64 hit):
     // its first kept item goes to the item list, the others (deferred) to
     // k_tri_def, which tests them only while the node pair has no hit.
-    const int kept = lane < batch ? __popcll(my_keep) : 0;
-    const bool defer = D.defer && l_inner != 0;
+    const int kept = __popcll(my_keep);
+    const int defer = D.defer && l_inner != 0 ? 1 : 0;
     const int mine = defer && kept > 1 ? 1 : kept, mdef = kept - mine;
-    const unsigned cmask =
-        lane < batch && (my_settled || my_keep != 0ull) ? child_mask(D, l_np, l_desc, l_offa, l_offb) : 0u;
-    const int nch = __popc(cmask);
-    const int incl = wave_incl_scan(mine), ich = wave_incl_scan(nch), idf = wave_incl_scan(mdef);
+    // The children: one per lane, 64 at a time; those spheres_apart_rel does
+    // not prove contact-free are listed.
+    const int cand = my_settled || kept ? (l_desc >> 1) & 15 : 0;
+    const int cand_incl = wave_incl_scan(cand), cands = rl(cand_incl, 63);
+    int nch = 0;
+    for (int q0 = 0; q0 < cands; q0 += 64) {
+      const int src = run_owner(s_own[wid], cand_incl - cand - q0, cand);
+      const int c = q0 + lane - __shfl(cand_incl - cand, src), desc = __shfl(l_desc, src);
+      const int pair = __shfl(l_pair, src), offa = __shfl(l_offa, src), offb = __shfl(l_offb, src);
+      bool keep = q0 + lane < cands;
+      if (keep && D.prune) {
+        const NP child = child_of(D.soup[w0 + src], desc, c, 0u);
+        float f[PF_FLOATS];
+        load_pose_f(D, pair, f);
+        keep = !spheres_apart_rel(f, D.nbound + NB_STRIDE * ((size_t)offa + child.na),
+                                  D.nbound + NB_STRIDE * ((size_t)offb + child.nb));
+      }
+      const unsigned long long m = __ballot(keep);
+      if (keep) s_u[wid].kid[nch + __popcll(m & lanes_below())] = (unsigned short)(c | src << 4);
+      nch += __popcll(m);
+    }
+    const int incl = wave_incl_scan(mine), idf = wave_incl_scan(mdef);
     const int par = it & 1;
-    if (lane == 63) s_tot[par][wid] = incl, s_ch[par][wid] = ich, s_df[par][wid] = idf;
+    if (lane == 63) s_tot[par][wid] = incl, s_ch[par][wid] = nch, s_df[par][wid] = idf;
     __syncthreads();
     if (threadIdx.x == 0) {  // one atomic for both ranges (same-address atomics from every block are costly)
       int sum = 0, sch = 0, sdf = 0;
@@ -1182,31 +1283,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))
       s_base[par] = base, s_chb[par] = chb, s_dfb[par] = dfb;
     }
     __syncthreads();
-    if (nch > 0) {
-      long long slot = (long long)s_chb[par] + ich - nch;
-      for (int v = 0; v < wid; ++v) slot += s_ch[par][v];
-      write_children(D, slot, l_np, l_desc, my_settled ? 0u : (uint32_t)(wl + 1), cmask);
+    long long cbase = (long long)s_chb[par];
+    for (int v = 0; v < wid; ++v) cbase += s_ch[par][v];
+    for (int q0 = 0; q0 < nch; q0 += 64) {
+      const int e = q0 + lane < nch ? s_u[wid].kid[q0 + lane] : 0, src = e >> 4;
+      const int desc = __shfl(l_desc, src), sure = __shfl(my_settled, src);
+      const long long slot = cbase + q0 + lane, w = w0 + src;
+      if (q0 + lane < nch && slot < D.cap_np)
+        D.soup_next[slot] = child_of(D.soup[w], desc, e & 15, sure ? 0u : (uint32_t)(w + 1));
     }
     long long base = (long long)s_base[par], dbase = (long long)s_dfb[par];
     for (int v = 0; v < wid; ++v) base += s_tot[par][v], dbase += s_df[par][v];
+    // the kept triangle pairs, one per lane, 64 at a time; a deferring node
+    // pair's first goes to the item list, its others to the deferred list
+    const int all_incl = incl + idf, all = rl(all_incl, 63), all_excl = all_incl - kept;
     const int excl = incl - mine, dexcl = idf - mdef;
-    const int defer_i = defer ? 1 : 0;
-    for (int k = 0; k < batch; ++k) {
-      const unsigned long long m = readlane_u64(my_keep, k);
-      if (m == 0ull) continue;
-      // deferring node pair: its lowest kept lane to the item list, the rest
-      // to the deferred list
-      const unsigned long long first = rl(defer_i, k) ? (m & (~m + 1ull)) : m;
-      const unsigned long long rest = m & ~first;
-      const DItem item{(uint32_t)(w0 + (long long)nw * k), (uint32_t)rl(l_pair, k),
-                       (uint32_t)(rl(l_offa, k) + rl(l_bka, k)), (uint32_t)(rl(l_offb, k) + rl(l_bkb, k)),
-                       (uint32_t)lane | (rl(l_inner, k) ? 256u : 0u)};
-      if ((first >> lane) & 1ull) {
-        const long long slot = base + rl(excl, k) + __popcll(first & lanes_below());
-        if (slot < D.cap_items) D.ditems[slot] = item;
-      } else if ((rest >> lane) & 1ull) {
-        const long long slot = dbase + rl(dexcl, k) + __popcll(rest & lanes_below());
-        if (slot < D.cap_items) D.ditems_def[slot] = item;
+    for (int q0 = 0; q0 < all; q0 += 64) {
+      const int src = run_owner(s_own[wid], all_excl - q0, kept);
+      const int r = q0 + lane - __shfl(all_excl, src);
+      const unsigned long long m = ((unsigned long long)(unsigned)__shfl((int)(my_keep >> 32), src) << 32) |
+                                   (unsigned)__shfl((int)(unsigned)my_keep, src);
+      const int ntb = __shfl(l_ntb, src), dfr = __shfl(defer, src);
+      const int at = __shfl(excl, src), dat = __shfl(dexcl, src);
+      const DItem item{(uint32_t)(w0 + src), (uint32_t)__shfl(l_pair, src),
+                       (uint32_t)__shfl(l_ga, src), (uint32_t)__shfl(l_gb, src),
+                       __shfl(l_inner, src) ? 256u : 0u};
+      if (q0 + lane < all) {
+        const int b = nth_bit(m, r), i = b / ntb, j = b - i * ntb;
+        const bool to_def = dfr && r > 0;
+        const long long slot = to_def ? dbase + dat + r - 1 : base + at + r;
+        if (slot < D.cap_items)
+          (to_def ? D.ditems_def : D.ditems)[slot] =
+              DItem{item.np, item.pair, item.ga, item.gb, item.sub | (uint32_t)(i << 3 | j)};
       }
     }
   }
@@ -3681,6 +3789,7 @@ struct d2_ctx {
   // pairs and clusters
   DBuf<int32_t> pairs, pair_info, cluster_of_pair;
   DBuf<double> max_time, pair_rec;
+  DBuf<float> pair_f;
   int n_pairs = 0, n_clusters = 0;
   // a pair list describes the uploaded bodies: a tree upload or a body upload
   // of another count invalidates it (and its clusters) until pairs come again
@@ -3927,6 +4036,7 @@ Dev make_dev(d2_ctx* c, int level, int discrete) {
   D.buckets = c->buckets.p;
   D.pair_info = c->pair_info.p;
   D.pair_rec = c->pair_rec.p;
+  D.pair_f = c->precision == D2_FP32 ? c->pair_f.p : nullptr;
   D.soup = c->soup_list[level & 1].p;
   D.conn = c->conn_list[level & 1].p;
   D.soup_next = c->soup_list[(level + 1) & 1].p;
@@ -3982,6 +4092,7 @@ int level_budget(const d2_ctx* c) { return std::min(MAX_LEVELS, c->pair_depth + 
 int prepare(d2_ctx* c) {
   const size_t np = (size_t)std::max(c->n_pairs, 1);
   const size_t g = (size_t)chunk_grid(c);
+  if (c->precision == D2_FP32) RC(ensure(c, c->pair_f, np * PF_STRIDE));
   for (int k = 0; k < 2; ++k) {
     RC(ensure(c, c->soup_list[k], c->cap));
     RC(ensure(c, c->conn_list[k], c->cap));
@@ -4801,7 +4912,7 @@ int d2_ctx_destroy(d2_ctx* c) {
   collect_timers(c);
   drop_graphs(c);
   release(c->nodes), release(c->buckets), release(c->fbuckets), release(c->stris), release(c->tree_off), release(c->body_tree), release(c->bodies);
-  release(c->pairs), release(c->pair_info), release(c->cluster_of_pair), release(c->max_time), release(c->pair_rec);
+  release(c->pairs), release(c->pair_info), release(c->cluster_of_pair), release(c->max_time), release(c->pair_rec), release(c->pair_f);
   for (int k = 0; k < 2; ++k) release(c->soup_list[k]), release(c->conn_list[k]);
   release(c->items), release(c->ditems), release(c->ditems_def), release(c->pt_items), release(c->ee_items), release(c->res), release(c->res_mask), release(c->np_hit), release(c->np_hit2), release(c->exp_desc);
   release(c->contacts), release(c->cnt), release(c->lvl), release(c->masks), release(c->conn_mask);

@@ -4097,7 +4097,7 @@ int prepare(d2_ctx* c) {
     RC(ensure(c, c->soup_list[k], c->cap));
     RC(ensure(c, c->conn_list[k], c->cap));
   }
-  RC(ensure(c, c->items, c->cap_items)); RC(ensure(c, c->pt_items, c->cap_items));
+  RC(ensure(c, c->items, c->cap_res)); RC(ensure(c, c->pt_items, c->cap_items));
   RC(ensure(c, c->ee_items, c->cap_items));
   if (c->precision == D2_FP32) {  // FP64: k_tri_full keeps no item list
     RC(ensure(c, c->ditems, c->cap_items));

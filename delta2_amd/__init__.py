@@ -47,7 +47,7 @@ class CapacityError(D2Error):
 
 
 class Tune(ctypes.Structure):
-    """Launch shapes (d2_tune): blocks of the chunked list kernels, of the
+    """Launch shapes (d2_tune): blocks of the list kernels, of the
     grid-stride kernels and of the per-pair post-processing."""
     _fields_ = [("chunk_blocks", ctypes.c_int), ("stream_blocks", ctypes.c_int), ("post_blocks", ctypes.c_int),
                 ("gate_phases", ctypes.c_int)]

@@ -220,10 +220,8 @@ D2_HD void corners_f(const tri<double>& T, float* c9) {
 // in world coordinates relative to b's start position at both ends (w[0..2]
 // a at t = 0, w[3..5] a at t = 1, w[6..8] b at t = 0, w[9..11] b at t = 1);
 // returns the magnitude of the transforms' inputs (the edge culls' extra).
-D2_HD float soup_world(const double* Ta0, const double* Ta1, const double* Tb0, const double* Tb1, const float* ca,
-                       const float* cb, float (*w)[3]) {
-  const M34f A0 = to_m34f(Ta0, Tb0), A1 = to_m34f(Ta1, Tb0);
-  const M34f B0 = to_m34f(Tb0, Tb0), B1 = to_m34f(Tb1, Tb0);
+D2_HD float soup_world(const M34f& A0, const M34f& A1, const M34f& B0, const M34f& B1, const float* ca, const float* cb,
+                       float (*w)[3]) {
   float extra = fmaxf(fmaxf(m34_mag(A0), m34_mag(A1)), m34_mag(B1));
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -233,14 +231,16 @@ D2_HD float soup_world(const double* Ta0, const double* Ta1, const double* Tb0, 
   }
   return extra;
 }
+D2_HD float soup_world(const double* Ta0, const double* Ta1, const double* Tb0, const double* Tb1, const float* ca,
+                       const float* cb, float (*w)[3]) {
+  return soup_world(to_m34f(Ta0, Tb0), to_m34f(Ta1, Tb0), to_m34f(Tb0, Tb0), to_m34f(Tb1, Tb0), ca, cb, w);
+}
 // The point-triangle slots: a's corners in b's frame against tb (its planes
 // sb, soup_tri), b's corners in a's frame against ta (sa).
-D2_HD unsigned soup_point_mask(const double* Mab0, const double* Mab1, const double* Mba0, const double* Mba1,
-                               const float* ca, const float* cb, const SoupTri& sa, const SoupTri& sb, float thr) {
+D2_HD unsigned soup_point_mask(const M34f& F0, const M34f& F1, const M34f& G0, const M34f& G1, const float* ca,
+                               const float* cb, const SoupTri& sa, const SoupTri& sb, float thr) {
   unsigned mask = 0u;
   float pa0[3][3], pa1[3][3], pb0[3][3], pb1[3][3];
-  const M34f F0 = to_m34f(Mab0, nullptr), F1 = to_m34f(Mab1, nullptr);
-  const M34f G0 = to_m34f(Mba0, nullptr), G1 = to_m34f(Mba1, nullptr);
   float mag = fmaxf(fmaxf(m34_mag(F0), m34_mag(F1)), fmaxf(m34_mag(G0), m34_mag(G1)));
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -268,7 +268,8 @@ D2_HD unsigned soup_cull_mask(const double* Ta0, const double* Ta1, const double
                               const tri<double>& ta, const tri<double>& tb, float thr) {
   float ca[9], cb[9];
   corners_f(ta, ca), corners_f(tb, cb);
-  unsigned mask = soup_point_mask(Mab0, Mab1, Mba0, Mba1, ca, cb, soup_tri(ta), soup_tri(tb), thr);
+  unsigned mask = soup_point_mask(to_m34f(Mab0, nullptr), to_m34f(Mab1, nullptr), to_m34f(Mba0, nullptr),
+                                  to_m34f(Mba1, nullptr), ca, cb, soup_tri(ta), soup_tri(tb), thr);
   float w[12][3];
   const float extra = soup_world(Ta0, Ta1, Tb0, Tb1, ca, cb, w);
   if (cull_tri_edges(w, w + 3, w + 6, w + 9, thr, extra)) return mask;  // all nine edge pairs culled at once

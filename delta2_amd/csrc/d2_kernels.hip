@@ -6,22 +6,20 @@
 // uneven the pairs are:
 //
 //   CCD level (compareTreesFullContinuous, full_tree_comparison.h:69-219)
-//     soup_cull    one wavefront per soup node pair, lane = triangle pair
-//                  (8x8): swept-AABB test, ballot/popcount compaction of the
-//                  overlapping triangle pairs into an item list
-//     soup_sub     one thread per (item, point-triangle sub-test)  6 per item,
-//                  and (other blocks) per (item, edge-edge sub-test) 9 per item
+//     ccd_cull     soup list: swept-AABB tests of the node pairs' triangle
+//                  pairs, the overlapping ones to the item list; connected
+//                  (leaf-leaf) list, other blocks: the leaf sub-tests the FP32
+//                  culls leave
+//     soup_keep    (FP32 form) one thread per item: the sub-tests the FP32
+//                  culls leave
+//     ccd_sub      one thread per FP64 sub-test, soup and leaf, point-triangle
+//                  and edge-edge; a leaf sub-test that hits is a contact
 //     soup_reduce  one thread per item: the reference's ordered selection of
-//                  the 15 sub-results, hit test, leaf-pair contact emission
-//     expand       one thread per node pair: children of hit node pairs
-//     leaf_enum    one wavefront per leaf-leaf node pair: enumerates its
-//                  vertex-triangle and edge-edge sub-tests
-//     leaf_sub     one thread per sub-test (point-triangle blocks, edge-edge
-//                  blocks), hit -> contact
+//                  the 15 sub-results, hit test, leaf-pair contact emission;
+//                  the children of hit node pairs to the next lists
 //   Discrete level (compareTreesFull, full_tree_comparison.h:13-67)
-//     tri_mask     one wavefront per node pair, lane = triangle pair: FP32
-//                  cull (or keep-all in FP64 mode), kept pairs to the item
-//                  list, children of node pairs that hit or may hit to the
+//     tri_mask     groups of 64 triangles per wavefront, lane = triangle pair:
+//                  FP32 cull, kept pairs to the item list, children of node pairs that hit or may hit to the
 //                  next list (dropped there if the parent did not hit)
 //     tri_dist     one thread per item: FP64 _comparisonDist, hit -> contact
 //                  (leaf-leaf) or the node pair's hit flag
@@ -98,6 +96,13 @@ enum : int {
   PR_STRIDE = 152
 };
 constexpr int PF_STRIDE = 32;  // PF_FLOATS in a cache line of their own
+// The CCD culls' pair record: eight 3x4 float matrices -- a's and b's poses at
+// both ends with b's start position as origin, and the frame changes -- and the
+// search distance.
+enum : int {
+  CF_A0 = 0, CF_A1 = 12, CF_B0 = 24, CF_B1 = 36, CF_MAB0 = 48, CF_MAB1 = 60, CF_MBA0 = 72, CF_MBA1 = 84,
+  CF_SEARCH = 96, CF_STRIDE = 100
+};
 constexpr int BUCKET = 88;
 constexpr int RES_SLOTS = 15;  // sub-results per soup triangle pair
 // Global counters (atomics) and per-level sizes.  Level L reads its list sizes
@@ -209,6 +214,58 @@ __device__ __forceinline__ int nth_bit(unsigned long long m, int r) {
   return pos;
 }
 
+// Walks a batch of up to 64 entries, one per lane, each wanting `slots` lanes
+// (at most 64; 0: none) and holding `jobs` jobs, in groups of consecutive
+// entries of at most 64 slots.  After next(): whether this lane's entry is in
+// the group, its first slot and job there, and the group's totals.  All lanes
+// call it.
+struct Groups {
+  int slots, jobs, slot_incl, job_incl, t0 = 0, j0 = 0;
+  bool in = false;
+  int ts = 0, js = 0, n_slots = 0, n_jobs = 0;
+  __device__ __forceinline__ Groups(int slots_, int jobs_) : slots(slots_), jobs(jobs_) {
+    slot_incl = wave_incl_scan(slots), job_incl = wave_incl_scan(jobs);
+  }
+  // fill: a few jobs over a multiple of 64 wait for the next group (an entry
+  // has at most 64 jobs)
+  __device__ __forceinline__ bool next(bool fill) {
+    if (t0 >= rl(slot_incl, 63)) return false;
+    ts = slot_incl - slots - t0, js = job_incl - jobs - j0;
+    in = slots > 0 && ts >= 0 && ts + slots <= 64;
+    int last = 63 - __clzll((long long)__ballot(in));
+    if (fill) {
+      const int over = rl(job_incl, last) - j0;
+      if (over > 64 && (over & 63) < 40) {
+        in = in && js + jobs <= (over & ~63);
+        last = 63 - __clzll((long long)__ballot(in));
+      }
+    }
+    n_slots = rl(slot_incl, last) - t0, n_jobs = rl(job_incl, last) - j0;
+    t0 += n_slots, j0 += n_jobs;
+    return true;
+  }
+  // This lane's entry's share (from bit 0) of 64 answers, the group's jobs
+  // from q0 on.
+  __device__ __forceinline__ unsigned long long share(unsigned long long answers, int q0) const {
+    const int d = js - q0;
+    if (!in || d >= 64 || d + jobs <= 0) return 0ull;
+    return (d >= 0 ? answers >> d : answers << -d) & (jobs < 64 ? (1ull << jobs) - 1ull : ~0ull);
+  }
+};
+// Tiles of a list of n entries over nblk blocks of nw wavefronts: up to 64
+// consecutive entries per wavefront, a block's wavefronts taking consecutive
+// ones, a block every nblk-th tile.
+struct Tiles {
+  long long n, step, b0;
+  int part;
+  __device__ __forceinline__ Tiles(long long n_, int blk, int nblk, int nw) : n(n_) {
+    const long long waves = (long long)nblk * nw;
+    part = n < 64 * waves ? (int)((n + waves - 1) / waves) : 64;
+    step = waves * part, b0 = (long long)blk * nw * part;
+  }
+  __device__ __forceinline__ long long first(int wid) const { return b0 + (long long)part * wid; }
+};
+
 // arr[key] = min(arr[key], v) for every lane (key -1: none).  Most lanes of a
 // wavefront often share one key (a pile is one cluster), and atomics on one
 // address take turns (6 ns each here): the lanes of the first keys met are
@@ -254,7 +311,7 @@ struct Dev {
   // pairs
   const int32_t* pair_info;  // a, b, node offset a, node offset b
   const double* pair_rec;
-  float* pair_f;               // FP32 form, discrete phase: pair_pose_f32 per pair (PF_STRIDE)
+  float* pair_f;               // FP32 form, per pair: pair_pose_f32 (discrete), the CF_ record (CCD)
   // work lists
   NP* soup;
   NP* conn;
@@ -263,8 +320,10 @@ struct Dev {
   Item* items;
   DItem* ditems;
   DItem* ditems_def;           // FP32 form: deferred items of inner node pairs (k_tri_def)
-  Item* pt_items;
+  Item* pt_items;              // CCD soup sub-tests that survive the FP32 culls, point and edge
   Item* ee_items;
+  Item* lpt_items;             // CCD leaf sub-tests, point and edge
+  Item* lee_items;
   double* res;  // [items][15][8]
   unsigned* res_mask;  // FP32 form: per soup item, the slots its FP32 culls keep
   int* np_hit;
@@ -274,10 +333,6 @@ struct Dev {
   ContactRec* contacts;
   unsigned long long* cnt;
   unsigned long long* lvl;
-  // per node pair counts, masks, and per-block partial sums of the counts
-  unsigned long long* masks;
-  int *cnt_a, *cnt_s, *cnt_c, *cnt_pt, *cnt_ee;
-  int *part_a, *part_s, *part_c, *part_pt, *part_ee;
   // per pair, min toc of the soup / connected pass (bits) and "a leaf pair
   // had hits in this pass"
   unsigned long long *pass_min_s, *pass_min_c;
@@ -291,7 +346,7 @@ struct Dev {
   int prune;                   // skip node pairs nodes_apart proves contact-free
   int defer;                   // FP32 form: inner node pairs send one item to k_tri_dist, the rest to k_tri_def
   int box_test;                // FP32 form: k_tri_mask tests arriving node pairs with boxes_apart_faces
-  unsigned long long* conn_mask;  // per connected node pair: surviving leaf sub-tests
+  int conn_blocks;             // CCD: the last blocks of k_ccd_cull, which take the connected list
   const int32_t* body_tree;
   int fp32;                    // FP32 culls of the CCD leaf sub-tests
   int n_pairs;
@@ -472,8 +527,19 @@ __global__ void __launch_bounds__(256) k_setup(Dev D, const int32_t* pairs, cons
         k[6] = so.t.x, k[7] = so.t.y, k[8] = so.t.z;  // PR_XA / PR_XB
       }
     }
-    if (!ccd && D.pair_f && end) {
-      // pair_pose_f32, each lane the half it has the pose of
+    if (D.pair_f && ccd) {  // the culls' record, each lane the two matrices it computed
+      float* f = D.pair_f + (size_t)CF_STRIDE * p;
+      const double org[3] = {rb[4], rb[5], rb[6]};  // b's start position
+      const double* M = pr + (of_a ? (end ? PR_MAB1 : PR_MAB0) : (end ? PR_MBA1 : PR_MBA0));
+      float* fw = f + (of_a ? (end ? CF_A1 : CF_A0) : (end ? CF_B1 : CF_B0));
+      float* fm = f + (of_a ? (end ? CF_MAB1 : CF_MAB0) : (end ? CF_MBA1 : CF_MBA0));
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          fw[4 * r + k] = (float)(k < 3 ? To[4 * r + k] : To[4 * r + 3] - org[r]), fm[4 * r + k] = (float)M[4 * r + k];
+      if (q == 0) f[CF_SEARCH] = (float)(ra[37] + rb[37]);
+    } else if (D.pair_f && end) {  // pair_pose_f32, each lane the half it has the pose of
       float* f = D.pair_f + (size_t)PF_STRIDE * p;
       const double t[3] = {so.t.x - sx.t.x, so.t.y - sx.t.y, so.t.z - sx.t.z};
 #pragma unroll
@@ -553,98 +619,6 @@ __device__ __forceinline__ void swept_box(const tri<double>& t, const double* m0
     o[k] = smin(lo, lo2) - g, o[3 + k] = smax(hi, hi2) + g;
   }
 }
-// One wavefront per soup node pair (chunked ranges), lane = triangle pair:
-// swept-AABB overlap mask, its popcount and the block partial; also folds the
-// connected pass of the previous level.  Lanes 0-7 build the swept boxes of
-// bucket a's triangles, lanes 8-15 bucket b's, into LDS; each triangle pair
-// then compares two of them.
-__global__ void __launch_bounds__(256) k_soup_cull(Dev D) {
-  __shared__ double s_box[4][16][6];
-  fold_pass(D, D.pair_rec, D.pass_min_c, D.pass_flag_c);
-  const long long n = D.n_soup();
-  const int lane = lane_id();
-  long long rb, re;
-  chunk_of(n, rb, re);
-  long long acc = 0;
-  // the wavefront index made visibly uniform: the node pair's record, nodes
-  // and poses then come through scalar loads into scalar registers
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  for (long long w = rb + wv; w < re; w += (blockDim.x >> 6)) {
-    NP np = D.soup[w];
-    const int32_t* pi = D.pair_info + 4 * np.pair;
-    const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
-    const NodeRec na = D.nodes[pi[2] + np.na];
-    const NodeRec nb = D.nodes[pi[3] + np.nb];
-    if (lane < 16) {
-      const bool side = lane >= 8;
-      const int k = lane & 7;
-      if (k < (side ? nb.ntris : na.ntris)) {
-        const double* bk = D.buckets + (size_t)BUCKET * (side ? pi[3] + nb.bucket : pi[2] + na.bucket);
-        swept_box(load_tri<double>(bk, k), side ? pr + PR_TB0 : pr + PR_TA0, side ? pr + PR_TB1 : pr + PR_TA1,
-                  side ? pr[PR_GEOB] : pr[PR_GEOA], s_box[wv][lane]);
-      }
-    }
-    wave_sync_lds();
-    int i = lane >> 3, j = lane & 7;
-    bool ok = i < na.ntris && j < nb.ntris;
-    bool hit = false;
-    if (ok) {
-      const double* A = s_box[wv][i];
-      const double* B = s_box[wv][8 + j];
-      hit = true;
-      for (int k = 0; k < 3; ++k) {  // bbox.h:8-23, a is "this"
-        bool o = (B[k] < A[k]) ? (B[3 + k] > A[k]) : (B[k] < A[3 + k]);
-        hit = hit && o;
-      }
-    }
-    wave_sync_lds();  // read before the next node pair overwrites
-    const unsigned long long m = __ballot(hit);
-    if (lane == 0) {
-      D.masks[w] = m;
-      D.cnt_a[w] = __popcll(m);
-      D.np_hit[w] = 0;
-      acc += __popcll(m);
-    }
-  }
-  // The overlapping triangle pairs of the block's range to the level's item
-  // list: one slot range per block (one atomic), in node-pair order within
-  // it; the list's order is free (contacts carry their emission keys).
-  __shared__ int toff[256];
-  __shared__ unsigned long long s_base;
-  const long long tot = block_sum(acc);
-  if (threadIdx.x == 0) {
-    unsigned long long base = 0;
-    if (tot) {
-      base = atomicAdd(&D.lvl[D.level * LV_STRIDE + LV_ITEMS], (unsigned long long)tot);
-      atomicAdd(&D.cnt[C_LVL_ITEMS], (unsigned long long)tot);
-      if ((long long)(base + tot) > D.cap_res) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
-    }
-    s_base = base;
-  }
-  __syncthreads();
-  if (tot == 0) return;
-  const int wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  long long carry = (long long)s_base;
-  for (long long t0 = rb; t0 < re; t0 += blockDim.x) {
-    const long long w = t0 + threadIdx.x;
-    int tile_total;
-    const int ex = block_scan(w < re ? D.cnt_a[w] : 0, tile_total);
-    toff[threadIdx.x] = ex;
-    __syncthreads();
-    const int in_tile = (int)((re - t0) < (long long)blockDim.x ? (re - t0) : (long long)blockDim.x);
-    for (int j = wid; j < in_tile; j += nw) {
-      const long long ww = t0 + j;
-      const unsigned long long m = D.masks[ww];
-      if ((m >> lane) & 1ull) {
-        const long long slot = carry + toff[j] + __popcll(m & lanes_below());
-        if (slot < D.cap_res) D.items[slot] = Item{(uint32_t)ww, (uint32_t)lane};
-      }
-    }
-    carry += tile_total;
-    __syncthreads();
-  }
-}
-
 __device__ __forceinline__ void store_res(double* r, double d, v3<double> P, v3<double> Q, double toc) {
   r[0] = d, r[1] = toc, r[2] = P.x, r[3] = P.y, r[4] = P.z, r[5] = Q.x, r[6] = Q.y, r[7] = Q.z;
 }
@@ -689,12 +663,300 @@ __device__ __forceinline__ SoupTri load_soup_tri(const float* st, size_t t) {
   S.m[7] = q2.w, S.m[8] = q3.x, S.o[0] = q3.y, S.o[1] = q3.z, S.o[2] = q3.w, S.eo = q4.x;
   return S;
 }
+// What a wavefront of k_ccd_cull keeps in LDS: the soup list's part, the
+// group's swept boxes and triangle pairs (slot of a's, slot of b's << 6); the
+// connected list's, the group's vertices at both ends (world, then the other
+// body's frame), its triangles' planes, per node pair the largest magnitude
+// (bits), and the surviving sub-tests on their way out.
+constexpr int LEAF_PT_BUF = 128, LEAF_EE_BUF = 256;
+union CullShare {
+  struct {
+    double box[64][6];
+    unsigned short job[256];
+  } s;
+  struct {
+    float v[64][12];
+    float t[21][20];
+    unsigned mag[64];
+    Item pt[LEAF_PT_BUF], ee[LEAF_EE_BUF];
+  } c;
+};
+// Soup list: per node pair the triangle pairs whose swept AABBs overlap, in
+// groups of at most 64 triangles: a lane builds one swept box, then the
+// triangle pairs compare boxes one per lane.  The overlapping ones go to the
+// level's item list, one slot range per block and round; the list's order is
+// free (contacts carry their emission keys).
+__device__ __forceinline__ void soup_cull_part(Dev& D, int nblk, CullShare& S, unsigned char* own) {
+  __shared__ int s_tot[2][4];
+  __shared__ unsigned long long s_base[2];
+  const int lane = lane_id(), wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const long long n = D.n_soup();
+  int it = 0;
+  for (Tiles T(n, blockIdx.x, nblk, 4); T.b0 < n; T.b0 += T.step, ++it) {
+    const long long w0 = T.first(wid), wl = w0 + lane;
+    const bool in_range = lane < T.part && wl < n;
+    int l_pair = 0, l_ga = 0, l_gb = 0, l_nta = 0, l_ntb = 0;
+    if (in_range) {
+      const NP np = D.soup[wl];
+      const int32_t* pi = D.pair_info + 4 * np.pair;
+      const NodeRec na = D.nodes[pi[2] + np.na];
+      const NodeRec nb = D.nodes[pi[3] + np.nb];
+      l_pair = (int)np.pair, l_ga = pi[2] + na.bucket, l_gb = pi[3] + nb.bucket, l_nta = na.ntris, l_ntb = nb.ntris;
+      D.np_hit[wl] = 0;
+    }
+    unsigned long long my_keep = 0;  // bit i * l_ntb + j
+    const int my_jobs = l_nta * l_ntb;
+    for (Groups g(my_jobs > 0 ? l_nta + l_ntb : 0, my_jobs); g.next(true);) {
+      const int src = run_owner(own, g.ts, g.in ? g.slots : 0);
+      const int start = __shfl(g.ts, src), jstart = __shfl(g.js, src);
+      const int pair = __shfl(l_pair, src), nta = __shfl(l_nta, src), ntb = __shfl(l_ntb, src);
+      const int ga = __shfl(l_ga, src), gb = __shfl(l_gb, src);
+      if (lane < g.n_slots) {
+        const int x = lane - start;
+        const bool side = x >= nta;
+        const int k = side ? x - nta : x;
+        const double* pr = D.pair_rec + (size_t)PR_STRIDE * pair;
+        const double* bk = D.buckets + (size_t)BUCKET * (side ? gb : ga);
+        swept_box(load_tri<double>(bk, k), side ? pr + PR_TB0 : pr + PR_TA0, side ? pr + PR_TB1 : pr + PR_TA1,
+                  side ? pr[PR_GEOB] : pr[PR_GEOA], S.s.box[lane]);
+        if (!side)
+          for (int j = 0; j < ntb; ++j)
+            S.s.job[jstart + k * ntb + j] = (unsigned short)(lane | ((start + nta + j) << 6));
+      }
+      wave_sync_lds();
+      for (int q0 = 0; q0 < g.n_jobs; q0 += 64) {
+        bool hit = false;
+        if (q0 + lane < g.n_jobs) {
+          const int job = S.s.job[q0 + lane];
+          const double* A = S.s.box[job & 63];
+          const double* B = S.s.box[job >> 6];
+          hit = true;
+          for (int k = 0; k < 3; ++k) {  // bbox.h:8-23, a is "this"
+            const bool o = (B[k] < A[k]) ? (B[3 + k] > A[k]) : (B[k] < A[3 + k]);
+            hit = hit && o;
+          }
+        }
+        my_keep |= g.share(__ballot(hit), q0);
+      }
+      wave_sync_lds();  // read before the next group overwrites
+    }
+    const int kept = __popcll(my_keep), incl = wave_incl_scan(kept), all = rl(incl, 63), par = it & 1;
+    if (lane == 0) s_tot[par][wid] = all;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int tot = s_tot[par][0] + s_tot[par][1] + s_tot[par][2] + s_tot[par][3];
+      unsigned long long base = 0;
+      if (tot) {
+        base = atomicAdd(&D.lvl[D.level * LV_STRIDE + LV_ITEMS], (unsigned long long)tot);
+        atomicAdd(&D.cnt[C_LVL_ITEMS], (unsigned long long)tot);
+        if ((long long)(base + tot) > D.cap_res) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
+      }
+      s_base[par] = base;
+    }
+    __syncthreads();
+    long long base = (long long)s_base[par];
+    for (int v = 0; v < wid; ++v) base += s_tot[par][v];
+    for (int q0 = 0; q0 < all; q0 += 64) {
+      const int src = run_owner(own, incl - kept - q0, kept);
+      const int r = q0 + lane - __shfl(incl - kept, src), ntb = __shfl(l_ntb, src);
+      const unsigned long long m = ((unsigned long long)(unsigned)__shfl((int)(my_keep >> 32), src) << 32) |
+                                   (unsigned)__shfl((int)(unsigned)my_keep, src);
+      if (q0 + lane < all && base + q0 + lane < D.cap_res) {
+        const int b = nth_bit(m, r), i = b / ntb;
+        D.items[base + q0 + lane] = Item{(uint32_t)(w0 + src), (uint32_t)(i << 3 | (b - i * ntb))};
+      }
+    }
+  }
+}
+
+// ------------------------------------------- FP32 culls of CCD leaf sub-tests
+// The bounds of d2_cull.hpp (soup_point_keep: plane side and edge
+// half-planes with each triangle's FP64-derived normals and its
+// float-barycentric acceptance bound; cull_edge_edge: separating axes).
+//
+// Connected list: the leaf sub-tests of every node pair (6nm point, 9nm edge;
+// the FP64 form keeps all) that the culls leave, to the level's two lists, in
+// groups of node pairs with at most 64 vertices: a lane transforms one vertex
+// (both ends, in world coordinates relative to b's start position and in the
+// other body's frame), another reads a triangle's planes, then the sub-tests
+// go one per lane, 64 at a time.  A leaf pair has about 13 vertices, 27 point
+// and 40 edge sub-tests: with a pass per node pair, most of its time was the
+// latency of the loads and 27 to 60 shuffles per sub-test (a pile's 2.7 M soup
+// and 2.6 M connected node pairs: 3.1 + 5.7 + 2.1 ms for the soup list, these
+// culls and their lists, 3.7 ms for all in this launch).
+// Survivors wait in LDS and leave together (an atomic on one address takes 6
+// ns of its turn).
+__device__ __forceinline__ M34f load_m34f(const float* p) {
+  const float4* q = reinterpret_cast<const float4*>(p);
+  const float4 a = q[0], b = q[1], c = q[2];
+  return M34f{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y, c.z, c.w}};
+}
+// Up to 64 sub-tests more to a wavefront's buffer of cap, which goes to the
+// list when another 64 might not fit.  All lanes call it.
+__device__ __forceinline__ void leaf_push(const Dev& D, bool keep, Item item, Item* buf, int cap, int& held, int slot_id,
+                                          Item* list) {
+  const unsigned long long m = __ballot(keep);
+  if (keep) buf[held + __popcll(m & lanes_below())] = item;
+  held += __popcll(m);
+  if (held <= cap - 64) return;
+  wave_sync_lds();
+  unsigned long long base = 0;
+  if (lane_id() == 0) {
+    base = atomicAdd(&D.lvl[D.level * LV_STRIDE + slot_id], (unsigned long long)held);
+    if ((long long)(base + held) > D.cap_items) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
+  }
+  base = readlane_u64(base, 0);
+  for (int i = lane_id(); i < held; i += 64)
+    if ((long long)base + i < D.cap_items) list[base + i] = buf[i];
+  held = 0;
+  wave_sync_lds();
+}
+__device__ __forceinline__ void leaf_cull_part(Dev& D, CullShare& S, unsigned char* own) {
+  __shared__ int s_held[2][4];
+  __shared__ unsigned long long s_out[2];
+  const int lane = lane_id(), wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const long long n = D.n_conn();
+  int held_pt = 0, held_ee = 0;
+  for (Tiles T(n, (int)blockIdx.x - ((int)gridDim.x - D.conn_blocks), D.conn_blocks, 4); T.b0 < n; T.b0 += T.step) {
+    const long long w0 = T.first(wid), wl = w0 + lane;
+    int l_pair = 0, l_ta = 0, l_tb = 0, l_n = 0, l_m = 0;  // l_ta, l_tb: global triangle 0 of the two leaves
+    float l_thr = 0.f;
+    if (lane < T.part && wl < n) {
+      const NP np = D.conn[wl];
+      const int32_t* pi = D.pair_info + 4 * np.pair;
+      const NodeRec na = D.nodes[pi[2] + np.na];
+      const NodeRec nb = D.nodes[pi[3] + np.nb];
+      l_pair = (int)np.pair, l_ta = 8 * (pi[2] + na.bucket), l_tb = 8 * (pi[3] + nb.bucket), l_n = na.ntris, l_m = nb.ntris;
+      if (D.fp32) l_thr = D.pair_f[(size_t)CF_STRIDE * np.pair + CF_SEARCH];
+    }
+    const int nm = l_n * l_m;
+    // s / n and s / m of sub-test numbers below 576 by multiplication: exact,
+    // the error s (65536 / d rounded up - 65536 / d) stays below 576 * 8 / 65536
+    const int inv_n = nm ? (65536 + l_n - 1) / l_n : 0, inv_m = nm ? (65536 + l_m - 1) / l_m : 0;
+    for (Groups g(nm > 0 ? 3 * (l_n + l_m) : 0, nm); g.next(false);) {
+      if (D.fp32) {
+        const int src = run_owner(own, g.ts, g.in ? g.slots : 0);
+        const int x = lane - __shfl(g.ts, src);
+        const int na = __shfl(l_n, src), ta = __shfl(l_ta, src), tb = __shfl(l_tb, src), pair = __shfl(l_pair, src);
+        S.c.mag[lane] = 0u;
+        wave_sync_lds();
+        const bool of_b = x >= 3 * na;
+        const int v = of_b ? x - 3 * na : x, tri = v / 3;
+        const size_t tk = (size_t)(of_b ? tb : ta) + tri;
+        if (lane < g.n_slots) {
+          const float* pf = D.fbuckets + (size_t)FB_STRIDE * tk + 3 * (v - 3 * tri);
+          const float p[3] = {pf[0], pf[1], pf[2]};  // the corner rounded to float
+          const float* cf = D.pair_f + (size_t)CF_STRIDE * pair;
+          const M34f W0 = load_m34f(cf + (of_b ? CF_B0 : CF_A0)), W1 = load_m34f(cf + (of_b ? CF_B1 : CF_A1));
+          const M34f F0 = load_m34f(cf + (of_b ? CF_MBA0 : CF_MAB0)), F1 = load_m34f(cf + (of_b ? CF_MBA1 : CF_MAB1));
+          float o[12];
+          xf_f(W0, p, o), xf_f(W1, p, o + 3), xf_f(F0, p, o + 6), xf_f(F1, p, o + 9);
+          float mag = fmaxf(fmaxf(amax3(o), amax3(o + 3)), fmaxf(amax3(o + 6), amax3(o + 9)));
+          mag = fmaxf(mag, fmaxf(fmaxf(fmaxf(m34_mag(W0), m34_mag(W1)), fmaxf(m34_mag(F0), m34_mag(F1))), amax3(p)));
+#pragma unroll
+          for (int q = 0; q < 12; ++q) S.c.v[lane][q] = o[q];
+          atomicMax(&S.c.mag[src], __float_as_uint(mag));
+        }
+        // the triangle of vertex slots 3 t .. 3 t + 2, by lane t
+        const int tt = __shfl((int)tk, lane < 21 ? 3 * lane : 63);
+        if (3 * lane < g.n_slots) {
+          const SoupTri t = load_soup_tri(D.stris, (size_t)tt);
+          float* o = S.c.t[lane];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) o[q] = t.n[q], o[13 + q] = t.o[q];
+          o[3] = t.d, o[16] = t.eo;
+#pragma unroll
+          for (int q = 0; q < 9; ++q) o[4 + q] = t.m[q];
+        }
+        wave_sync_lds();
+      }
+      for (int q0 = 0; q0 < 6 * g.n_jobs; q0 += 64) {  // point sub-tests
+        const int src = run_owner(own, 6 * g.js - q0, g.in ? 6 * g.jobs : 0);
+        const int sub = q0 + lane - 6 * __shfl(g.js, src);
+        bool keep = q0 + lane < 6 * g.n_jobs;
+        if (D.fp32) {
+          const int na = __shfl(l_n, src), nb = __shfl(l_m, src), vs = __shfl(g.ts, src);
+          const int in_ = __shfl(inv_n, src), im = __shfl(inv_m, src);
+          const float thr = __shfl(l_thr, src);
+          if (keep) {
+            const float margin = 1e-6f + 64.f * 5.9604645e-08f * __uint_as_float(S.c.mag[src]);
+            const bool of_b = sub >= 3 * na * nb;  // vertex of b against triangle of a
+            const int s2 = of_b ? sub - 3 * na * nb : sub;
+            const int v = (s2 * (of_b ? in_ : im)) >> 16, k = s2 - v * (of_b ? na : nb);
+            const float* f = S.c.v[vs + (of_b ? 3 * na : 0) + v] + 6;
+            const float* o = S.c.t[vs / 3 + (of_b ? 0 : na) + k];
+            SoupTri t;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) t.n[q] = o[q], t.o[q] = o[13 + q];
+            t.d = o[3], t.eo = o[16];
+#pragma unroll
+            for (int q = 0; q < 9; ++q) t.m[q] = o[4 + q];
+            keep = soup_point_keep(f, f + 3, t, thr, margin);
+          }
+        }
+        leaf_push(D, keep, Item{(uint32_t)(w0 + src), (uint32_t)sub}, S.c.pt, LEAF_PT_BUF, held_pt, LV_PT, D.lpt_items);
+      }
+      for (int q0 = 0; q0 < 9 * g.n_jobs; q0 += 64) {  // edge sub-tests
+        const int src = run_owner(own, 9 * g.js - q0, g.in ? 9 * g.jobs : 0);
+        const int sub = q0 + lane - 9 * __shfl(g.js, src);
+        bool keep = q0 + lane < 9 * g.n_jobs;
+        if (D.fp32) {
+          const int na = __shfl(l_n, src), nb = __shfl(l_m, src), vs = __shfl(g.ts, src), im = __shfl(inv_m, src);
+          const float thr = __shfl(l_thr, src);
+          if (keep) {
+            const float mag = __uint_as_float(S.c.mag[src]);
+            const int ea = ((sub * im) >> 16) / 3, eb = sub - 3 * nb * ea;
+            const int a1 = ea % 3 == 2 ? ea - 2 : ea + 1, b1 = eb % 3 == 2 ? eb - 2 : eb + 1;
+            const float* pa0 = S.c.v[vs + ea];
+            const float* pa1 = S.c.v[vs + a1];
+            const float* pb0 = S.c.v[vs + 3 * na + eb];
+            const float* pb1 = S.c.v[vs + 3 * na + b1];
+            keep = !cull_edge_edge(pa0, pa1, pa0 + 3, pa1 + 3, pb0, pb1, pb0 + 3, pb1 + 3, thr, mag);
+          }
+        }
+        leaf_push(D, keep, Item{(uint32_t)(w0 + src), (uint32_t)sub}, S.c.ee, LEAF_EE_BUF, held_ee, LV_EE, D.lee_items);
+      }
+      wave_sync_lds();  // read before the next group overwrites
+    }
+  }
+  // what is still held, one slot range per block and list
+  if (lane == 0) s_held[0][wid] = held_pt, s_held[1][wid] = held_ee;
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const int* h = s_held[threadIdx.x];
+    const int tot = h[0] + h[1] + h[2] + h[3];
+    unsigned long long base = 0;
+    if (tot) {
+      base = atomicAdd(&D.lvl[D.level * LV_STRIDE + (threadIdx.x ? LV_EE : LV_PT)], (unsigned long long)tot);
+      if ((long long)(base + tot) > D.cap_items) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
+    }
+    s_out[threadIdx.x] = base;
+  }
+  __syncthreads();
+  long long bp = (long long)s_out[0], be = (long long)s_out[1];
+  for (int v = 0; v < wid; ++v) bp += s_held[0][v], be += s_held[1][v];
+  for (int i = lane; i < held_pt; i += 64)
+    if (bp + i < D.cap_items) D.lpt_items[bp + i] = S.c.pt[i];
+  for (int i = lane; i < held_ee; i += 64)
+    if (be + i < D.cap_items) D.lee_items[be + i] = S.c.ee[i];
+}
+// The level's two lists in one launch: the last conn_blocks blocks take the
+// connected list, the others the soup list; all fold the previous level's
+// passes, which are complete.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) k_ccd_cull(Dev D) {
+  __shared__ CullShare s_share[4];
+  __shared__ unsigned char s_own[4][64];
+  fold_pass(D, D.pair_rec, D.pass_min_s, D.pass_flag_s);
+  fold_pass(D, D.pair_rec, D.pass_min_c, D.pass_flag_c);
+  const int wid = threadIdx.x >> 6, nblk = (int)gridDim.x - D.conn_blocks;
+  if ((int)blockIdx.x < nblk) soup_cull_part(D, nblk, s_share[wid], s_own[wid]);
+  else leaf_cull_part(D, s_share[wid], s_own[wid]);
+}
+
 // ------------------------------------------- FP32 culls of CCD soup sub-tests
 // FP32 form: one thread per soup item (triangle pair) runs the FP32 bounds of
 // its 15 sub-tests (k_soup_keep), keeps a 15-bit mask of the survivors per
-// item and appends them to two compact lists (point and edge sub-tests, the
-// leaf level's item lists, which this level's connected pass fills only
-// later); the FP64 sub-tests then run over those lists only, in full
+// item and appends them to two compact lists (point and edge sub-tests); the FP64 sub-tests then run over those lists only, in full
 // wavefronts, and k_soup_reduce selects over the surviving slots.  A culled
 // sub-test provably reports no distance below the search distance, so it
 // cannot be the winner of a hit (its slot would hold +inf, toc 1, which the
@@ -712,13 +974,16 @@ constexpr unsigned SOUP_EE_BITS = 0x739Cu;  // slots 5k+2+l (edge k of a, edge l
 // and, for the items it leaves, the per-edge culls packed over the
 // wavefront, nine per item, with the items' world corners staged in LDS),
 // then the two compact sub-test lists (wavefront prefix sums, one atomic per
-// wavefront and list; the lists' order is free, results go to fixed slots).
+// block and list; the lists' order is free, results go to fixed slots).
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) k_soup_keep(Dev D) {
   __shared__ float s_w[4][64][36];        // per wavefront: world corners of the items left for the per-edge culls
   __shared__ float s_thr[4][64];          // their search distances
   __shared__ float s_ex[4][64];           // and their transforms' input magnitudes
   __shared__ unsigned char s_fl[4][64];   // their lanes
   __shared__ unsigned s_em[4][64];        // per lane: surviving edge slots
+  __shared__ int s_pt[2][4], s_ee[2][4];  // survivors per wavefront and list
+  __shared__ unsigned long long s_at[2][2];
+  int par = 0;
   const long long n = D.n_res();
   const int lane = lane_id(), wv = threadIdx.x >> 6;
   unsigned long long* cpt = D.lvl + D.level * LV_STRIDE + LV_SPT;
@@ -726,13 +991,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
   for (long long b0 = (long long)blockIdx.x * blockDim.x; b0 < n; b0 += (long long)gridDim.x * blockDim.x) {
     const long long it = b0 + threadIdx.x;
     bool need = false;
-    const double* pr = nullptr;
+    const float* cf = nullptr;
     size_t ga = 0, gb = 0;  // global triangle indices (node * 8 + k) of the item's two triangles
     if (it < n) {
       const Item item = D.items[it];
       const NP np = D.soup[item.np];
       const int32_t* pi = D.pair_info + 4 * np.pair;
-      pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
+      cf = D.pair_f + (size_t)CF_STRIDE * np.pair;
       ga = 8 * (size_t)(pi[2] + D.nodes[pi[2] + np.na].bucket) + (item.sub >> 3);
       gb = 8 * (size_t)(pi[3] + D.nodes[pi[3] + np.nb].bucket) + (item.sub & 7);
     }
@@ -742,8 +1007,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
       if (it < n) {
         float ca[9], cb[9];
         load_corners_f(D.fbuckets, ga, ca), load_corners_f(D.fbuckets, gb, cb);
-        thr = (float)pr[PR_SEARCH];
-        extra = soup_world(pr + PR_TA0, pr + PR_TA1, pr + PR_TB0, pr + PR_TB1, ca, cb, w);
+        thr = cf[CF_SEARCH];
+        extra = soup_world(load_m34f(cf + CF_A0), load_m34f(cf + CF_A1), load_m34f(cf + CF_B0), load_m34f(cf + CF_B1),
+                           ca, cb, w);
         need = !cull_tri_edges(w, w + 3, w + 6, w + 9, thr, extra);
       }
       const unsigned long long tm = __ballot(need);
@@ -763,8 +1029,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
     if (it < n) {
       float ca[9], cb[9];
       load_corners_f(D.fbuckets, ga, ca), load_corners_f(D.fbuckets, gb, cb);
-      mask = soup_point_mask(pr + PR_MAB0, pr + PR_MAB1, pr + PR_MBA0, pr + PR_MBA1, ca, cb, load_soup_tri(D.stris, ga),
-                             load_soup_tri(D.stris, gb), (float)pr[PR_SEARCH]);
+      mask = soup_point_mask(load_m34f(cf + CF_MAB0), load_m34f(cf + CF_MAB1), load_m34f(cf + CF_MBA0),
+                             load_m34f(cf + CF_MBA1), ca, cb, load_soup_tri(D.stris, ga), load_soup_tri(D.stris, gb),
+                             cf[CF_SEARCH]);
     }
     wave_sync_lds();
     const int jobs = 9 * __popcll(__ballot(need));
@@ -781,19 +1048,28 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
     if (it < n) D.res_mask[it] = mask;
     const int mp = __popc(mask & SOUP_PT_BITS), me = __popc(mask & SOUP_EE_BITS);
     const int ip = wave_incl_scan(mp), ie = wave_incl_scan(me);
-    unsigned long long bp = 0ull, be = 0ull;
-    if (lane == 63) {
-      if (ip) bp = atomicAdd(cpt, (unsigned long long)ip);
-      if (ie) be = atomicAdd(cee, (unsigned long long)ie);
-      if ((long long)(bp + ip) > D.cap_items || (long long)(be + ie) > D.cap_items) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
+    if (lane == 63) s_pt[par][wv] = ip, s_ee[par][wv] = ie;
+    __syncthreads();
+    if (threadIdx.x < 2) {  // one atomic per block and list
+      const int* h = threadIdx.x ? s_ee[par] : s_pt[par];
+      const int tot = h[0] + h[1] + h[2] + h[3];
+      unsigned long long base = 0;
+      if (tot) {
+        base = atomicAdd(threadIdx.x ? cee : cpt, (unsigned long long)tot);
+        if ((long long)(base + tot) > D.cap_items) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
+      }
+      s_at[par][threadIdx.x] = base;
     }
-    long long sp = (long long)readlane_u64(bp, 63) + (ip - mp), se = (long long)readlane_u64(be, 63) + (ie - me);
+    __syncthreads();
+    long long sp = (long long)s_at[par][0] + (ip - mp), se = (long long)s_at[par][1] + (ie - me);
+    for (int v = 0; v < wv; ++v) sp += s_pt[par][v], se += s_ee[par][v];
     for (unsigned m = mask; m; m &= m - 1u) {
       const int s = __ffs(m) - 1;
       const bool pt = (SOUP_PT_BITS >> s) & 1u;
       const long long slot = pt ? sp++ : se++;
       if (slot < D.cap_items) (pt ? D.pt_items : D.ee_items)[slot] = Item{(uint32_t)it, (uint32_t)s};
     }
+    par ^= 1;
     wave_sync_lds();  // LDS read before the next round overwrites it
   }
 }
@@ -842,102 +1118,12 @@ __device__ __forceinline__ void soup_edge_one(Dev& D, long long it, int k, int l
   store_res(D.res + ((size_t)it * RES_SLOTS + 5 * k + 2 + l) * 8, d, P, Q, toc);
 }
 
-// The point sub-tests of the level: every item's six (FP64 form), or the
-// FP32 form's surviving list.
-__device__ __forceinline__ void soup_point_body(Dev& D, long long blk, long long nblk) {
-  if (D.fp32) {
-    const long long n = D.n_lv(LV_SPT);
-    for (long long t = blk * blockDim.x + threadIdx.x; t < n; t += nblk * blockDim.x) {
-      const Item e = D.pt_items[t];
-      soup_point_one(D, e.np, (int)e.sub / 5, (int)e.sub % 5);
-    }
-    return;
-  }
-  const long long total = D.n_res() * 6;
-  for (long long t = blk * blockDim.x + threadIdx.x; t < total; t += nblk * blockDim.x) {
-    const int s = (int)(t % 6);
-    soup_point_one(D, t / 6, s >> 1, s & 1);
-  }
-}
-
-// The edge sub-tests of the level: every item's nine (FP64 form), or the
-// FP32 form's surviving list.
-__device__ __forceinline__ void soup_edge_body(Dev& D, long long blk, long long nblk) {
-  if (D.fp32) {
-    const long long n = D.n_lv(LV_SEE);
-    for (long long t = blk * blockDim.x + threadIdx.x; t < n; t += nblk * blockDim.x) {
-      const Item e = D.ee_items[t];
-      soup_edge_one(D, e.np, (int)e.sub / 5, (int)e.sub % 5 - 2);
-    }
-    return;
-  }
-  const long long total = D.n_res() * 9;
-  for (long long t = blk * blockDim.x + threadIdx.x; t < total; t += nblk * blockDim.x) {
-    const int s = (int)(t % 9);
-    soup_edge_one(D, t / 9, s / 3, s % 3);
-  }
-}
-
-// Both kinds of sub-tests of the level's soup items in one launch: blocks
-// [0, g/2) take the point-triangle tests, [g/2, g) the edge-edge tests, so no
-// wavefront mixes the two code paths.
-__global__ void __launch_bounds__(256) k_soup_sub(Dev D) {
-  const int h = (int)(gridDim.x >> 1);
-  if ((int)blockIdx.x < h) soup_point_body(D, blockIdx.x, h);
-  else soup_edge_body(D, blockIdx.x - h, gridDim.x - h);
-}
-
-// triTriCCDLinear's selection over its 15 sub-results in the reference order
-// (continuous_comparison.h:680-779), hit test (continuous_comparison.h:817),
-// contact emission for leaf-leaf node pairs.
-__global__ void __launch_bounds__(256) k_soup_reduce(Dev D) {
-  const long long count = D.n_res();
-  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < count; t += (long long)gridDim.x * blockDim.x) {
-    Item item = D.items[t];
-    const double* r = D.res + (size_t)t * RES_SLOTS * 8;
-    double best = 1.0 / 0.0, toc = 1.0;
-    int win = -1;
-    const unsigned live = D.fp32 ? D.res_mask[t] : (1u << RES_SLOTS) - 1u;  // FP32 form: culled slots hold nothing
-    for (int s = 0; s < RES_SLOTS; ++s) {
-      if (!((live >> s) & 1u)) continue;
-      double d = r[8 * s], tc = r[8 * s + 1];
-      if (d < best || (d == best && tc < toc)) best = d, toc = tc, win = s;
-    }
-    NP np = D.soup[item.np];
-    const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
-    bool hit = best < pr[PR_SEARCH];
-    if (!hit) continue;
-    atomicOr(&D.np_hit[item.np], 1);
-    atomic_min_pos(&D.pass_min_s[np.pair], toc);
-    const int32_t* pi = D.pair_info + 4 * np.pair;
-    const NodeRec na = D.nodes[pi[2] + np.na];
-    const NodeRec nb = D.nodes[pi[3] + np.nb];
-    if (na.inner || nb.inner) continue;
-    D.pass_flag_s[np.pair] = 1;
-    unsigned long long slot = atomicAdd(&D.cnt[C_CONTACTS], 1ull);
-    if ((long long)slot >= D.cap_contacts) {
-      atomicOr(&D.cnt[C_OVERFLOW], D.discrete ? 2ull : 1ull);
-      continue;
-    }
-    atomicAdd(&D.pair_cnt[np.pair], 1);
-    ContactRec c;
-    c.key = make_key(2 * D.level, 0, np.key, (int)item.sub);
-    c.pair = (int32_t)np.pair, c.na = (int32_t)np.na, c.nb = (int32_t)np.nb, c.kind = 0;
-    c.ia = (int32_t)(item.sub >> 3), c.ib = (int32_t)(item.sub & 7), c.level = 2 * D.level, c.pad = 0;
-    const double* w = r + 8 * win;
-    c.r[0] = w[2], c.r[1] = w[3], c.r[2] = w[4], c.r[3] = w[5], c.r[4] = w[6], c.r[5] = w[7];
-    c.r[6] = pr[PR_GEOA], c.r[7] = pr[PR_GEOB], c.r[8] = 0.0, c.r[9] = 0.0, c.r[10] = toc;
-    D.contacts[slot] = c;
-  }
-}
-
 // ---------------------------------------------------- CCD leaf-leaf level
 // Sub-test numbering of a leaf pair with n (a) and m (b) triangles, in the
 // reference's order (continuous_comparison.h:855-907):
 //   [0, 3nm)        vertex v = s/m of a   vs triangle s%m of b
 //   [3nm, 6nm)      vertex v = s'/n of b  vs triangle s'%n of a
 //   edge list       edge s/(3m) of a      vs edge s%(3m) of b   (offset 6nm)
-// The sub-test items are written by k_level_write.
 __device__ __forceinline__ void emit_leaf(Dev& D, const NP& np, const double* pr, int kind, int ia, int ib, int sub,
                                           v3<double> A, v3<double> B, double toc) {
   unsigned long long slot = atomicAdd(&D.cnt[C_CONTACTS], 1ull);
@@ -955,86 +1141,95 @@ __device__ __forceinline__ void emit_leaf(Dev& D, const NP& np, const double* pr
   D.contacts[slot] = c;
 }
 
-__device__ __forceinline__ void leaf_point_body(Dev& D, long long blk, long long nblk) {
-  const long long count = D.n_lv(LV_PT);
-  for (long long t = blk * blockDim.x + threadIdx.x; t < count; t += nblk * blockDim.x) {
-    Item item = D.pt_items[t];
-    NP np = D.conn[item.np];
-    const int32_t* pi = D.pair_info + 4 * np.pair;
-    const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
-    const NodeRec na = D.nodes[pi[2] + np.na];
-    const NodeRec nb = D.nodes[pi[3] + np.nb];
-    const double* ba = D.buckets + (size_t)BUCKET * (pi[2] + na.bucket);
-    const double* bb = D.buckets + (size_t)BUCKET * (pi[3] + nb.bucket);
-    int s = (int)item.sub, n = na.ntris, m = nb.ntris;
-    v3<double> P, Q;
-    double toc = 1.0, d;
-    int kind, ia, ib;
-    if (s < 3 * n * m) {
-      int v = s / m, j = s % m;
-      d = point_tri(load_corner(ba, v / 3, v % 3), pr + PR_MAB0, pr + PR_MAB1, load_tri<double>(bb, j), pr + PR_TB0,
-                    pr + PR_TB1, P, Q, toc);
-      kind = 1, ia = v, ib = j;
+__device__ __forceinline__ void leaf_point_one(Dev& D, Item item) {
+  NP np = D.conn[item.np];
+  const int32_t* pi = D.pair_info + 4 * np.pair;
+  const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
+  const NodeRec na = D.nodes[pi[2] + np.na];
+  const NodeRec nb = D.nodes[pi[3] + np.nb];
+  const double* ba = D.buckets + (size_t)BUCKET * (pi[2] + na.bucket);
+  const double* bb = D.buckets + (size_t)BUCKET * (pi[3] + nb.bucket);
+  int s = (int)item.sub, n = na.ntris, m = nb.ntris;
+  v3<double> P, Q;
+  double toc = 1.0, d;
+  int kind, ia, ib;
+  if (s < 3 * n * m) {
+    int v = s / m, j = s % m;
+    d = point_tri(load_corner(ba, v / 3, v % 3), pr + PR_MAB0, pr + PR_MAB1, load_tri<double>(bb, j), pr + PR_TB0,
+                  pr + PR_TB1, P, Q, toc);
+    kind = 1, ia = v, ib = j;
+  } else {
+    int s2 = s - 3 * n * m, v = s2 / n, i = s2 % n;
+    d = point_tri(load_corner(bb, v / 3, v % 3), pr + PR_MBA0, pr + PR_MBA1, load_tri<double>(ba, i), pr + PR_TA0,
+                  pr + PR_TA1, P, Q, toc);
+    kind = 2, ia = i, ib = v;
+  }
+  if (d < pr[PR_SEARCH]) {
+    D.pass_flag_c[np.pair] = 1;
+    atomic_min_pos(&D.pass_min_c[np.pair], toc);
+    if (kind == 1) emit_leaf(D, np, pr, kind, ia, ib, s, P, Q, toc);
+    else emit_leaf(D, np, pr, kind, ia, ib, s, Q, P, toc);  // continuous_comparison.h:876
+  }
+}
+
+__device__ __forceinline__ void leaf_edge_one(Dev& D, Item item) {
+  NP np = D.conn[item.np];
+  const int32_t* pi = D.pair_info + 4 * np.pair;
+  const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
+  const NodeRec na = D.nodes[pi[2] + np.na];
+  const NodeRec nb = D.nodes[pi[3] + np.nb];
+  int s = (int)item.sub, n = na.ntris, m = nb.ntris;
+  int ea = s / (3 * m), eb = s % (3 * m);
+  const double* ba = D.buckets + (size_t)BUCKET * (pi[2] + na.bucket);
+  const double* bb = D.buckets + (size_t)BUCKET * (pi[3] + nb.bucket);
+  v3<double> a0 = load_corner(ba, ea / 3, ea % 3), a1 = load_corner(ba, ea / 3, (ea % 3 + 1) % 3);
+  v3<double> b0 = load_corner(bb, eb / 3, eb % 3), b1 = load_corner(bb, eb / 3, (eb % 3 + 1) % 3);
+  v3<double> P, Q;
+  double toc = 1.0;
+  double d = edge_edge(xform(pr + PR_TA0, a0), xform(pr + PR_TA0, a1), xform(pr + PR_TA1, a0), xform(pr + PR_TA1, a1),
+                       xform(pr + PR_TB0, b0), xform(pr + PR_TB0, b1), xform(pr + PR_TB1, b0), xform(pr + PR_TB1, b1),
+                       P, Q, toc);
+  if (d < pr[PR_SEARCH]) {
+    D.pass_flag_c[np.pair] = 1;
+    atomic_min_pos(&D.pass_min_c[np.pair], toc);
+    emit_leaf(D, np, pr, 3, ea, eb, 6 * n * m + s, Q, P, toc);  // continuous_comparison.h:903
+  }
+}
+// The level's FP64 sub-tests in one launch: the soup items' (the FP32 form's
+// surviving lists, or every item's six and nine) and the connected list's, point
+// and edge.  The four lists are dealt out 64 entries at a time, so no wavefront
+// mixes code paths and none waits for another list's end.
+__global__ void __launch_bounds__(256) k_ccd_sub(Dev D) {
+  const int lane = lane_id();
+  const long long se = D.fp32 ? D.n_lv(LV_SEE) : 9 * D.n_res(), sp = D.fp32 ? D.n_lv(LV_SPT) : 6 * D.n_res();
+  const long long le = D.n_lv(LV_EE), lp = D.n_lv(LV_PT);
+  const long long q1 = (se + 63) / 64, q2 = q1 + (le + 63) / 64, q3 = q2 + (sp + 63) / 64, q4 = q3 + (lp + 63) / 64;
+  const int nw = (int)(blockDim.x >> 6);
+  const long long first = (long long)blockIdx.x * nw + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  for (long long q = first; q < q4; q += (long long)gridDim.x * nw) {
+    if (q < q1) {
+      const long long t = 64 * q + lane;
+      if (t < se) {
+        const Item e = D.fp32 ? D.ee_items[t] : Item{(uint32_t)(t / 9), (uint32_t)(5 * (t % 9 / 3) + 2 + t % 3)};
+        soup_edge_one(D, e.np, (int)e.sub / 5, (int)e.sub % 5 - 2);
+      }
+    } else if (q < q2) {
+      const long long t = 64 * (q - q1) + lane;
+      if (t < le) leaf_edge_one(D, D.lee_items[t]);
+    } else if (q < q3) {
+      const long long t = 64 * (q - q2) + lane;
+      if (t < sp) {
+        const Item e = D.fp32 ? D.pt_items[t] : Item{(uint32_t)(t / 6), (uint32_t)(5 * (t % 6 / 2) + t % 2)};
+        soup_point_one(D, e.np, (int)e.sub / 5, (int)e.sub % 5);
+      }
     } else {
-      int s2 = s - 3 * n * m, v = s2 / n, i = s2 % n;
-      d = point_tri(load_corner(bb, v / 3, v % 3), pr + PR_MBA0, pr + PR_MBA1, load_tri<double>(ba, i), pr + PR_TA0,
-                    pr + PR_TA1, P, Q, toc);
-      kind = 2, ia = i, ib = v;
-    }
-    if (d < pr[PR_SEARCH]) {
-      D.pass_flag_c[np.pair] = 1;
-      atomic_min_pos(&D.pass_min_c[np.pair], toc);
-      if (kind == 1) emit_leaf(D, np, pr, kind, ia, ib, s, P, Q, toc);
-      else emit_leaf(D, np, pr, kind, ia, ib, s, Q, P, toc);  // continuous_comparison.h:876
+      const long long t = 64 * (q - q3) + lane;
+      if (t < lp) leaf_point_one(D, D.lpt_items[t]);
     }
   }
 }
 
-__device__ __forceinline__ void leaf_edge_body(Dev& D, long long blk, long long nblk) {
-  const long long count = D.n_lv(LV_EE);
-  for (long long t = blk * blockDim.x + threadIdx.x; t < count; t += nblk * blockDim.x) {
-    Item item = D.ee_items[t];
-    NP np = D.conn[item.np];
-    const int32_t* pi = D.pair_info + 4 * np.pair;
-    const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
-    const NodeRec na = D.nodes[pi[2] + np.na];
-    const NodeRec nb = D.nodes[pi[3] + np.nb];
-    int s = (int)item.sub, n = na.ntris, m = nb.ntris;
-    int ea = s / (3 * m), eb = s % (3 * m);
-    const double* ba = D.buckets + (size_t)BUCKET * (pi[2] + na.bucket);
-    const double* bb = D.buckets + (size_t)BUCKET * (pi[3] + nb.bucket);
-    v3<double> a0 = load_corner(ba, ea / 3, ea % 3), a1 = load_corner(ba, ea / 3, (ea % 3 + 1) % 3);
-    v3<double> b0 = load_corner(bb, eb / 3, eb % 3), b1 = load_corner(bb, eb / 3, (eb % 3 + 1) % 3);
-    v3<double> P, Q;
-    double toc = 1.0;
-    double d = edge_edge(xform(pr + PR_TA0, a0), xform(pr + PR_TA0, a1), xform(pr + PR_TA1, a0), xform(pr + PR_TA1, a1),
-                         xform(pr + PR_TB0, b0), xform(pr + PR_TB0, b1), xform(pr + PR_TB1, b0), xform(pr + PR_TB1, b1),
-                         P, Q, toc);
-    if (d < pr[PR_SEARCH]) {
-      D.pass_flag_c[np.pair] = 1;
-      atomic_min_pos(&D.pass_min_c[np.pair], toc);
-      emit_leaf(D, np, pr, 3, ea, eb, 6 * n * m + s, Q, P, toc);  // continuous_comparison.h:903
-    }
-  }
-}
-// The leaf-leaf sub-tests of the level in one launch, split by block as in
-// k_soup_sub.
-__global__ void __launch_bounds__(256) k_leaf_sub(Dev D) {
-  const int h = (int)(gridDim.x >> 1);
-  if ((int)blockIdx.x < h) leaf_point_body(D, blockIdx.x, h);
-  else leaf_edge_body(D, blockIdx.x - h, gridDim.x - h);
-}
-
-// ------------------------------------------- ordered enumeration/expansion
-// ------------------------------------------------ FP32 conservative cull
-// The discrete phase's FP32 classification of triangle pairs (certain miss,
-// FP64 test, certain hit) is in d2_cull.hpp: cull_prep, cull_margin,
-// cull_pair.
-
-// One wavefront per node pair (chunked ranges): which triangle pairs need the
-// FP64 test.  FP64 mode keeps every valid pair; FP32 mode drops certain
-// misses, and for node pairs with an inner node (they emit no contacts, only
-// "any hit" matters) a certain hit settles the node pair without FP64 work.
+// -------------------------------------------------------------- expansion
 __device__ __forceinline__ bool expand_side(const NodeRec& na, const NodeRec& nb) {
   return na.inner && (!nb.inner || na.depth < nb.depth);  // true: advance a
 }
@@ -1046,6 +1241,121 @@ __device__ __forceinline__ int expansion_desc(const NodeRec& na, const NodeRec& 
   const NodeRec& par = adv_a ? na : nb;
   return (adv_a ? 1 : 0) | (par.nchild << 1) | (par.child_first << 5);
 }
+// triTriCCDLinear's selection over its 15 sub-results in the reference order
+// (continuous_comparison.h:680-779), hit test (continuous_comparison.h:817),
+// contact emission for leaf-leaf node pairs.  Returns whether this is the first
+// hit found of a node pair with children to visit.
+__device__ __forceinline__ bool soup_reduce_one(Dev& D, long long t) {
+  Item item = D.items[t];
+  const double* r = D.res + (size_t)t * RES_SLOTS * 8;
+  double best = 1.0 / 0.0, toc = 1.0;
+  int win = -1;
+  const unsigned live = D.fp32 ? D.res_mask[t] : (1u << RES_SLOTS) - 1u;  // FP32 form: culled slots hold nothing
+  for (int s = 0; s < RES_SLOTS; ++s) {
+    if (!((live >> s) & 1u)) continue;
+    double d = r[8 * s], tc = r[8 * s + 1];
+    if (d < best || (d == best && tc < toc)) best = d, toc = tc, win = s;
+  }
+  NP np = D.soup[item.np];
+  const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
+  bool hit = best < pr[PR_SEARCH];
+  if (!hit) return false;
+  atomic_min_pos(&D.pass_min_s[np.pair], toc);
+  const int32_t* pi = D.pair_info + 4 * np.pair;
+  const NodeRec na = D.nodes[pi[2] + np.na];
+  const NodeRec nb = D.nodes[pi[3] + np.nb];
+  if (na.inner || nb.inner) return atomicOr(&D.np_hit[item.np], 1) == 0;
+  D.pass_flag_s[np.pair] = 1;
+  unsigned long long slot = atomicAdd(&D.cnt[C_CONTACTS], 1ull);
+  if ((long long)slot >= D.cap_contacts) {
+    atomicOr(&D.cnt[C_OVERFLOW], D.discrete ? 2ull : 1ull);
+    return false;
+  }
+  atomicAdd(&D.pair_cnt[np.pair], 1);
+  ContactRec c;
+  c.key = make_key(2 * D.level, 0, np.key, (int)item.sub);
+  c.pair = (int32_t)np.pair, c.na = (int32_t)np.na, c.nb = (int32_t)np.nb, c.kind = 0;
+  c.ia = (int32_t)(item.sub >> 3), c.ib = (int32_t)(item.sub & 7), c.level = 2 * D.level, c.pad = 0;
+  const double* w = r + 8 * win;
+  c.r[0] = w[2], c.r[1] = w[3], c.r[2] = w[4], c.r[3] = w[5], c.r[4] = w[6], c.r[5] = w[7];
+  c.r[6] = pr[PR_GEOA], c.r[7] = pr[PR_GEOB], c.r[8] = 0.0, c.r[9] = 0.0, c.r[10] = toc;
+  D.contacts[slot] = c;
+  return false;
+}
+// The children of the node pairs a block claimed (full_tree_comparison.h:26-62,
+// 99-150), one node pair per thread, to the next level's two lists: a child
+// pair goes to the soup list when either node is inner -- all of them when the
+// node that stays is inner, else the inner children of the one that advances.
+// One slot range per list and round; the lists' order is free.
+__device__ __forceinline__ void write_ccd_children(Dev& D, const unsigned* claim, int n_claim) {
+  __shared__ unsigned long long s_base[2];
+  for (int t0 = 0; t0 < n_claim; t0 += blockDim.x) {
+    const int t = t0 + threadIdx.x;
+    NP np{};
+    int ns = 0, nc = 0, first = 0;
+    bool adv_a = false, stay_inner = false;
+    unsigned kid = 0;
+    if (t < n_claim) {
+      np = D.soup[claim[t]];
+      const int32_t* pi = D.pair_info + 4 * np.pair;
+      const NodeRec na = D.nodes[pi[2] + np.na];
+      const NodeRec nb = D.nodes[pi[3] + np.nb];
+      adv_a = expand_side(na, nb);
+      stay_inner = adv_a ? nb.inner : na.inner;
+      const int nch = adv_a ? na.nchild : nb.nchild;
+      first = adv_a ? na.child_first : nb.child_first;
+      kid = stay_inner ? (1u << nch) - 1u : (unsigned)D.kid_inner[(adv_a ? pi[2] : pi[3]) + (adv_a ? np.na : np.nb)];
+      ns = __popc(kid), nc = nch - ns;
+    }
+    int tot;
+    const int ex = block_scan(ns | nc << 16, tot);  // (a block's sums stay below 2^16: 8 children x 256)
+    if (threadIdx.x < 2) {
+      const int k = threadIdx.x, sum = k ? tot >> 16 : tot & 0xffff;
+      unsigned long long base = 0;
+      if (sum) {
+        base = atomicAdd(&D.lvl[(D.level + 1) * LV_STRIDE + (k ? LV_CONN : LV_SOUP)], (unsigned long long)sum);
+        if ((long long)(base + sum) > D.cap_np) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
+      }
+      s_base[k] = base;
+    }
+    __syncthreads();
+    long long ps = (long long)s_base[0] + (ex & 0xffff), pc = (long long)s_base[1] + (ex >> 16);
+    for (int c = 0; c < ns + nc; ++c) {
+      const uint32_t id = (uint32_t)(first + c);
+      const bool to_soup = (kid >> c) & 1u;
+      const long long slot = to_soup ? ps++ : pc++;
+      if (slot < D.cap_np)
+        (to_soup ? D.soup_next : D.conn_next)[slot] =
+            NP{np.pair, adv_a ? id : np.na, adv_a ? np.nb : id, 0u, np.key * 8ull + (unsigned long long)c};
+    }
+    __syncthreads();  // s_base is read before the next round's is written
+  }
+}
+// The first hit of a node pair claims it; the claimed ones collect in LDS and
+// are expanded by whole blocks (a level is then complete without the two
+// launches that counted and wrote children in list order: on levels of up to
+// 26,000 node pairs writing alone took 18 us, claiming here adds 4).
+constexpr int CLAIM_CAP = 1024;
+__global__ void __launch_bounds__(256) k_soup_reduce(Dev D) {
+  __shared__ unsigned s_claim[CLAIM_CAP];
+  __shared__ int s_n;
+  const long long count = D.n_res();
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  for (long long b0 = (long long)blockIdx.x * blockDim.x; b0 < count; b0 += (long long)gridDim.x * blockDim.x) {
+    const long long t = b0 + threadIdx.x;
+    if (t < count && soup_reduce_one(D, t)) s_claim[atomicAdd(&s_n, 1)] = D.items[t].np;
+    __syncthreads();
+    const int n = s_n;
+    const bool last = b0 + (long long)gridDim.x * blockDim.x >= count;
+    if (n > CLAIM_CAP - (int)blockDim.x || (last && n)) {
+      write_ccd_children(D, s_claim, n);
+      if (threadIdx.x == 0) s_n = 0;
+    }
+    __syncthreads();
+  }
+}
+
 // The child c of a node pair of the discrete list.  Discrete lists: the
 // children of a node pair that hits or may hit take slots of the next list,
 // each naming its parent: parent 0 for a certain hit, list index + 1 when the
@@ -1067,6 +1377,12 @@ __device__ __forceinline__ void load_pose_f(const Dev& D, uint32_t pair, float* 
     f[4 * q] = v.x, f[4 * q + 1] = v.y, f[4 * q + 2] = v.z, f[4 * q + 3] = v.w;
   }
 }
+// ------------------------------------------------ FP32 conservative cull
+// Which triangle pairs of the discrete phase need the FP64 test (FP32 form;
+// the classification is in d2_cull.hpp: cull_prep, cull_apart, cull_sure):
+// certain misses are dropped, and for node pairs with an inner node (they emit
+// no contacts, only "any hit" matters) a certain hit settles the node pair
+// without FP64 work.
 static_assert(sizeof(CullTri) == 112, "prepared triangle: 28 dwords, a conflict-free LDS stride");
 // A wavefront takes the node pairs of a batch in groups of at most 64
 // triangles, both buckets' together: a lane prepares one triangle, then the
@@ -1102,12 +1418,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
   // offsets and node records of the wave's l-th node pair in one go, so the
   // per-node-pair dependent loads reduce to its pose and buckets.
   int it = 0;
-  const long long waves = (long long)gridDim.x * nw;
-  const int part = n < 64 * waves ? (int)((n + waves - 1) / waves) : 64;  // node pairs per wavefront
-  for (long long b0 = (long long)blockIdx.x * nw * part; b0 < n; b0 += waves * part, ++it) {
-    const long long w0 = b0 + (long long)part * wid;
+  for (Tiles T(n, blockIdx.x, gridDim.x, nw); T.b0 < n; T.b0 += T.step, ++it) {
+    const long long w0 = T.first(wid);
     const long long wl = w0 + lane;
-    const bool in_range = lane < part && wl < n;
+    const bool in_range = lane < T.part && wl < n;
     int l_pair = 0, l_ga = 0, l_gb = 0, l_nta = 0, l_ntb = 0, l_inner = 0, l_desc = 0;  // l_ga, l_gb: global buckets
     int l_offa = 0, l_offb = 0;
     if (in_range) {
@@ -1138,20 +1452,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
     }
     unsigned long long my_keep = 0;  // bit i * l_ntb + j: triangle i of a against j of b
     int my_settled = 0;
-    const int my_jobs = l_nta * l_ntb, my_tris = my_jobs > 0 ? l_nta + l_ntb : 0;
-    const int tri_incl = wave_incl_scan(my_tris), job_incl = wave_incl_scan(my_jobs);
-    const int tri_all = rl(tri_incl, 63);
-    for (int t0 = 0, j0 = 0; t0 < tri_all;) {
-      const int ts = tri_incl - my_tris - t0, js = job_incl - my_jobs - j0;
-      bool in = my_tris > 0 && ts >= 0 && ts + my_tris <= 64;
-      int last = 63 - __clzll((long long)__ballot(in));
-      // a few triangle pairs over a multiple of 64 wait for the next group
-      const int over = rl(job_incl, last) - j0;
-      if (over > 64 && (over & 63) < 40) {
-        in = in && js + my_jobs <= (over & ~63);
-        last = 63 - __clzll((long long)__ballot(in));
-      }
-      const int t1 = rl(tri_incl, last), j1 = rl(job_incl, last), jobs = j1 - j0;
+    const int my_jobs = l_nta * l_ntb;
+    for (Groups g(my_jobs > 0 ? l_nta + l_ntb : 0, my_jobs); g.next(true);) {
+      const int ts = g.ts, js = g.js, jobs = g.n_jobs;
+      const bool in = g.in;
       s_own[wid][lane] = 0;
       wave_sync_lds();
       if (in) s_own[wid][ts] = (unsigned char)(lane + 1);
@@ -1167,7 +1471,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
         const int jstart = __shfl(js, src), inner = __shfl(l_inner, src);
         const bool side = x >= nta;
         const int kk = side ? x - nta : x;
-        if (lane < t1 - t0) {
+        if (lane < g.n_slots) {
           CullTri mine{};
           // (b's rotation, no translation: b's position is the origin)
           const float4* pf = reinterpret_cast<const float4*>(D.pair_f + (size_t)PF_STRIDE * pair + (side ? PF_RB : PF_RA));
@@ -1203,10 +1507,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
           keep = !cull_apart(A, B, (float)(A.eps + B.eps));
         }
         const unsigned long long kept = __ballot(keep);
-        // this lane's node pair's share of the 64 answers
-        const int d = js - q0;
-        if (in && d < 64 && d + my_jobs > 0)
-          my_keep |= (d >= 0 ? kept >> d : kept << -d) & (my_jobs < 64 ? (1ull << my_jobs) - 1ull : ~0ull);
+        my_keep |= g.share(kept, q0);
         const bool more = keep && job >> 12;
         const unsigned long long m = __ballot(more);
         if (more) s_job[wid][left + __popcll(m & lanes_below())] = (unsigned short)job;
@@ -1226,7 +1527,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
         if (in && (s_sure[wid] >> ts & ((1ull << l_nta) - 1ull)) != 0ull) my_settled = 1;
       }
       wave_sync_lds();  // read before the next group overwrites
-      t0 = t1, j0 = j1;
     }
     if (my_settled) my_keep = 0ull;
     if (in_range) D.np_hit[wl] = my_settled;
@@ -1593,282 +1893,6 @@ __global__ void __launch_bounds__(256) k_tri_full(Dev D) {
   if (threadIdx.x == 0 && s_tested) {
     atomicAdd(&D.lvl[D.level * LV_STRIDE + LV_ITEMS], s_tested);
     atomicAdd(&D.cnt[C_LVL_ITEMS], s_tested);
-  }
-}
-
-// CCD levels: children of hit node pairs (full_tree_comparison.h:26-62,
-// 99-150) and the sub-tests of the connected (leaf-leaf) list, in two chunked
-// passes: counts + block partials, then writes at scanned offsets, which
-// keeps every list in the reference's breadth-first order (discrete levels
-// are expanded by k_tri_mask, or by k_disc_expand in FP64 mode).
-// ------------------------------------------- FP32 culls of CCD leaf sub-tests
-// The bounds of d2_cull.hpp (soup_point_keep: plane side and edge
-// half-planes with each triangle's FP64-derived normals and its
-// float-barycentric acceptance bound; cull_edge_edge: separating axes).
-// Per connected node pair, shared across its wavefront: lane v < 24 holds
-// vertex v of a's leaf (triangle v/3, corner v%3), lanes 24-47 those of b:
-// the vertex at both ends in world coordinates (relative to b's start
-// position) and in the other body's frame; lanes 48-55 / 56-63 hold
-// triangle k of a / b in its own frame: unit normal, plane offset, outward
-// unit edge normals and offsets.  A sub-test then reads what it needs by
-// shuffles.
-struct LeafShare {
-  float w0[3], w1[3], f0[3], f1[3];  // vertex lanes
-  SoupTri t;                         // triangle lanes (soup_tri: FP64 normals, float-barycentric bound)
-};
-struct LeafInfo {
-  int n, m;
-  float thr, margin, mag;  // mag: every magnitude of the node pair's FP32 transforms
-};
-__device__ LeafInfo leaf_share(const Dev& D, const NP& np, LeafShare& sh) {
-  const int lane = lane_id();
-  const int32_t* pi = D.pair_info + 4 * np.pair;
-  const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
-  const NodeRec na = D.nodes[pi[2] + np.na];
-  const NodeRec nb = D.nodes[pi[3] + np.nb];
-  const size_t ta0 = 8 * (size_t)(pi[2] + na.bucket), tb0 = 8 * (size_t)(pi[3] + nb.bucket);  // global triangle 0
-  LeafInfo I;
-  I.n = na.ntris, I.m = nb.ntris;
-  I.thr = (float)pr[PR_SEARCH];
-  float mag = 0.f;
-  for (int k = 0; k < 3; ++k) sh.w0[k] = sh.w1[k] = sh.f0[k] = sh.f1[k] = 0.f;
-  if (lane < 48) {
-    const bool of_b = lane >= 24;
-    const int v = of_b ? lane - 24 : lane;
-    if (v / 3 < (of_b ? I.m : I.n)) {
-      const float* pf = D.fbuckets + (size_t)FB_STRIDE * ((of_b ? tb0 : ta0) + v / 3) + 3 * (v % 3);
-      const float p[3] = {pf[0], pf[1], pf[2]};  // the corner rounded to float
-      const M34f W0 = to_m34f(of_b ? pr + PR_TB0 : pr + PR_TA0, pr + PR_TB0);
-      const M34f W1 = to_m34f(of_b ? pr + PR_TB1 : pr + PR_TA1, pr + PR_TB0);
-      const M34f F0 = to_m34f(of_b ? pr + PR_MBA0 : pr + PR_MAB0, nullptr);
-      const M34f F1 = to_m34f(of_b ? pr + PR_MBA1 : pr + PR_MAB1, nullptr);
-      xf_f(W0, p, sh.w0), xf_f(W1, p, sh.w1), xf_f(F0, p, sh.f0), xf_f(F1, p, sh.f1);
-      mag = fmaxf(fmaxf(amax3(sh.w0), amax3(sh.w1)), fmaxf(amax3(sh.f0), amax3(sh.f1)));
-      mag = fmaxf(mag, fmaxf(fmaxf(fmaxf(m34_mag(W0), m34_mag(W1)), fmaxf(m34_mag(F0), m34_mag(F1))), amax3(p)));
-    }
-    sh.t = SoupTri{};  // (vertex lanes: unused)
-  } else {
-    const bool of_b = lane >= 56;
-    const int k = lane & 7;
-    if (k < (of_b ? I.m : I.n)) {
-      const size_t tk = (of_b ? tb0 : ta0) + k;
-      float c9[9];
-      load_corners_f(D.fbuckets, tk, c9);
-      mag = fmaxf(amax3(c9), fmaxf(amax3(c9 + 3), amax3(c9 + 6)));
-      sh.t = load_soup_tri(D.stris, tk);
-    } else {
-      sh.t = SoupTri{};  // n = 0: never culled
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) mag = fmaxf(mag, __shfl_xor(mag, off));
-  I.mag = mag;
-  I.margin = 1e-6f + 64.f * 5.9604645e-08f * mag;
-  return I;
-}
-__device__ __forceinline__ void sh3(const float* v, int src, float* o) {
-  o[0] = __shfl(v[0], src), o[1] = __shfl(v[1], src), o[2] = __shfl(v[2], src);
-}
-// Point-triangle sub-test s survives (the bounds above: plane side, edge half-plane).
-// Every lane of the wavefront calls this (the shuffles need all lanes).
-__device__ bool leaf_point_keep(const LeafShare& sh, const LeafInfo& I, int s, bool active) {
-  const int n = I.n, m = I.m;
-  int vl, tl;
-  if (s < 3 * n * m) {
-    const int v = s / m, j = s % m;
-    vl = v, tl = 56 + j;  // vertex of a in b's frame, triangle of b
-  } else {
-    const int s2 = s - 3 * n * m, v = s2 / n, i = s2 % n;
-    vl = 24 + v, tl = 48 + i;
-  }
-  if (!active) vl = 0, tl = 48;
-  float p0[3], p1[3];
-  SoupTri t;
-  sh3(sh.f0, vl, p0), sh3(sh.f1, vl, p1), sh3(sh.t.n, tl, t.n);
-  t.d = __shfl(sh.t.d, tl), t.eo = __shfl(sh.t.eo, tl);
-  for (int q = 0; q < 3; ++q) sh3(sh.t.m + 3 * q, tl, t.m + 3 * q), t.o[q] = __shfl(sh.t.o[q], tl);
-  if (!active) return false;
-  return soup_point_keep(p0, p1, t, I.thr, I.margin);
-}
-__device__ bool leaf_edge_keep(const LeafShare& sh, const LeafInfo& I, int s, bool active) {
-  const int ea = active ? s / (3 * I.m) : 0, eb = active ? s % (3 * I.m) : 0;
-  const int a0 = 3 * (ea / 3) + ea % 3, a1 = 3 * (ea / 3) + (ea % 3 + 1) % 3;
-  const int b0 = 24 + 3 * (eb / 3) + eb % 3, b1 = 24 + 3 * (eb / 3) + (eb % 3 + 1) % 3;
-  float as0[3], as1[3], ae0[3], ae1[3], bs0[3], bs1[3], be0[3], be1[3];
-  sh3(sh.w0, a0, as0), sh3(sh.w0, a1, as1), sh3(sh.w1, a0, ae0), sh3(sh.w1, a1, ae1);
-  sh3(sh.w0, b0, bs0), sh3(sh.w0, b1, bs1), sh3(sh.w1, b0, be0), sh3(sh.w1, b1, be1);
-  if (!active) return false;
-  return !cull_edge_edge(as0, as1, ae0, ae1, bs0, bs1, be0, be1, I.thr, I.mag);
-}
-constexpr int CONN_MASK_WORDS = 16;  // 6 words of point sub-tests (<= 384), 9 of edge sub-tests (<= 576)
-
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) k_level_count(Dev D) {
-  {  // soup: children per destination list
-    const long long n = D.n_soup();
-    long long rb, re;
-    chunk_of(n, rb, re);
-    long long as = 0, ac = 0;
-    for (long long w = rb + threadIdx.x; w < re; w += blockDim.x) {
-      int ns = 0, nc = 0;
-      if (D.np_hit[w]) {
-        NP np = D.soup[w];
-        const int32_t* pi = D.pair_info + 4 * np.pair;
-        const NodeRec na = D.nodes[pi[2] + np.na];
-        const NodeRec nb = D.nodes[pi[3] + np.nb];
-        if (na.inner || nb.inner) {
-          // a child pair goes to the soup list when either node is inner:
-          // all of them when the node that stays is inner, else the inner
-          // children of the one that advances
-          const bool adv_a = expand_side(na, nb);
-          const NodeRec& par = adv_a ? na : nb;
-          const bool stay_inner = adv_a ? nb.inner : na.inner;
-          ns = stay_inner ? par.nchild : __popc((unsigned)D.kid_inner[(adv_a ? pi[2] : pi[3]) + (adv_a ? np.na : np.nb)]);
-          nc = par.nchild - ns;
-        }
-      }
-      D.cnt_s[w] = ns;
-      D.cnt_c[w] = nc;
-      as += ns, ac += nc;
-    }
-    const long long ts = block_sum(as), tc = block_sum(ac);
-    if (threadIdx.x == 0) D.part_s[blockIdx.x] = (int)ts, D.part_c[blockIdx.x] = (int)tc;
-  }
-  {
-    {  // connected list: sub-test counts
-      const long long n = D.n_conn();
-      long long rb, re;
-      chunk_of(n, rb, re);
-      long long ap = 0, ae = 0;  // lane 0 of each wavefront
-      const int lane = lane_id();
-      const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // uniform: scalar loads
-      for (long long w = rb + wv; w < re; w += (blockDim.x >> 6)) {  // one wavefront per node pair
-        const NP np = D.conn[w];
-        LeafShare sh;
-        LeafInfo L;
-        if (D.fp32) {
-          L = leaf_share(D, np, sh);  // reads the FP32 copies (FP32 contexts only)
-        } else {  // the FP64 form keeps every sub-test: only the sizes
-          const int32_t* pi = D.pair_info + 4 * np.pair;
-          L.n = D.nodes[pi[2] + np.na].ntris, L.m = D.nodes[pi[3] + np.nb].ntris;
-        }
-        const int npt = 6 * L.n * L.m, nee = 9 * L.n * L.m;
-        int kp = 0, ke = 0;
-        unsigned long long* mk = D.conn_mask + (size_t)CONN_MASK_WORDS * w;
-        for (int b0 = 0, wd = 0; b0 < npt; b0 += 64, ++wd) {
-          const int sb = b0 + lane;
-          const bool keep = D.fp32 ? leaf_point_keep(sh, L, sb, sb < npt) : sb < npt;
-          const unsigned long long bits = __ballot(keep);
-          if (lane == 0) mk[wd] = bits;
-          kp += __popcll(bits);
-        }
-        for (int b0 = 0, wd = 6; b0 < nee; b0 += 64, ++wd) {
-          const int sb = b0 + lane;
-          const bool keep = D.fp32 ? leaf_edge_keep(sh, L, sb, sb < nee) : sb < nee;
-          const unsigned long long bits = __ballot(keep);
-          if (lane == 0) mk[wd] = bits;
-          ke += __popcll(bits);
-        }
-        if (lane == 0) {
-          D.cnt_pt[w] = kp;
-          D.cnt_ee[w] = ke;
-          ap += kp, ae += ke;
-        }
-      }
-      const long long tp = block_sum(ap), te = block_sum(ae);
-      if (threadIdx.x == 0) D.part_pt[blockIdx.x] = (int)tp, D.part_ee[blockIdx.x] = (int)te;
-    }
-    fold_pass(D, D.pair_rec, D.pass_min_s, D.pass_flag_s);  // the soup pass of this level is complete
-  }
-}
-
-__global__ void __launch_bounds__(256) k_level_write(Dev D) {
-  __shared__ int toff_s[256], toff_c[256];
-  const int lane = lane_id(), wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  {
-    const long long n = D.n_soup();
-    long long rb, re, bs, ts, bc, tc;
-    chunk_of(n, rb, re);
-    partial_prefix(D.part_s, bs, ts);
-    partial_prefix(D.part_c, bc, tc);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      D.lvl[(D.level + 1) * LV_STRIDE + LV_SOUP] = (unsigned long long)ts;
-      D.lvl[(D.level + 1) * LV_STRIDE + LV_CONN] = (unsigned long long)tc;
-      if (ts > D.cap_np || tc > D.cap_np) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
-    }
-    for (long long t0 = rb; t0 < re; t0 += blockDim.x) {
-      const long long w = t0 + threadIdx.x;
-      int tts, ttc;
-      const int es = block_scan(w < re ? D.cnt_s[w] : 0, tts);
-      const int ec = block_scan(w < re ? D.cnt_c[w] : 0, ttc);
-      if (w < re && D.cnt_s[w] + D.cnt_c[w] > 0) {
-        NP np = D.soup[w];
-        const int32_t* pi = D.pair_info + 4 * np.pair;
-        const NodeRec na = D.nodes[pi[2] + np.na];
-        const NodeRec nb = D.nodes[pi[3] + np.nb];
-        bool adv_a = expand_side(na, nb);
-        const NodeRec& par = adv_a ? na : nb;
-        const bool stay_inner = adv_a ? nb.inner : na.inner;
-        const unsigned kid = D.kid_inner[(adv_a ? pi[2] : pi[3]) + (adv_a ? np.na : np.nb)];
-        long long ps = bs + es, pc = bc + ec;
-        for (int c = 0; c < par.nchild; ++c) {
-          uint32_t ca = adv_a ? (uint32_t)(par.child_first + c) : np.na;
-          uint32_t cb = adv_a ? np.nb : (uint32_t)(par.child_first + c);
-          NP child{np.pair, ca, cb, 0u, np.key * 8ull + (unsigned long long)c};
-          const bool to_soup = stay_inner || ((kid >> c) & 1u);
-          long long slot = to_soup ? ps++ : pc++;
-          if (slot < D.cap_np) (to_soup ? D.soup_next : D.conn_next)[slot] = child;
-        }
-      }
-      bs += tts, bc += ttc;
-    }
-  }
-  {
-    const long long n = D.n_conn();
-    long long rb, re, bp, tp, be, te;
-    chunk_of(n, rb, re);
-    partial_prefix(D.part_pt, bp, tp);
-    partial_prefix(D.part_ee, be, te);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      D.lvl[D.level * LV_STRIDE + LV_PT] = (unsigned long long)tp;
-      D.lvl[D.level * LV_STRIDE + LV_EE] = (unsigned long long)te;
-      if (tp > D.cap_items || te > D.cap_items) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
-    }
-    for (long long t0 = rb; t0 < re; t0 += blockDim.x) {
-      const long long w = t0 + threadIdx.x;
-      int ttp, tte;
-      const int ep = block_scan(w < re ? D.cnt_pt[w] : 0, ttp);
-      const int ee = block_scan(w < re ? D.cnt_ee[w] : 0, tte);
-      toff_s[threadIdx.x] = ep;
-      toff_c[threadIdx.x] = ee;
-      __syncthreads();
-      const int in_tile = (int)((re - t0) < (long long)blockDim.x ? (re - t0) : (long long)blockDim.x);
-      for (int j = wid; j < in_tile; j += nw) {  // one wavefront per connected node pair
-        const long long ww = t0 + j;
-        const NP cnp = D.conn[ww];
-        const int32_t* cpi = D.pair_info + 4 * cnp.pair;
-        const int nn = D.nodes[cpi[2] + cnp.na].ntris, mm = D.nodes[cpi[3] + cnp.nb].ntris;
-        const int npt = 6 * nn * mm, nee = 9 * nn * mm;
-        const unsigned long long* mkw = D.conn_mask + (size_t)CONN_MASK_WORDS * ww;
-        long long op = bp + toff_s[j], oe = be + toff_c[j];
-        for (int b0 = 0, wd = 0; b0 < npt; b0 += 64, ++wd) {  // surviving sub-tests in sub-test order
-          const int q = b0 + lane;
-          const unsigned long long mk = mkw[wd];
-          const bool keep = (mk >> lane) & 1ull;
-          const long long slot = op + __popcll(mk & lanes_below());
-          if (keep && slot < D.cap_items) D.pt_items[slot] = Item{(uint32_t)ww, (uint32_t)q};
-          op += __popcll(mk);
-        }
-        for (int b0 = 0, wd = 6; b0 < nee; b0 += 64, ++wd) {
-          const int q = b0 + lane;
-          const unsigned long long mk = mkw[wd];
-          const bool keep = (mk >> lane) & 1ull;
-          const long long slot = oe + __popcll(mk & lanes_below());
-          if (keep && slot < D.cap_items) D.ee_items[slot] = Item{(uint32_t)ww, (uint32_t)q};
-          oe += __popcll(mk);
-        }
-      }
-      bp += ttp, be += tte;
-      __syncthreads();
-    }
   }
 }
 
@@ -3796,15 +3820,14 @@ struct d2_ctx {
   bool pairs_valid = false;
   // work
   DBuf<NP> soup_list[2], conn_list[2];  // level l reads [l & 1] and writes [(l + 1) & 1]
-  DBuf<Item> items, pt_items, ee_items;
+  DBuf<Item> items, pt_items, ee_items, lpt_items, lee_items;
   DBuf<DItem> ditems;
   DBuf<DItem> ditems_def;  // FP32 form: deferred items of inner node pairs
   DBuf<double> res;
   DBuf<unsigned> res_mask;  // FP32 form: per soup item, the slots its FP32 culls keep
   DBuf<int> np_hit, np_hit2, exp_desc;
   DBuf<ContactRec> contacts;
-  DBuf<unsigned long long> cnt, lvl, masks, conn_mask;
-  DBuf<int> cnt_a, cnt_s, cnt_c, cnt_pt, cnt_ee, parts;
+  DBuf<unsigned long long> cnt, lvl;
   DBuf<unsigned long long> pass_min_s, pass_min_c;
   DBuf<int> pass_flag_s, pass_flag_c;
   DBuf<double> min_time, scale;
@@ -4046,6 +4069,8 @@ Dev make_dev(d2_ctx* c, int level, int discrete) {
   D.ditems_def = c->ditems_def.p;
   D.pt_items = c->pt_items.p;
   D.ee_items = c->ee_items.p;
+  D.lpt_items = c->lpt_items.p;
+  D.lee_items = c->lee_items.p;
   D.res = c->res.p;
   D.res_mask = c->res_mask.p;
   D.np_hit = (level & 1) ? c->np_hit2.p : c->np_hit.p;
@@ -4055,11 +4080,6 @@ Dev make_dev(d2_ctx* c, int level, int discrete) {
   D.contacts = c->contacts.p;
   D.cnt = c->cnt.p;
   D.lvl = c->lvl.p;
-  D.masks = c->masks.p;
-  D.cnt_a = c->cnt_a.p, D.cnt_s = c->cnt_s.p, D.cnt_c = c->cnt_c.p, D.cnt_pt = c->cnt_pt.p, D.cnt_ee = c->cnt_ee.p;
-  const int g = chunk_grid(c);
-  D.part_a = c->parts.p, D.part_s = c->parts.p + g, D.part_c = c->parts.p + 2 * g, D.part_pt = c->parts.p + 3 * g,
-  D.part_ee = c->parts.p + 4 * g;
   D.pass_min_s = c->pass_min_s.p, D.pass_min_c = c->pass_min_c.p;
   D.pass_flag_s = c->pass_flag_s.p, D.pass_flag_c = c->pass_flag_c.p;
   D.min_time = c->min_time.p;
@@ -4071,7 +4091,7 @@ Dev make_dev(d2_ctx* c, int level, int discrete) {
   D.prune = c->prune_on && !c->touch_on && c->nbound.p ? 1 : 0;  // accounting runs walk the reference's node pairs
   D.defer = c->defer_on && c->precision == D2_FP32 && c->ditems_def.p ? 1 : 0;  // per level: enqueue_level
   D.box_test = 1;
-  D.conn_mask = c->conn_mask.p;
+  D.conn_blocks = 0;
   D.body_tree = c->body_tree.p;
   D.fp32 = c->precision == D2_FP32 ? 1 : 0;
   D.n_pairs = c->n_pairs;
@@ -4092,21 +4112,20 @@ int level_budget(const d2_ctx* c) { return std::min(MAX_LEVELS, c->pair_depth + 
 int prepare(d2_ctx* c) {
   const size_t np = (size_t)std::max(c->n_pairs, 1);
   const size_t g = (size_t)chunk_grid(c);
-  if (c->precision == D2_FP32) RC(ensure(c, c->pair_f, np * PF_STRIDE));
+  if (c->precision == D2_FP32) RC(ensure(c, c->pair_f, np * std::max((int)PF_STRIDE, (int)CF_STRIDE)));
   for (int k = 0; k < 2; ++k) {
     RC(ensure(c, c->soup_list[k], c->cap));
     RC(ensure(c, c->conn_list[k], c->cap));
   }
-  RC(ensure(c, c->items, c->cap_res)); RC(ensure(c, c->pt_items, c->cap_items));
-  RC(ensure(c, c->ee_items, c->cap_items));
-  if (c->precision == D2_FP32) {  // FP64: k_tri_full keeps no item list
+  RC(ensure(c, c->items, c->cap_res)); RC(ensure(c, c->lpt_items, c->cap_items));
+  RC(ensure(c, c->lee_items, c->cap_items));
+  if (c->precision == D2_FP32) {  // FP64: k_tri_full keeps no item list, and every soup sub-test runs
+    RC(ensure(c, c->pt_items, c->cap_items));
+    RC(ensure(c, c->ee_items, c->cap_items));
     RC(ensure(c, c->ditems, c->cap_items));
     RC(ensure(c, c->ditems_def, c->cap_items));
   }
-  RC(ensure(c, c->np_hit, c->cap)); RC(ensure(c, c->np_hit2, c->cap)); RC(ensure(c, c->exp_desc, c->cap)); RC(ensure(c, c->masks, c->cap));
-  RC(ensure(c, c->cnt_a, c->cap)); RC(ensure(c, c->cnt_s, c->cap)); RC(ensure(c, c->cnt_c, c->cap));
-  RC(ensure(c, c->cnt_pt, c->cap)); RC(ensure(c, c->cnt_ee, c->cap)); RC(ensure(c, c->parts, 5 * g));
-  RC(ensure(c, c->conn_mask, (size_t)c->cap * CONN_MASK_WORDS));
+  RC(ensure(c, c->np_hit, c->cap)); RC(ensure(c, c->np_hit2, c->cap)); RC(ensure(c, c->exp_desc, c->cap));
   RC(ensure(c, c->contacts, c->cap_contacts)); RC(ensure(c, c->cnt, C_COUNT));
   RC(ensure(c, c->hscratch, 6 * (size_t)c->cap_contacts));
   RC(ensure(c, c->lvl, (size_t)2 * (MAX_LEVELS + 1) * LV_STRIDE));
@@ -4148,9 +4167,8 @@ void scan_host_n(d2_ctx* c, const int* in, int* out, long long n, unsigned long 
 // Launch grids of one level: the tuned block counts are the caps; a level
 // that was small in the last run of its phase gets fewer blocks (at least 16,
 // in powers of two, with 25% headroom): the culling kernels keep about one
-// node pair per wavefront (they are latency-bound, so as many wavefronts as
-// there is work), the count/write pair one soup node pair per thread or one
-// connected node pair per wavefront, the stream kernels one unit per thread.
+// node pair per wavefront (they are latency-bound on small levels, so as many
+// wavefronts as there is work), the others one unit per thread.
 // Any grid gives the same results; only the time changes.
 // def: k_tri_def's grid, 0 where the level defers nothing; box: whether
 // k_tri_mask runs the face-axis box test.  Both pay on large levels only (on
@@ -4158,26 +4176,28 @@ void scan_host_n(d2_ctx* c, const int* in, int* out, long long n, unsigned long 
 // they save), judged by the last run's sizes of the level: at least 64 K
 // items, at least 256 K node pairs.
 struct LevelGrids {
-  int cull, expand, stream, def, box;
+  int cull, conn, stream, sub, def, box;
 };
 LevelGrids level_grids(const d2_ctx* c, int discrete, int level) {
-  LevelGrids g{chunk_grid(c), chunk_grid(c), stream_grid(c), stream_grid(c), 1};
+  LevelGrids g{chunk_grid(c), chunk_grid(c), stream_grid(c), 2 * stream_grid(c), stream_grid(c), 1};
   const int ph = discrete ? 0 : 1;
   if (!c->prev_ok[ph] || level > MAX_LEVELS) return g;
   const long long* v = c->prev_lv[ph][level];
-  const long long ns = v[LV_SOUP], nc = v[LV_CONN];
-  const long long units = discrete ? v[LV_ITEMS] : std::max(std::max(9 * v[LV_ITEMS], v[LV_PT]), v[LV_EE]);
+  const long long ns = v[LV_SOUP];
   auto fit = [](long long n, long long per, int hi) {
     long long b = 16;
     while (b < hi && b * per < n + n / 4) b <<= 1;
     return (int)std::min<long long>(b, hi);
   };
   g.cull = fit(ns, 4, g.cull);
-  g.expand = fit(std::max((ns + 63) / 64, nc), 4, g.expand);
-  g.stream = fit(units, 256, g.stream);
+  g.conn = fit(v[LV_CONN], 4, g.conn);
+  g.stream = fit(v[LV_ITEMS], 256, g.stream);
   if (discrete) {
     g.def = v[LV_ITEMS] + v[LV_DEF] >= (1ll << 16) ? fit(v[LV_DEF], 256, g.def) : 0;
     g.box = ns >= (1ll << 18) ? 1 : 0;
+  } else {
+    const long long soup = c->precision == D2_FP32 ? v[LV_SPT] + v[LV_SEE] : 15 * v[LV_ITEMS];
+    g.sub = fit(soup + v[LV_PT] + v[LV_EE], 256, g.sub);
   }
   return g;
 }
@@ -4185,7 +4205,7 @@ unsigned long long grids_hash(const d2_ctx* c, int discrete, int levels) {
   unsigned long long h = 1469598103934665603ull;
   for (int l = 0; l < levels; ++l) {
     const LevelGrids g = level_grids(c, discrete, l);
-    h = (h ^ (unsigned long long)((((g.cull * 131071ll + g.expand) * 131071ll + g.stream) * 131071ll + g.def) * 2 +
+    h = (h ^ (unsigned long long)(((((g.cull * 131071ll + g.conn) * 131071ll + g.stream) * 131071ll + g.sub) * 131071ll + g.def) * 2 +
                                   g.box)) *
         1099511628211ull;
   }
@@ -4250,7 +4270,7 @@ void enqueue_level(d2_ctx* c, int level, int discrete) {
   if (c->touch_on && !c->capturing) touch_level(c, level, discrete);
   Dev D = make_dev(c, level, discrete);
   const LevelGrids G = level_grids(c, discrete, level);
-  const int cg = G.cull, eg = G.expand, sg = G.stream;
+  const int cg = G.cull, sg = G.stream;
   D.defer = D.defer && G.def > 0 ? 1 : 0;
   D.box_test = G.box;
   if (discrete && c->precision == D2_FP32) {
@@ -4261,22 +4281,16 @@ void enqueue_level(d2_ctx* c, int level, int discrete) {
     if (D.prune) timed_launch(c, K_TRI_FULL, k_tri_full<true>, dim3(cg), dim3(256), D);
     else timed_launch(c, K_TRI_FULL, k_tri_full<false>, dim3(cg), dim3(256), D);
   } else {
-    timed_launch(c, K_SOUP_CULL, k_soup_cull, dim3(cg), dim3(256), D);
+    // the connected list of level 0 is empty (roots go to the soup list)
+    D.conn_blocks = level > 0 ? G.conn : 0;
+    timed_launch(c, K_SOUP_CULL, k_ccd_cull, dim3(cg + D.conn_blocks), dim3(256), D);
     if (D.fp32) timed_launch(c, K_SOUP_KEEP, k_soup_keep, dim3(sg), dim3(256), D);  // FP32 culls + survivor lists
-    timed_launch(c, K_SOUP_EDGE, k_soup_sub, dim3(2 * sg), dim3(256), D);  // point and edge sub-tests
+    timed_launch(c, K_SOUP_EDGE, k_ccd_sub, dim3(G.sub), dim3(256), D);
     timed_launch(c, K_SOUP_REDUCE, k_soup_reduce, dim3(sg), dim3(256), D);
   }
-  if (discrete && c->precision != D2_FP32) {
+  if (discrete && c->precision != D2_FP32) {  // FP32 discrete levels are expanded by k_tri_mask
     Timer tm(c, K_EXPAND, 0.0);
     hipLaunchKernelGGL(k_disc_expand, dim3(cg), dim3(256), 0, c->stream, D);
-  } else if (!discrete) {  // FP32 discrete levels are expanded by k_tri_mask
-    Timer tm(c, K_EXPAND, 0.0);
-    hipLaunchKernelGGL(k_level_count, dim3(eg), dim3(256), 0, c->stream, D);
-    hipLaunchKernelGGL(k_level_write, dim3(eg), dim3(256), 0, c->stream, D);
-  }
-  if (!discrete) {
-    // the connected list of level 0 is empty (roots go to the soup list)
-    if (level > 0) timed_launch(c, K_LEAF_EDGE, k_leaf_sub, dim3(2 * sg), dim3(256), D);
   }
 }
 
@@ -4914,9 +4928,8 @@ int d2_ctx_destroy(d2_ctx* c) {
   release(c->nodes), release(c->buckets), release(c->fbuckets), release(c->stris), release(c->tree_off), release(c->body_tree), release(c->bodies);
   release(c->pairs), release(c->pair_info), release(c->cluster_of_pair), release(c->max_time), release(c->pair_rec), release(c->pair_f);
   for (int k = 0; k < 2; ++k) release(c->soup_list[k]), release(c->conn_list[k]);
-  release(c->items), release(c->ditems), release(c->ditems_def), release(c->pt_items), release(c->ee_items), release(c->res), release(c->res_mask), release(c->np_hit), release(c->np_hit2), release(c->exp_desc);
-  release(c->contacts), release(c->cnt), release(c->lvl), release(c->masks), release(c->conn_mask);
-  release(c->cnt_a), release(c->cnt_s), release(c->cnt_c), release(c->cnt_pt), release(c->cnt_ee), release(c->parts);
+  release(c->items), release(c->ditems), release(c->ditems_def), release(c->pt_items), release(c->ee_items), release(c->lpt_items), release(c->lee_items), release(c->res), release(c->res_mask), release(c->np_hit), release(c->np_hit2), release(c->exp_desc);
+  release(c->contacts), release(c->cnt), release(c->lvl);
   release(c->pass_min_s), release(c->pass_min_c), release(c->pass_flag_s), release(c->pass_flag_c);
   release(c->min_time), release(c->scale);
   release(c->pair_cnt), release(c->pair_off), release(c->pair_fill), release(c->perm), release(c->keep),

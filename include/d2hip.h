@@ -86,8 +86,8 @@ int d2_set_capacity(d2_ctx* ctx, int64_t entries);
 int d2_set_auto_grow(d2_ctx* ctx, int on);
 
 /* Launch shapes (no reference counterpart: the reference runs on the CPU).
- * chunk_blocks: blocks of the chunked list kernels (1-4096; a list is split
- * into that many contiguous ranges); stream_blocks: blocks of the
+ * chunk_blocks: blocks of the list kernels (1-4096; each takes its share of
+ * a list); stream_blocks: blocks of the
  * grid-stride kernels (1-16384); post_blocks: 256-thread blocks of the
  * per-pair post-processing (1-16384).  Defaults: 4, 8 and 16 per CU.
  * Results do not depend on them; d2_autotune picks them by timing. */

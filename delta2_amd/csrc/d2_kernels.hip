@@ -2035,11 +2035,14 @@ __global__ void __launch_bounds__(256) k_touch_count(const unsigned* nodes_bits,
 // The plugin point's unit of work (strategy::ContactDetectionStrategy::
 // findContactsBucketComparison, contact_detection_strategy.h:11, and its
 // implementation comparison_dist.h:205-240): a list of node pairs of two
-// bodies compared at the bodies' future states.  One wavefront per node pair,
-// lane 8 i + j tests triangle i of a against triangle j of b in FP64
-// (tri_tri_dist); a node pair's hits take one slot range (one atomic), and
-// k_bucket_scan / k_bucket_place put them in the reference's order: node-pair
-// order, then i, then j -- the lane order.
+// bodies compared at the bodies' future states.  A wavefront takes consecutive
+// node pairs in groups of at most 64 triangle pairs, one per lane, each tested
+// in FP64 (tri_tri_dist): the latency of that test's serial chain bounds short
+// lists, and a wavefront per node pair left 59 of 64 lanes idle at the leaves
+// (6,007 node pairs: 83 -> 29 us).  A node pair's hits are
+// consecutive slots of its wavefront's range (one atomic), and k_bucket_scan /
+// k_bucket_place put them in the reference's order: node-pair order, then i,
+// then j -- the lane order.
 struct BucketArgs {
   const int32_t* np_list;  // [n][2] node indices within the two trees
   int n;
@@ -2063,42 +2066,57 @@ __global__ void __launch_bounds__(256) k_bucket_pairs(BucketArgs A) {
     pose(quat{sb[0], sb[1], sb[2], sb[3]}, v3<double>{sb[4], sb[5], sb[6]}, sT + 16);
   }
   __syncthreads();
-  const int lane = lane_id();
-  const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const long long n_waves = ((long long)gridDim.x * blockDim.x) >> 6;
+  __shared__ unsigned char s_own[4][64];
+  const int lane = lane_id(), wid = threadIdx.x >> 6;
   const double geo_a = A.body_a[37], geo_b = A.body_b[37];
   const double search = (double)(float)(geo_a + geo_b);  // float search distance (comparison_dist.h:207)
-  const int i = lane >> 3, j = lane & 7;
-  for (long long k = wave; k < A.n; k += n_waves) {
-    const int la = A.np_list[2 * k], lb = A.np_list[2 * k + 1];
-    const NodeRec na = A.nodes[A.off_a + la];
-    const NodeRec nb = A.nodes[A.off_b + lb];
-    const double* ba = A.buckets + (size_t)BUCKET * (A.off_a + na.bucket);
-    const double* bb = A.buckets + (size_t)BUCKET * (A.off_b + nb.bucket);
-    bool hit = false;
-    v3<double> P{0, 0, 0}, Q{0, 0, 0};
-    if (i < na.ntris && j < nb.ntris) {
-      const tri<double> TA = xform(sT, load_tri<double>(ba, i));
-      const tri<double> TB = xform(sT + 16, load_tri<double>(bb, j));
-      const double d = tri_tri_dist(TA, TB, P, Q);
-      hit = d < (search + ba[72 + i]) + bb[72 + j];
+  for (Tiles T(A.n, blockIdx.x, gridDim.x, 4); T.b0 < A.n; T.b0 += T.step) {
+    const long long w0 = T.first(wid), wl = w0 + lane;
+    const bool in_range = lane < T.part && wl < A.n;
+    int l_a = 0, l_b = 0, l_ga = 0, l_gb = 0, l_m = 0, jobs = 0;
+    if (in_range) {
+      l_a = A.np_list[2 * wl], l_b = A.np_list[2 * wl + 1];
+      const NodeRec na = A.nodes[A.off_a + l_a];
+      const NodeRec nb = A.nodes[A.off_b + l_b];
+      l_ga = A.off_a + na.bucket, l_gb = A.off_b + nb.bucket, l_m = nb.ntris;
+      jobs = na.ntris * nb.ntris;
+      if (jobs == 0) A.base[wl] = 0, A.count[wl] = 0;
     }
-    const unsigned long long mask = __ballot(hit);
-    const int cnt = __popcll(mask);
-    unsigned long long b0 = 0;
-    if (lane == 0 && cnt) b0 = atomicAdd(A.counter, (unsigned long long)cnt);
-    b0 = readlane_u64(b0, 0);
-    if (lane == 0) A.base[k] = (long long)b0, A.count[k] = cnt;
-    if (hit) {
-      const long long slot = (long long)b0 + __popcll(mask & lanes_below());
-      if (slot < A.cap) {
-        ContactRec c;
-        c.key = 0ull;
-        c.pair = 0, c.na = la, c.nb = lb, c.kind = 0, c.ia = i, c.ib = j, c.level = 0, c.pad = 0;
-        c.r[0] = P.x, c.r[1] = P.y, c.r[2] = P.z, c.r[3] = Q.x, c.r[4] = Q.y, c.r[5] = Q.z;
-        c.r[6] = geo_a + ba[72 + i], c.r[7] = geo_b + bb[72 + j];  // Contact(P, Q, geo + eps, ..., inner eps)
-        c.r[8] = ba[80 + i], c.r[9] = bb[80 + j], c.r[10] = 0.0;
-        A.hits[slot] = c;
+    for (Groups g(jobs, jobs); g.next(false);) {  // a triangle pair per lane
+      const int src = run_owner(s_own[wid], g.js, g.in ? g.jobs : 0);
+      const int r = lane - __shfl(g.js, src), m = __shfl(l_m, src);
+      const int la = __shfl(l_a, src), lb = __shfl(l_b, src), ga = __shfl(l_ga, src), gb = __shfl(l_gb, src);
+      const double* ba = A.buckets + (size_t)BUCKET * ga;
+      const double* bb = A.buckets + (size_t)BUCKET * gb;
+      bool hit = false;
+      int i = 0, j = 0;
+      v3<double> P{0, 0, 0}, Q{0, 0, 0};
+      if (lane < g.n_jobs) {
+        i = r / m, j = r - i * m;
+        const tri<double> TA = xform(sT, load_tri<double>(ba, i));
+        const tri<double> TB = xform(sT + 16, load_tri<double>(bb, j));
+        const double d = tri_tri_dist(TA, TB, P, Q);
+        hit = d < (search + ba[72 + i]) + bb[72 + j];
+      }
+      const unsigned long long mask = __ballot(hit);
+      unsigned long long b0 = 0;
+      if (lane == 0 && mask) b0 = atomicAdd(A.counter, (unsigned long long)__popcll(mask));
+      b0 = readlane_u64(b0, 0);
+      if (g.in) {
+        A.base[wl] = (long long)b0 + __popcll(mask & ((1ull << g.js) - 1ull));
+        A.count[wl] = __popcll(g.share(mask, 0));
+      }
+      if (hit) {
+        const long long slot = (long long)b0 + __popcll(mask & lanes_below());
+        if (slot < A.cap) {
+          ContactRec c;
+          c.key = 0ull;
+          c.pair = 0, c.na = la, c.nb = lb, c.kind = 0, c.ia = i, c.ib = j, c.level = 0, c.pad = 0;
+          c.r[0] = P.x, c.r[1] = P.y, c.r[2] = P.z, c.r[3] = Q.x, c.r[4] = Q.y, c.r[5] = Q.z;
+          c.r[6] = geo_a + ba[72 + i], c.r[7] = geo_b + bb[72 + j];  // Contact(P, Q, geo + eps, ..., inner eps)
+          c.r[8] = ba[80 + i], c.r[9] = bb[80 + j], c.r[10] = 0.0;
+          A.hits[slot] = c;
+        }
       }
     }
   }
@@ -2135,28 +2153,27 @@ __global__ void __launch_bounds__(256) k_filter_load(int n, const double* reals,
 // reference's cumulative counts (pair_used_out[k] = hits up to and including
 // node pair k, comparison_dist.h:238); one block.
 __global__ void __launch_bounds__(1024) k_bucket_scan(int n, const int* count, long long* off, int32_t* used) {
-  __shared__ long long s[1024];
-  const int t = threadIdx.x;
-  const int per = (n + 1023) / 1024;
-  const int b = t * per, e = b + per < n ? b + per : n;
-  long long sum = 0;
-  for (int k = b; k < e; ++k) sum += count[k];
-  s[t] = sum;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {  // inclusive scan of the chunk sums
-    const long long v = t >= d ? s[t - d] : 0;
-    __syncthreads();
-    s[t] += v;
-    __syncthreads();
-  }
-  long long run = t ? s[t - 1] : 0;
-  for (int k = b; k < e; ++k) {
-    off[k] = run;
-    run += count[k];
-    used[k] = (int32_t)run;
+  constexpr int K = 8;  // node pairs per thread and round, read at once
+  long long carry = 0;
+  for (int b0 = 0; b0 < n; b0 += K * 1024) {
+    const int per = n - b0 < K * 1024 ? (n - b0 + 1023) / 1024 : K;
+    const int b = b0 + (int)threadIdx.x * per;
+    int v[K], sum = 0, total;
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = k < per && b + k < n ? count[b + k] : 0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) sum += v[k];
+    long long run = carry + block_scan(sum, total);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k >= per || b + k >= n) break;
+      off[b + k] = run;
+      run += v[k];
+      used[b + k] = (int32_t)run;
+    }
+    carry += total;
   }
 }
-
 // Each node pair's hits from their provisional slots to their final rows, in
 // the flat contact layout (8 int32 + 11 doubles per hit).
 __global__ void __launch_bounds__(256) k_bucket_place(int n, const long long* base, const int* count,
@@ -4984,8 +5001,9 @@ int bucket_run(d2_ctx* c, const BucketScratch& S, int a, int b, int n, const int
   A.off_a = c->host_tree_off[c->host_body_tree[a]], A.off_b = c->host_tree_off[c->host_body_tree[b]];
   A.body_a = c->bodies.p + 40 * (size_t)a, A.body_b = c->bodies.p + 40 * (size_t)b;
   A.hits = S.hits, A.cap = S.cap_hits, A.counter = S.counter, A.base = S.base, A.count = S.count;
-  const int blocks = (int)std::min<long long>((n + 3) / 4, (long long)c->cus * 8);
-  hipLaunchKernelGGL(k_bucket_pairs, dim3(blocks), dim3(256), 0, c->stream, A);
+  const int blocks = (int)std::min<long long>((n + 3) / 4, (long long)c->cus * 8);  // a node pair per wavefront
+  // two wavefronts per SIMD (what fits), then several node pairs per wavefront
+  hipLaunchKernelGGL(k_bucket_pairs, dim3(std::min(blocks, c->cus * 2)), dim3(256), 0, c->stream, A);
   hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, c->stream, n, (const int*)S.count, S.off, S.used);
   HIPCHK(c, hipGetLastError());
   unsigned long long hits = 0;

@@ -1625,6 +1625,73 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
 }
 
 
+// tri_tri_dist by the four lanes of a quad (each with the whole operands; the
+// fourth does the first's share again): lane q takes corner q of either
+// triangle against the other's plane, a's edge q against b's three edges, and
+// edge q of either triangle through the other, a third of the serial chain.
+// The quad then picks what the sequential walk keeps: of the candidate
+// distances the smallest, the earliest of equal ones; of the piercings the last.
+__device__ __forceinline__ double quad_bcast(double v, int from) {
+  return __shfl(v, (lane_id() & ~3) | from);
+}
+// aq, ae, bq, be: corners q and q + 1 of a and b (read and transformed again by
+// the caller: choosing them from a and b puts the triangles in scratch memory).
+__device__ __forceinline__ int quad_share() {
+  const int k = lane_id() & 3;
+  return k == 3 ? 0 : k;
+}
+__device__ __forceinline__ double tri_tri_dist_quad(const tri<double>& a, const tri<double>& b, v3<double> aq,
+                                                    v3<double> ae, v3<double> bq, v3<double> be, v3<double>& P,
+                                                    v3<double>& Q) {
+  const int q = quad_share();
+  double best = 1.0 / 0.0;
+  int at = 99;  // place in the sequential order
+  bool in;
+  {
+    const v3<double> p = project_plane(a, bq, in);
+    const double d = vlen(sub(p, bq));
+    if (in && d < best) P = p, Q = bq, best = d, at = q;
+  }
+  {
+    const v3<double> p = project_plane(b, aq, in);
+    const double d = vlen(sub(aq, p));
+    if (in && d < best) P = aq, Q = p, best = d, at = 3 + q;
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    v3<double> x, y;
+    const double d = seg_closest(aq, ae, corner(b, j), corner(b, (j + 1) % 3), x, y);
+    if (d < best) P = x, Q = y, best = d, at = 6 + 3 * q + j;
+  }
+  int pierce = 0;  // 1 + place in the sequential order
+  v3<double> X{0, 0, 0};
+  bool tinf, hit;
+  double t = segment_hit(a, bq, be, tinf, hit);
+  if (hit) X = lerp(bq, be, t), pierce = 1 + q;
+  t = segment_hit(b, aq, ae, tinf, hit);
+  if (hit) X = lerp(aq, ae, t), pierce = 4 + q;
+  int win = 0, wp = 0;
+  double wd = quad_bcast(best, 0);
+  int wa = __shfl(at, lane_id() & ~3), wv = __shfl(pierce, lane_id() & ~3);
+#pragma unroll
+  for (int l = 1; l < 3; ++l) {
+    const double od = quad_bcast(best, l);
+    const int oa = __shfl(at, (lane_id() & ~3) | l), ov = __shfl(pierce, (lane_id() & ~3) | l);
+    if (od < wd || (od == wd && oa < wa)) wd = od, wa = oa, win = l;
+    if (ov > wv) wv = ov, wp = l;
+  }
+  P = v3<double>{quad_bcast(P.x, win), quad_bcast(P.y, win), quad_bcast(P.z, win)};
+  Q = v3<double>{quad_bcast(Q.x, win), quad_bcast(Q.y, win), quad_bcast(Q.z, win)};
+  X = v3<double>{quad_bcast(X.x, wp), quad_bcast(X.y, wp), quad_bcast(X.z, wp)};
+  if (wv > 0) P = Q = X;
+  return vlen(sub(P, Q));
+}
+// Items up to which the FP64 triangle tests take a quad each instead of a lane:
+// half of what leaves every SIMD its two wavefronts (what the test's registers
+// allow).  A launch of 1,000 to 16,000 items takes 15.8 us with a lane per item,
+// 12.5 with a quad; at 22,000 to 31,000 both take the same, above a quad loses
+// (three lanes repeat the loads and the planes).  A 100-body step: 808 -> 785 us.
+constexpr long long QUAD_ITEMS = 1 << 14;
 // The FP64 test of one item (comparison_dist.h:205-240's leaf test): the
 // reference's triangle distance at the phase's poses against search + eps_a
 // + eps_b.
@@ -1634,7 +1701,7 @@ struct ItemTest {
   int i, j;
   bool hit;
 };
-__device__ __forceinline__ ItemTest item_test(const Dev& D, const DItem& item) {
+template <bool QUAD> __device__ __forceinline__ ItemTest item_test(const Dev& D, const DItem& item) {
   ItemTest r;
   const double* pr = D.pair_rec + (size_t)PR_STRIDE * item.pair;
   const double* ba = D.buckets + (size_t)BUCKET * item.ga;
@@ -1643,13 +1710,21 @@ __device__ __forceinline__ ItemTest item_test(const Dev& D, const DItem& item) {
   r.i = sub >> 3, r.j = sub & 7;
   const tri<double> A = xform(pr + PR_TA1, load_tri<double>(ba, r.i));
   const tri<double> B = xform(pr + PR_TB1, load_tri<double>(bb, r.j));
-  const double d = tri_tri_dist(A, B, r.P, r.Q);
+  double d;
+  if (QUAD) {
+    const int q = quad_share(), e = q == 2 ? 0 : q + 1;
+    d = tri_tri_dist_quad(A, B, xform(pr + PR_TA1, load_corner(ba, r.i, q)), xform(pr + PR_TA1, load_corner(ba, r.i, e)),
+                          xform(pr + PR_TB1, load_corner(bb, r.j, q)), xform(pr + PR_TB1, load_corner(bb, r.j, e)), r.P,
+                          r.Q);
+  } else {
+    d = tri_tri_dist(A, B, r.P, r.Q);
+  }
   r.ea = ba[72 + r.i], r.eb = bb[72 + r.j];
   r.hit = d < (pr[PR_SEARCH] + r.ea) + r.eb;
   return r;
 }
 // FP64 triangle-pair distances of the level's items (grid-stride).
-__global__ void __launch_bounds__(256) k_tri_dist(Dev D) {
+template <bool QUAD> __global__ void __launch_bounds__(256) k_tri_dist(Dev D) {
   const unsigned long long pack = D.lv(D.level, LV_PACK);
   const long long n_items = (long long)(pack & 0xffffffffull);
   const long long count = n_items < D.cap_items ? n_items : D.cap_items;
@@ -1658,10 +1733,11 @@ __global__ void __launch_bounds__(256) k_tri_dist(Dev D) {
     D.lvl[(D.level + 1) * LV_STRIDE + LV_SOUP] = pack >> 32;
     atomicAdd(&D.cnt[C_LVL_ITEMS], (unsigned long long)n_items);
   }
-  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < count; t += (long long)gridDim.x * blockDim.x) {
+  const long long stride = (long long)gridDim.x * blockDim.x / (QUAD ? 4 : 1);
+  for (long long t = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / (QUAD ? 4 : 1); t < count; t += stride) {
     const DItem item = D.ditems[t];
-    const ItemTest r = item_test(D, item);
-    if (!r.hit) continue;
+    const ItemTest r = item_test<QUAD>(D, item);
+    if (!r.hit || (QUAD && (threadIdx.x & 3))) continue;
     D.np_hit[item.np] = 1;
     if (item.sub & 256u) continue;  // an inner node: the hit only expands the node pair
     unsigned long long slot = atomicAdd(&D.cnt[C_CONTACTS], 1ull);
@@ -1713,7 +1789,7 @@ __global__ void __launch_bounds__(256) k_tri_def(Dev D) {
       const int take = qn < 64 ? qn : 64;
       if (lane < take) {
         const DItem item = D.ditems_def[s_q[wid][lane]];
-        if (D.np_hit[item.np] == 0 && item_test(D, item).hit) D.np_hit[item.np] = 1;
+        if (D.np_hit[item.np] == 0 && item_test<false>(D, item).hit) D.np_hit[item.np] = 1;
       }
       const int rest = qn - take;  // below 64: move it to the queue's front
       const uint32_t v = lane < rest ? s_q[wid][take + lane] : 0u;
@@ -4249,10 +4325,10 @@ void scan_host_n(d2_ctx* c, const int* in, int* out, long long n, unsigned long 
 // they save), judged by the last run's sizes of the level: at least 64 K
 // items, at least 256 K node pairs.
 struct LevelGrids {
-  int cull, conn, stream, sub, def, box;
+  int cull, conn, stream, sub, def, box, quad;
 };
 LevelGrids level_grids(const d2_ctx* c, int discrete, int level) {
-  LevelGrids g{chunk_grid(c), chunk_grid(c), stream_grid(c), 2 * stream_grid(c), stream_grid(c), 1};
+  LevelGrids g{chunk_grid(c), chunk_grid(c), stream_grid(c), 2 * stream_grid(c), stream_grid(c), 1, 0};
   const int ph = discrete ? 0 : 1;
   if (!c->prev_ok[ph] || level > MAX_LEVELS) return g;
   const long long* v = c->prev_lv[ph][level];
@@ -4264,7 +4340,8 @@ LevelGrids level_grids(const d2_ctx* c, int discrete, int level) {
   };
   g.cull = fit(ns, 4, g.cull);
   g.conn = fit(v[LV_CONN], 4, g.conn);
-  g.stream = fit(v[LV_ITEMS], 256, g.stream);
+  if (discrete && v[LV_ITEMS] <= QUAD_ITEMS) g.quad = 1;
+  g.stream = fit(v[LV_ITEMS], g.quad ? 64 : 256, g.stream);
   if (discrete) {
     g.def = v[LV_ITEMS] + v[LV_DEF] >= (1ll << 16) ? fit(v[LV_DEF], 256, g.def) : 0;
     g.box = ns >= (1ll << 18) ? 1 : 0;
@@ -4278,8 +4355,8 @@ unsigned long long grids_hash(const d2_ctx* c, int discrete, int levels) {
   unsigned long long h = 1469598103934665603ull;
   for (int l = 0; l < levels; ++l) {
     const LevelGrids g = level_grids(c, discrete, l);
-    h = (h ^ (unsigned long long)(((((g.cull * 131071ll + g.conn) * 131071ll + g.stream) * 131071ll + g.sub) * 131071ll + g.def) * 2 +
-                                  g.box)) *
+    h = (h ^ (unsigned long long)(((((g.cull * 131071ll + g.conn) * 131071ll + g.stream) * 131071ll + g.sub) * 131071ll + g.def) * 4 +
+                                  2 * g.quad + g.box)) *
         1099511628211ull;
   }
   return h;
@@ -4348,7 +4425,7 @@ void enqueue_level(d2_ctx* c, int level, int discrete) {
   D.box_test = G.box;
   if (discrete && c->precision == D2_FP32) {
     timed_launch(c, K_TRI_MASK, k_tri_mask, dim3(cg), dim3(256), D);
-    timed_launch(c, K_TRI_DIST, k_tri_dist, dim3(sg), dim3(256), D);
+    timed_launch(c, K_TRI_DIST, G.quad ? k_tri_dist<true> : k_tri_dist<false>, dim3(sg), dim3(256), D);
     if (D.defer) timed_launch(c, K_TRI_DEF, k_tri_def, dim3(G.def), dim3(256), D);
   } else if (discrete) {  // as many wavefronts as there are node pairs, up to the tuned blocks
     if (D.prune) timed_launch(c, K_TRI_FULL, k_tri_full<true>, dim3(cg), dim3(256), D);

@@ -4355,9 +4355,8 @@ unsigned long long grids_hash(const d2_ctx* c, int discrete, int levels) {
   unsigned long long h = 1469598103934665603ull;
   for (int l = 0; l < levels; ++l) {
     const LevelGrids g = level_grids(c, discrete, l);
-    h = (h ^ (unsigned long long)(((((g.cull * 131071ll + g.conn) * 131071ll + g.stream) * 131071ll + g.sub) * 131071ll + g.def) * 4 +
-                                  2 * g.quad + g.box)) *
-        1099511628211ull;
+    for (int f : {g.cull, g.conn, g.stream, g.sub, g.def, 2 * g.quad + g.box})
+      h = (h ^ (unsigned long long)f) * 1099511628211ull;
   }
   return h;
 }

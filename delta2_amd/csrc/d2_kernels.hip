@@ -4028,6 +4028,7 @@ struct d2_ctx {
   // learned gate
   DBuf<float> tree_radius, tree_eps_out, hv, feat, pred;
   DBuf<int32_t> hv_off;
+  bool big_hulls = false;  // some tree's hull has more vertices than k_certify takes
   DBuf<int> cert;  // per pair: 1 = traverse (not certified)
   int gate_phases = 3;       // bit 0: CCD phase, bit 1: discrete phase
   DBuf<float> mlp_w, mlp_m, mlp_v, mlp_wf, mlp_grad;
@@ -4613,11 +4614,15 @@ void enqueue_gate(d2_ctx* c, const PhaseSpec& ph) {
                          FeatIn{c->pairs.p, c->bodies.p, c->body_tree.p, c->tree_radius.p, mt});
     }
     // at most CERT_LIST pairs per block; the kept pairs are the phase's roots
-    const int grid = std::max(std::max(1, std::min(np, c->cus * 8)), (np + CERT_LIST - 1) / CERT_LIST);
-    hipLaunchKernelGGL(k_certify, dim3(grid), dim3(256), 0, c->stream, np, c->pair_info.p, c->body_tree.p,
-                       c->pair_rec.p, c->pred.p, c->gate_t, c->gate_s, c->hv_off.p, c->hv.p, c->tree_eps_out.p,
-                       ph.discrete ? 1 : 0, c->cert.p, c->cnt.p + (ph.discrete ? C_GATED_DISC : C_GATED_CCD), D.soup,
-                       c->lvl.p + LV_SOUP);
+    const CertIn C{np, c->pair_info.p, c->body_tree.p, c->pair_rec.p, c->pred.p, c->gate_t, c->gate_s,
+                   c->hv_off.p, c->hv.p, c->tree_eps_out.p, ph.discrete ? 1 : 0};
+    unsigned long long* counts = c->cnt.p + (ph.discrete ? C_GATED_DISC : C_GATED_CCD);
+    const int fill = (np + CERT_LIST - 1) / CERT_LIST;
+    const int waves = std::max(std::max(1, std::min((np + 3) / 4, c->cus * 8)), fill);
+    hipLaunchKernelGGL(k_certify, dim3(waves), dim3(256), 0, c->stream, C, c->cert.p, counts, D.soup, c->lvl.p + LV_SOUP);
+    if (c->big_hulls)
+      hipLaunchKernelGGL(k_certify_block, dim3(std::max(std::max(1, std::min(np, c->cus * 8)), fill)), dim3(256), 0,
+                         c->stream, C, c->cert.p, counts, D.soup, c->lvl.p + LV_SOUP);
   }
 }
 
@@ -4966,6 +4971,7 @@ hipError_t copy_out(d2_ctx* c, std::initializer_list<CopyOut> parts, int max_thr
   std::atomic<size_t> launched[2] = {{0}, {0}};  // per half, windows launched into it so far: w + 1 of the last
   std::atomic<int> err{(int)hipSuccess};
   auto launch = [&](size_t w) {  // window w, into half w & 1 (window w - 2 has been copied on)
+    if (w > 1) (void)hipSetDevice(c->device);  // (maybe one of the threads below)
     CopyJob K = J;
     K.off = w * window, K.end = std::min<unsigned long long>(total, K.off + window);
     K.dst = c->stage + (w & 1) * window, K.count = c->stage_cnt + (w & 1) * per, K.flag = c->stage_flag + (w & 1) * per;
@@ -4992,7 +4998,6 @@ hipError_t copy_out(d2_ctx* c, std::initializer_list<CopyOut> parts, int max_thr
     }
   };
   auto work = [&] {
-    (void)hipSetDevice(c->device);
     for (size_t k; (k = next.fetch_add(1)) < chunks;) {
       const size_t w = k / per;
       if (!arrived(w, k % per)) return;
@@ -5558,6 +5563,8 @@ int d2_trees_upload(d2_ctx* c, int n_trees, const int32_t* tree_node_offset, con
   HIPCHK(c, hipMemcpyAsync(c->tb_box.p, tbox.data(), sizeof(float) * tbox.size(), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->tb_rad.p, trad.data(), sizeof(double) * n_trees, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->tree_depth_d.p, depth.data(), sizeof(int32_t) * n_trees, hipMemcpyHostToDevice, c->stream));
+  c->big_hulls = false;
+  for (int t = 0; t < n_trees; ++t) c->big_hulls = c->big_hulls || hv_off[t + 1] - hv_off[t] > CERT_WAVEV;
   RC(ensure(c, c->hv, std::max<size_t>(hv.size(), 3))); RC(ensure(c, c->hv_off, n_trees + 1));
   RC(ensure(c, c->tree_radius, n_trees)); RC(ensure(c, c->tree_eps_out, n_trees));
   HIPCHK(c, hipMemcpyAsync(c->hv.p, hv.data(), sizeof(float) * hv.size(), hipMemcpyHostToDevice, c->stream));

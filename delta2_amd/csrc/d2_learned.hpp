@@ -385,8 +385,7 @@ __global__ void k_mlp_round(const float* w, short* wb, float* wf) {
 //     union of a's two poses and b;
 //   a's frame: the same with the bodies swapped.
 // The discrete phase needs one bound: the two bodies at the future poses.
-// One block per pair; a set's vertices are transformed into LDS once; axes
-// come from Gilbert's minimum-norm-point iteration on the difference set
+// A set's vertices are transformed once; axes come from Gilbert's minimum-norm-point iteration on the difference set
 // (every iterate's axis gives a sound bound, the best one is kept).
 constexpr int CERT_MAXV = 1024;  // vertices per body held in LDS; larger bodies are not certified
 __device__ __forceinline__ void cert_mat(const double* m, const double* origin, float* o) {
@@ -395,31 +394,69 @@ __device__ __forceinline__ void cert_mat(const double* m, const double* origin, 
     o[4 * r + 3] = (float)(m[4 * r + 3] - (origin ? origin[r] : 0.0));
   }
 }
-// LDS copy of n body-frame vertices under the 3x4 matrix m (identity when null).
-__device__ void cert_load(const float* v, int n, const float* m, float* out, float& mag) {
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const float x = v[3 * k], y = v[3 * k + 1], z = v[3 * k + 2];
-    float o0 = x, o1 = y, o2 = z;
-    if (m) {
-      o0 = (m[0] * x + m[1] * y) + (m[2] * z + m[3]);
-      o1 = (m[4] * x + m[5] * y) + (m[6] * z + m[7]);
-      o2 = (m[8] * x + m[9] * y) + (m[10] * z + m[11]);
-    }
-    out[3 * k] = o0, out[3 * k + 1] = o1, out[3 * k + 2] = o2;
-    mag = fmaxf(mag, fmaxf(fabsf(o0), fmaxf(fabsf(o1), fabsf(o2))));
+// A vertex set under a pose.  CertBlock: a block's, in LDS; CertWave: a
+// wavefront's, in registers (vertex lane + 64 k in slot k), up to CERT_WAVEV.
+constexpr int CERT_SLOTS = 4, CERT_WAVEV = 64 * CERT_SLOTS;
+struct CertBlock {
+  float* v;
+  int n;
+};
+struct CertWave {
+  float v[CERT_SLOTS][3];
+  int n;
+};
+__device__ __forceinline__ void cert_move(const float* v, const float* m, float* o, float& mag) {
+  const float x = v[0], y = v[1], z = v[2];
+  o[0] = x, o[1] = y, o[2] = z;
+  if (m) {
+    o[0] = (m[0] * x + m[1] * y) + (m[2] * z + m[3]);
+    o[1] = (m[4] * x + m[5] * y) + (m[6] * z + m[7]);
+    o[2] = (m[8] * x + m[9] * y) + (m[10] * z + m[11]);
+  }
+  mag = fmaxf(mag, fmaxf(fabsf(o[0]), fmaxf(fabsf(o[1]), fabsf(o[2]))));
+}
+// n body-frame vertices under the 3x4 matrix m (as they are when null).
+__device__ __forceinline__ void cert_load(const float* v, int n, const float* m, CertBlock& S, float& mag) {
+  S.n = n;
+  for (int k = threadIdx.x; k < n; k += blockDim.x) cert_move(v + 3 * k, m, S.v + 3 * k, mag);
+}
+__device__ __forceinline__ void cert_load(const float* v, int n, const float* m, CertWave& S, float& mag) {
+  S.n = n;
+#pragma unroll
+  for (int k = 0; k < CERT_SLOTS; ++k) {
+    S.v[k][0] = S.v[k][1] = S.v[k][2] = 0.f;
+    if (lane_id() + 64 * k < n) cert_move(v + 3 * (lane_id() + 64 * k), m, S.v[k], mag);
   }
 }
-// Block-wide extreme of u.x over sets S[0..ns) (sign +1: max, -1: min) and
-// the point attaining it.
-__device__ float cert_extreme(const float* const* S, const int* n, int ns, const float* u, float sign, float* pt,
-                              float* red) {
+// Largest magnitude of all lanes' (block: and the sets are complete).
+__device__ __forceinline__ float cert_mag(const CertBlock&, float m, float* mag_red) {
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) mag_red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  float r = 0.f;
+  for (int i = 0; i < (int)(blockDim.x >> 6); ++i) r = fmaxf(r, mag_red[i]);
+  return r;
+}
+__device__ __forceinline__ float cert_mag(const CertWave&, float m, float*) {
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  return m;
+}
+__device__ __forceinline__ void cert_reuse(const CertBlock&) { __syncthreads(); }  // before a set is loaded anew
+__device__ __forceinline__ void cert_reuse(const CertWave&) {}
+// Extreme of u.x over A (and B: TWO) (sign +1: max, -1: min) and the point
+// attaining it; of equal ones the first vertex's, A's before B's.
+template <bool TWO>
+__device__ float cert_extreme(const CertBlock& A, const CertBlock& B, const float* u, float sign, float* pt, float* red) {
   float best = -3.4e38f, bp[3] = {0.f, 0.f, 0.f};
-  for (int s = 0; s < ns; ++s)
-    for (int k = threadIdx.x; k < n[s]; k += blockDim.x) {
-      const float* q = S[s] + 3 * k;
+  for (int s = 0; s < (TWO ? 2 : 1); ++s) {
+    const CertBlock& S = s ? B : A;
+    for (int k = threadIdx.x; k < S.n; k += blockDim.x) {
+      const float* q = S.v + 3 * k;
       const float pr = sign * ((u[0] * q[0] + u[1] * q[1]) + u[2] * q[2]);
       if (pr > best) best = pr, bp[0] = q[0], bp[1] = q[1], bp[2] = q[2];
     }
+  }
   for (int off = 32; off > 0; off >>= 1) {
     const float ob = __shfl_xor(best, off);
     const float o0 = __shfl_xor(bp[0], off), o1 = __shfl_xor(bp[1], off), o2 = __shfl_xor(bp[2], off);
@@ -437,13 +474,42 @@ __device__ float cert_extreme(const float* const* S, const int* n, int ns, const
   pt[0] = red[4 * w + 1], pt[1] = red[4 * w + 2], pt[2] = red[4 * w + 3];
   return sign * red[4 * w];
 }
-// Separation bound of P below Q along u: (min_Q u.q - max_P u.p) / |u|, and
-// the support points.
-__device__ float cert_axis(const float* const* P, const int* nP, int nsP, const float* const* Q, const int* nQ, int nsQ,
-                           const float* u, float* pp, float* qq, float* red) {
+template <bool TWO>
+__device__ __forceinline__ float cert_extreme(const CertWave& A, const CertWave& B, const float* u, float sign, float* pt,
+                                              float*) {
+  float best = -3.4e38f, bp[3] = {0.f, 0.f, 0.f};
+  int bv = 1 << 20;
+#pragma unroll
+  for (int k = 0; k < CERT_SLOTS; ++k) {
+    const int v = lane_id() + 64 * k;
+#pragma unroll
+    for (int s = 0; s < (TWO ? 2 : 1); ++s) {
+      const CertWave& S = s ? B : A;
+      const float* q = S.v[k];
+      const float pr = sign * ((u[0] * q[0] + u[1] * q[1]) + u[2] * q[2]);
+      if (v < S.n && pr > best) best = pr, bp[0] = q[0], bp[1] = q[1], bp[2] = q[2], bv = v;
+    }
+  }
+  float top = best;
+  for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
+  unsigned long long m = __ballot(best == top);
+  int l = __ffsll((long long)m) - 1;
+  for (m &= m - 1ull; m; m &= m - 1ull) {
+    const int o = __ffsll((long long)m) - 1;
+    if (rl(bv, o) < rl(bv, l)) l = o;
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) pt[k] = __int_as_float(rl(__float_as_int(bp[k]), l));
+  return sign * top;
+}
+// Separation bound of P (P0, P1: TWO) below Q along u: (min_Q u.q - max_P u.p)
+// / |u|, and the support points.
+template <bool TWO, class Set>
+__device__ __forceinline__ float cert_axis(const Set& P0, const Set& P1, const Set& Q, const float* u, float* pp, float* qq,
+                                           float* red) {
   const float nu = sqrtf((u[0] * u[0] + u[1] * u[1]) + u[2] * u[2]);
-  const float hp = cert_extreme(P, nP, nsP, u, 1.f, pp, red);
-  const float lq = cert_extreme(Q, nQ, nsQ, u, -1.f, qq, red);
+  const float hp = cert_extreme<TWO>(P0, P1, u, 1.f, pp, red);
+  const float lq = cert_extreme<false>(Q, Q, u, -1.f, qq, red);
   return nu > 1e-30f ? (lq - hp) / nu : -3.4e38f;
 }
 // Gilbert's minimum-norm-point iteration on the difference set Q - P from the
@@ -454,17 +520,19 @@ __device__ float cert_axis(const float* const* P, const int* nP, int nsP, const 
 // With stop >= 0 the iteration ends as soon as the answer to "best > stop"
 // is known: a gap above stop, or an iterate x with |x| <= stop (x lies in the
 // hull of the difference set, so no axis can separate it by more than |x|).
-__device__ float cert_gilbert(const float* const* P, const int* nP, int nsP, const float* const* Q, const int* nQ,
-                              int nsQ, const float* x0, int iters, float* u_out, float* red, float stop = -1.f) {
+template <bool TWO, class Set>
+__device__ __forceinline__ float cert_gilbert(const Set& P0, const Set& P1, const Set& Q, const float* x0, int iters,
+                                              float* u_out, float* red, float stop = -1.f) {
   float x[3] = {x0[0], x0[1], x0[2]};
   float best = -3.4e38f;
   u_out[0] = x[0], u_out[1] = x[1], u_out[2] = x[2];
+#pragma unroll 1
   for (int it = 0; it < iters; ++it) {
     const float xx = (x[0] * x[0] + x[1] * x[1]) + x[2] * x[2];
     if (!(xx > 1e-30f)) break;
     if (stop >= 0.f && it > 0 && xx <= stop * stop) break;
     float pp[3], qq[3];
-    const float g = cert_axis(P, nP, nsP, Q, nQ, nsQ, x, pp, qq, red);
+    const float g = cert_axis<TWO>(P0, P1, Q, x, pp, qq, red);
     if (g > best) best = g, u_out[0] = x[0], u_out[1] = x[1], u_out[2] = x[2];
     if (stop >= 0.f && best > stop) break;
     const float sd[3] = {qq[0] - pp[0], qq[1] - pp[1], qq[2] - pp[2]};
@@ -480,126 +548,158 @@ __device__ float cert_gilbert(const float* const* P, const int* nP, int nsP, con
 }
 // Per-time world bound: min over the two instants of the separation along one
 // axis, the axis taken from each instant's own Gilbert iteration.
-__device__ float cert_gap_timed(const float* P0, const float* P1, int nP, const float* Q0, const float* Q1, int nQ,
-                                const float* x0, const float* x1, int iters, float* red) {
-  const float* Ps[2] = {P0, P1};
-  const float* Qs[2] = {Q0, Q1};
+template <class Set>
+__device__ __forceinline__ float cert_gap_timed(const Set& P0, const Set& P1, const Set& Q0, const Set& Q1, const float* x0,
+                                                const float* x1, int iters, float* red) {
   float ax[3][3];
-  for (int k = 0; k < 2; ++k) (void)cert_gilbert(Ps + k, &nP, 1, Qs + k, &nQ, 1, k ? x1 : x0, iters, ax[k], red);
+  (void)cert_gilbert<false>(P0, P0, Q0, x0, iters, ax[0], red);
+  (void)cert_gilbert<false>(P1, P1, Q1, x1, iters, ax[1], red);
   const float n0 = sqrtf((ax[0][0] * ax[0][0] + ax[0][1] * ax[0][1]) + ax[0][2] * ax[0][2]);
   const float n1 = sqrtf((ax[1][0] * ax[1][0] + ax[1][1] * ax[1][1]) + ax[1][2] * ax[1][2]);
+#pragma unroll
   for (int r = 0; r < 3; ++r) ax[2][r] = (n0 > 0.f ? ax[0][r] / n0 : 0.f) + (n1 > 0.f ? ax[1][r] / n1 : 0.f);
   float best = -3.4e38f;
+#pragma unroll
   for (int c = 0; c < 3; ++c) {
     float pp[3], qq[3];
-    const float g0 = cert_axis(Ps, &nP, 1, Qs, &nQ, 1, ax[c], pp, qq, red);
-    const float g1 = cert_axis(Ps + 1, &nP, 1, Qs + 1, &nQ, 1, ax[c], pp, qq, red);
+    const float g0 = cert_axis<false>(P0, P0, Q0, ax[c], pp, qq, red);
+    const float g1 = cert_axis<false>(P1, P1, Q1, ax[c], pp, qq, red);
     best = fmaxf(best, fminf(g0, g1));
   }
   return best;
 }
 constexpr int CERT_ITERS = 16;
-constexpr int CERT_LIST = 1024;  // pairs per block at most (the grid is sized for it)
+constexpr int CERT_LIST = 1024;  // pairs per block at most (the grids are sized for it)
+// Whether a pair's bodies (hull vertices va, vb) are provably apart by more
+// than thr: CCD (mode 0) or at the future poses (mode 1).  S: the sets' storage.
+template <class Set>
+__device__ __forceinline__ bool cert_pair(int mode, const double* pr, const float* va, int na, const float* vb, int nb,
+                                          float thr, Set (&S)[4], float* red, float* mag_red) {
+  const float EPSF = 5.9604645e-08f;
+  float m0[12], m1[12], m2[12], m3[12], u[3], ax[3];
+  float mag = 0.f;
+  if (mode != 0) {
+    const double o[3] = {pr[PR_TB1 + 3], pr[PR_TB1 + 7], pr[PR_TB1 + 11]};
+    cert_mat(pr + PR_TA1, o, m0), cert_mat(pr + PR_TB1, o, m1);
+    cert_load(va, na, m0, S[0], mag), cert_load(vb, nb, m1, S[1], mag);
+    const float M = cert_mag(S[0], mag, mag_red);
+    for (int k = 0; k < 3; ++k) u[k] = m1[4 * k + 3] - m0[4 * k + 3];
+    const float margin = 1e-6f + 64.f * EPSF * M;
+    return cert_gilbert<false>(S[0], S[0], S[1], u, CERT_ITERS, ax, red, thr + margin) - margin > thr;
+  }
+  const double o[3] = {pr[PR_TB0 + 3], pr[PR_TB0 + 7], pr[PR_TB0 + 11]};
+  cert_mat(pr + PR_TA0, o, m0), cert_mat(pr + PR_TA1, o, m1), cert_mat(pr + PR_TB0, o, m2), cert_mat(pr + PR_TB1, o, m3);
+  cert_load(va, na, m0, S[0], mag), cert_load(va, na, m1, S[1], mag);
+  cert_load(vb, nb, m2, S[2], mag), cert_load(vb, nb, m3, S[3], mag);
+  const float M = cert_mag(S[0], mag, mag_red);
+  {  // world, per instant: (a at start, b at start), (a at end, b at end)
+    float x0[3], x1[3];
+    for (int k = 0; k < 3; ++k) x0[k] = m2[4 * k + 3] - m0[4 * k + 3], x1[k] = m3[4 * k + 3] - m1[4 * k + 3];
+    if (!(cert_gap_timed(S[0], S[1], S[2], S[3], x0, x1, CERT_ITERS, red) - (1e-6f + 64.f * EPSF * M) > thr)) return false;
+  }
+#pragma unroll 1
+  for (int f = 0; f < 2; ++f) {  // a's two poses in b's frame against b, then the other way round
+    cert_reuse(S[0]);
+    mag = 0.f;
+    cert_mat(pr + (f ? PR_MBA0 : PR_MAB0), nullptr, m0), cert_mat(pr + (f ? PR_MBA1 : PR_MAB1), nullptr, m1);
+    const float* v = f ? vb : va;
+    const int n = f ? nb : na;
+    cert_load(v, n, m0, S[0], mag), cert_load(v, n, m1, S[1], mag);
+    cert_load(f ? va : vb, f ? na : nb, nullptr, S[2], mag);
+    const float M2 = cert_mag(S[0], mag, mag_red);
+    for (int k = 0; k < 3; ++k) u[k] = -0.5f * (m0[4 * k + 3] + m1[4 * k + 3]);
+    if (!(cert_gilbert<true>(S[0], S[1], S[2], u, CERT_ITERS, ax, red) - (1e-6f + 64.f * EPSF * M2) > thr)) return false;
+  }
+  return true;
+}
+struct CertIn {
+  int n_pairs;
+  const int32_t *pair_info, *body_tree;
+  const double* pair_rec;
+  const float* Y;
+  float t_gate, s_gate;
+  const int32_t* hv_off;
+  const float *hv, *tree_eps_out;
+  int mode;
+};
+// A pair's part in the certificate: 0 not proposed, or proposed with hulls
+// beyond CERT_MAXV (kept); 1 a wavefront's, 2 a block's.
+__device__ __forceinline__ int cert_kind(const CertIn& C, int p, bool& gated, int& ta, int& tb, int& na, int& nb) {
+  gated = !C.Y || (C.Y[2 * p] >= C.s_gate && C.Y[2 * p + 1] >= C.t_gate);
+  ta = C.body_tree[C.pair_info[4 * p]], tb = C.body_tree[C.pair_info[4 * p + 1]];
+  na = C.hv_off[ta + 1] - C.hv_off[ta], nb = C.hv_off[tb + 1] - C.hv_off[tb];
+  const int m = na > nb ? na : nb;
+  return !gated || m > CERT_MAXV ? 0 : m > CERT_WAVEV ? 2 : 1;
+}
 
 // gate: the MLP outputs (y0 >= s_gate and y1 >= t_gate), or every pair when
 // null.  keep[p] = 0 for a certified pair, 1 otherwise.  counters[0..1]:
 // proposed / certified pairs.  The kept pairs are the phase's roots: each
 // block appends its kept pairs to soup with one atomic on *n_soup (zeroed by
 // the phase's set-up; the discrete and CCD lists need no order).
-__global__ void __launch_bounds__(256) k_certify(int n_pairs, const int32_t* pair_info, const int32_t* body_tree,
-                                                 const double* pair_rec, const float* Y, float t_gate, float s_gate,
-                                                 const int32_t* hv_off, const float* hv, const float* tree_eps_out,
-                                                 int mode, int* keep, unsigned long long* counters, NP* soup,
+//
+// A wavefront per pair while both hulls have at most 256 vertices: they sit in
+// its registers, and a support point is a few products and one reduction.  A
+// block per pair met two barriers for each of the ~100 support points of a CCD
+// certificate (1,773 pairs, 548 of them proposed: 183 -> 78 us); k_certify_block still takes the larger hulls.
+__global__ void __launch_bounds__(256) k_certify(CertIn C, int* keep, unsigned long long* counters, NP* soup,
                                                  unsigned long long* n_soup) {
+  __shared__ int s_kept[CERT_LIST];
+  __shared__ int s_nk, s_cnt[2];
+  __shared__ unsigned long long s_base;
+  if (threadIdx.x == 0) s_nk = 0, s_cnt[0] = 0, s_cnt[1] = 0;
+  __syncthreads();
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  for (int p = 4 * (int)blockIdx.x + wv; p < C.n_pairs; p += 4 * (int)gridDim.x) {
+    bool gated;
+    int ta, tb, na, nb;
+    const int kind = cert_kind(C, p, gated, ta, tb, na, nb);
+    if (kind == 2) continue;
+    bool ok = false;
+    if (kind == 1) {
+      CertWave S[4];
+      ok = cert_pair(C.mode, C.pair_rec + (size_t)PR_STRIDE * p, C.hv + 3 * (size_t)C.hv_off[ta], na,
+                     C.hv + 3 * (size_t)C.hv_off[tb], nb,
+                     (float)C.pair_rec[(size_t)PR_STRIDE * p + PR_SEARCH] + C.tree_eps_out[ta] + C.tree_eps_out[tb], S,
+                     nullptr, nullptr);
+    }
+    if (lane_id() == 0) {
+      keep[p] = ok ? 0 : 1;
+      if (!ok) s_kept[atomicAdd(&s_nk, 1)] = p;
+      if (gated) atomicAdd(&s_cnt[0], 1);
+      if (ok) atomicAdd(&s_cnt[1], 1);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s_base = s_nk ? atomicAdd(n_soup, (unsigned long long)s_nk) : 0ull;
+    if (s_cnt[0]) atomicAdd(&counters[0], (unsigned long long)s_cnt[0]);
+    if (s_cnt[1]) atomicAdd(&counters[1], (unsigned long long)s_cnt[1]);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < s_nk; i += blockDim.x)
+    soup[s_base + i] = NP{(uint32_t)s_kept[i], 0u, 0u, 0u, 0ull};
+}
+// The pairs k_certify leaves: a hull of more than 256 vertices (a block each).
+__global__ void __launch_bounds__(256) k_certify_block(CertIn C, int* keep, unsigned long long* counters, NP* soup,
+                                                       unsigned long long* n_soup) {
   __shared__ float buf[4][3 * CERT_MAXV];
   __shared__ float red[4 * 16];
   __shared__ float mag_red[16];
   __shared__ int s_kept[CERT_LIST];
   __shared__ int s_nk;
   __shared__ unsigned long long s_base;
-  const float EPSF = 5.9604645e-08f;
   if (threadIdx.x == 0) s_nk = 0;
-  for (int p = blockIdx.x; p < n_pairs; p += gridDim.x) {
-    const bool gated = !Y || (Y[2 * p] >= s_gate && Y[2 * p + 1] >= t_gate);
-    const int a = pair_info[4 * p], b = pair_info[4 * p + 1];
-    const int ta = body_tree[a], tb = body_tree[b];
-    const int na = hv_off[ta + 1] - hv_off[ta], nb = hv_off[tb + 1] - hv_off[tb];
-    if (!gated || na > CERT_MAXV || nb > CERT_MAXV) {
-      if (threadIdx.x == 0) {
-        keep[p] = 1;
-        s_kept[s_nk++] = p;
-        if (gated) atomicAdd(&counters[0], 1ull);
-      }
-      continue;
-    }
-    const double* pr = pair_rec + (size_t)PR_STRIDE * p;
-    const float thr = (float)pr[PR_SEARCH] + tree_eps_out[ta] + tree_eps_out[tb];
-    const float* va = hv + 3 * (size_t)hv_off[ta];
-    const float* vb = hv + 3 * (size_t)hv_off[tb];
-    float m0[12], m1[12], m2[12], m3[12], u[3];
-    float mag = 0.f;
-    bool ok = true;
-    auto finish_mag = [&]() {  // block maximum of the coordinate magnitudes
-      float m = mag;
-      for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-      __syncthreads();
-      if ((threadIdx.x & 63) == 0) mag_red[threadIdx.x >> 6] = m;
-      __syncthreads();
-      float r = 0.f;
-      for (int i = 0; i < (int)(blockDim.x >> 6); ++i) r = fmaxf(r, mag_red[i]);
-      return r;
-    };
-    if (mode == 0) {
-      const double o[3] = {pr[PR_TB0 + 3], pr[PR_TB0 + 7], pr[PR_TB0 + 11]};
-      cert_mat(pr + PR_TA0, o, m0), cert_mat(pr + PR_TA1, o, m1), cert_mat(pr + PR_TB0, o, m2), cert_mat(pr + PR_TB1, o, m3);
-      cert_load(va, na, m0, buf[0], mag), cert_load(va, na, m1, buf[1], mag);
-      cert_load(vb, nb, m2, buf[2], mag), cert_load(vb, nb, m3, buf[3], mag);
-      const float M = finish_mag();
-      {  // world, per instant: (a at start, b at start), (a at end, b at end)
-        float x0[3], x1[3];
-        for (int k = 0; k < 3; ++k) x0[k] = m2[4 * k + 3] - m0[4 * k + 3], x1[k] = m3[4 * k + 3] - m1[4 * k + 3];
-        ok = cert_gap_timed(buf[0], buf[1], na, buf[2], buf[3], nb, x0, x1, CERT_ITERS, red) -
-                 (1e-6f + 64.f * EPSF * M) > thr;
-      }
-      if (ok) {  // a's two poses in b's frame against b
-        __syncthreads();
-        mag = 0.f;
-        cert_mat(pr + PR_MAB0, nullptr, m0), cert_mat(pr + PR_MAB1, nullptr, m1);
-        cert_load(va, na, m0, buf[0], mag), cert_load(va, na, m1, buf[1], mag), cert_load(vb, nb, nullptr, buf[2], mag);
-        const float M2 = finish_mag();
-        for (int k = 0; k < 3; ++k) u[k] = -0.5f * (m0[4 * k + 3] + m1[4 * k + 3]);
-        const float* P[2] = {buf[0], buf[1]};
-        const float* Q[1] = {buf[2]};
-        const int nP[2] = {na, na}, nQ[1] = {nb};
-        float ax[3];
-        ok = cert_gilbert(P, nP, 2, Q, nQ, 1, u, CERT_ITERS, ax, red) - (1e-6f + 64.f * EPSF * M2) > thr;
-      }
-      if (ok) {  // b's two poses in a's frame against a
-        __syncthreads();
-        mag = 0.f;
-        cert_mat(pr + PR_MBA0, nullptr, m0), cert_mat(pr + PR_MBA1, nullptr, m1);
-        cert_load(vb, nb, m0, buf[0], mag), cert_load(vb, nb, m1, buf[1], mag), cert_load(va, na, nullptr, buf[2], mag);
-        const float M3 = finish_mag();
-        for (int k = 0; k < 3; ++k) u[k] = -0.5f * (m0[4 * k + 3] + m1[4 * k + 3]);
-        const float* P[2] = {buf[0], buf[1]};
-        const float* Q[1] = {buf[2]};
-        const int nP[2] = {nb, nb}, nQ[1] = {na};
-        float ax[3];
-        ok = cert_gilbert(P, nP, 2, Q, nQ, 1, u, CERT_ITERS, ax, red) - (1e-6f + 64.f * EPSF * M3) > thr;
-      }
-    } else {
-      const double o[3] = {pr[PR_TB1 + 3], pr[PR_TB1 + 7], pr[PR_TB1 + 11]};
-      cert_mat(pr + PR_TA1, o, m0), cert_mat(pr + PR_TB1, o, m1);
-      cert_load(va, na, m0, buf[0], mag), cert_load(vb, nb, m1, buf[1], mag);
-      const float M = finish_mag();
-      for (int k = 0; k < 3; ++k) u[k] = m1[4 * k + 3] - m0[4 * k + 3];
-      const float* P[1] = {buf[0]};
-      const float* Q[1] = {buf[1]};
-      const int nP[1] = {na}, nQ[1] = {nb};
-      float ax[3];
-      const float margin = 1e-6f + 64.f * EPSF * M;
-      ok = cert_gilbert(P, nP, 1, Q, nQ, 1, u, CERT_ITERS, ax, red, thr + margin) - margin > thr;
-    }
+  for (int p = blockIdx.x; p < C.n_pairs; p += gridDim.x) {
+    bool gated;
+    int ta, tb, na, nb;
+    if (cert_kind(C, p, gated, ta, tb, na, nb) != 2) continue;
+    CertBlock S[4] = {{buf[0], 0}, {buf[1], 0}, {buf[2], 0}, {buf[3], 0}};
+    const bool ok = cert_pair(C.mode, C.pair_rec + (size_t)PR_STRIDE * p, C.hv + 3 * (size_t)C.hv_off[ta], na,
+                              C.hv + 3 * (size_t)C.hv_off[tb], nb,
+                              (float)C.pair_rec[(size_t)PR_STRIDE * p + PR_SEARCH] + C.tree_eps_out[ta] +
+                                  C.tree_eps_out[tb],
+                              S, red, mag_red);
     if (threadIdx.x == 0) {
       keep[p] = ok ? 0 : 1;
       if (!ok) s_kept[s_nk++] = p;

@@ -837,8 +837,28 @@ __device__ __forceinline__ void leaf_cull_part(Dev& D, CullShare& S, unsigned ch
     // s / n and s / m of sub-test numbers below 576 by multiplication: exact,
     // the error s (65536 / d rounded up - 65536 / d) stays below 576 * 8 / 65536
     const int inv_n = nm ? (65536 + l_n - 1) / l_n : 0, inv_m = nm ? (65536 + l_m - 1) / l_m : 0;
+    if (!D.fp32) {  // every sub-test: the batch's places are known at once, one atomic per list
+      const int incl = wave_incl_scan(nm), first = incl - nm, all = rl(incl, 63);
+      unsigned long long base = 0;
+      if (all && lane < 2) {
+        base = atomicAdd(&D.lvl[D.level * LV_STRIDE + (lane ? LV_EE : LV_PT)], (unsigned long long)((lane ? 9 : 6) * all));
+        if ((long long)(base + (lane ? 9 : 6) * all) > D.cap_items) atomicOr(&D.cnt[C_OVERFLOW], 1ull);
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int k = e ? 9 : 6;
+        const long long b = (long long)readlane_u64(base, e);
+        for (int q0 = 0; q0 < k * all; q0 += 64) {
+          const int src = run_owner(own, k * first - q0, k * nm);
+          const int sub = q0 + lane - k * __shfl(first, src);
+          if (q0 + lane < k * all && b + q0 + lane < D.cap_items)
+            (e ? D.lee_items : D.lpt_items)[b + q0 + lane] = Item{(uint32_t)(w0 + src), (uint32_t)sub};
+        }
+      }
+      continue;
+    }
     for (Groups g(nm > 0 ? 3 * (l_n + l_m) : 0, nm); g.next(false);) {
-      if (D.fp32) {
+      {
         const int src = run_owner(own, g.ts, g.in ? g.slots : 0);
         const int x = lane - __shfl(g.ts, src);
         const int na = __shfl(l_n, src), ta = __shfl(l_ta, src), tb = __shfl(l_tb, src), pair = __shfl(l_pair, src);
@@ -878,7 +898,7 @@ __device__ __forceinline__ void leaf_cull_part(Dev& D, CullShare& S, unsigned ch
         const int src = run_owner(own, 6 * g.js - q0, g.in ? 6 * g.jobs : 0);
         const int sub = q0 + lane - 6 * __shfl(g.js, src);
         bool keep = q0 + lane < 6 * g.n_jobs;
-        if (D.fp32) {
+        {
           const int na = __shfl(l_n, src), nb = __shfl(l_m, src), vs = __shfl(g.ts, src);
           const int in_ = __shfl(inv_n, src), im = __shfl(inv_m, src);
           const float thr = __shfl(l_thr, src);
@@ -904,7 +924,7 @@ __device__ __forceinline__ void leaf_cull_part(Dev& D, CullShare& S, unsigned ch
         const int src = run_owner(own, 9 * g.js - q0, g.in ? 9 * g.jobs : 0);
         const int sub = q0 + lane - 9 * __shfl(g.js, src);
         bool keep = q0 + lane < 9 * g.n_jobs;
-        if (D.fp32) {
+        {
           const int na = __shfl(l_n, src), nb = __shfl(l_m, src), vs = __shfl(g.ts, src), im = __shfl(inv_m, src);
           const float thr = __shfl(l_thr, src);
           if (keep) {
@@ -1981,37 +2001,42 @@ __global__ void __launch_bounds__(256) k_tri_full(Dev D) {
 // Eight lanes per node pair, one per child: each tests its own child's bounds
 // and writes it (18.1 us a launch when one lane walked a node pair's children,
 // 8.7 us now, on levels of up to 20 000 node pairs).
+// Large levels take up to 8 rounds of 32 node pairs per atomic and barrier.
 __global__ void __launch_bounds__(256) k_disc_expand(Dev D) {
   __shared__ int s_tot[4];
   __shared__ unsigned long long s_base;
   const long long n = D.n_soup();
   const int lane = lane_id(), wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int c = lane & 7;
-  const long long stride = (long long)gridDim.x * (blockDim.x >> 3);
-  for (long long b0 = (long long)blockIdx.x * (blockDim.x >> 3); b0 < n; b0 += stride) {  // block-uniform
-    const long long w = b0 + (threadIdx.x >> 3);
-    NP child{};
-    bool keep = false;
-    if (w < n && D.np_hit[w]) {
-      const int desc = D.exp_desc[w];
-      const NP np = D.soup[w];
-      if (c < ((desc >> 1) & 15)) {
-        const bool adv_a = desc & 1;
-        const uint32_t id = (uint32_t)((desc >> 5) + c);
-        child = NP{np.pair, adv_a ? id : np.na, adv_a ? np.nb : id, 0u, np.key * 8ull + (unsigned long long)c};
-        keep = true;
-        if (D.prune) {
-          const int32_t* pi = D.pair_info + 4 * np.pair;
-          const double* pr = D.pair_rec + (size_t)PR_STRIDE * np.pair;
+  constexpr int K = 8;
+  const long long turn = (long long)gridDim.x * 32;  // node pairs of one round of all blocks
+  const int rounds = n >= K * turn ? K : (int)((n + turn - 1) / turn);
+  for (long long b0 = (long long)blockIdx.x * 32 * rounds; b0 < n; b0 += turn * rounds) {  // block-uniform
+    unsigned long long m[K];
+    int cnt = 0;
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+      m[r] = 0ull;
+      if (r >= rounds) continue;
+      const long long w = b0 + 32 * r + (threadIdx.x >> 3);
+      bool keep = false;
+      if (w < n && D.np_hit[w]) {
+        const int desc = D.exp_desc[w];
+        keep = c < ((desc >> 1) & 15);
+        if (keep && D.prune) {
+          const NP child = child_of(D.soup[w], desc, c, 0u);
+          const int32_t* pi = D.pair_info + 4 * child.pair;
+          const double* pr = D.pair_rec + (size_t)PR_STRIDE * child.pair;
           const float* ba = D.nbound + NB_STRIDE * ((size_t)pi[2] + child.na);
           const float* bb = D.nbound + NB_STRIDE * ((size_t)pi[3] + child.nb);
           keep = !(spheres_apart(pr + PR_TA1, pr + PR_TB1, ba, bb, pr[PR_SEARCH]) ||
                    nodes_apart(pr + PR_TA1, pr + PR_TB1, ba, bb, pr[PR_SEARCH]));
         }
       }
+      m[r] = __ballot(keep);
+      cnt += __popcll(m[r]);
     }
-    const unsigned long long m = __ballot(keep);
-    if (lane == 0) s_tot[wid] = __popcll(m);
+    if (lane == 0) s_tot[wid] = cnt;
     __syncthreads();
     if (threadIdx.x == 0) {
       int tot = 0;
@@ -2024,10 +2049,18 @@ __global__ void __launch_bounds__(256) k_disc_expand(Dev D) {
       s_base = base;
     }
     __syncthreads();
-    long long slot = (long long)s_base + __popcll(m & lanes_below());
+    long long slot = (long long)s_base;
     for (int v = 0; v < wid; ++v) slot += s_tot[v];
-    if (keep && slot < D.cap_np) D.soup_next[slot] = child;
-    __syncthreads();  // s_tot and s_base are rewritten by the next round
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+      const long long at = slot + __popcll(m[r] & lanes_below());
+      if ((m[r] >> lane) & 1ull && at < D.cap_np) {
+        const long long w = b0 + 32 * r + (threadIdx.x >> 3);
+        D.soup_next[at] = child_of(D.soup[w], D.exp_desc[w], c, 0u);
+      }
+      slot += __popcll(m[r]);
+    }
+    __syncthreads();  // s_tot and s_base are rewritten by the next tile
   }
 }
 

@@ -2001,7 +2001,8 @@ __global__ void __launch_bounds__(256) k_tri_full(Dev D) {
 // Eight lanes per node pair, one per child: each tests its own child's bounds
 // and writes it (18.1 us a launch when one lane walked a node pair's children,
 // 8.7 us now, on levels of up to 20 000 node pairs).
-// Large levels take up to 8 rounds of 32 node pairs per atomic and barrier.
+// Large levels take up to 8 rounds of 32 node pairs per atomic and barrier (a
+// step of 48 scenes without pruning: 2.85 -> 0.63 ms).
 __global__ void __launch_bounds__(256) k_disc_expand(Dev D) {
   __shared__ int s_tot[4];
   __shared__ unsigned long long s_base;

@@ -3945,9 +3945,10 @@ struct Sig {
   int learned = -1;
   float gate_t = 0.f, gate_s = 0.f;
   int cl_dev = -1;  // clusters built on the device (first members known)
+  int big_hulls = -1;  // the gate's certificate has its second launch (k_certify_block)
   unsigned long long grids = 0;  // hash of the per-level launch grids
   bool operator==(const Sig& o) const {
-    return grids == o.grids && cl_dev == o.cl_dev && levels[0] == o.levels[0] && levels[1] == o.levels[1] && learned == o.learned && gate_t == o.gate_t &&
+    return grids == o.grids && cl_dev == o.cl_dev && big_hulls == o.big_hulls && levels[0] == o.levels[0] && levels[1] == o.levels[1] && learned == o.learned && gate_t == o.gate_t &&
            gate_s == o.gate_s && n_pairs == o.n_pairs && n_bodies == o.n_bodies && n_clusters == o.n_clusters && max_depth == o.max_depth &&
            precision == o.precision && filter == o.filter && dt == o.dt &&
            tune.chunk_blocks == o.tune.chunk_blocks && tune.stream_blocks == o.tune.stream_blocks &&
@@ -4800,6 +4801,7 @@ int run_graph(d2_ctx* c, int kind, int filter, float dt) {
   sig.tune = c->tune;
   sig.learned = (c->learned_on && c->mlp_ready) ? c->gate_phases : 0, sig.gate_t = c->gate_t, sig.gate_s = c->gate_s;
   sig.cl_dev = kind == RUN_STEP && c->clusters_on_device ? 1 : 0;
+  sig.big_hulls = sig.learned && c->big_hulls ? 1 : 0;
   for (int i = 0; i < n; ++i) sig.levels[i] = std::min(c->phase_levels[ph[i].slot], budget);
   for (int i = 0; i < n; ++i)
     sig.grids = (sig.grids * 31 + grids_hash(c, ph[i].discrete, sig.levels[i])) * 31 + post_grid(c, ph[i].post_mode);

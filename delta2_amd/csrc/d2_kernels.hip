@@ -2580,7 +2580,9 @@ __device__ __forceinline__ unsigned long long greedy_keep(int m, const unsigned 
 // 16 u cmax + 1e-6 search away from the search distance is decided, and only
 // the others run the FP64 test (25 FP64 instructions per test were most of
 // the greedy pass).  Distances that FP32 cannot hold, and negative or infinite
-// search distances, always run it.
+// search distances, always run it, and so do search distances of at most
+// 1e-15 m (0 aside, which nothing is nearer than): their squares go under
+// FP32's normal numbers from 1e-19 m on.
 struct NearTest {
   double mx, my, mz, search;
   float fx, fy, fz, lo2, hi2;
@@ -2592,7 +2594,7 @@ __device__ __forceinline__ NearTest near_test(double mx, double my, double mz, d
   const float s = (float)search, err = 16.f * 5.9604645e-08f * cmax + 1e-6f * s;
   const float lo = s - err, hi = s + err;
   t.lo2 = lo > 0.f ? lo * lo * (1.f - 1e-6f) : -1.f, t.hi2 = hi * hi * (1.f + 1e-6f);
-  t.exact = __ballot(!(search >= 0.0 && search < 1e15 && cmax < 1e15f)) != 0ull;
+  t.exact = __ballot(!((search == 0.0 || search > 1e-15) && search < 1e15 && cmax < 1e15f)) != 0ull;
   return t;
 }
 __device__ __forceinline__ float rlf(float v, int l) { return __int_as_float(rl(__float_as_int(v), l)); }

@@ -545,7 +545,9 @@ __global__ void __launch_bounds__(256) k_bp_gather(int n_items, const int* item_
 // stale parent is still an ancestor, and whether a root found this way is one
 // still is decided by the CAS that hooks it.  Loads at device scope, all
 // ending on the largest component's root, queued on one line: 260 us of
-// unions for 120 k pairs of 65 536 bodies against 102 us.
+// unions for 120 k pairs of 65 536 bodies against 102 us.  The halved paths
+// are stored at device scope, as the CAS is: words that other wavefronts,
+// behind other L2 caches, read and hook.
 __device__ __forceinline__ int cc_load(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
@@ -553,7 +555,7 @@ __device__ __forceinline__ int cc_find(int* parent, int x) {
   int p = cc_load(&parent[x]);
   while (p != x) {
     const int g = cc_load(&parent[p]);
-    if (g != p) __hip_atomic_store(&parent[x], g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    if (g != p) __hip_atomic_store(&parent[x], g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     x = p, p = g;
   }
   return x;

@@ -18,7 +18,9 @@
 // is always the smallest index of its tree), clusters numbered by their
 // smallest member, roll-back of the members to the cluster's earliest time.
 
-constexpr int BP_SEG = 512;  // bodies one item of a static body sweeps (4096 left 48 wavefronts to finish 100 us after the rest)
+// Bodies one item of a static body sweeps: the least of BP_SEG_MIN, twice that,
+// ... BP_SEG_MAX that leaves at most BP_SEG_ITEMS items (bp_segment).
+constexpr int BP_SEG_MIN = 512, BP_SEG_MAX = 4096, BP_SEG_ITEMS = 1 << 15;
 constexpr int BP_WAVE_CAP = 512;  // partners a wave sorts in LDS
 enum BpRed : int {  // reductions over the non-static bodies' boxes
   BR_EXT = 0,       // largest box extent (float bits, non-negative)
@@ -293,7 +295,7 @@ __device__ __forceinline__ bool bp_collide(int a, int b, int mode, double t, con
   return s >= 0.0 && s < window;
 }
 
-// Items: one per non-static body, ceil((n - 1 - a) / BP_SEG) (at least one)
+// Items: one per non-static body, ceil((n - 1 - a) / seg) (at least one)
 // per static body a, in body order; item_body / item_seg describe them.
 // Each item's wave writes its partners to a chunk of `chunk` allocated with
 // one atomic and records the chunk position, the count and whether the chunk
@@ -331,7 +333,7 @@ __device__ __forceinline__ void lds_rank_sort(int* buf, int cnt) {
 }
 
 struct BpIn {
-  int n, mode;
+  int n, mode, seg;
   double t;
   const double* bodies;
   const double* last;
@@ -390,8 +392,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))
       long long lo = 0;
       int total = 0, n_cand;
       if (sweep) {
-        lo = (long long)a + 1 + (long long)item_seg[it] * BP_SEG;
-        const long long hi = lo + BP_SEG < in.n ? lo + BP_SEG : in.n;
+        lo = (long long)a + 1 + (long long)item_seg[it] * in.seg;
+        const long long hi = lo + in.seg < in.n ? lo + in.seg : in.n;
         n_cand = hi > lo ? (int)(hi - lo) : 0;
       } else {
         long long c0[3];

@@ -4048,7 +4048,7 @@ struct d2_ctx {
   DBuf<int32_t> tree_depth_d, group;
   bool has_groups = false;
   std::vector<int> host_static;
-  int n_items = 0;
+  int n_items = 0, bp_seg = BP_SEG_MIN;
   DBuf<int> bp_statics, bp_item_body, bp_item_seg, bp_item_cnt, bp_item_sorted, bp_item_off, bp_meta, bp_slot,
       bp_rank, bp_counts, bp_start, bp_red;
   DBuf<long long> bp_item_pos;
@@ -4174,6 +4174,22 @@ template <class T> void release(DBuf<T>& b) {
   if (b.p) (void)hipFree(b.p);
   b.p = nullptr;
   b.n = 0;
+}
+
+// The segment length of the static bodies' sweeps.  Few statics need short
+// segments to fill the chip (3 among 65,536 bodies: 290 us a broad phase with
+// 512 bodies a segment, 298 with 4096, 509 with 32768); with many the items
+// themselves cost, on the host at each upload and in the kernels' per-item
+// arrays (30,000 among 65,536: 4.1 ms of upload and 7.8 ms of broad phase
+// with 512, 2.1 and 5.9 ms with 4096).
+int bp_segment(const std::vector<int>& statics, int n_bodies) {
+  int seg = BP_SEG_MIN;
+  for (; seg < BP_SEG_MAX; seg *= 2) {
+    long long items = 0;
+    for (int a : statics) items += (n_bodies - 1 - a + seg - 1) / seg;
+    if (items <= BP_SEG_ITEMS) break;
+  }
+  return seg;
 }
 
 int grid_for(d2_ctx* c, long long threads, int block = 256) {
@@ -5637,14 +5653,16 @@ int d2_bodies_upload(d2_ctx* c, int n_bodies, const int32_t* tree_of_body, const
   for (int i = 0; i < n_bodies; ++i) std::memcpy(&last[14 * (size_t)i], records + 40 * (size_t)i, 14 * sizeof(double));
   RC(ensure(c, c->last_state, 14 * (size_t)n_bodies));
   HIPCHK(c, hipMemcpyAsync(c->last_state.p, last.data(), sizeof(double) * last.size(), hipMemcpyHostToDevice, c->stream));
-  // broad-phase work items: one per non-static body, one per BP_SEG later
+  // broad-phase work items: one per non-static body, one per bp_seg later
   // bodies for a static one (it sweeps all of them)
   c->host_static.clear();
+  for (int i = 0; i < n_bodies; ++i)
+    if (records[40 * (size_t)i + 38] != 0.0) c->host_static.push_back(i);
+  const int seg = c->bp_seg = bp_segment(c->host_static, n_bodies);
   std::vector<int> ib, is;
   for (int i = 0; i < n_bodies; ++i) {
     if (records[40 * (size_t)i + 38] != 0.0) {
-      c->host_static.push_back(i);
-      const int segs = std::max(1, (n_bodies - 1 - i + BP_SEG - 1) / BP_SEG);
+      const int segs = std::max(1, (n_bodies - 1 - i + seg - 1) / seg);
       for (int q = 0; q < segs; ++q) ib.push_back(i), is.push_back(q);
     } else {
       ib.push_back(i), is.push_back(0);
@@ -6119,7 +6137,7 @@ int d2_broad_phase(d2_ctx* c, int mode, double t, int64_t* n_pairs_out) {
     hipLaunchKernelGGL(k_bp_scatter, dim3(g), dim3(256), 0, c->stream, n, c->bp_box.p, c->bp_meta.p, c->bp_slot.p,
                        c->bp_rank.p, c->bp_start.p, c->bp_members.p);
     BpIn in;
-    in.n = n, in.mode = mode, in.t = t, in.bodies = c->bodies.p, in.last = c->last_state.p, in.box = c->bp_box.p;
+    in.n = n, in.mode = mode, in.seg = c->bp_seg, in.t = t, in.bodies = c->bodies.p, in.last = c->last_state.p, in.box = c->bp_box.p;
     in.R = c->bp_R.p, in.meta = c->bp_meta.p, in.statics = c->bp_statics.p, in.n_static = (int)c->host_static.size();
     in.red = c->bp_red.p, in.T = T, in.keys = c->bp_keys.p, in.counts = c->bp_counts.p, in.start = c->bp_start.p;
     in.members = c->bp_members.p;

@@ -541,26 +541,24 @@ __global__ void __launch_bounds__(256) k_bp_gather(int n_items, const int* item_
 }
 
 // ---------------------------------------------------------------- clusters
-// The root of x, halving the path on the way: every visited node is pointed
-// at its grandparent.  The loads may come from the caches (wavefront scope):
-// a node's parent only ever changes to an ancestor with a smaller index, so a
-// stale parent is still an ancestor, and whether a root found this way is one
-// still is decided by the CAS that hooks it.  Loads at device scope, all
-// ending on the largest component's root, queued on one line: 260 us of
-// unions for 120 k pairs of 65 536 bodies against 102 us.  The halved paths
-// are stored at device scope, as the CAS is: words that other wavefronts,
-// behind other L2 caches, read and hook.
+// The root of x; x is then pointed at it.  The loads may come from the caches
+// (wavefront scope): a node's parent only ever changes to an ancestor with a
+// smaller index, so a stale parent is still an ancestor, and whether a root
+// found this way is one still is decided by the CAS that hooks it.  Loads at
+// device scope, all ending on the largest component's root, queued on one
+// line: 260 us of unions for 120 k pairs of 65 536 bodies against 105 us.  The
+// shortened path is stored at device scope, as the CAS is: words that other
+// wavefronts, behind other L2 caches, read and hook.  (Halving the whole path
+// stores more: 116 to 121 us.)
 __device__ __forceinline__ int cc_load(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
-__device__ __forceinline__ int cc_find(int* parent, int x) {
-  int p = cc_load(&parent[x]);
-  while (p != x) {
-    const int g = cc_load(&parent[p]);
-    if (g != p) __hip_atomic_store(&parent[x], g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    x = p, p = g;
-  }
-  return x;
+template <bool SHORTEN = true> __device__ __forceinline__ int cc_find(int* parent, int x) {
+  const int p = cc_load(&parent[x]);
+  int r = p;
+  for (int g; (g = cc_load(&parent[r])) != r;) r = g;
+  if (SHORTEN && r != p) __hip_atomic_store(&parent[x], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return r;
 }
 __global__ void k_cc_init(int n, int* parent) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) parent[i] = i;
@@ -590,7 +588,7 @@ __global__ void k_cc_union(int n_pairs, const int32_t* pairs, const double* bodi
 }
 __global__ void k_cc_roots(int n, const double* bodies, int* parent, int* label, int* is_root) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int r = cc_find(parent, i);
+    const int r = cc_find<false>(parent, i);  // (paths are short by now: 5 us, 14 us with the stores)
     label[i] = r;
     is_root[i] = (r == i && bodies[40 * (size_t)i + 38] == 0.0) ? 1 : 0;
   }

@@ -3341,7 +3341,8 @@ __global__ void k_project(int n, double* bodies, const double* step, int skip_st
 
 // ------------------------------------------- sequential impulses (the solver)
 // After a filtered step: the clusters' pair lists, particles and hit counts,
-// then a block per cluster runs SequentialImpulses::solve (d2_solver.hpp).
+// then a block per cluster, or a lane per cluster where many are small, runs
+// SequentialImpulses::solve (d2_solver.hpp).
 struct SolveArgs {
   int n_pairs, n_clusters, n_bodies;
   const int32_t* pairs;
@@ -3383,9 +3384,10 @@ struct SolveArgs {
   double* hB;   // [hits][3]
   double* heps; // [hits]
   double* hkey; // [hits] |A - B| / (eps_a + eps_b)
-  double* hhot;   // [hits][CH] (clusters above the LDS capacity)
-  double* hcold;  // [hits][CC]
-  double* ps;     // [2 n_pairs][SP] (clusters above the LDS capacity)
+  double* hs;     // [hits][SH]: per cluster its CH records (unless in LDS), then its CC records
+  double* ps;     // [2 n_pairs][SP] (unless in LDS)
+  int* hist;      // [SV_BINS] clusters by size class
+  int small;      // clusters up to this size are k_sv_solve_small's (-1: none)
   double* out;  // [hits][11], cluster-gathered order
   WarmTable warm;
 };
@@ -3453,12 +3455,19 @@ __global__ void k_sv_count(SolveArgs A) {
     }
   }
 }
+// A cluster's size for the choice of its solver: its hits and its pairs.
+constexpr int SV_BINS = 6;  // sizes up to 2, 4, 8, 16, 32, above
+__device__ __forceinline__ int sv_size(const SolveArgs& A, int k) {
+  return (A.ccount[k + 1] - A.ccount[k]) + (A.chits[k + 1] - A.chits[k]);
+}
 // ccount / chits hold the exclusive offsets here (poff / hoff).  The pairs to
 // their clusters, the dynamic bodies to their clusters' particles (which
 // particle is which changes no result).
 __global__ void k_sv_place(SolveArgs A) {
-  const int n = A.n_pairs > A.n_bodies ? A.n_pairs : A.n_bodies;
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
+  int n = A.n_pairs > A.n_bodies ? A.n_pairs : A.n_bodies;
+  n = A.n_clusters > n ? A.n_clusters : n;
+  for (int p0 = blockIdx.x * blockDim.x; p0 < n; p0 += gridDim.x * blockDim.x) {  // block-uniform
+    const int p = p0 + threadIdx.x;
     if (p < A.n_pairs) {
       const int k = A.cluster_of_pair[p];
       A.cpairs[A.ccount[k] + atomicAdd(&A.cfill[k], 1)] = p;
@@ -3468,7 +3477,40 @@ __global__ void k_sv_place(SolveArgs A) {
       A.loc[p] = q;
       A.pbody[2 * (size_t)A.ccount[k] + q] = p;
     }
+    if (p0 >= A.n_clusters) continue;
+    int bin = -1;
+    if (p < A.n_clusters) {
+      const int size = sv_size(A, p);
+      for (bin = 0; bin < SV_BINS - 1 && size > 2 << bin;) ++bin;
+    }
+    for (int b = 0; b < SV_BINS; ++b) {
+      const unsigned long long m = __ballot(bin == b);
+      if (m && lane_id() == 0) atomicAdd(&A.hist[b], __popcll(m));
+    }
   }
+}
+// Hit H (contact position t of the pair with local particles la, lb), as the
+// cluster's solve takes it.
+__device__ __forceinline__ void sv_take_hit(const SolveArgs& A, size_t H, int t, int la, int lb, int row, int cnt) {
+  const ContactRec& c = A.contacts[A.perm[t]];
+  for (int j = 0; j < 3; ++j) A.hA[3 * H + j] = c.r[j], A.hB[3 * H + j] = c.r[3 + j];
+  A.heps[H] = c.r[6] + c.r[7];
+  A.hkey[H] = vlen(sub(v3<double>{c.r[0], c.r[1], c.r[2]}, v3<double>{c.r[3], c.r[4], c.r[5]})) / A.heps[H];
+  A.hl[2 * H] = la, A.hl[2 * H + 1] = lb;
+  A.hrow[H] = row;
+  A.hpc[H] = cnt;
+}
+// Cluster k's solve, once its nh hits from h0 on and np particles are gathered.
+__device__ __forceinline__ ClusterSolve sv_cluster(const SolveArgs& A, int k, int h0, int nh, int p0, int np) {
+  ClusterSolve S;
+  S.nh = nh, S.np = np;
+  S.hA = A.hA + 3 * (size_t)h0, S.hB = A.hB + 3 * (size_t)h0, S.heps = A.heps + h0, S.hl = A.hl + 2 * (size_t)h0;
+  S.hpc = A.hpc + h0;
+  S.ord = A.ord + h0, S.pbody = A.pbody + 2 * (size_t)p0, S.bodies = A.bodies, S.mass = A.mass, S.fric = A.fric;
+  S.t = A.cluster_step[k], S.g = v3<double>{A.gx, A.gy, A.gz}, S.warm = A.warm;
+  S.hs = A.hs + (size_t)SH * h0, S.ps = A.ps + (size_t)SP * 2 * p0;
+  S.out_h = A.out + 11 * (size_t)h0;
+  return S;
 }
 struct KeyLess {
   const double* k;
@@ -3714,6 +3756,7 @@ __global__ void __launch_bounds__(256) k_sv_solve(SolveArgs A) {
   __shared__ int s_np;
   const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
   for (int k = blockIdx.x; k < A.n_clusters; k += gridDim.x) {
+    if (sv_size(A, k) <= A.small) continue;
     const int p0 = A.ccount[k], np_k = A.ccount[k + 1] - p0;
     const int h0 = A.chits[k], nh = A.chits[k + 1] - h0;
     const int* cu = A.cpairs + p0;
@@ -3787,14 +3830,7 @@ __global__ void __launch_bounds__(256) k_sv_solve(SolveArgs A) {
         const unsigned long long m = __ballot(take);
         if (take) {
           const int q = n + __popcll(m & lanes_below());
-          const size_t H = (size_t)h0 + A.phit[p0 + i] + q;
-          const ContactRec& c = A.contacts[A.perm[t]];
-          for (int j = 0; j < 3; ++j) A.hA[3 * H + j] = c.r[j], A.hB[3 * H + j] = c.r[3 + j];
-          A.heps[H] = c.r[6] + c.r[7];
-          A.hkey[H] = vlen(sub(v3<double>{c.r[0], c.r[1], c.r[2]}, v3<double>{c.r[3], c.r[4], c.r[5]})) / A.heps[H];
-          A.hl[2 * H] = la, A.hl[2 * H + 1] = lb;
-          A.hrow[H] = row + q;
-          A.hpc[H] = cnt;
+          sv_take_hit(A, (size_t)h0 + A.phit[p0 + i] + q, t, la, lb, row + q, cnt);
         }
         n += __popcll(m);
       }
@@ -3845,15 +3881,8 @@ __global__ void __launch_bounds__(256) k_sv_solve(SolveArgs A) {
       }
     }
     __syncthreads();
-    ClusterSolve S;
-    S.nh = nh, S.np = np;
-    S.hA = A.hA + 3 * (size_t)h0, S.hB = A.hB + 3 * (size_t)h0, S.heps = A.heps + h0, S.hl = A.hl + 2 * (size_t)h0;
-    S.hpc = A.hpc + h0;
-    S.ord = ord, S.pbody = pb, S.bodies = A.bodies, S.mass = A.mass, S.fric = A.fric;
-    S.t = A.cluster_step[k], S.g = v3<double>{A.gx, A.gy, A.gz}, S.warm = A.warm;
-    S.hs = nullptr, S.ps = nullptr;
-    S.out_h = A.out + 11 * (size_t)h0;
-    double* cold = A.hcold + (size_t)CC * h0;
+    const ClusterSolve S = sv_cluster(A, k, h0, nh, p0, np);
+    double* cold = S.hs + (size_t)CH * nh;
     // during the schedule the particles' ints share C's memory, the level
     // counts P's (both are filled only after it)
     int* ci = reinterpret_cast<int*>(L.C);
@@ -3866,13 +3895,56 @@ __global__ void __launch_bounds__(256) k_sv_solve(SolveArgs A) {
       static_assert(sizeof(L.C) >= 2 * CI * sizeof(int) && sizeof(L.P) >= PI * sizeof(int) &&
                         SV_CAPH * CH >= TILE, "schedule scratch in LDS");
       int* pi = A.pint + 3 * 2 * (size_t)p0 + k;  // [np + 1] csr offsets, [np] levels, [np] cursors
-      ok = sv_solve_block(S, A.hhot + (size_t)CH * h0, cold, A.ps + (size_t)SP * 2 * p0, wi + 4 * (size_t)nh, wi,
+      ok = sv_solve_block(S, S.hs, cold, S.ps, wi + 4 * (size_t)nh, wi,
                           wi + nh, wi + 2 * (size_t)nh, A.lvlo + h0 + k, pi, np <= CI ? ci : pi + np + 1,
                           np <= CI ? ci + CI : pi + 2 * (size_t)np + 1,
                           nh <= PI ? reinterpret_cast<int*>(L.P) : A.cntl + h0, n_dyn, s_misc, false);
     }
     if (tid == 0) A.status[k] = ok ? 1 : 0;
     __syncthreads();  // LDS is reused by the next cluster
+  }
+}
+// The clusters of size A.small at most, one lane each: gathered, sorted and
+// walked contact by contact.
+__global__ void __launch_bounds__(64) k_sv_solve_small(SolveArgs A) {
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < A.n_clusters; k += gridDim.x * blockDim.x) {
+    if (sv_size(A, k) > A.small) continue;
+    const int p0 = A.ccount[k], np_k = A.ccount[k + 1] - p0;
+    const int h0 = A.chits[k], nh = A.chits[k + 1] - h0;
+    int* cp = A.cps + p0;
+    int* pb = A.pbody + 2 * (size_t)p0;
+    const int n_dyn = A.cpart[k];
+    int np = n_dyn, n = 0;
+    for (int i = 0; i < np_k; ++i) {  // the pairs in index order
+      const int x = A.cpairs[p0 + i];
+      int at = i;
+      for (; at > 0 && cp[at - 1] > x; --at) cp[at] = cp[at - 1];
+      cp[at] = x;
+    }
+    for (int i = 0; i < np_k; ++i) {
+      const int p = cp[i];
+      int l[2];
+      for (int e = 0; e < 2; ++e) {  // a static body: one particle per cluster it touches
+        const int b = A.pairs[2 * p + e];
+        if (A.bodies[40 * (size_t)b + 38] == 0.0) {
+          l[e] = A.loc[b];
+        } else {
+          int q = n_dyn;
+          while (q < np && pb[q] != b) ++q;
+          if (q == np) pb[np++] = b;
+          l[e] = q;
+        }
+      }
+      int row = A.out_off[p];
+      for (int t = A.pair_off[p]; t < A.pair_off[p + 1]; ++t) {
+        if (!A.keep[t]) continue;
+        sv_take_hit(A, (size_t)h0 + n, t, l[0], l[1], row++, A.kept_cnt[p]);
+        A.ord[h0 + n] = n;
+        ++n;
+      }
+    }
+    StdSort<KeyLess>{A.ord + h0, KeyLess{A.hkey + h0}}.sort(0, nh);
+    A.status[k] = solve_cluster(sv_cluster(A, k, h0, nh, p0, np)) ? 1 : 0;
   }
 }
 // Bodies in no pair: a cluster of their own without contacts (gravity only).
@@ -4028,7 +4100,7 @@ struct d2_ctx {
   DBuf<double> sv_mass, sv_fric;
   DBuf<int> sv_ccount, sv_chits, sv_poff, sv_hoff, sv_cfill, sv_cpairs, sv_inpair, sv_loc, sv_status, sv_flag;
   DBuf<int> sv_hl, sv_ord, sv_hrow, sv_hpc, sv_pbody, sv_cpart, sv_cps, sv_ploc, sv_phit, sv_hint, sv_lvlo, sv_cntl, sv_pint;
-  DBuf<double> sv_hA, sv_hB, sv_heps, sv_hkey, sv_hhot, sv_hcold, sv_ps, sv_out, sv_out_csr;
+  DBuf<double> sv_hA, sv_hB, sv_heps, sv_hkey, sv_hs, sv_ps, sv_out, sv_out_csr;
   DBuf<unsigned long long> warm_keys, warm_used;
   DBuf<double> warm_vals;
   int last_kind = -1;         // kind of the last finished run
@@ -5094,6 +5166,29 @@ int read_out(d2_ctx* c, std::initializer_list<CopyOut> parts, int max_threads) {
   return e == hipSuccess ? D2_OK : fail(c, D2_ERR_HIP, std::string("reading results: ") + hipGetErrorString(e));
 }
 
+// Which clusters a lane each solves, by size (SV_BINS classes), the others a
+// block each.  A lane takes 1.5 to 6 times as long for a cluster as a block
+// does (below, us for clusters of each class: measured with spheres in single
+// layers and stacks on a floor), but hardly longer for thousands of clusters
+// than for one, while two blocks fit a CU: 10,000 single spheres on a floor
+// take 5.0 ms with a block each and 0.5 ms with a lane each, 8,192 stacks of
+// two 8.5 and 1.8 ms, 512 of them 0.7 and 1.6 ms.
+int sv_small_size(const d2_ctx* c, const int* hist) {
+  constexpr double LANE[SV_BINS - 1] = {350, 1600, 3000, 5000, 17000};
+  constexpr double BLOCK[SV_BINS] = {240, 720, 1100, 1300, 2900, 6000};
+  int best = -1;
+  double best_us = 0.0, lane = 0.0, n_lane = 0.0;
+  for (int b = -1; b < SV_BINS - 1; ++b) {  // classes up to b by lanes
+    if (b >= 0 && hist[b]) lane = LANE[b], n_lane += hist[b];
+    double one = 0.0, all = 0.0;  // the others' longest, and their share of the chip
+    for (int k = b + 1; k < SV_BINS; ++k)
+      if (hist[k]) one = BLOCK[k], all += 0.7 * hist[k] * BLOCK[k] / (2.0 * c->cus);
+    const double us = lane * (1.0 + n_lane / 20000.0) + std::max(one, all);
+    if (b < 0 || us < best_us) best = b < 0 ? -1 : 2 << b, best_us = us;
+  }
+  return best;
+}
+
 // ---- bucket-level entry: scratch and one call
 struct BucketScratch {
   int32_t* np;       // [cap_np][2] staged node pairs
@@ -5284,7 +5379,7 @@ int d2_ctx_destroy(d2_ctx* c) {
       release(c->sv_hoff), release(c->sv_cfill), release(c->sv_cpairs), release(c->sv_inpair), release(c->sv_loc),
       release(c->sv_status), release(c->sv_flag), release(c->sv_hl), release(c->sv_ord), release(c->sv_hrow),
       release(c->sv_hpc), release(c->sv_pbody), release(c->sv_hA), release(c->sv_hB), release(c->sv_heps),
-      release(c->sv_hkey), release(c->sv_hhot), release(c->sv_hcold), release(c->sv_ps), release(c->sv_out),
+      release(c->sv_hkey), release(c->sv_hs), release(c->sv_ps), release(c->sv_out),
       release(c->sv_out_csr), release(c->sv_cpart), release(c->sv_cps), release(c->sv_ploc), release(c->sv_phit),
       release(c->sv_hint), release(c->sv_lvlo), release(c->sv_cntl), release(c->sv_pint),
       release(c->warm_keys), release(c->warm_used), release(c->warm_vals);
@@ -5727,13 +5822,13 @@ int d2_solve(d2_ctx* c, const double* gravity, int32_t* cluster_status, int* n_f
   RC(ensure(c, c->sv_ccount, nk + 1)); RC(ensure(c, c->sv_chits, nk + 1)); RC(ensure(c, c->sv_poff, nk + 1));
   RC(ensure(c, c->sv_hoff, nk + 1)); RC(ensure(c, c->sv_cfill, nk)); RC(ensure(c, c->sv_status, nk));
   RC(ensure(c, c->sv_cpairs, std::max(np, 1))); RC(ensure(c, c->sv_pbody, 2 * (size_t)std::max(np, 1)));
-  RC(ensure(c, c->sv_inpair, nb)); RC(ensure(c, c->sv_loc, nb)); RC(ensure(c, c->sv_flag, 1));
+  RC(ensure(c, c->sv_inpair, nb)); RC(ensure(c, c->sv_loc, nb)); RC(ensure(c, c->sv_flag, 1 + SV_BINS));
   RC(ensure(c, c->out_off, (size_t)np + 1));
   const size_t H = (size_t)std::max<long long>(nh, 1);
   RC(ensure(c, c->sv_hl, 2 * H)); RC(ensure(c, c->sv_ord, H)); RC(ensure(c, c->sv_hrow, H)); RC(ensure(c, c->sv_hpc, H));
   RC(ensure(c, c->sv_hA, 3 * H)); RC(ensure(c, c->sv_hB, 3 * H)); RC(ensure(c, c->sv_heps, H)); RC(ensure(c, c->sv_hkey, H));
   const size_t P = (size_t)std::max(np, 1), K = (size_t)std::max(nk, 1);
-  RC(ensure(c, c->sv_hhot, (size_t)CH * H)); RC(ensure(c, c->sv_hcold, (size_t)CC * H)); RC(ensure(c, c->sv_out, 11 * H));
+  RC(ensure(c, c->sv_hs, (size_t)SH * H)); RC(ensure(c, c->sv_out, 11 * H));
   RC(ensure(c, c->sv_ps, (size_t)SP * 2 * P)); RC(ensure(c, c->sv_cpart, K)); RC(ensure(c, c->sv_cps, P));
   RC(ensure(c, c->sv_ploc, 2 * P)); RC(ensure(c, c->sv_phit, P)); RC(ensure(c, c->sv_hint, 6 * H));
   RC(ensure(c, c->sv_lvlo, H + K)); RC(ensure(c, c->sv_cntl, H)); RC(ensure(c, c->sv_pint, 6 * P + K));
@@ -5748,26 +5843,33 @@ int d2_solve(d2_ctx* c, const double* gravity, int32_t* cluster_status, int* n_f
   A.inpair = c->sv_inpair.p, A.loc = c->sv_loc.p, A.status = c->sv_status.p;
   A.hl = c->sv_hl.p, A.ord = c->sv_ord.p, A.hrow = c->sv_hrow.p, A.hpc = c->sv_hpc.p, A.pbody = c->sv_pbody.p;
   A.hA = c->sv_hA.p, A.hB = c->sv_hB.p, A.heps = c->sv_heps.p, A.hkey = c->sv_hkey.p;
-  A.hhot = c->sv_hhot.p, A.hcold = c->sv_hcold.p, A.cpart = c->sv_cpart.p, A.cps = c->sv_cps.p;
+  A.hs = c->sv_hs.p, A.cpart = c->sv_cpart.p, A.cps = c->sv_cps.p;
   A.ploc = c->sv_ploc.p, A.phit = c->sv_phit.p, A.hint = c->sv_hint.p, A.lvlo = c->sv_lvlo.p;
   A.cntl = c->sv_cntl.p, A.pint = c->sv_pint.p;
   A.ps = c->sv_ps.p, A.out = c->sv_out.p, A.warm = warm_table(c), A.flag = c->sv_flag.p;
+  A.hist = c->sv_flag.p + 1, A.small = -1;
   auto fill = [&](int* p, long long n, int v) {
     hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(c, n)), dim3(256), 0, c->stream, p, n, v);
   };
   fill(A.ccount, nk + 1, 0), fill(A.chits, nk + 1, 0), fill(A.cfill, nk, 0);
-  fill(A.inpair, nb, 0), fill(A.cpart, nk, 0), fill(c->sv_flag.p, 1, 0);
+  fill(A.inpair, nb, 0), fill(A.cpart, nk, 0), fill(c->sv_flag.p, 1 + SV_BINS, 0);
   hipLaunchKernelGGL(k_sv_count, dim3(grid_for(c, np)), dim3(256), 0, c->stream, A);
   scan_host_n(c, c->sv_ccount.p, c->sv_poff.p, nk, nullptr);
   scan_host_n(c, c->sv_chits.p, c->sv_hoff.p, nk, nullptr);
   scan_host_n(c, c->kept_cnt.p, c->out_off.p, np, nullptr);
   SolveArgs B = A;
   B.ccount = c->sv_poff.p, B.chits = c->sv_hoff.p;  // the offsets from here on
-  hipLaunchKernelGGL(k_sv_place, dim3(grid_for(c, std::max(np, nb))), dim3(256), 0, c->stream, B);
-  int bad = 0;
-  RC(read_out(c, {{&bad, c->sv_flag.p, sizeof(int)}}));
-  if (bad) return fail(c, D2_ERR_ARG, "d2_solve: a dynamic body's pairs lie in more than one cluster");
-  hipLaunchKernelGGL(k_sv_solve, dim3(std::max(1, std::min(nk, 16 * c->cus))), dim3(256), 0, c->stream, B);
+  hipLaunchKernelGGL(k_sv_place, dim3(grid_for(c, std::max(std::max(np, nb), nk))), dim3(256), 0, c->stream, B);
+  int head[1 + SV_BINS] = {};  // the flag, the clusters by size class
+  RC(read_out(c, {{head, c->sv_flag.p, sizeof(head)}}));
+  if (head[0]) return fail(c, D2_ERR_ARG, "d2_solve: a dynamic body's pairs lie in more than one cluster");
+  B.small = sv_small_size(c, head + 1);
+  int n_small = 0;
+  for (int b = 0; b < SV_BINS - 1 && 2 << b <= B.small; ++b) n_small += head[1 + b];
+  if (n_small > 0)
+    hipLaunchKernelGGL(k_sv_solve_small, dim3(grid_for(c, nk, 64)), dim3(64), 0, c->stream, B);
+  if (n_small < nk)
+    hipLaunchKernelGGL(k_sv_solve, dim3(std::max(1, std::min(nk, 16 * c->cus))), dim3(256), 0, c->stream, B);
   hipLaunchKernelGGL(k_sv_free, dim3(grid_for(c, nb)), dim3(256), 0, c->stream, B);
   HIPCHK(c, hipGetLastError());
   std::vector<int32_t> st(std::max(nk, 1));

@@ -15,8 +15,9 @@
 //
 // The arithmetic is in per-contact and per-particle functions (sv_*).  Two
 // walks call them: solve_cluster below, one thread contact by contact (the
-// host's check against the oracle), and the device's k_sv_solve, a block per
-// cluster, which runs contacts that share no dynamic particle side by side.
+// device's k_sv_solve_small, a lane per cluster, and the host's check against
+// the oracle), and the device's k_sv_solve, a block per cluster, which runs
+// contacts that share no dynamic particle side by side.
 //
 // What does not change during a solve is formed once.  The torques of offset
 // impulses stay zero, so a particle's predicted rotation is the same in every
@@ -160,7 +161,7 @@ struct ClusterSolve {
   double t;
   v3<double> g;
   WarmTable warm;
-  double* hs;  // scratch per hit (sorted position): [nh][SH]
+  double* hs;  // scratch per hit (sorted position): [nh][CH], then [nh][CC]
   double* ps;  // scratch per particle: [np][SP]
   double* out_h;  // [nh][11]
 };
@@ -364,8 +365,8 @@ D2_HD void sv_store_out(const double* c, const double* k, double* o) {
 D2_HD bool solve_cluster(const ClusterSolve& S) {
   const int nh = S.nh, np = S.np;
   const double t = S.t;
-  auto hot = [&](int c) { return S.hs + (size_t)SH * c; };
-  auto cold = [&](int c) { return S.hs + (size_t)SH * c + CH; };
+  auto hot = [&](int c) { return S.hs + (size_t)CH * c; };
+  auto cold = [&](int c) { return S.hs + (size_t)CH * nh + (size_t)CC * c; };
   auto part = [&](int c, int side) { return S.ps + (size_t)SP * S.hl[2 * S.ord[c] + side]; };
   auto is_static = [&](int k) { return S.bodies[40 * (size_t)S.pbody[k] + 38] != 0.0; };
   for (int c = 0; c < nh; ++c)

@@ -3994,9 +3994,12 @@ namespace {
 const char* kKernelNames[] = {"setup", "soup_cull", "soup_point", "soup_edge", "soup_reduce", "expand",
                               "leaf_point", "leaf_edge", "tri_mask", "tri_enum", "tri_dist", "post", "post_pairs",
                               "cluster", "gate", "tri_full", "soup_keep", "tri_def"};
-// K_TRI_ENUM launches nothing (the enumeration is part of k_tri_mask); its
-// item count is the discrete node pairs received, kept for instrumentation.
-// FP64 contexts run K_TRI_FULL (k_tri_full) in place of K_TRI_MASK + K_TRI_DIST.
+// Some launch nothing and only count: K_TRI_ENUM the discrete node pairs
+// received (part of k_tri_mask), K_SOUP_POINT, K_LEAF_POINT and K_LEAF_EDGE
+// their sub-tests (part of k_ccd_sub, which K_SOUP_EDGE times over all four
+// kinds).  K_SOUP_CULL is k_ccd_cull, over both lists.  FP64 contexts run
+// K_TRI_FULL (k_tri_full) and K_EXPAND (k_disc_expand) in place of K_TRI_MASK +
+// K_TRI_DIST; the other forms expand in the kernels that find the hits.
 enum KId { K_SETUP, K_SOUP_CULL, K_SOUP_POINT, K_SOUP_EDGE, K_SOUP_REDUCE, K_EXPAND, K_LEAF_POINT, K_LEAF_EDGE,
            K_TRI_MASK, K_TRI_ENUM, K_TRI_DIST, K_POST, K_POST_PAIRS, K_CLUSTER, K_GATE, K_TRI_FULL, K_SOUP_KEEP, K_TRI_DEF,
            K_NUM };
@@ -4756,22 +4759,24 @@ void add_level_items(d2_ctx* c, int level, int discrete) {
   const unsigned long long* s = c->host_lvl + level * LV_STRIDE;
   if (discrete && c->precision != D2_FP32) {
     c->k_items[K_TRI_FULL] += (double)s[LV_ITEMS];
+    c->k_items[K_EXPAND] += (double)s[LV_SOUP];
   } else if (discrete) {
     c->k_items[K_TRI_MASK] += (double)s[LV_SOUP];
     c->k_items[K_TRI_ENUM] += (double)s[LV_SOUP];
     c->k_items[K_TRI_DIST] += (double)s[LV_ITEMS];
     c->k_items[K_TRI_DEF] += (double)s[LV_DEF];
   } else {
-    c->k_items[K_SOUP_CULL] += (double)s[LV_SOUP];
     const bool fp32 = c->precision == D2_FP32;  // FP32 form: the sub-tests its culls keep
+    const double point = fp32 ? (double)s[LV_SPT] : 6.0 * (double)s[LV_ITEMS];
+    const double edge = fp32 ? (double)s[LV_SEE] : 9.0 * (double)s[LV_ITEMS];
+    c->k_items[K_SOUP_CULL] += (double)s[LV_SOUP] + (double)s[LV_CONN];
     if (fp32) c->k_items[K_SOUP_KEEP] += (double)s[LV_ITEMS];
-    c->k_items[K_SOUP_POINT] += fp32 ? (double)s[LV_SPT] : 6.0 * (double)s[LV_ITEMS];
-    c->k_items[K_SOUP_EDGE] += fp32 ? (double)s[LV_SPT] + (double)s[LV_SEE] : 15.0 * (double)s[LV_ITEMS];
+    c->k_items[K_SOUP_POINT] += point;
+    c->k_items[K_SOUP_EDGE] += (point + edge) + ((double)s[LV_PT] + (double)s[LV_EE]);
     c->k_items[K_SOUP_REDUCE] += (double)s[LV_ITEMS];
     c->k_items[K_LEAF_POINT] += (double)s[LV_PT];
     c->k_items[K_LEAF_EDGE] += (double)s[LV_EE];
   }
-  c->k_items[K_EXPAND] += (double)s[LV_SOUP];
 }
 
 struct CopyOut {  // bytes (a multiple of 4) of device memory for the host; none when dst is null

@@ -385,8 +385,11 @@ int d2_ccd(d2_ctx* ctx, int n_pairs, const int32_t* pairs, const double* max_tim
 
 /* ---- instrumentation ---------------------------------------------------- */
 /* When on, every kernel launch is bracketed by HIP events on the context's
- * stream; d2_kernel_stats returns per-kernel launch counts and summed
- * milliseconds (index order: d2_kernel_name(i)). */
+ * stream; d2_kernel_stats returns per-kernel launch counts, summed
+ * milliseconds and the items these launches took (index order:
+ * d2_kernel_name(i)).  A kernel without launches only counts: "tri_enum" the
+ * discrete node pairs, "soup_point", "leaf_point" and "leaf_edge" sub-tests
+ * that the launches named "soup_edge" run with all the others of a level. */
 int d2_set_profiling(d2_ctx* ctx, int on);
 int d2_num_kernels(void);
 const char* d2_kernel_name(int i);
@@ -399,8 +402,10 @@ int d2_reset_stats(d2_ctx* ctx);
  * per level 0..16 eight sizes (soup node pairs, connected node pairs, items,
  * point and edge sub-tests, 3 reserved) of the discrete phase (of the CCD
  * phase for d2_ccd_run), then the same table of the last CCD phase (its
- * contact count in the last field of level 0).  Copies min(n, total) values;
- * returns the total. */
+ * contact count in the last field of level 0).  A discrete level's items are
+ * the triangle pairs its bounds left to the FP64 test (every one in the FP64
+ * form without pruning), those that FP32 levels defer not counted.  Copies
+ * min(n, total) values; returns the total. */
 int d2_run_info(const d2_ctx* ctx, int64_t* info, int n);
 /* Subtree pruning of the discrete traversal (no reference counterpart; on by
  * default): a node pair whose leaf triangles are provably farther apart than

@@ -44,11 +44,11 @@
 #include <random>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <initializer_list>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -5155,7 +5155,7 @@ hipError_t copy_out(d2_ctx* c, std::initializer_list<CopyOut> parts, int max_thr
   for (int t = 1; t < threads; ++t) {
     try {
       pool[t] = std::thread(work);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {  // (nothing may unwind past the joinable threads)
       break;  // the threads there are do the work
     }
   }

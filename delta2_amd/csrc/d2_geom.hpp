@@ -185,9 +185,10 @@ D2_HD bool nodes_apart(const double* Ta, const double* Tb, const float* ba, cons
   }
   return gap > thr;
 }
-// nodes_apart over the six face axes only (each box's three face normals):
-// what the FP32 form's mask kernel asks of every node pair on arrival, in FP32
-// (boxes_apart_faces_rel below).  The face axes find nearly all of the separations
+// nodes_apart over the six face axes only (each box's three face normals): in
+// FP64 what the FP32 form's mask kernel asks of every node pair on arrival
+// (boxes_apart_faces_rel below, which the checks hold against this; no kernel
+// calls it).  The face axes find nearly all of the separations
 // the edge axes add to the spheres' (on a 4096-body funnel pile 98% for
 // funnel pairs, 92% for body pairs).  b's offset along its own face normal
 // j (Rb's column j) is taken as that column times the centre difference.
@@ -243,8 +244,9 @@ D2_HD bool spheres_apart(const double* Ta, const double* Tb, const float* ba, co
   }
   return sqrt(s2) - ((double)ba[7] + (double)bb[7]) > thr;
 }
-// spheres_apart in FP32.  Each world
-// coordinate w = R c + t is off by at most 8 u (|R c|_1 + |t|) after the
+// spheres_apart in FP32 from the poses themselves (no kernel calls it: they
+// hold float records, spheres_apart_rel below; the geometry check does).  Each
+// world coordinate w = R c + t is off by at most 8 u (|R c|_1 + |t|) after the
 // rounding of the pose, the product and the sums (u = 2^-24), so the centre
 // distance by at most 16 u m + 5 u |d| with m the sum of |w| over both
 // centres; the test demands 32 u (m + |d|) beyond the FP64 threshold.
@@ -265,6 +267,7 @@ D2_HD bool spheres_apart_f32(const double* Ta, const double* Tb, const float* ba
 // A pair's poses for the discrete phase's FP32 tests, PF_FLOATS floats: a's
 // rotation (rows), a's translation relative to b's, b's rotation, the search
 // distance (a float to begin with), in the frame with b's position as origin.
+// (k_setup writes them lane by lane; the checks use pair_pose_f32.)
 constexpr int PF_RA = 0, PF_TR = 9, PF_RB = 12, PF_SEARCH = 21, PF_FLOATS = 24;
 D2_HD void pair_pose_f32(const double* Ta, const double* Tb, float search, float* f) {
   for (int r = 0; r < 3; ++r) {

@@ -315,7 +315,7 @@ struct Dev {
   // pairs
   const int32_t* pair_info;  // a, b, node offset a, node offset b
   const double* pair_rec;
-  float* pair_f;               // FP32 form, per pair: pair_pose_f32 (discrete), the CF_ record (CCD)
+  float* pair_f;               // FP32 form, per pair: the PF_ record (discrete, pair_pose_f32's), the CF_ record (CCD)
   // work lists
   NP* soup;
   NP* conn;
@@ -349,7 +349,7 @@ struct Dev {
   const uint8_t* kid_inner;    // per node: bit c set when child c is an inner node
   int prune;                   // skip node pairs nodes_apart proves contact-free
   int defer;                   // FP32 form: inner node pairs send one item to k_tri_dist, the rest to k_tri_def
-  int box_test;                // FP32 form: k_tri_mask tests arriving node pairs with boxes_apart_faces
+  int box_test;                // FP32 form: k_tri_mask tests arriving node pairs with boxes_apart_faces_rel
   int conn_blocks;             // CCD: the last blocks of k_ccd_cull, which take the connected list
   const int32_t* body_tree;
   int fp32;                    // FP32 culls of the CCD leaf sub-tests
@@ -2955,7 +2955,7 @@ __global__ void __launch_bounds__(NT) k_pair_finish_block(int n_pairs, const int
   for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
     const int p = list ? list[it] : it;
     const int b = pair_off[p], e = pair_off[p + 1], n = e - b;
-    if (n > CAP) {  // to the second launch: its LDS pass, or (above its capacity) one lane per pair
+    if (n > CAP) {  // to the second launch: its LDS pass, or (above its capacity) a block per pair
       if (tid == 0) {
         if (n > POST_CAP_LARGE) huge[atomicAdd(n_huge, 1)] = p;
         else over[atomicAdd(n_over, 1)] = p;
@@ -4586,9 +4586,9 @@ int post_grid(const d2_ctx* c, int mode) {
 
 // The per-pair finishing launches over contacts, pair_off and perm: pairs up to
 // 512 contacts in the first (wblocks blocks), those up to 2048 in the second
-// launch's LDS pass, larger ones by the second launch's per-pair forms (with
-// the filter, one lane per pair; n_big[0..1] count the two lists, zeroed
-// before).  mode 1 applies filterContacts(.., margin).
+// launch's LDS pass, larger ones by the second launch's per-pair forms, a
+// 1024-thread block per pair (n_big[0..1] count the two lists, zeroed before).
+// mode 1 applies filterContacts(.., margin).
 HugeScratch huge_scratch(d2_ctx* c) {
   const size_t m = c->hscratch.n / 6;
   int* h = c->hscratch.p;
@@ -4633,9 +4633,8 @@ int enqueue_post(d2_ctx* c, int mode) {
     Timer tm(c, K_POST_PAIRS, (double)np);
     const int wblocks = std::max(1, std::min(np, c->tune.post_blocks));
     // pairs above the first launch's capacity (512 contacts): the second
-    // launch's 2048-contact LDS pass (list big); above that, one block per
-    // pair, or one lane per pair with the filter (list huge, filled by the
-    // first launch only)
+    // launch's 2048-contact LDS pass (list big); above that, its per-pair
+    // forms on global scratch (list huge, filled by the first launch only)
     // the filter's kept total accumulates into C_OUT (zeroed by k_setup); the
     // output offsets are scanned when the contacts are read (d2_result_contacts)
     unsigned long long* kept_total = filtered ? c->cnt.p + C_OUT : nullptr;

@@ -541,15 +541,16 @@ __global__ void __launch_bounds__(256) k_bp_gather(int n_items, const int* item_
 }
 
 // ---------------------------------------------------------------- clusters
-// The root of x; x is then pointed at it.  The loads may come from the caches
-// (wavefront scope): a node's parent only ever changes to an ancestor with a
-// smaller index, so a stale parent is still an ancestor, and whether a root
-// found this way is one still is decided by the CAS that hooks it.  Loads at
-// device scope, all ending on the largest component's root, queued on one
-// line: 260 us of unions for 120 k pairs of 65 536 bodies against 105 us.  The
-// shortened path is stored at device scope, as the CAS is: words that other
-// wavefronts, behind other L2 caches, read and hook.  (Halving the whole path
-// stores more: 116 to 121 us.)
+// The root of x; x is then pointed at it if it is more than two nodes below.
+// The loads may come from the caches (wavefront scope): a node's parent only
+// ever changes to an ancestor with a smaller index, so a stale parent is still
+// an ancestor, and whether a root found this way is one still is decided by
+// the CAS that hooks it.  Loads at device scope, all ending on the largest
+// component's root, queued on one line: 260 us of unions for 120 k pairs of
+// 65 536 bodies against 88 us.  The shortened path is stored at device scope,
+// as the CAS is: words that other wavefronts, behind other L2 caches, read and
+// hook.  (With the store on every path of two nodes and more 108 us, halving
+// the whole path 116 to 121 us.)
 __device__ __forceinline__ int cc_load(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
@@ -558,9 +559,9 @@ __device__ __forceinline__ void cc_store(int* p, int v) {
 }
 __device__ __forceinline__ int cc_find(int* parent, int x) {
   const int p = cc_load(&parent[x]);
-  int r = p;
-  for (int g; (g = cc_load(&parent[r])) != r;) r = g;
-  if (r != p) cc_store(&parent[x], r);
+  int r = p, hops = 0;
+  for (int g; (g = cc_load(&parent[r])) != r; ++hops) r = g;
+  if (hops > 1) cc_store(&parent[x], r);
   return r;
 }
 // The same for the pass after the unions: paths are short by then (4.9 us; 14
